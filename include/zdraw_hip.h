@@ -437,7 +437,8 @@ void zdraw_hip_attention_tail_plan(uint64_t tiles, uint32_t cus, uint32_t key_bl
  * activations: the tiles are 256 x 256; a last round that fills at most half the CUs runs as
  * *splits ranges of k per tile (at most 8, at least four 64-wide slabs each) whose fp32
  * partial tiles are added in range order; nothing is split when k is not a multiple of 64,
- * when fewer than 160 tiles exist, or under the eight-wave build. */
+ * when fewer than 160 tiles exist, or under the eight-wave build. (A product that other tiles
+ * fit better does not run on 256-tiles and splits nothing.) */
 void zdraw_hip_gemm_tail_plan(uint32_t m, uint32_t k, uint32_t n, uint32_t groups, uint32_t cus, uint32_t* tail_tiles,
                               uint32_t* splits);
 

@@ -36,6 +36,10 @@ void zdraw_hip_set_attention_variant(int variant);
  * each (default); 0 = eight waves, 64 x 128 each. */
 void zdraw_hip_set_gemm_build(int build);
 
+/* The tile of C (rows x columns) that `groups` (1..3) side-by-side products C[m][n] =
+ * A[m][k] x W[n][k]^T run on, on a device with `cus` compute units. Host arithmetic only. */
+void zdraw_hip_gemm_tile(uint32_t m, uint32_t k, uint32_t n, uint32_t groups, uint32_t cus, uint32_t* rows, uint32_t* cols);
+
 /* How many query tiles (128 rows) of the last wide-head launch had a score outgrow its row's
  * fixed reference point and were formed again by the running-maximum kernel (waits for that
  * launch). 0 on ordinary data; -1 if no wide-head launch has been made or the read failed. */

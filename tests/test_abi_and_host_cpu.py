@@ -90,6 +90,24 @@ def test_gemm_tail_plan_of_the_projection_shapes():
         assert (t == 0 and s == 1) or (tiles >= 160 and t == tiles % 256 and 2 <= s <= 8 and t * s <= 256 and 32 // s >= 4)
 
 
+def test_gemm_tile_of_the_projection_shapes():
+    # 256 CUs: few rows take small tiles so that every CU has one, many rows the 256-tiles
+    L = hip.lib()
+
+    def tile(m, k, n, groups=1, cus=256):
+        r, c = C.c_uint32(99), C.c_uint32(99)
+        L.zdraw_hip_gemm_tile(m, k, n, groups, cus, C.byref(r), C.byref(c))
+        return r.value, c.value
+
+    assert tile(4608, 3072, 3072, 3) == tile(4608, 12288, 3072) == tile(4608, 3840, 3840, 3) == (256, 256)
+    assert tile(512, 3072, 3072, 3) == (128, 160)   # 232 tiles
+    assert tile(512, 3072, 3072) == (64, 96)        # 256 tiles
+    assert tile(1024, 3072, 3072, 3) == (256, 160)  # 240 tiles
+    assert tile(77, 3072, 3072) == (64, 64)
+    assert tile(4608, 3076, 3072) != (256, 256)     # k not a multiple of 64: never the 256-tiles
+    assert tile(0, 64, 64) == (0, 0) and tile(64, 64, 64, 4) == (0, 0)
+
+
 def test_tail_plan_of_the_baseline_shapes():
     # 256 CUs, one 256-row tile per workgroup: which last rounds are split along the keys
     L = hip.lib()

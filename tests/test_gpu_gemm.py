@@ -530,3 +530,57 @@ def test_k_split_last_round_of_a_group(ctx):
     assert L.zdraw_hip_dispatch_count() == d0
     for b in [ab, wb] + cbs:
         b.release()
+
+
+# one problem per tile of the pipelined kernel: more than one tile each way, a ragged last row and
+# column of tiles, and a k of three slabs (fewer than the LDS holds) or of 3.125 (the last slab
+# keeps one of its eight chunks)
+TILE_CASES = [((64, 64), 72, 73, 1), ((64, 96), 199, 1349, 3), ((128, 64), 1797, 202, 3), ((128, 96), 259, 1794, 3),
+              ((128, 128), 522, 1636, 3), ((128, 160), 899, 1304, 3), ((128, 192), 902, 1601, 3),
+              ((192, 192), 1299, 1357, 3), ((256, 160), 1546, 1738, 3)]
+
+
+@pytest.mark.parametrize("tile,m,n,count", TILE_CASES, ids=[f"{t[0]}x{t[1]}" for t, *_ in TILE_CASES])
+@pytest.mark.parametrize("k", [192, 200, 520])
+@pytest.mark.parametrize("c_dtype", [hip.F32, hip.BF16])
+def test_every_tile_of_the_pipelined_kernel(ctx, tile, m, n, count, k, c_dtype):
+    # Every product of the group on sampled rows (first, last, the edges of tiles and of their waves)
+    # against the oracle on the same rounded operands: only the order of 32-bit sums differs, so the
+    # bar is that of `check` above; 16-bit results may differ by one place. What lies past k in a
+    # row (here NaN, in a wider A and W) must not count; the columns past n stay untouched.
+    L = hip.lib()
+    r, c = C.c_uint32(), C.c_uint32()
+    L.zdraw_hip_gemm_tile(m, k, n, count, 256, C.byref(r), C.byref(c))
+    if k < 512:
+        assert (r.value, c.value) == tile
+    rng = np.random.default_rng(m + n + k)
+    lda = ldw = k + 8
+    ldc = n + (3 if c_dtype == hip.F32 else 5)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    w = rng.standard_normal((count, n, k), dtype=np.float32) * np.float32(k ** -0.5)
+    a_bits, ar = to16(a, hip.W_BF16)
+    w_bits, wr = to16(w, hip.W_BF16)
+    pad = lambda x, width: np.concatenate([x, np.full(x.shape[:-1] + (width - k,), 0x7FC0, np.uint16)], axis=-1)
+    ab, wb = ctx.buffer(pad(a_bits, lda)), ctx.buffer(pad(w_bits, ldw))
+    esz = 4 if c_dtype == hip.F32 else 2
+    cbs = [ctx.buffer(np.full(m * ldc * esz, 0x5A, np.uint8)) for _ in range(count)]
+    ps = [hip.GemmParams(m, k, n, hip.W_BF16, hip.GEMM_HALF, i * n * ldw * 2) for i in range(count)]
+    ext = hip.GemmExt(0, 0, lda, ldw, ldc, hip.BF16, c_dtype)
+    batch = L.zdraw_hip_batch_begin(ctx.queue)
+    rc = L.zdraw_hip_run_gemm_group_ext_enc(batch, ab.handle, (C.c_void_p * count)(*([wb.handle] * count)),
+                                            (C.c_void_p * count)(*(b.handle for b in cbs)),
+                                            (C.POINTER(hip.GemmParams) * count)(*(C.pointer(p) for p in ps)), count, C.byref(ext))
+    assert L.zdraw_hip_batch_end(batch) == 0
+    assert rc == 0, hip.last_error()
+    rows = sorted({0, 15, 16, tile[0] // 2 - 1, tile[0] // 2, tile[0] - 1, tile[0], m // 2, m - 2, m - 1} & set(range(m)))
+    for i in range(count):
+        raw = cbs[i].read(np.uint8, (m, ldc * esz))
+        assert (raw[:, n * esz:] == 0x5A).all(), "columns past n were written"
+        got = raw[:, :n * esz].copy().view(np.float32) if c_dtype == hip.F32 else host.bf16_bits_to_f32(raw[:, :n * esz].copy().view(np.uint16))
+        assert np.isfinite(got).all()
+        want = zo.linear_batch(np.ascontiguousarray(ar[rows]), wr[i])
+        s = np.sqrt(k) * np.sqrt(np.mean(ar.astype(np.float64) ** 2)) * np.sqrt(np.mean(wr[i].astype(np.float64) ** 2))
+        place = 0.0 if c_dtype == hip.F32 else 2.0 ** -8 * np.abs(want)  # half a unit in the last place of bf16
+        assert (np.abs(got[rows] - want) <= 2e-5 * s + 1e-6 + place).all(), f"product {i}: max {np.abs(got[rows] - want).max():.3e}"
+    for b in [ab, wb] + cbs:
+        b.release()

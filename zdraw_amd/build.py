@@ -71,11 +71,11 @@ def _device_asm(src: str, extra_flags=()) -> list[str]:
     return _ASM_CACHE[key]
 
 
-def m0_writes(src: str = os.path.join(CSRC, "gemm_half.hip"), kernel_substr: str = "gemm_ring_kernel", extra_flags=()) -> list[str]:
-    """Compiles `src` to gfx950 assembly and lists, for the kernels whose symbol contains
-    `kernel_substr`, every instruction that writes M0 other than the source's own
-    `s_mov_b32 m0, <sgpr>` + `s_nop 0` pair (attn_device.hpp, lds_dma_base). The four-wave GEMM
-    keeps M0 live across several loads without the compiler knowing; a write of the compiler's
+def m0_writes(src: str = os.path.join(CSRC, "gemm_half.hip"), kernels: str = "gemm_(ring|pipe)_kernel", extra_flags=()) -> list[str]:
+    """Compiles `src` to gfx950 assembly and lists, for the kernels whose symbol matches
+    `kernels`, every instruction that writes M0 other than the source's own
+    `s_mov_b32 m0, <sgpr>` + `s_nop 0` pair (attn_device.hpp, lds_dma_base). The four-wave GEMMs
+    keep M0 live across several loads without the compiler knowing; a write of the compiler's
     own in between would send those loads elsewhere in LDS."""
     import re
     lines = [l.split(";")[0].strip() for l in _device_asm(src, extra_flags)]
@@ -87,7 +87,7 @@ def m0_writes(src: str = os.path.join(CSRC, "gemm_half.hip"), kernel_substr: str
         if text.endswith(":") and not text.startswith("."):
             kernel = text[:-1]
             continue
-        if kernel_substr not in kernel or not writes.match(text):
+        if not re.search(kernels, kernel) or not writes.match(text):
             continue
         own = re.match(r"^s_mov_b32\s+m0\s*,\s*s\d+$", text) and i + 1 < len(lines) and lines[i + 1] == "s_nop 0"
         if not own:

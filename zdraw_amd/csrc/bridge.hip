@@ -971,7 +971,6 @@ int enqueue_gemm_group(void* a, void* const* ws, void* const* cs, const uint64_t
     g.tiles_n = (int32_t)((p->n + (uint32_t)gemm_tile_cols() - 1) / (uint32_t)gemm_tile_cols());
     if ((uint64_t)g.tiles_n * (uint64_t)groups * ((p->m + (uint32_t)gemm_tile_rows() - 1) / (uint32_t)gemm_tile_rows()) > 0x7fffffffull)
         return unavailable("grid too large");
-    int a_eff = (int)x->a_dtype;
     if (const size_t rb = gemm_round_bytes(g, (int)x->a_dtype)) {
         // f32 activations are rounded to the weight's type once, into scratch slot 6, and the
         // product then runs as for 16-bit activations
@@ -981,13 +980,13 @@ int enqueue_gemm_group(void* a, void* const* ws, void* const* cs, const uint64_t
             return ZDRAW_HIP_ERR_HANDLE;
         }
         g.a16 = a16->ptr;
-        a_eff = (int)wt;
     }
-    {
-        // a last round of tiles that fills at most half the CUs runs split along k; its fp32
+    g.shape = gemm_shape(g, queue->dev->cus);
+    if (g.shape < 0) {
+        // a last round of 256-tiles that fills at most half the CUs runs split along k; its fp32
         // partial tiles go through scratch slot 5
         int tail = 0, splits = 1;
-        gemm_tail_plan(g, a_eff, queue->dev->cus, &tail, &splits);
+        gemm_tail_plan(g, queue->dev->cus, &tail, &splits);
         if (splits > 1) {
             Buffer* part = queue_scratch(queue, 5, gemm_part_bytes(tail, splits));
             if (!part) {
@@ -1824,9 +1823,21 @@ void zdraw_hip_gemm_tail_plan(uint32_t m, uint32_t k, uint32_t n, uint32_t group
     g.groups = (int32_t)groups;
     int t = 0, s = 1;
     if (m && k && n && groups >= 1 && groups <= 3 && m <= 0x7fffffffu && k <= 0x7fffffffu && n <= 0x7fffffffu)
-        gemm_tail_plan(g, (int)ZDRAW_HIP_BF16, (int)cus, &t, &s);
+        gemm_tail_plan(g, (int)cus, &t, &s);
     if (tail_tiles) *tail_tiles = (uint32_t)t;
     if (splits) *splits = (uint32_t)s;
+}
+
+void zdraw_hip_gemm_tile(uint32_t m, uint32_t k, uint32_t n, uint32_t groups, uint32_t cus, uint32_t* rows, uint32_t* cols) {
+    GemmArgs g;
+    memset(&g, 0, sizeof(g));
+    g.m = (int32_t)m; g.k = (int32_t)k; g.n = (int32_t)n;
+    g.groups = (int32_t)groups;
+    int r = 0, c = 0;
+    if (m && k && n && groups >= 1 && groups <= 3 && m <= 0x7fffffffu && k <= 0x7fffffffu && n <= 0x7fffffffu)
+        gemm_shape_tile(gemm_shape(g, (int)cus), &r, &c);
+    if (rows) *rows = (uint32_t)r;
+    if (cols) *cols = (uint32_t)c;
 }
 
 void zdraw_hip_attention_tail_plan(uint64_t tiles, uint32_t cus, uint32_t key_blocks, uint32_t* tail_tiles,

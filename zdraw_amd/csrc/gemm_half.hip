@@ -7,20 +7,15 @@
 // input and drain the attention output (klein/zflux2_resident.zig:1473-1513,
 // 1986-1998). Both operands are K-major (activation rows and weight rows are
 // contiguous in k), which is exactly the register layout of the 16-bit MFMAs
-// (v_mfma_f32_16x16x32 in the direct-to-LDS builds, v_mfma_f32_32x32x16 in the
-// register-staged one): a lane supplies 8 consecutive k of one row.
+// (v_mfma_f32_16x16x32): a lane supplies 8 consecutive k of one row.
 //
-// Three builds share the tile walk, the operand layout and the epilogue:
-//   * f32 activations, or k not a multiple of 64: workgroup tile 256 x 256, K slabs of
-//     64, 8 waves as 4 (M) x 2 (N), a wave owns 64 x 128 of C; global loads (buffer
-//     loads, scalar slab offset) run two slabs ahead in registers and are rounded to the
-//     weight's 16-bit type on the way into padded LDS rows (144 bytes: 16-lane b128
-//     fragment reads hit 16 distinct bank groups), so no conversion pass is needed;
-//   * 16-bit activations, whole slabs, enough 256-tiles to fill the chip (the default for
-//     the projections): 4 waves, one per SIMD, each owning 128 x 128 of C, slabs fetched
-//     from global memory straight into swizzled, unpadded LDS rows (gemm_ring_kernel);
-//     the same tile with 8 waves is kept behind a knob;
-//   * the same with too few 256-tiles: 128 x 128 tiles, 4 waves, two workgroups per CU;
+// Two kernels share the tile walk, the operand layout and the schedule (four waves, one per SIMD,
+// slabs of 64 k fetched from global memory straight into swizzled, unpadded LDS rows):
+//   * gemm_ring_kernel: 256 x 256 tiles, each wave 128 x 128 of C; an eight-wave build of that tile
+//     is kept behind a knob;
+//   * gemm_pipe_kernel: nine tiles from 64 x 64 to 256 x 160 with three or four slabs in LDS, for
+//     problems that do not fill the chip with 256-tiles, and for any k that is not a multiple of 64;
+//   * f32 activations are rounded to the weight's type by a launch of their own;
 //   * two or three products of one A with equal shapes (q/k/v, gate/up) run as one launch
 //     whose tiles cover all of them;
 //   * fixed summation order and no atomics (a thinly filled last round is cut along k and
@@ -28,58 +23,16 @@
 #include "attn_device.hpp"
 #include "gemm_kernel.h"
 
+#include <cmath>
+
 namespace zdraw {
 
 namespace gemm {
 
 constexpr int BM = 256, BN = 256, BK = 64;
-constexpr int NT = 512;
-constexpr int PITCH = BK + 8;                  // elements per LDS row
-constexpr int STAGE_ELEMS = (BM + BN) * PITCH; // A rows then W rows
-constexpr size_t kLdsBytes = 2 * (size_t)STAGE_ELEMS * 2;
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-
-// 8 consecutive k of one row as they come from memory.
-template <typename T> struct Chunk { u32x4 r; };
-template <> struct Chunk<float> { f32x4 a, b; };
-
-template <typename T>
-__device__ __forceinline__ Chunk<T> ld_chunk(rsrc_t rsrc, unsigned voff, unsigned soff) {
-    Chunk<T> x;
-    if constexpr (std::is_same<T, float>::value) {
-        x.a = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)voff, (int)soff, 0));
-        x.b = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(voff + 16), (int)soff, 0));
-    } else {
-        x.r = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)voff, (int)soff, 0));
-    }
-    return x;
-}
-
-// The chunk as 8 packed 16-bit values of the compute type.
-template <typename T, bool F16>
-__device__ __forceinline__ u32x4 to_half8(const Chunk<T>& x, bool keep) {
-    u32x4 r;
-    if constexpr (std::is_same<T, float>::value) {
-        f32x8 v;
-#pragma unroll
-        for (int i = 0; i < 4; i++) { v[i] = x.a[i]; v[4 + i] = x.b[i]; }
-        if constexpr (F16) r = __builtin_bit_cast(u32x4, __builtin_convertvector(v, f16x8));
-        else r = __builtin_bit_cast(u32x4, __builtin_convertvector(v, bf16x8));
-    } else {
-        r = x.r;
-    }
-    return keep ? r : u32x4{0u, 0u, 0u, 0u};
-}
-
-template <bool F16>
-__device__ __forceinline__ f32x16 mfma(const u32x4& a, const u32x4& b, const f32x16& c) {
-    if constexpr (F16)
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
 
 // v_mfma_f32_16x16x32: a lane supplies 8 consecutive k (chunk lane / 16 of the 32) of row lane % 16
 // and receives, of the 16 x 16 result, row lane % 16 of the second operand against rows
@@ -88,7 +41,7 @@ __device__ __forceinline__ f32x16 mfma(const u32x4& a, const u32x4& b, const f32
 // Written as assembly with the accumulator tied to the result: given the builtin, the compiler
 // picks the three-address form for these 64 four-register accumulators and then moves them
 // around the accumulation file inside the loop (several copies per MFMA). The compiler inserts
-// no hazard waits around assembly: the caller keeps dependent MFMAs apart (here 64 MFMAs) and
+// no hazard waits around assembly: the caller keeps dependent MFMAs apart (here at least four MFMAs) and
 // calls mfma16_drain() in the same basic block as the last MFMA, before control can reach code
 // the compiler may have placed on its own (copies or spills of the accumulators at a join): a
 // result read within the MFMA's four passes is the old value.
@@ -99,45 +52,6 @@ __device__ __forceinline__ void mfma16(const u32x4& a, const u32x4& b, f32x4& c)
 }
 __device__ __forceinline__ void mfma16_drain() {
     asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
-}
-
-// A wave's (32 TM) x (32 TN) block of C. The MFMAs take the W fragment as their first
-// operand, so a lane holds row row0 + 32 i + l32 of C and, in register 4 r + jj of tile
-// (i, j), column col0 + 32 j + 8 r + 4 h + jj: four consecutive columns per r, stored as
-// one 8- or 16-byte vector where the row pitch and the base allow it.
-template <bool F16, typename TC, int TM, int TN>
-__device__ __forceinline__ void store_tile(const GemmArgs& g, void* c, const f32x16 (&acc)[TM][TN], int row0, int col0, int l32, int h) {
-    // uniform over the launch: every group of four columns starts aligned for a vector store
-    const bool vec = (g.ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(c) % (4 * sizeof(TC))) == 0);
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-        const int row = row0 + i * 32 + l32;
-        if (row >= g.m) continue;
-        TC* const crow = reinterpret_cast<TC*>(c) + (int64_t)row * g.ldc;
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int col = col0 + j * 32 + 8 * r + 4 * h;
-                const f32x4 v = f32x4{acc[i][j][4 * r], acc[i][j][4 * r + 1], acc[i][j][4 * r + 2], acc[i][j][4 * r + 3]};
-                if (vec && col + 3 < g.n) {
-                    if constexpr (std::is_same<TC, float>::value) *reinterpret_cast<f32x4*>(crow + col) = v;
-                    else if constexpr (F16) *reinterpret_cast<f16x4*>(crow + col) = __builtin_convertvector(v, f16x4);
-                    else *reinterpret_cast<bf16x4*>(crow + col) = __builtin_convertvector(v, bf16x4);
-                } else {
-#pragma unroll
-                    for (int jj = 0; jj < 4; jj++) {
-                        if (col + jj < g.n) {
-                            TC* dst = crow + col + jj;
-                            if constexpr (std::is_same<TC, float>::value) *dst = v[jj];
-                            else if constexpr (F16) *reinterpret_cast<_Float16*>(dst) = (_Float16)v[jj];
-                            else *reinterpret_cast<bf16_t*>(dst) = (bf16_t)v[jj];
-                        }
-                    }
-                }
-            }
-        }
-    }
 }
 
 // A wave's (16 TI) x (16 TJ) block of C from 16 x 16 x 32 MFMAs. They take the W fragment as
@@ -174,26 +88,24 @@ __device__ __forceinline__ void store_tile16(const GemmArgs& g, void* c, const f
     }
 }
 
-// The same block for a 16-bit C, as whole rows of the block (32 TJ bytes: 256 for TJ = 8, 128
-// for TJ = 4): the wave turns 32 rows at a time (two rows of tiles) through LDS of its own
-// (32 x 32 TJ bytes at lds_wave), so it needs no barrier of its own; the caller sees to it that
-// nobody else uses that LDS any more. Staged rows are unpadded; the 16-byte chunk c of row r
-// sits at c ^ (r & 15) in 256-byte rows and at c ^ ((r >> 1) & 7) in 128-byte rows, which
-// spreads both the 8-byte writes (16 rows x 2 halves per half wave) and the row-wise reads over
+// A 128-column block of a 16-bit C, as whole rows of the block (256 bytes): the wave turns 32 rows
+// at a time (two rows of tiles) through 8 KB of LDS of its own at lds_wave, so it needs no barrier
+// of its own; the caller sees to it that nobody else uses that LDS any more. Staged rows are
+// unpadded; the 16-byte chunk c of row r sits at c ^ (r & 15), which spreads both the 8-byte writes (16 rows x 2 halves per half wave) and the row-wise reads over
 // all banks. A wave's LDS operations complete in order, so the reads of one pass see its
 // writes and the next pass's writes follow its reads. Rows of C that do not start on 16 bytes,
 // and the columns past n, are stored element by element.
-constexpr int kEpiWaveBytes = 32 * 256;
-template <bool F16, typename TC, int TI, int TJ>
-__device__ __forceinline__ void store_tile_lds16(const GemmArgs& g, void* c, const f32x4 (&acc)[TI][TJ], unsigned lds_wave, int row0, int col0, int lane) {
+template <bool F16, typename TC, int TI>
+__device__ __forceinline__ void store_tile_lds16(const GemmArgs& g, void* c, const f32x4 (&acc)[TI][8], unsigned lds_wave, int row0, int col0, int lane) {
     static_assert(sizeof(TC) == 2, "16-bit C only");
-    static_assert((TJ == 8 || TJ == 4) && TI % 2 == 0, "blocks of 128 or 64 columns, rows in pairs of tiles");
+    static_assert(TI % 2 == 0, "rows in pairs of tiles");
+    constexpr int TJ = 8;
     constexpr int ROWB = 32 * TJ;   // bytes per staged row
     constexpr int NCH = 2 * TJ;     // 16-byte chunks per row
     constexpr int RPI = 64 / NCH;   // rows per read-back instruction
     typedef __attribute__((address_space(3))) u32x2* lds_u32x2_t;
     typedef const __attribute__((address_space(3))) u32x4* lds_u32x4_t;
-    auto swz = [](int r) { return TJ == 8 ? (r & 15) : ((r >> 1) & 7); };
+    auto swz = [](int r) { return r & 15; };
     const int c16 = lane & 15, q = lane >> 4;
     // write: row 16 (i & 1) + c16, bytes 32 j + 8 q .. + 8 = chunk 2 j + q / 2, half q & 1
     const unsigned wbase = lds_wave + (unsigned)(c16 * ROWB + (q & 1) * 8);
@@ -214,7 +126,7 @@ __device__ __forceinline__ void store_tile_lds16(const GemmArgs& g, void* c, con
                 u32x2 pk;
                 if constexpr (F16) pk = __builtin_bit_cast(u32x2, __builtin_convertvector(v, f16x4));
                 else pk = __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
-                // (rows 16 .. 31 swizzle as rows 0 .. 15 do: both forms of swz ignore bit 4)
+                // (rows 16 .. 31 swizzle as rows 0 .. 15 do)
                 *(lds_u32x2_t)(wbase + (unsigned)(ii * 16 * ROWB) + (((unsigned)(2 * j) ^ wsw) * 16u)) = pk;
             }
         __builtin_amdgcn_sched_barrier(0); // (keeps the scheduler from reading every accumulator out at once)
@@ -235,6 +147,102 @@ __device__ __forceinline__ void store_tile_lds16(const GemmArgs& g, void* c, con
 #pragma unroll
                 for (int e = 0; e < 8; e++)
                     if (col + e < g.n) dst[e] = (unsigned short)(v[p2][e >> 1] >> (16 * (e & 1)));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// A 128-column block of f32 C in the same way: 16 rows (8 KB) at a time, the 16-byte chunk c of
+// row r at c ^ (r & 7) (eight rows written at once hit eight different chunks; the swizzle stays
+// inside 128 bytes, so an instruction still stores two whole 512-byte rows).
+template <int TI>
+__device__ __forceinline__ void store_tile_lds32(const GemmArgs& g, void* c, const f32x4 (&acc)[TI][8], unsigned lds_wave, int row0, int col0, int lane) {
+    typedef __attribute__((address_space(3))) f32x4* lds_f32x4_t;
+    const int c16 = lane & 15, q = lane >> 4;
+    const bool vec = (g.ldc % 4 == 0) && (reinterpret_cast<uintptr_t>(c) % 16 == 0);
+#pragma unroll
+    for (int i = 0; i < TI; i++) {
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            *(lds_f32x4_t)(lds_wave + (unsigned)(c16 * 512) + (unsigned)(((4 * j + q) ^ (c16 & 7)) * 16)) = acc[i][j];
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 v[8];
+#pragma unroll
+        for (int p = 0; p < 8; p++) v[p] = *(lds_f32x4_t)(lds_wave + (unsigned)(p * 1024 + lane * 16));
+#pragma unroll
+        for (int p = 0; p < 8; p++) {
+            const int r = 2 * p + (lane >> 5);
+            const int row = row0 + 16 * i + r, col = col0 + (((lane & 31) ^ (r & 7)) * 4);
+            if (row >= g.m || col >= g.n) continue;
+            float* const dst = reinterpret_cast<float*>(c) + (int64_t)row * g.ldc + col;
+            if (vec && col + 4 <= g.n) {
+                *reinterpret_cast<f32x4*>(dst) = v[p];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (col + e < g.n) dst[e] = v[p][e];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// The same for either type of C and any TJ, with padded rows instead of a swizzle: two rows of
+// tiles at a time go through 32 x (16 TJ sizeof(TC) + 16) bytes of LDS of the wave's own at
+// lds_wave and leave as whole rows of the block, 16 bytes per lane. (Stored from the registers a
+// lane's four columns make every instruction 16 separate pieces of 32 or 64 bytes, which the
+// CU's address unit takes one by one: a 256 x 160 tile of bf16 took 6 us that way.)
+template <typename TC, int TJ>
+constexpr int rows_wave_bytes() { return 32 * (16 * TJ * (int)sizeof(TC) + 16); }
+template <bool F16, typename TC, int TI, int TJ>
+__device__ __forceinline__ void store_rows_lds(const GemmArgs& g, void* c, const f32x4 (&acc)[TI][TJ], unsigned lds_wave, int row0, int col0, int lane) {
+    constexpr int ES = (int)sizeof(TC);
+    constexpr int PITCH = 16 * TJ * ES + 16; // bytes per staged row
+    constexpr int CPR = TJ * ES;             // 16-byte chunks per row
+    constexpr int PER = 16 / ES;             // elements per chunk
+    static_assert(TI % 2 == 0, "rows of tiles in pairs");
+    typedef __attribute__((address_space(3))) u32x2* lds_u32x2_t;
+    typedef __attribute__((address_space(3))) f32x4* lds_f32x4_t;
+    typedef const __attribute__((address_space(3))) u32x4* lds_u32x4_t;
+    const int c16 = lane & 15, q = lane >> 4;
+    const unsigned wbase = lds_wave + (unsigned)(c16 * PITCH + 4 * q * ES);
+    // (uniform over the launch: rows of C start on 16 bytes; otherwise element by element)
+    const bool vec = ((g.ldc * ES) % 16 == 0) && (reinterpret_cast<uintptr_t>(c) % 16 == 0);
+#pragma unroll
+    for (int ip = 0; ip < TI / 2; ip++) {
+#pragma unroll
+        for (int ii = 0; ii < 2; ii++)
+#pragma unroll
+            for (int j = 0; j < TJ; j++) {
+                const f32x4 v = acc[2 * ip + ii][j];
+                const unsigned at = wbase + (unsigned)(ii * 16 * PITCH + j * 16 * ES);
+                if constexpr (ES == 4) *(lds_f32x4_t)at = v;
+                else if constexpr (F16) *(lds_u32x2_t)at = __builtin_bit_cast(u32x2, __builtin_convertvector(v, f16x4));
+                else *(lds_u32x2_t)at = __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
+            }
+        __builtin_amdgcn_sched_barrier(0); // (keeps the scheduler from reading every accumulator out at once)
+        u32x4 v[CPR / 2];
+#pragma unroll
+        for (int p = 0; p < CPR / 2; p++) {
+            const int x = 64 * p + lane;
+            v[p] = *(lds_u32x4_t)(lds_wave + (unsigned)((x / CPR) * PITCH + (x % CPR) * 16));
+        }
+#pragma unroll
+        for (int p = 0; p < CPR / 2; p++) {
+            const int x = 64 * p + lane;
+            const int row = row0 + 32 * ip + x / CPR, col = col0 + (x % CPR) * PER;
+            if (row >= g.m || col >= g.n) continue;
+            TC* const dst = reinterpret_cast<TC*>(c) + (int64_t)row * g.ldc + col;
+            if (vec && col + PER <= g.n) {
+                *reinterpret_cast<u32x4*>(dst) = v[p];
+            } else {
+#pragma unroll
+                for (int e = 0; e < PER; e++) {
+                    if (col + e >= g.n) break;
+                    if constexpr (ES == 4) reinterpret_cast<unsigned*>(dst)[e] = v[p][e];
+                    else reinterpret_cast<unsigned short*>(dst)[e] = (unsigned short)(v[p][e >> 1] >> (16 * (e & 1)));
+                }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -271,126 +279,9 @@ __device__ __forceinline__ void tile_coords(int logical, int tiles_m, int tiles_
     tn = strip * kStrip + (r - tm * width);
 }
 
-// TA: float or a 16-bit type (then it is the compute type); F16: compute type is
-// IEEE half instead of bf16; TC: float or a 16-bit type.
-template <typename TA, bool F16, typename TC>
-__global__ void __launch_bounds__(NT, 2) gemm_kernel(const GemmArgs g) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    unsigned short* const lds = reinterpret_cast<unsigned short*>(smem);
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int l32 = lane & 31;
-    const int h = lane >> 5;
-    const int wm = wave >> 1, wn = wave & 1;
-
-    const int logical = logical_tile((int)blockIdx.x, (int)gridDim.x);
-    const int tiles_row = g.tiles_n * g.groups;
-    int tm, tn;
-    tile_coords(logical, (g.m + BM - 1) / BM, tiles_row, tm, tn);
-    const int grp = tn / g.tiles_n;
-    tn -= grp * g.tiles_n;
-    const void* const wp = grp == 0 ? g.w : g.w_more[grp - 1];
-    void* const cp = grp == 0 ? g.c : g.c_more[grp - 1];
-    const int m0 = tm * BM, n0 = tn * BN;
-
-    // ---- staging: thread t owns 16-byte chunk t%8 of rows t/8 + 64 j (j < 4) of the A slab and of the W slab
-    constexpr unsigned ea = sizeof(TA);
-    const unsigned a_span = ((unsigned)(g.m - 1) * (unsigned)g.lda + (unsigned)g.k) * ea;
-    const unsigned w_span = ((unsigned)(g.n - 1) * (unsigned)g.ldw + (unsigned)g.k) * 2u;
-    const rsrc_t a_rsrc = make_rsrc(g.a, a_span);
-    const rsrc_t w_rsrc = make_rsrc(wp, w_span);
-    const int lr = tid >> 3;
-    const int kc = tid & 7;
-    unsigned a_off[4], w_off[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int ar = min(m0 + lr + 64 * j, g.m - 1); // rows past the edge re-read the last row; never stored
-        const int wr = min(n0 + lr + 64 * j, g.n - 1);
-        a_off[j] = ((unsigned)ar * (unsigned)g.lda + (unsigned)(kc * 8)) * ea;
-        w_off[j] = ((unsigned)wr * (unsigned)g.ldw + (unsigned)(kc * 8)) * 2u;
-    }
-    const int nslab = (g.k + BK - 1) / BK;
-
-    Chunk<TA> ra[4];
-    Chunk<unsigned short> rw[4];
-    auto load_slab = [&](int s) __attribute__((always_inline)) {
-        const int ss = s < nslab ? s : nslab - 1; // past the end: a harmless re-read
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            ra[j] = ld_chunk<TA>(a_rsrc, a_off[j], (unsigned)ss * (BK * ea));
-            rw[j] = ld_chunk<unsigned short>(w_rsrc, w_off[j], (unsigned)ss * (BK * 2u));
-        }
-    };
-    auto store_slab = [&](int s) __attribute__((always_inline)) {
-        unsigned short* st = lds + (s & 1) * STAGE_ELEMS;
-        // chunks past k contribute zeros; only the last slab of a k that is not a multiple of 64 has any
-        const bool ragged = (s + 1) * BK > g.k; // wave-uniform
-        const bool keep = !ragged || s * BK + kc * 8 < g.k;
-        if (ragged) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                *reinterpret_cast<u32x4*>(st + (lr + 64 * j) * PITCH + kc * 8) = to_half8<TA, F16>(ra[j], keep);
-                *reinterpret_cast<u32x4*>(st + (BM + lr + 64 * j) * PITCH + kc * 8) = to_half8<unsigned short, F16>(rw[j], keep);
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                *reinterpret_cast<u32x4*>(st + (lr + 64 * j) * PITCH + kc * 8) = to_half8<TA, F16>(ra[j], true);
-                *reinterpret_cast<u32x4*>(st + (BM + lr + 64 * j) * PITCH + kc * 8) = to_half8<unsigned short, F16>(rw[j], true);
-            }
-        }
-    };
-
-    f32x16 acc[2][4];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
-
-    load_slab(0);
-    store_slab(0);
-    load_slab(1);
-    __syncthreads();
-
-    const int a_frag = (wm * 64 + l32) * PITCH + 8 * h;
-    const int w_frag = (BM + wn * 128 + l32) * PITCH + 8 * h;
-    for (int s = 0; s < nslab; s++) {
-        const unsigned short* st = lds + (s & 1) * STAGE_ELEMS;
-#pragma unroll
-        for (int kk = 0; kk < BK / 16; kk++) {
-            u32x4 af[2], wf[4];
-#pragma unroll
-            for (int i = 0; i < 2; i++) af[i] = *reinterpret_cast<const u32x4*>(st + a_frag + i * 32 * PITCH + kk * 16);
-#pragma unroll
-            for (int j = 0; j < 4; j++) wf[j] = *reinterpret_cast<const u32x4*>(st + w_frag + j * 32 * PITCH + kk * 16);
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] = mfma<F16>(wf[j], af[i], acc[i][j]);
-            if (kk == 0) {
-                // slab s+1 (in registers since the previous iteration) goes to the other stage,
-                // whose readers finished before the last barrier; then slab s+2 starts loading.
-                // The fences keep the loads here: sunk to the end of the iteration they would
-                // be waited for as soon as they are issued.
-                __builtin_amdgcn_sched_barrier(0);
-                store_slab(s + 1);
-                load_slab(s + 2);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        __syncthreads();
-    }
-
-    store_tile<F16, TC, 2, 4>(g, cp, acc, m0 + wm * 64, n0 + wn * 128, l32, h);
-}
-
-// The same tile with 16-bit activations and k a multiple of 64: both slabs go
-// from global memory straight into LDS (buffer_load ... lds), no staging
-// registers and no LDS store instructions. Such a load writes lane i's 16 bytes
+// The eight-wave build (k a multiple of 64; kept behind a knob). Both slabs go from global
+// memory straight into LDS (buffer_load ... lds), no staging registers and no LDS store
+// instructions; the other kernels use the same layout. Such a load writes lane i's 16 bytes
 // at (LDS base) + 16 i, so rows are 128 bytes with no padding and bank conflicts
 // are avoided by a swizzle instead: the 16-byte chunk c of row r lives at chunk
 // position c ^ ((r >> 1) & 7); the lane that fills position p of row r fetches
@@ -399,11 +290,10 @@ __global__ void __launch_bounds__(NT, 2) gemm_kernel(const GemmArgs g) {
 constexpr int DMA_STAGE_BYTES = (BM + BN) * BK * 2; // 64 KB
 constexpr size_t kDmaLdsBytes = 2 * (size_t)DMA_STAGE_BYTES;
 
-// TB x TB tile of C, WM x WN waves, a wave owns (TB / WM) x (TB / WN). Built as 256 with
-// 4 x 2 waves (two per SIMD, 64 x 128 each) and as 128 with 2 x 2 waves (64 x 64 each, 64 KB
-// of LDS, two workgroups per CU) for problems with too few 256-tiles to fill the chip.
-template <bool F16, typename TC, int WM, int WN, int TB>
+// 256 x 256 tile of C, 4 x 2 waves (two per SIMD, 64 x 128 each).
+template <bool F16, typename TC, int WM, int WN>
 __global__ void __launch_bounds__(WM * WN * 64, 2) gemm_dma_kernel(const GemmArgs g) {
+    constexpr int TB = 256;
     constexpr int STAGE_BYTES = 2 * TB * BK * 2; // A rows then W rows
     constexpr int NW = WM * WN;
     constexpr int TM = TB / WM / 16, TN = TB / WN / 16; // 16 x 16 MFMA tiles per wave
@@ -504,31 +394,30 @@ __global__ void __launch_bounds__(WM * WN * 64, 2) gemm_dma_kernel(const GemmArg
         __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): slab s+1 has landed
         __syncthreads();
     }
-    if constexpr (sizeof(TC) == 2 && TB == 128) {
-        // the loop's last barrier has left the stages idle; each wave stages 32 rows of its block in them
-        static_assert((size_t)WM * WN * 32 * (32 * TN) <= 2 * (size_t)(2 * TB * BK * 2), "staging exceeds the slab stages");
-        store_tile_lds16<F16, TC, TM, TN>(g, cp, acc, lds_address(smem) + (unsigned)wave * (32 * 32 * TN),
-                                          m0 + wm * (16 * TM), n0 + wn * (16 * TN), lane);
-    } else {
-        store_tile16<F16, TC, TM, TN>(g, cp, acc, m0 + wm * (16 * TM), n0 + wn * (16 * TN), lane);
-    }
+    store_tile16<F16, TC, TM, TN>(g, cp, acc, m0 + wm * (16 * TM), n0 + wn * (16 * TN), lane);
 }
 
 // ---------------------------------------------------------------------------
 // Four-wave build: one wave per SIMD, each owning 128 x 128 of C as 8 x 8 tiles of
 // v_mfma_f32_16x16x32 (256 accumulation registers; 16 fragment reads per 64 MFMAs, a third
-// fewer LDS bytes per MFMA than the 8-wave builds). One wave per SIMD has no neighbour to hide
+// fewer LDS bytes per MFMA than the 8-wave build). One wave per SIMD has no neighbour to hide
 // its waits, so the schedule leaves none. A 64-wide slab is two 32-wide steps of 64 MFMAs; the
 // 16 fragments of the next step are read one per two MFMAs under the first half of the current
 // one. The slab's one barrier sits in its FIRST step, after the 40th MFMA, when the slab's last
-// fragments are in registers: it both frees the slab's LDS stage for slab s + 2 and makes slab
-// s + 1 visible, whose first fragments are read under the second step. The 16 loads of slab
-// s + 2 follow the barrier one per four MFMAs (the CU's address unit takes 16 cycles per 1 KB
-// load and the four waves issue in the same phase: 64 cycles per round of loads). The loop is
-// unrolled over the two stages, so every LDS address is a pointer plus a constant. Same
-// 128-byte swizzled rows and two 64 KB stages as the direct-to-LDS build above; behind them
-// 8 KB per wave for the epilogue of a 16-bit C.
-constexpr size_t kRingLdsBytes = 2 * (size_t)DMA_STAGE_BYTES + 4 * (size_t)kEpiWaveBytes; // 160 KB
+// fragments are in registers: it both frees the slab's LDS slots and makes slab s + 1 visible,
+// whose first fragments are read under the second step. The 16 loads into the freed slots follow
+// the barrier one per four MFMAs (the CU's address unit takes 16 cycles per 1 KB load and the
+// four waves issue in the same phase: 64 cycles per round of loads).
+// The LDS is five slots of one operand's slab (32 KB), W and A of the slabs going round in turn:
+// into the two slots slab s frees go A of slab s + 2, which has 96 MFMAs (0.6-0.8 us) to arrive,
+// and W of slab s + 3, which has 224 (weights come from memory, 0.6 us away when it is idle).
+// With two whole stages, where all loads of slab s + 2 went out after the barrier and the last had
+// 64 MFMAs, cold weights cost 8-16 % (same shapes with weights in the last-level cache: 204 / 246 us
+// against 221 / 285 for 4608 x 3072 x 9216 and 4608 x 12288 x 3072); now 4-10 % (195 / 234, 204 / 259).
+// The loop is unrolled over the five slots, so every LDS address is a pointer plus a constant. Same
+// 128-byte swizzled rows as the direct-to-LDS build above.
+constexpr int SLOT = BM * BK * 2; // one operand's half of a slab: 32 KB
+constexpr size_t kRingLdsBytes = 5 * (size_t)SLOT; // 160 KB
 template <bool F16, typename TC>
 __global__ void __launch_bounds__(256, 1) gemm_ring_kernel(const GemmArgs g) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -585,29 +474,24 @@ __global__ void __launch_bounds__(256, 1) gemm_ring_kernel(const GemmArgs g) {
     if (splits > 1) {
         const int per = (nslab + splits - 1) / splits;
         slab0 = part_id * per;
-        nslab = max(min(nslab - slab0, per), 0);
+        // (uniform, but the division runs on the vector unit)
+        nslab = __builtin_amdgcn_readfirstlane(max(min(nslab - slab0, per), 0));
+        slab0 = __builtin_amdgcn_readfirstlane(slab0);
     }
     const unsigned fetch_lds = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)wave * (64 * BK * 2));
-    // slabs past the end re-fetch the last slab into a stage nobody reads any more
-    // the i-th (i < 16) of the loads that bring this wave's part of slab s in, in the order A rows
-    // 0..31 of the wave's 64, W rows 0..31, A rows 32..63, W rows 32..63 (eight rows a load); the
-    // loads of a run must be issued in order, the first sets M0 for the rest
-    auto fetch_one = [&](int s, int i) __attribute__((always_inline)) {
-        const unsigned uo = (unsigned)min(slab0 + max(s < nslab ? s : nslab - 1, 0), g.k / BK - 1) * (BK * 2u);
-        const int run = i >> 2, jj = i & 3;
-        const bool is_w = run & 1;
-        const int j = (run >> 1) * 4 + jj;
-        if (jj == 0) lds_dma_base(fetch_lds + (unsigned)(s & 1) * DMA_STAGE_BYTES + (is_w ? BM * BK * 2 : 0) + (unsigned)(run >> 1) * (32 * BK * 2));
+    // the i-th (i < 8) of the loads that bring this wave's rows of an operand's slab s into slot `slot`
+    // (eight rows a load), in order: the first of every four sets M0 for the rest. Slabs past the end
+    // re-fetch the last one into a slot nobody reads any more.
+    auto fetch_one = [&](bool is_w, int s, int slot, int i) __attribute__((always_inline)) {
+        // (uniform, but the compiler may have formed it in a vector register)
+        const unsigned uo = __builtin_amdgcn_readfirstlane((unsigned)min(slab0 + max(s < nslab ? s : nslab - 1, 0), g.k / BK - 1) * (BK * 2u));
+        if ((i & 3) == 0) lds_dma_base(fetch_lds + (unsigned)(slot * SLOT + (i >> 2) * (32 * BK * 2)));
         const u32x4& rsrc = is_w ? w_rsrc : a_rsrc;
-        const unsigned off = is_w ? w_off[j] : a_off[j];
-        if (jj == 0) load_to_lds_16_at<0>(rsrc, off, uo);
-        if (jj == 1) load_to_lds_16_at<1024>(rsrc, off, uo);
-        if (jj == 2) load_to_lds_16_at<2048>(rsrc, off, uo);
-        if (jj == 3) load_to_lds_16_at<3072>(rsrc, off, uo);
-    };
-    auto fetch_slab = [&](int s) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 16; i++) fetch_one(s, i);
+        const unsigned off = is_w ? w_off[i] : a_off[i];
+        if ((i & 3) == 0) load_to_lds_16_at<0>(rsrc, off, uo);
+        if ((i & 3) == 1) load_to_lds_16_at<1024>(rsrc, off, uo);
+        if ((i & 3) == 2) load_to_lds_16_at<2048>(rsrc, off, uo);
+        if ((i & 3) == 3) load_to_lds_16_at<3072>(rsrc, off, uo);
     };
 
     f32x4 acc[8][8];
@@ -618,41 +502,47 @@ __global__ void __launch_bounds__(256, 1) gemm_ring_kernel(const GemmArgs g) {
 
     // fragment addresses: row (.. + c16), logical chunk 4 ks + q4 (ks < 2) at c ^ ((row >> 1) & 7);
     // a tile row adds 16 rows = 2 KB. (Pointers, so that the constant parts go into the
-    // instruction's offset field; a stage is 64 KB, beyond that field: one pointer per stage.)
+    // instruction's offset field; that field reaches 64 KB: one pointer per two slots.)
     typedef const __attribute__((address_space(3))) unsigned char* lds_byte_t;
     typedef const __attribute__((address_space(3))) u32x4* lds_u32x4_t;
     const lds_byte_t lds_base = (lds_byte_t)smem;
     const int sw = (c16 >> 1) & 7;
-    lds_byte_t fa[2][2], fw[2][2]; // [stage][ks]
+    lds_byte_t fa[3][2], fw[3][2]; // [slot / 2][ks]
 #pragma unroll
-    for (int st = 0; st < 2; st++)
+    for (int sp = 0; sp < 3; sp++)
 #pragma unroll
         for (int ks = 0; ks < 2; ks++) {
             const int pos = ((4 * ks + q4) ^ sw) * 16;
-            fa[st][ks] = lds_base + (st * DMA_STAGE_BYTES + (wm * 128 + c16) * (BK * 2) + pos);
-            fw[st][ks] = lds_base + (st * DMA_STAGE_BYTES + BM * BK * 2 + (wn * 128 + c16) * (BK * 2) + pos);
+            fa[sp][ks] = lds_base + (2 * sp * SLOT + (wm * 128 + c16) * (BK * 2) + pos);
+            fw[sp][ks] = lds_base + (2 * sp * SLOT + (wn * 128 + c16) * (BK * 2) + pos);
         }
     struct Frag { u32x4 a[8], w[8]; };
-    // the r-th of the 16 reads of a fragment set
-    auto read_one = [&](Frag& f, int st, int ks, int r) __attribute__((always_inline)) {
-        if (r < 8) f.a[r] = *(lds_u32x4_t)(fa[st][ks] + r * 16 * (BK * 2));
-        else f.w[r - 8] = *(lds_u32x4_t)(fw[st][ks] + (r - 8) * 16 * (BK * 2));
+    // the r-th of the 16 reads of a fragment set; W and A of slab s are in slots 2 s and 2 s + 1 (mod 5)
+    auto read_one = [&](Frag& f, int a_slot, int w_slot, int ks, int r) __attribute__((always_inline)) {
+        if (r < 8) f.a[r] = *(lds_u32x4_t)(fa[a_slot >> 1][ks] + ((a_slot & 1) * SLOT + r * 16 * (BK * 2)));
+        else f.w[r - 8] = *(lds_u32x4_t)(fw[w_slot >> 1][ks] + ((w_slot & 1) * SLOT + (r - 8) * 16 * (BK * 2)));
     };
-    // One 32-wide step: 64 MFMAs on `cur`, the 16 reads of `nxt` under the first 32 of them.
-    // FIRST (the slab's first step): the barrier after the 40th MFMA, then loads 0..5 of slab
-    // s + 2, one per four MFMAs; the second step sends loads 6..15.
-    auto mfma_step = [&](auto first_c, auto st_c, auto ks_c, const Frag& cur, Frag& nxt, int s) __attribute__((always_inline)) {
+    // One 32-wide step of slab s (P = s mod 5): 64 MFMAs on `cur`, the 16 reads of `nxt` under the
+    // first 32 of them. FIRST (the slab's first step): the barrier after the 40th MFMA, then the first
+    // 6 of the 16 loads that go into the slab's two slots, one per four MFMAs; the second step sends
+    // the other 10.
+    auto mfma_step = [&](auto first_c, auto p_c, const Frag& cur, Frag& nxt, int s) __attribute__((always_inline)) {
         constexpr bool FIRST = decltype(first_c)::value;
-        constexpr int NST = decltype(st_c)::value, NKS = decltype(ks_c)::value; // where nxt is read from
+        constexpr int P = decltype(p_c)::value;
+        constexpr int NP = FIRST ? P : (P + 1) % 5; // the slab nxt belongs to
+        auto send = [&](int i) __attribute__((always_inline)) {
+            if (i < 8) fetch_one(false, s + 2, (2 * P) % 5, i);
+            else fetch_one(true, s + 3, (2 * P + 1) % 5, i - 8);
+        };
 #pragma unroll
         for (int t = 0; t < 64; t++) {
-            if (FIRST && t >= 40 && (t & 3) == 0) fetch_one(s + 2, (t - 40) >> 2);
-            if (!FIRST && (t & 3) == 1 && t < 40) fetch_one(s + 2, 6 + (t >> 2));
-            if ((t & 1) == 0 && t < 32) read_one(nxt, NST, NKS, t >> 1);
+            if (FIRST && t >= 40 && (t & 3) == 0) send((t - 40) >> 2);
+            if (!FIRST && (t & 3) == 1 && t < 40) send(6 + (t >> 2));
+            if ((t & 1) == 0 && t < 32) read_one(nxt, (2 * NP + 1) % 5, (2 * NP) % 5, FIRST ? 1 : 0, t >> 1);
             mfma16<F16>(cur.w[t & 7], cur.a[t >> 3], acc[t >> 3][t & 7]);
             __builtin_amdgcn_sched_barrier(0);
             if (FIRST && t == 39) {
-                __builtin_amdgcn_s_waitcnt(0x0070); // vmcnt(0) lgkmcnt(0)
+                __builtin_amdgcn_s_waitcnt(0x0078); // vmcnt(8) lgkmcnt(0): all but W of slab s + 2 has landed
                 asm volatile("" ::: "memory");
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
@@ -661,28 +551,43 @@ __global__ void __launch_bounds__(256, 1) gemm_ring_kernel(const GemmArgs g) {
         }
     };
 
-    fetch_slab(0);
-    fetch_slab(1);
-    __builtin_amdgcn_s_waitcnt(0x4F70); // vmcnt(16): slab 0 has landed
+#pragma unroll
+    for (int i = 0; i < 8; i++) fetch_one(true, 0, 0, i);
+#pragma unroll
+    for (int i = 0; i < 8; i++) fetch_one(false, 0, 1, i);
+#pragma unroll
+    for (int i = 0; i < 8; i++) fetch_one(true, 1, 2, i);
+#pragma unroll
+    for (int i = 0; i < 8; i++) fetch_one(false, 1, 3, i);
+#pragma unroll
+    for (int i = 0; i < 8; i++) fetch_one(true, 2, 4, i);
+    __builtin_amdgcn_s_waitcnt(0x4F78); // vmcnt(24): slab 0 has landed
     __syncthreads();
     Frag f0, f1;
 #pragma unroll
-    for (int r = 0; r < 16; r++) read_one(f0, 0, 0, r);
+    for (int r = 0; r < 16; r++) read_one(f0, 1, 0, 0, r);
+    auto slab = [&](auto p_c, int s) __attribute__((always_inline)) {
+        mfma_step(std::true_type{}, p_c, f0, f1, s);
+        mfma_step(std::false_type{}, p_c, f1, f0, s);
+    };
     typedef std::integral_constant<int, 0> I0;
     typedef std::integral_constant<int, 1> I1;
+    typedef std::integral_constant<int, 2> I2;
+    typedef std::integral_constant<int, 3> I3;
+    typedef std::integral_constant<int, 4> I4;
     int s = 0;
-    for (; s + 1 < nslab; s += 2) {
-        mfma_step(std::true_type{}, I0{}, I1{}, f0, f1, s);
-        mfma_step(std::false_type{}, I1{}, I0{}, f1, f0, s);
-        mfma_step(std::true_type{}, I1{}, I1{}, f0, f1, s + 1);
-        mfma_step(std::false_type{}, I0{}, I0{}, f1, f0, s + 1);
-        mfma16_drain(); // (24 cycles per two slabs: whatever follows the loop body may read the accumulators)
+    for (; s + 5 <= nslab; s += 5) {
+        slab(I0{}, s);
+        slab(I1{}, s + 1);
+        slab(I2{}, s + 2);
+        slab(I3{}, s + 3);
+        slab(I4{}, s + 4);
+        mfma16_drain(); // (24 cycles per five slabs: whatever follows the loop body may read the accumulators)
     }
-    if (s < nslab) {
-        mfma_step(std::true_type{}, I0{}, I1{}, f0, f1, s);
-        mfma_step(std::false_type{}, I1{}, I0{}, f1, f0, s);
-        mfma16_drain();
-    }
+    if (s < nslab) { slab(I0{}, s); mfma16_drain(); }
+    if (s + 1 < nslab) { slab(I1{}, s + 1); mfma16_drain(); }
+    if (s + 2 < nslab) { slab(I2{}, s + 2); mfma16_drain(); }
+    if (s + 3 < nslab) { slab(I3{}, s + 3); mfma16_drain(); }
     __builtin_amdgcn_s_waitcnt(0x0F70); // no direct load may outlive the workgroup's LDS
     if (splits > 1) {
         // partial tile in the accumulation layout: [tile][part][wave][i][j][lane] x 16 bytes,
@@ -695,10 +600,190 @@ __global__ void __launch_bounds__(256, 1) gemm_ring_kernel(const GemmArgs g) {
             for (int j = 0; j < 8; j++) dst[(i * 8 + j) * 64] = acc[i][j];
         return;
     }
-    if constexpr (sizeof(TC) == 2)
-        store_tile_lds16<F16, TC, 8, 8>(g, cp, acc, lds0 + 2u * DMA_STAGE_BYTES + (unsigned)wave * kEpiWaveBytes, m0 + wm * 128, n0 + wn * 128, lane);
-    else
-        store_tile16<F16, TC, 8, 8>(g, cp, acc, m0 + wm * 128, n0 + wn * 128, lane);
+    // (this wave's 8 KB of the slot that A of slab `nslab` went to: only this wave's loads write them,
+    // they have landed, and nobody needs what is there)
+    const unsigned epi_lds = fetch_lds + (unsigned)(((2 * nslab + 1) % 5) * SLOT);
+    if constexpr (sizeof(TC) == 2) store_tile_lds16<F16, TC, 8>(g, cp, acc, epi_lds, m0 + wm * 128, n0 + wn * 128, lane);
+    else store_tile_lds32<8>(g, cp, acc, epi_lds, m0 + wm * 128, n0 + wn * 128, lane);
+}
+
+// ---------------------------------------------------------------------------
+// Problems with too few 256-tiles to fill the chip: the four-wave schedule of gemm_ring_kernel
+// for any tile of (32 TI) x (32 TJ), one workgroup per CU, each wave (16 TI) x (16 TJ) of C. A
+// smaller tile spends fewer cycles on a slab than the slab takes to arrive, so the LDS holds ST
+// slabs and ST - 1 of them are on their way while one is worked on.
+//   slab s, first step: the MFMAs of its k 0..31 on f0; its k 32..63 fragments are read into f1;
+//     after the last of those reads the slab's one barrier (this wave's part of slab s + 1 has
+//     landed, everybody has slab s in registers: its stage is free);
+//   second step: the MFMAs on f1, the k 0..31 fragments of slab s + 1 are read into f0;
+//   from the barrier on, one load of slab s + ST per four MFMAs (the pace of the CU's address
+//     unit); what is left of them goes out in the next slab's first step, ahead of its barrier.
+constexpr int vm_lgkm0(int vm) { return (vm & 15) | 0x70 | ((vm >> 4) << 14); }           // vmcnt(vm) lgkmcnt(0)
+constexpr int vm_only(int vm) { return (vm & 15) | 0xF70 | ((vm >> 4) << 14); }           // vmcnt(vm)
+constexpr size_t pipe_lds_bytes(int ti, int tj, int st) { return (size_t)st * (size_t)(ti + tj) * 32 * BK * 2; }
+
+template <bool F16, typename TC, int TI, int TJ, int ST, bool RAG>
+__global__ void __launch_bounds__(256, 1) gemm_pipe_kernel(const GemmArgs g) {
+    constexpr int TBM = 32 * TI, TBN = 32 * TJ;
+    constexpr int STAGE = (TBM + TBN) * BK * 2; // bytes: A rows then W rows
+    constexpr int NM = TI * TJ;                 // MFMAs of a step
+    constexpr int NR = TI + TJ;                 // fragment reads of a step
+    constexpr int NL = TI + TJ;                 // loads of a wave per slab
+    constexpr int RS = NM >= 32 ? 2 : 1;        // MFMAs per fragment read
+    constexpr int TB = (NR - 1) * RS + 5 < NM - 1 ? (NR - 1) * RS + 5 : NM - 1; // the barrier follows this MFMA of the first step
+    constexpr int LS = 2 * NM / NL < 4 ? 2 * NM / NL : 4; // MFMAs per load
+    // load i goes out ahead of MFMA TB + 1 + LS i, counted from the start of the slab that frees its stage
+    constexpr int IW = (2 * NM - (TB + 1) + LS - 1) / LS < NL ? (2 * NM - (TB + 1) + LS - 1) / LS : NL; // loads that go out within that slab
+    static_assert(LS >= 1 && TB + 1 + LS * (NL - 1) <= 2 * NM + TB, "all loads of a slab are out by the next barrier");
+    static_assert((ST - 1) * NL <= 63, "vmcnt counts to 63");
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int c16 = lane & 15;
+    const int q4 = lane >> 4;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int tiles_row = g.tiles_n * g.groups;
+    const int tiles_m = (g.m + TBM - 1) / TBM;
+    int tm, tn;
+    tile_coords(logical_tile((int)blockIdx.x, (int)gridDim.x), tiles_m, tiles_row, tm, tn);
+    const int grp = tn / g.tiles_n;
+    tn -= grp * g.tiles_n;
+    const void* const wp = grp == 0 ? g.w : g.w_more[grp - 1];
+    void* const cp = grp == 0 ? g.c : g.c_more[grp - 1];
+    const int m0 = tm * TBM, n0 = tn * TBN;
+
+    const unsigned a_span = ((unsigned)(g.m - 1) * (unsigned)g.lda + (unsigned)g.k) * 2u;
+    const unsigned w_span = ((unsigned)(g.n - 1) * (unsigned)g.ldw + (unsigned)g.k) * 2u;
+    // loads in runs of four under one M0, as in gemm_ring_kernel
+    constexpr unsigned kBias = 3 * 1024;
+    const u32x4 a_rsrc = make_rsrc_words(reinterpret_cast<const unsigned char*>(g.a) - kBias, a_span + kBias);
+    const u32x4 w_rsrc = make_rsrc_words(reinterpret_cast<const unsigned char*>(wp) - kBias, w_span + kBias);
+    const unsigned lds0 = lds_address(smem);
+    // wave w fills rows 8 TI w + 8 j + lane / 8 (j < TI) of the A slab and rows 8 TJ w + .. of the W slab
+    unsigned a_off[TI], w_off[TJ];
+#pragma unroll
+    for (int j = 0; j < TI; j++) {
+        const int r = wave * (8 * TI) + j * 8 + (lane >> 3);
+        const int c = (lane & 7) ^ ((r >> 1) & 7);
+        const int ar = min(m0 + r, g.m - 1); // rows past the edge re-read the last row; never stored
+        a_off[j] = ((unsigned)ar * (unsigned)g.lda + (unsigned)(c * 8)) * 2u + kBias - (unsigned)(j & 3) * 1024u;
+    }
+#pragma unroll
+    for (int j = 0; j < TJ; j++) {
+        const int r = wave * (8 * TJ) + j * 8 + (lane >> 3);
+        const int c = (lane & 7) ^ ((r >> 1) & 7);
+        const int wr = min(n0 + r, g.n - 1);
+        w_off[j] = ((unsigned)wr * (unsigned)g.ldw + (unsigned)(c * 8)) * 2u + kBias - (unsigned)(j & 3) * 1024u;
+    }
+    const int nslab = (g.k + BK - 1) / BK;
+    const unsigned a_lds = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)wave * (8 * TI * BK * 2));
+    const unsigned w_lds = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)(TBM * BK * 2) + (unsigned)wave * (8 * TJ * BK * 2));
+    // the i-th (i < NL) load of this wave's part of slab s into stage st: A rows, then W rows; within an
+    // operand in order, the first of every four sets M0 for the rest. Slabs past the end re-fetch the
+    // last one into a stage nobody reads any more.
+    auto fetch_one = [&](int s, int st, int i) __attribute__((always_inline)) {
+        const unsigned uo = (unsigned)(s < nslab ? s : nslab - 1) * (BK * 2u);
+        const bool is_w = i >= TI;
+        const int j = is_w ? i - TI : i;
+        if ((j & 3) == 0) lds_dma_base((is_w ? w_lds : a_lds) + (unsigned)(st * STAGE + (j >> 2) * 4096));
+        const u32x4& rsrc = is_w ? w_rsrc : a_rsrc;
+        const unsigned off = is_w ? w_off[is_w ? j : 0] : a_off[is_w ? 0 : j];
+        if ((j & 3) == 0) load_to_lds_16_at<0>(rsrc, off, uo);
+        if ((j & 3) == 1) load_to_lds_16_at<1024>(rsrc, off, uo);
+        if ((j & 3) == 2) load_to_lds_16_at<2048>(rsrc, off, uo);
+        if ((j & 3) == 3) load_to_lds_16_at<3072>(rsrc, off, uo);
+    };
+
+    f32x4 acc[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < TJ; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    typedef const __attribute__((address_space(3))) unsigned char* lds_byte_t;
+    typedef const __attribute__((address_space(3))) u32x4* lds_u32x4_t;
+    const lds_byte_t lds_base = (lds_byte_t)smem;
+    const int sw = (c16 >> 1) & 7;
+    lds_byte_t fa[ST][2], fw[ST][2]; // [stage][ks]: row (.. + c16), logical chunk 4 ks + q4 at c ^ ((row >> 1) & 7)
+#pragma unroll
+    for (int st = 0; st < ST; st++)
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+            const int pos = ((4 * ks + q4) ^ sw) * 16;
+            fa[st][ks] = lds_base + (st * STAGE + (wm * (16 * TI) + c16) * (BK * 2) + pos);
+            fw[st][ks] = lds_base + (st * STAGE + TBM * BK * 2 + (wn * (16 * TJ) + c16) * (BK * 2) + pos);
+        }
+    struct Frag { u32x4 a[TI], w[TJ]; };
+    auto read_one = [&](Frag& f, int st, int ks, int r) __attribute__((always_inline)) {
+        if (r < TI) f.a[r] = *(lds_u32x4_t)(fa[st][ks] + r * 16 * (BK * 2));
+        else f.w[r - TI] = *(lds_u32x4_t)(fw[st][ks] + (r - TI) * 16 * (BK * 2));
+    };
+    Frag f0, f1;
+    // one step of slab s (in stage S0): FIRST = the MFMAs on its k 0..31
+    auto step = [&](auto first_c, auto st_c, Frag& cur, Frag& nxt, int s) __attribute__((always_inline)) {
+        constexpr bool FIRST = decltype(first_c)::value;
+        if constexpr (RAG) {
+            // the last slab of a k that is not a multiple of 64: what lies past k in a row (the next
+            // row, or what the descriptor's bound made of it) must not count
+            if (s == nslab - 1) {
+                const bool keep = s * BK + (FIRST ? 0 : 32) + 8 * q4 < g.k;
+#pragma unroll
+                for (int i = 0; i < TI; i++) cur.a[i] = keep ? cur.a[i] : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int j = 0; j < TJ; j++) cur.w[j] = keep ? cur.w[j] : u32x4{0u, 0u, 0u, 0u};
+            }
+        }
+        constexpr int S0 = decltype(st_c)::value;
+        constexpr int SN = (S0 + 1) % ST;           // stage of slab s + 1
+        constexpr int SP = (S0 + ST - 1) % ST;      // of slab s - 1, which slab s - 1 + ST takes
+#pragma unroll
+        for (int t = 0; t < NM; t++) {
+            const int late = 2 * NM + t - (TB + 1); // loads of slab s - 1 + ST that are still to go out
+            if (FIRST && t <= TB && late % LS == 0 && late / LS >= IW && late / LS < NL) fetch_one(s - 1 + ST, SP, late / LS);
+            const int own = (FIRST ? t : NM + t) - (TB + 1);
+            if (own >= 0 && own % LS == 0 && own / LS < IW) fetch_one(s + ST, S0, own / LS);
+            if (t % RS == 0 && t / RS < NR) read_one(nxt, FIRST ? S0 : SN, FIRST ? 1 : 0, t / RS);
+            mfma16<F16>(cur.w[t % TJ], cur.a[t / TJ], acc[t / TJ][t % TJ]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (FIRST && t == TB) {
+                __builtin_amdgcn_s_waitcnt(vm_lgkm0((ST - 2) * NL));
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    auto slab = [&](auto st_c, int s) __attribute__((always_inline)) {
+        step(std::true_type{}, st_c, f0, f1, s);
+        step(std::false_type{}, st_c, f1, f0, s);
+    };
+
+#pragma unroll
+    for (int st = 0; st < ST; st++)
+#pragma unroll
+        for (int i = 0; i < (st < ST - 1 ? NL : IW); i++) fetch_one(st, st, i); // (the rest of the last one goes out in slab 0)
+    __builtin_amdgcn_s_waitcnt(vm_only((ST - 2) * NL + IW)); // slab 0 has landed
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < NR; r++) read_one(f0, 0, 0, r);
+    int s = 0;
+    for (; s + ST <= nslab; s += ST) {
+        slab(std::integral_constant<int, 0>{}, s);
+        slab(std::integral_constant<int, 1>{}, s + 1);
+        if constexpr (ST > 2) slab(std::integral_constant<int, 2 % ST>{}, s + 2);
+        if constexpr (ST > 3) slab(std::integral_constant<int, 3 % ST>{}, s + 3);
+        static_assert(ST >= 2 && ST <= 4, "two to four stages");
+        mfma16_drain(); // whatever follows the loop body may read the accumulators
+    }
+    if (s < nslab) { slab(std::integral_constant<int, 0>{}, s); mfma16_drain(); }
+    if constexpr (ST > 2) if (s + 1 < nslab) { slab(std::integral_constant<int, 1>{}, s + 1); mfma16_drain(); }
+    if constexpr (ST > 3) if (s + 2 < nslab) { slab(std::integral_constant<int, 2 % ST>{}, s + 2); mfma16_drain(); }
+    __builtin_amdgcn_s_waitcnt(0x0F70); // this wave's direct loads (re-fetches past the end) have landed
+    __syncthreads();                    // and everybody's: the stages are idle
+    static_assert(4 * rows_wave_bytes<TC, TJ>() <= ST * STAGE, "the epilogue's rows fit the stages");
+    store_rows_lds<F16, TC, TI, TJ>(g, cp, acc, lds0 + (unsigned)(wave * rows_wave_bytes<TC, TJ>()), m0 + wm * (16 * TI), n0 + wn * (16 * TJ), lane);
 }
 
 // Adds the parts of the k-split tiles in part order and writes C. A workgroup takes the 32 x
@@ -812,69 +897,94 @@ __global__ void __launch_bounds__(256) gemm_round_kernel(const float* a, int64_t
 // schedule above 1047-1248; four waves with the simple loop of the eight-wave build 960-1120.
 constexpr int DMA_WM = 4, DMA_WN = 2;
 
-static int g_gemm_build = 1; // 256-tiles of 16-bit activations: 1 = four-wave build (default), 0 = eight-wave build (measurement knob)
+static int g_gemm_build = 1; // 256-tiles: 1 = four-wave build (default), 0 = eight-wave build (measurement knob)
 
-constexpr size_t kSmallLdsBytes = 2 * (size_t)(2 * 128 * BK * 2); // two stages of a 128-tile
+// The tiles gemm_pipe_kernel is built for: (32 ti) x (32 tj) with st slabs in LDS, what one slab of
+// it takes when weights come from memory (us, every CU busy) and what a tile costs beside its slabs.
+// A slab's time is close to its bytes (A and W rows of 128 bytes) at 55-60 GB/s: a CU has at most
+// 32 KB of loads in flight, in order, and memory answers after 600 ns (350 ns from the last-level
+// cache, 190 ns from L2: 93 and 173 GB/s). So a tile's bytes per FLOP decide, and they fall with its
+// size, until there are fewer tiles than CUs.
+struct PipeShape { int ti, tj, st; float slab_us, fix_us; };
+constexpr PipeShape kPipe[] = {
+    {2, 2, 4, 0.30f, 4.0f}, {2, 3, 4, 0.31f, 4.0f}, {4, 2, 4, 0.385f, 4.5f}, {4, 3, 4, 0.446f, 4.5f}, {4, 4, 4, 0.54f, 5.0f},
+    {4, 5, 4, 0.66f, 5.0f}, {4, 6, 3, 0.74f, 5.5f}, {6, 6, 3, 0.83f, 6.0f}, {8, 5, 3, 0.88f, 6.5f},
+};
+constexpr int kPipeShapes = (int)(sizeof(kPipe) / sizeof(kPipe[0]));
+constexpr int kRingShape = -1;
+// The same for the 256-tiles of gemm_ring_kernel; a last round split along k also pays for its
+// partial tiles' way through memory and for the merge.
+constexpr float kRingSlabUs = 1.28f, kRingFixUs = 8.0f, kRingSplitUs = 28.0f;
 
-template <typename TA, bool F16, typename TC>
-static hipError_t launch_one(const GemmArgs& g0, hipStream_t stream) {
-    GemmArgs g = g0;
-    const int64_t tiles256 = (int64_t)((g.m + 255) / 256) * ((g.n + 255) / 256) * g.groups;
-    if constexpr (!std::is_same<TA, float>::value) {
-        // fewer 256-tiles than five eighths of the CUs: 128-tiles, two workgroups per CU
-        if (g.k % BK == 0 && tiles256 < 160) {
-            g.tiles_n = (g.n + 127) / 128;
-            const int64_t nwg = (int64_t)((g.m + 127) / 128) * g.tiles_n * g.groups;
-            if (nwg <= 0 || nwg > 0x7fffffff) return hipErrorInvalidValue;
-            gemm_dma_kernel<F16, TC, 2, 2, 128><<<dim3((unsigned)nwg), dim3(256), kSmallLdsBytes, stream>>>(g);
-            return hipGetLastError();
-        }
-    }
-    g.tiles_n = (g.n + BN - 1) / BN;
-    const int64_t nwg = tiles256;
+template <bool F16, typename TC, int I, bool RAG>
+static const void* pipe_entry() {
+    return reinterpret_cast<const void*>(&gemm_pipe_kernel<F16, TC, kPipe[I].ti, kPipe[I].tj, kPipe[I].st, RAG>);
+}
+
+template <bool F16, typename TC, bool RAG>
+static hipError_t launch_pipe(GemmArgs g, hipStream_t stream) {
+    const PipeShape& p = kPipe[g.shape];
+    g.tiles_n = (g.n + 32 * p.tj - 1) / (32 * p.tj);
+    const int64_t nwg = (int64_t)((g.m + 32 * p.ti - 1) / (32 * p.ti)) * g.tiles_n * g.groups;
     if (nwg <= 0 || nwg > 0x7fffffff) return hipErrorInvalidValue;
-    if constexpr (!std::is_same<TA, float>::value) {
-        if (g_gemm_build == 1 && g.k % BK == 0) {
-            // one launch: (splits > 1) the tiles of the last round in parts, the whole tiles behind them; then the merge
-            const int tail = g0.splits > 1 ? g0.tile_base : 0; // the planner leaves the tail size in tile_base
-            if (tail < 0 || tail > nwg || g0.splits > kMaxKSplits || (tail > 0 && g0.part == nullptr)) return hipErrorInvalidValue;
-            const int64_t whole = nwg - tail;
-            g.tile_base = (int32_t)whole;
-            g.splits = tail > 0 ? g0.splits : 1;
-            g.part_wgs = tail > 0 ? (int32_t)(((int64_t)tail * g0.splits + 7) & ~(int64_t)7) : 0;
-            if (whole + g.part_wgs > 0x7fffffff) return hipErrorInvalidValue;
-            gemm_ring_kernel<F16, TC><<<dim3((unsigned)(whole + g.part_wgs)), dim3(256), kRingLdsBytes, stream>>>(g);
-            if (tail > 0) {
-                hipError_t e = hipGetLastError();
-                if (e != hipSuccess) return e;
-                gemm_merge_kernel<F16, TC><<<dim3((unsigned)tail * 16u), dim3(256), 0, stream>>>(g);
-            }
-            return hipGetLastError();
-        }
-        if (g.k % BK == 0) { // whole slabs of 16-bit activations: the direct-to-LDS build
-            gemm_dma_kernel<F16, TC, DMA_WM, DMA_WN, 256><<<dim3((unsigned)nwg), dim3(DMA_WM * DMA_WN * 64), kDmaLdsBytes, stream>>>(g);
-            return hipGetLastError();
-        }
+    const dim3 grid((unsigned)nwg), block(256);
+    const size_t lds = pipe_lds_bytes(p.ti, p.tj, p.st);
+    switch (g.shape) {
+#define ZD_PIPE(I) \
+    case I: gemm_pipe_kernel<F16, TC, kPipe[I].ti, kPipe[I].tj, kPipe[I].st, RAG><<<grid, block, lds, stream>>>(g); break;
+    ZD_PIPE(0) ZD_PIPE(1) ZD_PIPE(2) ZD_PIPE(3) ZD_PIPE(4) ZD_PIPE(5) ZD_PIPE(6) ZD_PIPE(7) ZD_PIPE(8)
+#undef ZD_PIPE
+    default: return hipErrorInvalidValue;
     }
-    gemm_kernel<TA, F16, TC><<<dim3((unsigned)nwg), dim3(NT), kLdsBytes, stream>>>(g);
+    static_assert(kPipeShapes == 9, "one case per shape");
     return hipGetLastError();
 }
 
-template <typename TA, bool F16, typename TC>
-static hipError_t raise_lds() {
-    if constexpr (!std::is_same<TA, float>::value) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dma_kernel<F16, TC, DMA_WM, DMA_WN, 256>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDmaLdsBytes);
-        if (e != hipSuccess) return e;
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dma_kernel<F16, TC, 2, 2, 128>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLdsBytes);
-        if (e != hipSuccess) return e;
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ring_kernel<F16, TC>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRingLdsBytes);
-        if (e != hipSuccess) return e;
+template <bool F16, typename TC>
+static hipError_t launch_one(const GemmArgs& g0, hipStream_t stream) {
+    GemmArgs g = g0;
+    if (g.k % BK != 0) return launch_pipe<F16, TC, true>(g, stream);
+    if (g.shape != kRingShape) return launch_pipe<F16, TC, false>(g, stream);
+    g.tiles_n = (g.n + BN - 1) / BN;
+    const int64_t nwg = (int64_t)((g.m + BM - 1) / BM) * g.tiles_n * g.groups;
+    if (nwg <= 0 || nwg > 0x7fffffff) return hipErrorInvalidValue;
+    if (g_gemm_build != 1) {
+        gemm_dma_kernel<F16, TC, DMA_WM, DMA_WN><<<dim3((unsigned)nwg), dim3(DMA_WM * DMA_WN * 64), kDmaLdsBytes, stream>>>(g);
+        return hipGetLastError();
     }
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<TA, F16, TC>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
+    // one launch: (splits > 1) the tiles of the last round in parts, the whole tiles behind them; then the merge
+    const int tail = g0.splits > 1 ? g0.tile_base : 0; // the planner leaves the tail size in tile_base
+    if (tail < 0 || tail > nwg || g0.splits > kMaxKSplits || (tail > 0 && g0.part == nullptr)) return hipErrorInvalidValue;
+    const int64_t whole = nwg - tail;
+    g.tile_base = (int32_t)whole;
+    g.splits = tail > 0 ? g0.splits : 1;
+    g.part_wgs = tail > 0 ? (int32_t)(((int64_t)tail * g0.splits + 7) & ~(int64_t)7) : 0;
+    if (whole + g.part_wgs > 0x7fffffff) return hipErrorInvalidValue;
+    gemm_ring_kernel<F16, TC><<<dim3((unsigned)(whole + g.part_wgs)), dim3(256), kRingLdsBytes, stream>>>(g);
+    if (tail > 0) {
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        gemm_merge_kernel<F16, TC><<<dim3((unsigned)tail * 16u), dim3(256), 0, stream>>>(g);
+    }
+    return hipGetLastError();
+}
+
+template <bool F16, typename TC, int I>
+static hipError_t raise_pipe() {
+    const int lds = (int)pipe_lds_bytes(kPipe[I].ti, kPipe[I].tj, kPipe[I].st);
+    hipError_t e = hipFuncSetAttribute(pipe_entry<F16, TC, I, false>(), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e == hipSuccess) e = hipFuncSetAttribute(pipe_entry<F16, TC, I, true>(), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if constexpr (I + 1 < kPipeShapes) return e == hipSuccess ? raise_pipe<F16, TC, I + 1>() : e;
+    return e;
+}
+template <bool F16, typename TC>
+static hipError_t raise_lds() {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dma_kernel<F16, TC, DMA_WM, DMA_WN>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDmaLdsBytes);
+    if (e != hipSuccess) return e;
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ring_kernel<F16, TC>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRingLdsBytes);
+    return e == hipSuccess ? raise_pipe<F16, TC, 0>() : e;
 }
 
 } // namespace gemm
@@ -882,14 +992,14 @@ static hipError_t raise_lds() {
 int gemm_tile_rows() { return gemm::BM; }
 int gemm_tile_cols() { return gemm::BN; }
 
-// Only the four-wave build splits (16-bit activations, whole slabs, enough tiles for 256-tiles).
+// Only the four-wave build splits (whole slabs, enough tiles for 256-tiles).
 // A last round that fills at most half the CUs is cut along k so that it fills them: the round
 // then costs 1 / splits of a tile's time plus the partial tiles' trip through memory (256 KB
 // per part, which is why the number of parts is kept small and a fuller round is left whole).
-void gemm_tail_plan(const GemmArgs& g, int a_dtype, int cus, int* tail_tiles, int* splits) {
+void gemm_tail_plan(const GemmArgs& g, int cus, int* tail_tiles, int* splits) {
     *tail_tiles = 0;
     *splits = 1;
-    if (a_dtype == kF32 || gemm::g_gemm_build != 1 || g.k % gemm::BK != 0 || cus <= 0) return;
+    if (gemm::g_gemm_build != 1 || g.k % gemm::BK != 0 || cus <= 0) return;
     const int64_t tiles = (int64_t)((g.m + 255) / 256) * ((g.n + 255) / 256) * g.groups;
     if (tiles < 160 || tiles > 0x7fffffff) return;
     const int tail = (int)(tiles % cus);
@@ -906,20 +1016,50 @@ size_t gemm_part_bytes(int tail_tiles, int splits) {
     return (size_t)tail_tiles * splits * gemm::BM * gemm::BN * sizeof(float);
 }
 
-size_t gemm_round_bytes(const GemmArgs& g, int a_dtype) {
-    // Whole slabs (the direct-to-LDS builds need them) and at least one full tile each way. The
-    // pass moves 6 bytes per element of A through memory; measured at 4608 rows it pays at every
-    // shape tried (n = 9216: 0.268 -> 0.263 ms with f32 C; k = 12288, n = 3072: 0.384 -> 0.372;
-    // k = n = 3840: 0.225 -> 0.155, where it also opens the way to the k-split last round).
-    if (a_dtype != kF32 || g.k % gemm::BK != 0 || g.m < 256 || g.n < 256) return 0;
-    return (size_t)g.m * (size_t)g.k * 2;
+// The tile whose estimate (rounds of tiles over the CUs, each its slabs and its fixed part) is the
+// smallest. The estimates are within 10 % of what was measured for 77 to 4608 rows, 3072 and 3840
+// columns once and three times, k 3072 to 12288, and put the measured best first or within 3 % of it
+// (us, cold weights, bf16; the 128-tiles with one slab in flight that did all of these before, or the
+// 256-tiles, in brackets): 512 x 3072 x 3 x 3072 128 x 160 tiles 40 (51), 512 x 3072 x 3072 64 x 96
+// 20 (47), 1024 x 3072 x 3 x 3072 256 x 160 56 (86), 1024 x 3072 x 3072 128 x 96 28 (47), 77 x 3072 x
+// 3 x 3072 64 x 96 20 (48), 2816 x 12288 x 3072 192 x 192 164 (238), 2304 x 3840 x 3840 192 x 192 61 (95).
+int gemm_shape(const GemmArgs& g, int cus) {
+    using namespace gemm;
+    if (cus <= 0) return 0;
+    auto count = [&](int rows, int cols) { return (int64_t)((g.m + rows - 1) / rows) * ((g.n + cols - 1) / cols) * g.groups; };
+    const int nslab = (g.k + BK - 1) / BK;
+    const int64_t tiles256 = count(BM, BN);
+    int best = kRingShape;
+    float best_us = INFINITY;
+    if (g.k % BK == 0) {
+        if (g_gemm_build != 1 && tiles256 >= 160) return kRingShape;
+        int tail = 0, splits = 1;
+        gemm_tail_plan(g, cus, &tail, &splits);
+        const float round_us = (float)nslab * kRingSlabUs + kRingFixUs;
+        best_us = splits > 1 ? (float)(tiles256 / cus) * round_us + (float)((nslab + splits - 1) / splits) * kRingSlabUs + kRingSplitUs
+                             : (float)((tiles256 + cus - 1) / cus) * round_us;
+    }
+    for (int i = 0; i < kPipeShapes; i++) {
+        const int64_t rounds = (count(32 * kPipe[i].ti, 32 * kPipe[i].tj) + cus - 1) / cus;
+        const float us = (float)rounds * ((float)nslab * kPipe[i].slab_us + kPipe[i].fix_us);
+        if (us < best_us) { best_us = us; best = i; }
+    }
+    return best;
 }
+void gemm_shape_tile(int shape, int* rows, int* cols) {
+    *rows = shape < 0 ? gemm::BM : 32 * gemm::kPipe[shape].ti;
+    *cols = shape < 0 ? gemm::BN : 32 * gemm::kPipe[shape].tj;
+}
+
+// f32 activations are rounded to the weight's type once, ahead of the product.
+size_t gemm_round_bytes(const GemmArgs& g, int a_dtype) { return a_dtype == kF32 ? (size_t)g.m * (size_t)g.k * 2 : 0; }
 
 hipError_t launch_gemm(const GemmArgs& g0, int a_dtype, int w_dtype, int c_dtype, hipStream_t stream) {
     using namespace gemm;
     typedef unsigned short h16; // a 16-bit operand in the compute type (bf16 or f16 per the weight)
     GemmArgs g = g0;
-    if (a_dtype == kF32 && g.a16 != nullptr && gemm_round_bytes(g, a_dtype) != 0) {
+    if (a_dtype == kF32) {
+        if (g.a16 == nullptr) return hipErrorInvalidValue;
         const dim3 grid((unsigned)g.m, (unsigned)((g.k + 4095) / 4096));
         if (w_dtype == kF16)
             gemm_round_kernel<true><<<grid, dim3(256), 0, stream>>>(static_cast<const float*>(g.a), g.lda, static_cast<h16*>(g.a16), g.m, g.k);
@@ -929,18 +1069,15 @@ hipError_t launch_gemm(const GemmArgs& g0, int a_dtype, int w_dtype, int c_dtype
         if (e != hipSuccess) return e;
         g.a = g.a16;
         g.lda = g.k;
-        a_dtype = w_dtype;
+    } else if (a_dtype != w_dtype) {
+        return hipErrorInvalidValue;
     }
     if (w_dtype == kBF16) {
-        if (a_dtype == kF32 && c_dtype == kF32) return launch_one<float, false, float>(g, stream);
-        if (a_dtype == kF32 && c_dtype == kBF16) return launch_one<float, false, h16>(g, stream);
-        if (a_dtype == kBF16 && c_dtype == kF32) return launch_one<h16, false, float>(g, stream);
-        if (a_dtype == kBF16 && c_dtype == kBF16) return launch_one<h16, false, h16>(g, stream);
+        if (c_dtype == kF32) return launch_one<false, float>(g, stream);
+        if (c_dtype == kBF16) return launch_one<false, h16>(g, stream);
     } else if (w_dtype == kF16) {
-        if (a_dtype == kF32 && c_dtype == kF32) return launch_one<float, true, float>(g, stream);
-        if (a_dtype == kF32 && c_dtype == kF16) return launch_one<float, true, h16>(g, stream);
-        if (a_dtype == kF16 && c_dtype == kF32) return launch_one<h16, true, float>(g, stream);
-        if (a_dtype == kF16 && c_dtype == kF16) return launch_one<h16, true, h16>(g, stream);
+        if (c_dtype == kF32) return launch_one<true, float>(g, stream);
+        if (c_dtype == kF16) return launch_one<true, h16>(g, stream);
     }
     return hipErrorInvalidValue;
 }
@@ -951,14 +1088,10 @@ hipError_t gemm_setup() {
     using namespace gemm;
     typedef unsigned short h16;
     hipError_t e;
-    if ((e = raise_lds<float, false, float>()) != hipSuccess) return e;
-    if ((e = raise_lds<float, false, h16>()) != hipSuccess) return e;
-    if ((e = raise_lds<h16, false, float>()) != hipSuccess) return e;
-    if ((e = raise_lds<h16, false, h16>()) != hipSuccess) return e;
-    if ((e = raise_lds<float, true, float>()) != hipSuccess) return e;
-    if ((e = raise_lds<float, true, h16>()) != hipSuccess) return e;
-    if ((e = raise_lds<h16, true, float>()) != hipSuccess) return e;
-    if ((e = raise_lds<h16, true, h16>()) != hipSuccess) return e;
+    if ((e = raise_lds<false, float>()) != hipSuccess) return e;
+    if ((e = raise_lds<false, h16>()) != hipSuccess) return e;
+    if ((e = raise_lds<true, float>()) != hipSuccess) return e;
+    if ((e = raise_lds<true, h16>()) != hipSuccess) return e;
     return hipSuccess;
 }
 

@@ -13,7 +13,7 @@ struct GemmArgs {
     const void* w;   // weights, row-major [n][ldw]
     void* c;         // output, row-major [m][ldc]
     int32_t m, n, k;
-    int32_t pad0;
+    int32_t shape;   // which kernel and tile (gemm_shape)
     int64_t lda, ldw, ldc;
     int32_t tiles_n; // column tiles of one group (grid = tiles_m * tiles_n * groups)
     int32_t groups;  // 1..3 products sharing A and every dimension: group i > 0 uses w_more[i-1], c_more[i-1]
@@ -31,10 +31,14 @@ struct GemmArgs {
     int32_t part_wgs; // set by the launcher
     int32_t pad1;
     // f32 activations: room for A rounded to the weight's type, [m][k] 16-bit (gemm_round_bytes
-    // says how much; null: A is rounded block by block on its way into LDS instead)
+    // says how much)
     void* a16;
 };
 
+// Kernel and tile for this product on a device with `cus` compute units (GemmArgs::shape): -1 the
+// 256-tiles of gemm_ring_kernel, otherwise an entry of gemm_pipe_kernel's table of tiles.
+int gemm_shape(const GemmArgs& args, int cus);
+void gemm_shape_tile(int shape, int* rows, int* cols);
 int gemm_tile_rows();
 int gemm_tile_cols();
 // a_dtype: kF32 or the weight's type; w_dtype: kF16 or kBF16; c_dtype: kF32 or the weight's type.
@@ -43,10 +47,9 @@ hipError_t gemm_setup();
 // How launch_gemm would split the last round of this product on a device with `cus` compute
 // units: *tail_tiles tiles in *splits parts each (splits 1: no split), and the bytes of fp32
 // partial tiles that needs.
-void gemm_tail_plan(const GemmArgs& args, int a_dtype, int cus, int* tail_tiles, int* splits);
+void gemm_tail_plan(const GemmArgs& args, int cus, int* tail_tiles, int* splits);
 size_t gemm_part_bytes(int tail_tiles, int splits);
-// Bytes of scratch launch_gemm wants for rounding f32 activations once, ahead of the product
-// (0: not worth it or not possible for this shape).
+// Bytes of scratch launch_gemm needs for f32 activations rounded ahead of the product (0: none).
 size_t gemm_round_bytes(const GemmArgs& args, int a_dtype);
 void gemm_set_build(int build); // 256-tiles of 16-bit activations: 1 = four-wave build (default), 0 = eight-wave build
 
