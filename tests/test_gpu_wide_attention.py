@@ -44,6 +44,23 @@ def test_wide_head_matches_oracle_on_every_row(ctx, tokens):
     assert np.array_equal(got, again)
 
 
+# Numbers of key blocks that the number of ranges does not divide (the last range is shorter),
+# half a query tile left over, three to seven ranges, and both sides of the length
+# where two ranges a tile outgrow one round; rows of the first, a middle and the last tile.
+@pytest.mark.parametrize("tokens", [704, 1344, 1984, 3008, 8256, 16448])
+def test_wide_head_uneven_key_ranges_sampled_rows_and_rerun(ctx, tokens):
+    rng = np.random.default_rng(90 + tokens)
+    q, k, v = draw(rng, tokens)
+    cfg = host.Config(tokens, 1, 1, 512)
+    got = ctx.run(q, k, v, cfg).reshape(tokens, 1, 512)
+    again = ctx.run(q, k, v, cfg).reshape(tokens, 1, 512)
+    assert got.tobytes() == again.tobytes()
+    rows = [0, 31, 127, tokens // 2, tokens - 65, tokens - 64, tokens - 1]
+    want = zo.attention_token_list(q, k, v, zo.Config(tokens, 1, 1, 512), rows)
+    refimpl.check_close(got[rows], want.reshape(len(rows), 1, 512), f"wide head, {tokens} tokens")
+    assert (np.abs(got).max(axis=(1, 2)) > 0).all()
+
+
 def test_wide_head_reference_case_sampled_rows_and_rerun(ctx):
     # metal/mattn_test.zig:138-230
     tokens = 6208

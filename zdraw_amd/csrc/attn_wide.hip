@@ -19,9 +19,9 @@
 //     registers where they are (given the builtin the compiler moves such tuples about and
 //     spills); nothing else may touch those registers between such an MFMA and the wait that
 //     ends the step (zdraw_amd.build.tied_mfma_hazards checks the compiled code);
-//   * a query tile's keys are split over at least two workgroups (256 workgroups at 16384
-//     tokens: one per CU), each leaving its unnormalised O and its (reference point, row sum)
-//     in scratch; wide_merge_kernel combines the ranges in range order;
+//   * a query tile's keys are split over up to eight workgroups (two at 16384 tokens: 256
+//     workgroups, one per CU; wide_splits), each leaving its unnormalised O and its (reference
+//     point, row sum) in scratch; wide_merge_kernel combines the ranges in range order;
 //   * per 32-key block a wave forms S^T = K Q^T (32 MFMAs; scores transposed, so a lane owns
 //     one query and P^T is the next MFMA's B operand without an LDS round trip) with the online
 //     softmax of the previous block in their shadow, then adds V^T P^T to O^T (32 MFMAs);
@@ -34,6 +34,8 @@
 //     fragments are in registers: the V fragments of the product are read under the rest;
 //   * fixed block order and fixed summation order: bit-identical from run to run.
 #include "attn_device.hpp"
+
+#include <cmath>
 
 namespace zdraw {
 
@@ -125,12 +127,18 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
     const int wave = tid >> 6;
     const int l32 = lane & 31;
     const int h = lane >> 5;
-    // workgroup = (query tile, key range); a.splits is a power of two
+    // workgroup = (key range, query tile), range-major, and each XCD takes one contiguous run of
+    // that order (workgroups go to the XCDs in turn): the workgroups behind one L2 walk the same
+    // range, so a K/V block comes in once per XCD, not once per range as well.
     const int nsp = a.splits > 1 ? a.splits : 1;
-    const int lg = __builtin_ctz((unsigned)nsp); // (shifts: an integer division would run on the vector unit)
-    const int part = (int)blockIdx.x & (nsp - 1);
-    const int q0 = ((int)blockIdx.x >> lg) * BQ + 32 * wave;        // this wave's query rows
-    const int per = (a.tokens / KB + nsp - 1) >> lg;
+    const int tiles = (int)gridDim.x / nsp;
+    const int xcd = (int)blockIdx.x & 7, xrem = (int)gridDim.x & 7;
+    const int logical = ((int)blockIdx.x >> 3) + xcd * ((int)gridDim.x >> 3) + min(xcd, xrem);
+    // (uniform, but the divisions run on the vector unit)
+    const int part = __builtin_amdgcn_readfirstlane(logical / tiles);
+    const int tile = logical - part * tiles;
+    const int q0 = tile * BQ + 32 * wave;                           // this wave's query rows
+    const int per = __builtin_amdgcn_readfirstlane((a.tokens / KB + nsp - 1) / nsp);
     const int blk0 = part * per;                                    // this range's first key block
     const int nblk = max(min(a.tokens / KB - blk0, per), 1);        // and how many it has (the host gives every range some)
 
@@ -333,7 +341,7 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
     // ---- epilogue: O = O^T / l, or the range's share as it stands
     const float l_tot = pair_sum(l_run);
     // a row sum past 2^kHeadroom (or not a number): some score left the reach of the fixed reference
-    if (__any(!(l_tot <= kRowSumLimit)) && lane == 0) a.redo[(int)blockIdx.x >> lg] = 1;
+    if (__any(!(l_tot <= kRowSumLimit)) && lane == 0) a.redo[tile] = 1;
     if (q0 + l32 >= a.tokens) return;
     if (nsp > 1) {
         float* op = a.part_o + ((int64_t)part * a.tokens + (q0 + l32)) * WD + 4 * h;
@@ -652,15 +660,31 @@ hipError_t launch_wide_round(const WidePrepArgs& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Key ranges per query tile (one workgroup each): doubled while the launch still fits the
-// device's CUs once and every range keeps at least eight key blocks. 16384 tokens are 128 tiles
-// of two ranges, one workgroup per CU; 4096 tokens (the mid-block at 512 px) 32 tiles of eight.
+// Key ranges per query tile (one workgroup each, of equal length but for the last, at least eight
+// blocks): the number whose estimate is the smallest. A full round over the CUs takes kFullUs per
+// block of a range (the power limit), a thinly filled one kThinUs (a wave's own chain), in between
+// in proportion; every range's share of O goes to memory and back once. The constants are a fit to
+// 1 to 8 ranges of 256 to 18432 tokens; the rule's pick is the measured best or within 4 % of it.
+// (A power of two that divides the blocks, which this was before, left 6208 tokens, 194 blocks, at
+// two ranges and 98 workgroups: call 163 us against 118 with four; 18432 tokens at one range:
+// 678 against 610 with three.)
 int wide_splits(int tokens, int cus) {
+    constexpr float kFullUs = 1.6f, kThinUs = 1.16f, kRoundUs = 4.0f, kMergeUs = 3.0f, kShareBytesPerUs = 2.0e6f;
+    if (cus <= 0) return 1;
     const int tiles = (tokens + wide::BQ - 1) / wide::BQ;
     const int nblk = tokens / wide::KB;
-    int s = 1;
-    while (s < wide::kMaxSplits && tiles * (s * 2) <= cus && nblk / (s * 2) >= 8 && nblk % (s * 2) == 0) s *= 2;
-    return s;
+    int best = 1;
+    float best_us = INFINITY;
+    for (int s = 1; s <= wide::kMaxSplits; s++) {
+        const int per = (nblk + s - 1) / s;
+        if (s > 1 && (per < 8 || (s - 1) * per >= nblk)) continue; // (no empty range)
+        const int rounds = tiles * s / cus, last = tiles * s % cus;
+        float us = (float)rounds * ((float)per * kFullUs + kRoundUs);
+        if (last) us += (float)per * fmaxf(kThinUs, kFullUs * (float)last / (float)cus) + kRoundUs;
+        if (s > 1) us += kMergeUs + (float)s * (float)tokens * (float)(wide::WD * sizeof(float)) / kShareBytesPerUs;
+        if (us < best_us) { best_us = us; best = s; }
+    }
+    return best;
 }
 size_t wide_part_bytes(int tokens, int splits) {
     return splits > 1 ? (size_t)splits * (size_t)tokens * (wide::WD + 2) * sizeof(float) : 0;
@@ -669,7 +693,8 @@ size_t wide_part_bytes(int tokens, int splits) {
 hipError_t launch_wide_attention(const WideArgs& a, hipStream_t stream) {
     if (a.tokens <= 0 || a.tokens % wide_block_rows() != 0) return hipErrorInvalidValue;
     const int nsp = a.splits > 1 ? a.splits : 1;
-    if (nsp > wide::kMaxSplits || (nsp & (nsp - 1)) != 0 || (a.tokens / wide::KB) % nsp != 0) return hipErrorInvalidValue;
+    const int nblk = a.tokens / wide::KB;
+    if (nsp > wide::kMaxSplits || (nsp - 1) * ((nblk + nsp - 1) / nsp) >= nblk) return hipErrorInvalidValue; // every range has a block
     if (nsp > 1 && (a.part_o == nullptr || a.part_ml == nullptr)) return hipErrorInvalidValue;
     const unsigned tiles = (unsigned)((a.tokens + wide::BQ - 1) / wide::BQ);
     if (a.redo == nullptr) return hipErrorInvalidValue;
@@ -679,9 +704,12 @@ hipError_t launch_wide_attention(const WideArgs& a, hipStream_t stream) {
     if (nsp > 1) {
         const int64_t threads = (int64_t)a.tokens * (wide::WD / 4);
         const dim3 mgrid((unsigned)((threads + 255) / 256));
-        if (nsp == 2) wide::wide_merge_kernel<2><<<mgrid, dim3(256), 0, stream>>>(a);
-        else if (nsp == 4) wide::wide_merge_kernel<4><<<mgrid, dim3(256), 0, stream>>>(a);
-        else wide::wide_merge_kernel<8><<<mgrid, dim3(256), 0, stream>>>(a);
+        switch (nsp) {
+#define ZD_MERGE(N) case N: wide::wide_merge_kernel<N><<<mgrid, dim3(256), 0, stream>>>(a); break;
+        ZD_MERGE(2) ZD_MERGE(3) ZD_MERGE(4) ZD_MERGE(5) ZD_MERGE(6) ZD_MERGE(7) ZD_MERGE(8)
+#undef ZD_MERGE
+        }
+        static_assert(wide::kMaxSplits == 8, "one case per number of ranges");
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     // flagged tiles (none on ordinary data) are formed again, over whatever the launches above left there

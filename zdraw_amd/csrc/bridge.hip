@@ -841,14 +841,15 @@ int enqueue_wide(Queue* queue, void* q, void* k, void* v, void* out, const Zdraw
     a.redo = static_cast<int*>(redo->ptr);
     a.splits = wide_splits(a.tokens, queue->dev->cus);
     if (a.splits > 1) {
-        // a short sequence runs as key ranges whose shares go through scratch slot 3
+        // key ranges leave their shares in scratch slot 3; without room for them the keys stay whole
         Buffer* part = queue_scratch(queue, 3, wide_part_bytes(a.tokens, a.splits));
         if (!part) {
-            set_err("scratch allocation failed");
-            return ZDRAW_HIP_ERR_HANDLE;
+            (void)hipGetLastError(); // or the next launch would report the failed allocation
+            a.splits = 1;
+        } else {
+            a.part_o = static_cast<float*>(part->ptr);
+            a.part_ml = a.part_o + (size_t)a.splits * (size_t)a.tokens * (size_t)wide_head_dim();
         }
-        a.part_o = static_cast<float*>(part->ptr);
-        a.part_ml = a.part_o + (size_t)a.splits * (size_t)a.tokens * (size_t)wide_head_dim();
     }
     TracePair tp{nullptr, nullptr};
     if (g_trace && hipEventCreate(&tp.a) == hipSuccess && hipEventCreate(&tp.b) == hipSuccess)
