@@ -776,6 +776,51 @@ def _plain_fused(ctx, q, k, v, *, valid=0, in_dtype, key_pad=None, knob=0):
     return out
 
 
+# Masked key lists: mask bytes of any non-zero value, segments whose mask starts off every alignment
+# (odd token counts), a block that the limit cuts, blocks without any admitted key at the start, in
+# the middle and at the end, more blocks than a workgroup has threads (16 384 keys), lists shorter
+# and longer than the 64 positions a wave holds at a time. Sampled rows against float64 on the
+# bf16-rounded operands; the bf16 attention bar.
+@pytest.mark.parametrize("tokens,valid,heads,bounded", [(33, 0, 2, True), (487, 470, 2, False), (2081, 0, 2, True), (2500, 2301, 1, False),
+                                                        (4133, 0, 1, True), (16419, 0, 1, True), (17001, 16990, 1, False)])
+def test_masked_key_lists_sampled_rows(ctx, tokens, valid, heads, bounded):
+    L = hip.lib()
+    rng = np.random.default_rng(tokens)
+    batch, shape = 2, (2, tokens, heads, 128)
+    scale = np.float32(0.35 if bounded else 1.0)
+    bits = [host.f32_to_bf16_bits(rng.standard_normal(shape, dtype=np.float32) * scale) for _ in range(3)]
+    q, k, v = (host.bf16_bits_to_f32(b).reshape(shape) for b in bits)
+    pad = (rng.integers(1, 256, (batch, tokens)) * (rng.random((batch, tokens)) < 0.02)).astype(np.uint8)
+    pad[0, : tokens // 5] = rng.integers(1, 256, tokens // 5)
+    pad[1, tokens // 2: tokens // 2 + tokens // 7] = 128
+    pad[1, tokens - tokens // 9:] = 1
+    pad[:, tokens // 3] = 0  # some key stays
+    bufs = [ctx.buffer(b) for b in bits] + [ctx.buffer(pad), ctx.buffer(nbytes=q.size * 4)]
+    p = hip.AttnParams(tokens, heads, heads, 128, 0, valid)
+    x = hip.AttnExt()
+    for s_ in (x.q_stride, x.k_stride, x.v_stride, x.out_stride):
+        s_[0], s_[1], s_[2] = tokens * heads * 128, heads * 128, 128
+    x.batch, x.in_dtype, x.out_dtype, x.qk_mode = batch, hip.BF16, hip.F32, hip.QK_NONE
+    x.score_bound, x.mask_batch_bytes = 40.0 if bounded else 0.0, tokens
+    ops = hip.QkOperands()
+    ops.key_pad = bufs[3].handle
+    rc = L.zdraw_hip_run_attention_fused(ctx.queue, bufs[0].handle, bufs[1].handle, bufs[2].handle, bufs[4].handle, C.byref(p), C.byref(x),
+                                         C.byref(ops))
+    assert rc == 0, hip.last_error()
+    got = bufs[4].read(np.float32, shape)
+    rows = sorted({0, 31, tokens // 2, tokens - 2, tokens - 1})
+    for seg in range(batch):
+        keep = pad[seg] == 0
+        keep[valid or tokens:] = False
+        for head in range(heads):
+            s = q[seg, rows, head].astype(np.float64) @ k[seg, keep, head].astype(np.float64).T / np.sqrt(128.0)
+            w = np.exp(s - s.max(axis=1, keepdims=True))
+            want = (w / w.sum(axis=1, keepdims=True)) @ v[seg, keep, head].astype(np.float64)
+            refimpl.check_close(got[seg, rows, head], want.astype(np.float32), f"segment {seg}, head {head}")
+    for b in bufs:
+        b.release()
+
+
 # first, a middle and the last key block; rising, so that the reference moves at each of them
 PLANT_CASES = [
     # name, tokens, heads, in_dtype, valid, planted (key, nats), whole tiles only (knob 2)

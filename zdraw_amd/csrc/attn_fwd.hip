@@ -149,7 +149,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     bf16_t* const Vs = Ks + NST * KSTAGE;
     unsigned short* const blocks = reinterpret_cast<unsigned short*>(Vs + NST * VSTAGE);
     unsigned* const bmask = reinterpret_cast<unsigned*>(blocks + MAX_BLOCKS); // bit j: key j of the block is excluded
-    __shared__ int s_nblocks;
+    __shared__ int s_count[MASKED ? MAX_BLOCKS / 64 : 1]; // admitted blocks of every 64
 
     unsigned long long clk_c0 = 0, clk_r0 = 0;
     if (a.clock_probe) {
@@ -203,31 +203,53 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     const unsigned char* const kp = a.key_pad ? a.key_pad + (int64_t)seg * a.mask_bs : nullptr;
     int nblk = nb_all;
     if constexpr (MASKED) {
-        // exclusion mask of every key block (padding mask, key limit, tail), two blocks per wave pass
-        for (int t2 = wave; 2 * t2 < nb_all; t2 += NW) {
-            const int key = t2 * 64 + lane;
-            const bool bad = key >= a.key_limit || (kp != nullptr && kp[key < a.key_limit ? key : 0] != 0);
-            const unsigned long long m = __ballot(bad);
-            if (lane == 0) {
-                bmask[2 * t2] = (unsigned)m;
-                if (2 * t2 + 1 < MAX_BLOCKS) bmask[2 * t2 + 1] = (unsigned)(m >> 32);
+        // A thread forms the exclusion mask (padding mask, key limit, tail) of one block in NT: all
+        // of a workgroup's mask bytes are one memory round trip. (A byte per lane and a ballot per
+        // two blocks, as this was at first, took a round trip for every 16 blocks, ahead of the
+        // first K/V fetch: the same call 263 -> 252 us, two segments of 8704 tokens 1579 -> 1476.)
+#pragma clang loop unroll(disable)
+        for (int t0 = wave * 64; t0 < nb_all; t0 += NT) {
+            const int t = t0 + lane;
+            const int left = a.key_limit - t * KB; // keys of the block below the limit, if not whole
+            unsigned mask = left >= KB ? 0u : left <= 0 ? 0xffffffffu : 0xffffffffu << left;
+            if (kp != nullptr) {
+                const unsigned char* const src = kp + (int64_t)t * KB;
+                if (left >= KB) {
+                    u32x4 w[2];
+                    __builtin_memcpy(w, src, KB); // (no alignment is promised)
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        const unsigned x = w[i >> 2][i & 3];
+                        const unsigned z = ((((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u) >> 7; // bits 0, 8, 16, 24: the byte is not zero
+                        mask |= ((z | (z >> 7) | (z >> 14) | (z >> 21)) & 15u) << (4 * i);
+                    }
+                } else if (left > 0) { // the block that holds the limit: nothing past it is read
+                    unsigned char byte[KB];
+#pragma unroll
+                    for (int i = 0; i < KB; i++) byte[i] = src[min(i, left - 1)];
+#pragma unroll
+                    for (int i = 0; i < KB; i++) mask |= byte[i] != 0 ? 1u << i : 0u;
+                }
             }
+            if (t < nb_all) bmask[t] = mask;
+            const int admitted = __popcll(__ballot(mask != 0xffffffffu)); // (past nb_all: nothing is)
+            if (lane == 0) s_count[t0 / 64] = admitted;
         }
         __syncthreads();
         if (kp) { // compact the blocks that admit at least one key
-            if (wave == 0) {
-                int count = 0;
-                for (int base = 0; base < nb_all; base += 64) {
-                    const int t = base + lane;
-                    const bool act = t < nb_all && bmask[t < nb_all ? t : 0] != 0xffffffffu;
-                    const unsigned long long m = __ballot(act);
-                    if (act) blocks[count + __popcll(m & ((1ull << lane) - 1ull))] = (unsigned short)t;
-                    count += __popcll(m);
-                }
-                if (lane == 0) s_nblocks = count;
+#pragma clang loop unroll(disable)
+            for (int t0 = wave * 64; t0 < nb_all; t0 += NT) {
+                const int t = t0 + lane;
+                int at = 0;
+                for (int g = 0; g < t0 / 64; g++) at += s_count[g];
+                const bool act = t < nb_all && bmask[t < nb_all ? t : 0] != 0xffffffffu;
+                const unsigned long long m = __ballot(act);
+                if (act) blocks[at + __popcll(m & ((1ull << lane) - 1ull))] = (unsigned short)t;
             }
+            nblk = 0;
+            for (int g = 0; g < (nb_all + 63) / 64; g++) nblk += s_count[g];
+            nblk = __builtin_amdgcn_readfirstlane(nblk);
             __syncthreads();
-            nblk = __builtin_amdgcn_readfirstlane(s_nblocks);
         }
     }
     // a key-split workgroup walks positions [i0, i0 + nblk) of the list
@@ -237,8 +259,24 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
         i0 = split * per;
         nblk = max(min(nblk - i0, per), 0);
     }
-    // wave-uniform by construction; readfirstlane lets the compiler keep it in scalar registers
-    auto block_of = [&](int i) -> int { return (MASKED && kp) ? __builtin_amdgcn_readfirstlane((int)blocks[i + i0]) : i + i0; };
+    // Masked builds: lane i of two registers holds the block and the exclusion mask of list position
+    // list_base + i, and a step takes its own by v_readlane. (Read from LDS in the step, as they
+    // were at first, each made the wave wait for every fragment read in flight: a Klein 1024^2
+    // call with masked text keys 278 -> 263 us.) Reloaded every 32 positions or so; a trip of the
+    // main loop and the remainder behind it look at most 51 positions past list_base.
+    int list_base = 0;
+    unsigned list_blk = 0, list_mask = 0;
+    auto list_load = [&](int base) __attribute__((always_inline)) {
+        list_base = base;
+        const int i = min(base + lane, nblk - 1); // positions past the end repeat the last one
+        list_blk = kp ? (unsigned)blocks[i + i0] : (unsigned)(i + i0);
+        list_mask = bmask[list_blk];
+    };
+    if constexpr (MASKED) {
+        if (nblk > 0) list_load(0);
+    }
+    // (i from list_base to list_base + 63)
+    auto block_of = [&](int i) -> int { return MASKED ? __builtin_amdgcn_readlane((int)list_blk, i - list_base) : i + i0; };
 
     // ---- Q rows -> B-operand registers: qf[qi][s], lane: query 32*qi + l32, dims 16s + 8h .. +7
     // The workgroup's query rows are prepared in the layout that coalesces: 16 lanes per
@@ -582,11 +620,6 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
         }
     };
 
-    unsigned badm_cur = 0; // exclusion mask of the block whose scores the next step exponentiates
-    if constexpr (MASKED) {
-        if (nblk > 0) badm_cur = bmask[block_of(0)];
-    }
-
     // One pipeline step for list position b: consumes S(b) and P(b-1),
     // produces S(b+1) and P(b). The three streams are independent, so the
     // step is laid out by hand as 16 slots, each fenced from the next:
@@ -646,7 +679,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
 
         if constexpr (MASKED) {
             // excluded keys (padding mask, key limit, tail) -> -inf; bit kk of badm = key kk of the block
-            const unsigned badm = __builtin_amdgcn_readfirstlane(badm_cur); // fetched from LDS during the previous step
+            const unsigned badm = (unsigned)__builtin_amdgcn_readlane((int)list_mask, b - list_base);
             if (badm != 0u) { // wave-uniform: most blocks exclude nothing
 #pragma unroll
                 for (int qi = 0; qi < QB; qi++)
@@ -755,9 +788,6 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             // ring: block b+AHEAD (in this register set since two steps ago) goes to its stage,
             // whose previous tenant's last reader (V, NST-AHEAD-1 steps back) is at least one
             // barrier behind; then the set starts loading block b+AHEAD+2
-            if constexpr (MASKED) {
-                if (g == 10) badm_cur = bmask[block_of(b + 1 < nblk ? b + 1 : nblk - 1)];
-            }
             if constexpr (DMA) {
                 if (g == STORE_SLOT) dma_fetch(b + AHEAD, stage_of(AHEAD));
             } else {
@@ -950,6 +980,9 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
         int b = 0;
         // (builds that prepare K inside the block load carry too much state for a full turn)
         for (; KMODE == kQkNone && b + NST <= nblk; b += NST) {
+            if constexpr (MASKED) {
+                if (b - list_base >= 32) list_load(b);
+            }
             step(std::integral_constant<int, 0>{}, b, sets[0], NST != 8, s_a, s_b, p_a, p_b);
             step(std::integral_constant<int, 1>{}, b + 1, sets[1], true, s_b, s_a, p_b, p_a);
             step(std::integral_constant<int, 2>{}, b + 2, sets[0], NST != 8, s_a, s_b, p_a, p_b);
@@ -962,6 +995,9 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             }
         }
         for (; b + 1 < nblk; b += 2) {
+            if constexpr (MASKED && KMODE != kQkNone) {
+                if (b - list_base >= 32) list_load(b);
+            }
             step(Dyn{}, b, sets[0], NST != 8, s_a, s_b, p_a, p_b);
             step(Dyn{}, b + 1, sets[1], true, s_b, s_a, p_b, p_a);
         }
