@@ -821,6 +821,64 @@ def test_masked_key_lists_sampled_rows(ctx, tokens, valid, heads, bounded):
         b.release()
 
 
+# Launches of few tiles run 128 query rows per workgroup and two groups of waves over half of the
+# keys each: one key block (the second group has none), an odd number of blocks (an idle last step),
+# fewer blocks than ring stages and a whole turn of the ring more, half a tile left over, a half
+# whose keys are all masked, parts of a split tile on top (two heads from 640 tokens on); both
+# softmax forms, both score types, every type of output. Sampled rows against float64 on the
+# operands as given; the bf16 attention bar.
+@pytest.mark.parametrize("bounded", [True, False])
+@pytest.mark.parametrize("tokens,heads,dead,in_dtype,out_dtype", [
+    (1, 1, None, hip.BF16, hip.F32), (32, 2, None, hip.BF16, hip.BF16), (33, 3, None, hip.BF16, hip.F16), (96, 2, None, hip.F16, hip.F32),
+    (128, 24, None, hip.BF16, hip.BF16), (129, 5, (0, 64), hip.BF16, hip.F32), (160, 2, (64, 159), hip.F16, hip.F16),
+    (257, 3, (0, 257), hip.BF16, hip.F32), (288, 30, None, hip.BF16, hip.BF16), (320, 2, (0, 200), hip.BF16, hip.BF16),
+    (1024, 2, None, hip.BF16, hip.F32), (1501, 2, (700, 1500), hip.BF16, hip.BF16)])
+def test_two_key_groups_sampled_rows(ctx, tokens, heads, dead, in_dtype, out_dtype, bounded):
+    L = hip.lib()
+    rng = np.random.default_rng(tokens + heads)
+    shape = (tokens, heads, 128)
+    scale = np.float32(0.35 if bounded else 1.0)
+    draws = [rng.standard_normal(shape, dtype=np.float32) * scale for _ in range(3)]
+    if in_dtype == hip.BF16:
+        raw = [host.f32_to_bf16_bits(a) for a in draws]
+        q, k, v = (host.bf16_bits_to_f32(b).reshape(shape) for b in raw)
+    else:
+        raw = [a.astype(np.float16) for a in draws]
+        q, k, v = (b.astype(np.float32) for b in raw)
+    keep = np.ones(tokens, bool)
+    ops = hip.QkOperands()
+    bufs = [ctx.buffer(b) for b in raw] + [ctx.buffer(nbytes=q.size * (4 if out_dtype == hip.F32 else 2))]
+    if dead:
+        keep[dead[0]:dead[1]] = False
+        bufs.append(ctx.buffer((~keep).astype(np.uint8)))
+        ops.key_pad = bufs[4].handle
+    p = hip.AttnParams(tokens, heads, heads, 128, 0, 0)
+    x = hip.AttnExt()
+    for s_ in (x.q_stride, x.k_stride, x.v_stride, x.out_stride):
+        s_[0], s_[1], s_[2] = 0, heads * 128, 128
+    x.batch, x.in_dtype, x.out_dtype, x.qk_mode, x.score_bound = 1, in_dtype, out_dtype, hip.QK_NONE, 40.0 if bounded else 0.0
+    outs = []
+    for _ in range(2):
+        rc = L.zdraw_hip_run_attention_fused(ctx.queue, bufs[0].handle, bufs[1].handle, bufs[2].handle, bufs[3].handle, C.byref(p), C.byref(x),
+                                             C.byref(ops))
+        assert rc == 0, hip.last_error()
+        if out_dtype == hip.BF16:
+            outs.append(host.bf16_bits_to_f32(bufs[3].read(np.uint16, shape)).reshape(shape))
+        else:
+            outs.append(bufs[3].read(np.float32 if out_dtype == hip.F32 else np.float16, shape).astype(np.float32))
+    assert np.array_equal(outs[0], outs[1])
+    rows = sorted({0, tokens // 2, max(tokens - 2, 0), tokens - 1, min(31, tokens - 1), min(127, tokens - 1)})
+    for head in range(heads):
+        want = np.zeros((len(rows), 128))
+        if keep.any():
+            s = q[rows, head].astype(np.float64) @ k[keep, head].astype(np.float64).T / np.sqrt(128.0)
+            w = np.exp(s - s.max(axis=1, keepdims=True))
+            want = (w / w.sum(axis=1, keepdims=True)) @ v[keep, head].astype(np.float64)
+        refimpl.check_close(outs[0][rows, head], want.astype(np.float32), f"head {head}")
+    for b in bufs:
+        b.release()
+
+
 # first, a middle and the last key block; rising, so that the reference moves at each of them
 PLANT_CASES = [
     # name, tokens, heads, in_dtype, valid, planted (key, nats), whole tiles only (knob 2)

@@ -33,6 +33,8 @@
 //     atomics, so the output is bit-identical from run to run.
 #include "attn_device.hpp"
 
+#include <cmath>
+
 namespace zdraw {
 
 namespace fwd {
@@ -107,21 +109,27 @@ __device__ __forceinline__ void pin(T& v) {
 // v_mfma_f32_32x32x16_f16: three more mantissa bits on every score at the same MFMA rate. P and
 // V stay bf16 (P reaches 2^64 in the bounded form). Only for the direct-to-LDS build, where the
 // operands' bits go from memory to the MFMA untouched.
-template <typename TIn, int KMODE, bool MASKED, bool BOUNDED, int QB, int NW, bool SF16 = false>
+//
+// KG = 2 (prepared operands, QB=1, NW=8): 128 query rows per workgroup and two groups of four
+// waves, each over half of the keys, merged in LDS at the end: half the steps per workgroup and
+// twice the workgroups, for launches that leave CUs idle (launch_attention, shape 2). Every group
+// has a four-stage ring of its own and all of the schedule below; a step ends in a barrier.
+template <typename TIn, int KMODE, bool MASKED, bool BOUNDED, int QB, int NW, bool SF16 = false, int KG = 1>
 __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(const AttnArgs a) {
     constexpr int NT = NW * 64;
     constexpr int QR = 32 * QB;       // query rows per wave
-    constexpr int BQ = NW * QR;       // query rows per workgroup
+    constexpr int BQ = NW / KG * QR;  // query rows per workgroup
     constexpr int CPT = 512 / NT;     // 8-element chunks of K (and of V) per thread per block
     constexpr int TPK = 16 / CPT;     // threads sharing one key row
-    constexpr int NST = ring_stages(QB, NW);
-    constexpr bool XSTEP = NST == 8;          // fragment reads run ahead across step boundaries
+    constexpr int NST = KG == 2 ? 4 : ring_stages(QB, NW); // ring stages of a key group
+    constexpr bool XSTEP = NST == 8 || KG == 2; // fragment reads run ahead across step boundaries
     // Prepared bf16 operands (K pre-pass mode) skip the registers: each wave moves four K rows and four V rows of a block from global
     // memory straight into the ring (buffer_load ... lds). Such a load puts lane i's
     // 16 bytes at base + 16 i, so rows are 256 bytes without padding and bank
     // conflicts are avoided by swizzling the 16-byte chunk position instead:
     // K chunk c of row r sits at c ^ (r & 15), V chunk c of row r at c ^ ((r & 3) << 2).
     constexpr bool DMA = kDirectLds && std::is_same<TIn, bf16_t>::value && KMODE == kQkNone && NW == 8 && QB == 1;
+    static_assert(KG == 1 || DMA, "key groups exist for the direct-to-LDS build only");
     static_assert(!SF16 || DMA, "half-precision score operands exist for the direct-to-LDS build only");
     // The product O^T += V^T P^T on v_mfma_f32_16x16x32 (the scores keep the 32 x 32 x 16 form, in
     // which a lane owns one query). The 16 x 16 form moves half the accumulator bytes per FLOP
@@ -131,7 +139,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     // room take it: prepared operands, and not the running maximum together with a mask (that
     // build then spills inside the loop). (Giving the scores that form too would double the MFMA
     // instructions on a vector issue port that the softmax already half fills.)
-    constexpr bool PV16 = DMA && (BOUNDED || !MASKED);
+    constexpr bool PV16 = DMA && (!MASKED || (BOUNDED && KG == 1));
     constexpr int KSTAGE = DMA ? KB * D : KS_ELEMS; // elements per ring stage
     constexpr int VSTAGE = DMA ? KB * D : VS_ELEMS;
     // a block enters the ring AHEAD steps before S needs its K (direct loads: one more step, to land)
@@ -146,8 +154,8 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     constexpr int STORE_SLOT = kStoreSlot; // slot after which the ring store is issued
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     bf16_t* const Ks = reinterpret_cast<bf16_t*>(smem);
-    bf16_t* const Vs = Ks + NST * KSTAGE;
-    unsigned short* const blocks = reinterpret_cast<unsigned short*>(Vs + NST * VSTAGE);
+    bf16_t* const Vs = Ks + KG * NST * KSTAGE;
+    unsigned short* const blocks = reinterpret_cast<unsigned short*>(Vs + KG * NST * VSTAGE);
     unsigned* const bmask = reinterpret_cast<unsigned*>(blocks + MAX_BLOCKS); // bit j: key j of the block is excluded
     __shared__ int s_count[MASKED ? MAX_BLOCKS / 64 : 1]; // admitted blocks of every 64
 
@@ -161,6 +169,8 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     const int wave = tid >> 6;
     const int l32 = lane & 31;
     const int h = lane >> 5;
+    const int grp = KG == 2 ? __builtin_amdgcn_readfirstlane(wave >> 2) : 0; // key group
+    const int gw = KG == 2 ? (wave & 3) : wave;                              // wave within it = its 32 query rows
 
     // XCD-aware remap: consecutive logical ids (one head's query blocks) share an XCD's L2
     int logical;
@@ -187,13 +197,14 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     const int qb = logical - bh * a.nqb;
     const int seg = bh / a.heads;
     const int head = bh - seg * a.heads;
-    const int q0 = qb * BQ + wave * QR;
+    const int q0 = qb * BQ + gw * QR;
 
     // The pipeline's first O update multiplies P = 0 by the V stage of "block -1":
     // that stage must hold finite numbers, so it is zeroed. (The last S update
     // reads a K stage past the end; its result is discarded.)
-    {
-        u32x4* z = reinterpret_cast<u32x4*>(Vs + (NST - 1) * VSTAGE);
+#pragma unroll
+    for (int g = 0; g < KG; g++) {
+        u32x4* z = reinterpret_cast<u32x4*>(Vs + (g * NST + NST - 1) * VSTAGE);
         constexpr int n16 = (int)(VSTAGE * sizeof(bf16_t) / 16);
         for (int i = tid; i < n16; i += NT) z[i] = u32x4{0u, 0u, 0u, 0u};
     }
@@ -259,6 +270,16 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
         i0 = split * per;
         nblk = max(min(nblk - i0, per), 0);
     }
+    // a key group walks the first or the second half of them: nblk steps for both, of which the last
+    // is idle (every key excluded) where the second half is the shorter
+    int nown = nblk;
+    if constexpr (KG == 2) {
+        const int total = nblk;
+        nblk = (total + 1) >> 1;
+        nown = grp == 0 ? nblk : total - nblk;
+        if (grp != 0 && nown > 0) i0 += nblk; // (with no block of its own it re-fetches the first group's)
+    }
+    const int last_own = KG == 2 ? max(nown - 1, 0) : nblk - 1; // positions past the end repeat the last one
     // Masked builds: lane i of two registers holds the block and the exclusion mask of list position
     // list_base + i, and a step takes its own by v_readlane. (Read from LDS in the step, as they
     // were at first, each made the wave wait for every fragment read in flight: a Klein 1024^2
@@ -268,7 +289,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     unsigned list_blk = 0, list_mask = 0;
     auto list_load = [&](int base) __attribute__((always_inline)) {
         list_base = base;
-        const int i = min(base + lane, nblk - 1); // positions past the end repeat the last one
+        const int i = min(base + lane, last_own);
         list_blk = kp ? (unsigned)blocks[i + i0] : (unsigned)(i + i0);
         list_mask = bmask[list_blk];
     };
@@ -435,25 +456,46 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     // i % NST; the lane that fills chunk position p of row r fetches the chunk that the
     // swizzle places there. In the block that holds the last row, rows past the sequence
     // re-read the last row (they are masked before the softmax).
-    const int dma_row = 4 * wave + (lane >> 4);
+    // (KG = 2: four waves fill a block, each K rows dma_row and + 16, V rows dma_vrow and + 8, so
+    // that a lane's chunk is the same in both)
+    const int dma_row = 4 * gw + (lane >> 4);
+    const int dma_vrow0 = KG == 2 ? 16 * (gw >> 1) + 4 * (gw & 1) : 4 * gw;
+    const int dma_vrow = dma_vrow0 + (lane >> 4);
     const unsigned dma_k_chunk = (unsigned)(((lane & 15) ^ (dma_row & 15)) * 8);
     // (PV16: a row's 16-dim halves also swap with bit 4 of the row, so that the lane groups that
     // read rows 16 apart hit different banks)
-    const unsigned dma_v_chunk = (unsigned)(((lane & 15) ^ ((dma_row & 3) << 2) ^ (PV16 ? (((dma_row >> 4) & 1) << 1) : 0)) * 8);
+    const unsigned dma_v_chunk = (unsigned)(((lane & 15) ^ ((dma_vrow & 3) << 2) ^ (PV16 ? (((dma_vrow >> 4) & 1) << 1) : 0)) * 8);
     const unsigned dma_k_off = ((unsigned)dma_row * (unsigned)a.k_ts + dma_k_chunk) * 2u;
-    const unsigned dma_v_off = ((unsigned)dma_row * (unsigned)a.v_ts + dma_v_chunk) * 2u;
+    const unsigned dma_v_off = ((unsigned)dma_vrow * (unsigned)a.v_ts + dma_v_chunk) * 2u;
     const int dma_tail_row = min(dma_row, last_row - last_blk * KB);
     const unsigned dma_k_off_tail = ((unsigned)dma_tail_row * (unsigned)a.k_ts + dma_k_chunk) * 2u;
     const unsigned dma_v_off_tail = ((unsigned)dma_tail_row * (unsigned)a.v_ts + dma_v_chunk) * 2u;
     const u32x4 dma_k_rsrc = make_rsrc_words(reinterpret_cast<const TIn*>(a.k) + (int64_t)seg * a.k_bs + (int64_t)head * a.k_hs, k_span);
     const u32x4 dma_v_rsrc = make_rsrc_words(reinterpret_cast<const TIn*>(a.v) + (int64_t)seg * a.v_bs + (int64_t)head * a.v_hs, v_span);
-    // LDS byte addresses of this wave's four rows in stage 0 of the K ring and of the V ring
-    const unsigned dma_k_lds = __builtin_amdgcn_readfirstlane(lds_address(Ks) + (unsigned)(4 * wave * D * 2));
-    const unsigned dma_v_lds = __builtin_amdgcn_readfirstlane(lds_address(Vs) + (unsigned)(4 * wave * D * 2));
+    // LDS byte addresses of this wave's first four rows in stage 0 of its group's K ring and V ring
+    const unsigned dma_k_lds = __builtin_amdgcn_readfirstlane(lds_address(Ks + grp * NST * KSTAGE) + (unsigned)(4 * gw * D * 2));
+    const unsigned dma_v_lds = __builtin_amdgcn_readfirstlane(lds_address(Vs + grp * NST * VSTAGE) + (unsigned)(dma_vrow0 * D * 2));
     // which: 1 = the K block, 2 = the V block, 3 = both
     auto dma_fetch_part = [&](int i, int stage, int which) __attribute__((always_inline)) {
-        const int ii = i < nblk ? i : nblk - 1; // past the end: a harmless re-fetch into a dead stage
+        const int ii = min(i, last_own); // past the end: a harmless re-fetch into a dead stage
         const int blk = block_of(ii);
+        if constexpr (KG == 2) { // eight rows per wave and operand: two loads, 16 rows of K and 8 of V apart
+            const bool tail = MASKED && blk >= last_blk; // wave-uniform
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                if (which & 1) {
+                    const unsigned lds = dma_k_lds + (unsigned)(stage * (KSTAGE * 2) + j * 16 * D * 2);
+                    if (!tail) load_to_lds_16(dma_k_rsrc, lds, dma_k_off, (unsigned)blk * k_blk_bytes + (unsigned)j * (k_blk_bytes >> 1));
+                    else load_to_lds_16(dma_k_rsrc, lds, ((unsigned)min(dma_row + 16 * j, last_row - last_blk * KB) * (unsigned)a.k_ts + dma_k_chunk) * 2u, (unsigned)blk * k_blk_bytes);
+                }
+                if (which & 2) {
+                    const unsigned lds = dma_v_lds + (unsigned)(stage * (VSTAGE * 2) + j * 8 * D * 2);
+                    if (!tail) load_to_lds_16(dma_v_rsrc, lds, dma_v_off, (unsigned)blk * v_blk_bytes + (unsigned)j * (v_blk_bytes >> 2));
+                    else load_to_lds_16(dma_v_rsrc, lds, ((unsigned)min(dma_vrow + 8 * j, last_row - last_blk * KB) * (unsigned)a.v_ts + dma_v_chunk) * 2u, (unsigned)blk * v_blk_bytes);
+                }
+            }
+            return;
+        }
         unsigned ko = dma_k_off, vo = dma_v_off;
         if constexpr (MASKED) {
             const bool tail = blk >= last_blk; // wave-uniform
@@ -509,12 +551,12 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
 #pragma unroll
     for (int s = 0; s < 8; s++) {
         const int col = DMA ? (((2 * s + h) ^ (l32 & 15)) * 8) : (8 * h + 16 * s);
-        kfo[s] = lds_address(Ks) + (unsigned)((l32 * KROW + col) * 2);
+        kfo[s] = lds_address(Ks + grp * NST * KSTAGE) + (unsigned)((l32 * KROW + col) * 2);
     }
 #pragma unroll
     for (int blk = 0; blk < 4; blk++) {
         const int col = (DMA ? ((blk ^ tr_row) * 32) : (32 * blk)) + tr_col; // (4 h + tr_row) & 3 == tr_row
-        vfo[blk] = lds_address(Vs) + (unsigned)(((4 * h + tr_row) * VROW + col) * 2);
+        vfo[blk] = lds_address(Vs + grp * NST * VSTAGE) + (unsigned)(((4 * h + tr_row) * VROW + col) * 2);
     }
     // PV16: the patch for output tile dt = 2 blk + x: the 16 lanes of group g4 take keys vkey0 + 8
     // half + tr_row (vkey0 = 0, 16, 4, 20: the keys whose probabilities the group holds as the
@@ -526,7 +568,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
 #pragma unroll
         for (int x = 0; x < 2; x++) {
             const int col = (blk ^ tr_row) * 32 + (x ^ (g4 & 1)) * 16 + 4 * (lane & 3); // (vkey0 + tr_row) & 3 == tr_row
-            vfo16[blk][x] = lds_address(Vs) + (unsigned)(((vkey0 + tr_row) * VROW + col) * 2);
+            vfo16[blk][x] = lds_address(Vs + grp * NST * VSTAGE) + (unsigned)(((vkey0 + tr_row) * VROW + col) * 2);
         }
     typedef const __attribute__((address_space(3))) bf16x8* lds_bf16x8_t;
     typedef __attribute__((address_space(3))) s16x4* lds_s16x4_t;
@@ -677,9 +719,10 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             if (MFMA_PRIO) __builtin_amdgcn_s_setprio(0);
         };
 
-        if constexpr (MASKED) {
+        if constexpr (MASKED || KG == 2) {
             // excluded keys (padding mask, key limit, tail) -> -inf; bit kk of badm = key kk of the block
-            const unsigned badm = (unsigned)__builtin_amdgcn_readlane((int)list_mask, b - list_base);
+            unsigned badm = MASKED ? (unsigned)__builtin_amdgcn_readlane((int)list_mask, b - list_base) : 0u;
+            if (KG == 2 && b >= nown) badm = 0xffffffffu; // the idle step of the shorter half
             if (badm != 0u) { // wave-uniform: most blocks exclude nothing
 #pragma unroll
                 for (int qi = 0; qi < QB; qi++)
@@ -789,7 +832,14 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             // whose previous tenant's last reader (V, NST-AHEAD-1 steps back) is at least one
             // barrier behind; then the set starts loading block b+AHEAD+2
             if constexpr (DMA) {
-                if (g == STORE_SLOT) dma_fetch(b + AHEAD, stage_of(AHEAD));
+                if constexpr (KG == 2) {
+                    // K(b) and V(b-2) have had their last reader before the barrier that ended step b-1;
+                    // what is requested here is waited for by the barrier that ends step b+1
+                    if (g == STORE_SLOT) dma_fetch_part(b + 4, stage_of(4), 1);
+                    if (g == STORE_SLOT + 4) dma_fetch_part(b + 2, stage_of(2), 2);
+                } else if (g == STORE_SLOT) {
+                    dma_fetch(b + AHEAD, stage_of(AHEAD));
+                }
             } else {
                 if (g == STORE_SLOT) stage_store(regs, stage_of(AHEAD));
                 if (g == STORE_SLOT + 1) stage_load(regs, b + AHEAD + 2);
@@ -888,7 +938,8 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                 asm volatile("" ::: "memory");
                 // direct loads: all but this step's two must have landed (vmcnt(2)); a block is
                 // first read two barriers after it was requested
-                if constexpr (DMA) __builtin_amdgcn_s_waitcnt(0x0F72);
+                // (KG = 2: all but this step's four; a block is first read one barrier after that)
+                if constexpr (DMA) __builtin_amdgcn_s_waitcnt(KG == 2 ? 0x0F74 : 0x0F72);
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
             } else {
@@ -907,12 +958,17 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             // and is their only reader, so it needs no barrier for them, only its own vmcnt.
             const unsigned q_span = ((unsigned)(a.tokens - 1) * (unsigned)a.q_ts + D) * 2u;
             const u32x4 q_rsrc = make_rsrc_words(reinterpret_cast<const bf16_t*>(a.q) + (int64_t)seg * a.q_bs + (int64_t)head * a.q_hs, q_span);
+            // (KG = 2: the two waves of the same rows bring half of them each into one such area: V
+            // stage 2 of the first group, and behind the lists.)
             const unsigned q_lds = __builtin_amdgcn_readfirstlane(
-                wave < 3   ? lds_address(Ks) + (unsigned)((5 + wave) * (KSTAGE * 2))
+                KG == 2    ? (gw < 3 ? lds_address(Vs) + (unsigned)(KG * NST * (VSTAGE * 2) + (int)kListBytes + gw * (KB * D * 2))
+                                     : lds_address(Vs) + (unsigned)(2 * (VSTAGE * 2)))
+                : wave < 3 ? lds_address(Ks) + (unsigned)((5 + wave) * (KSTAGE * 2))
                 : wave < 5 ? lds_address(Vs) + (unsigned)((5 + wave - 3) * (VSTAGE * 2))
                            : lds_address(Vs) + (unsigned)(NST * (VSTAGE * 2) + (int)kListBytes + (wave - 5) * (KB * D * 2)));
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
+            for (int jj = 0; jj < 8 / KG; jj++) {
+                const int j = KG == 2 ? jj + 4 * grp : jj;
                 const int r = 4 * j + (lane >> 4);
                 const int qrow = min(q0 + r, a.tokens - 1); // rows past the sequence re-read the last row (never stored)
                 const unsigned off = ((unsigned)qrow * (unsigned)a.q_ts + (unsigned)(((lane & 15) ^ (r & 15)) * 8)) * 2u;
@@ -923,16 +979,25 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             // for here; the rest of the first AHEAD blocks (4 loads) is covered by the wait before
             // the barrier that ends step 1. Every workgroup of a round starts at once, so these
             // first loads arrive at the rate of memory, not at its latency.
-            static_assert(AHEAD == 5, "the prologue's load count assumes five blocks ahead");
-            dma_fetch_part(0, 0, 3);
-            dma_fetch_part(1, 1, 3);
-            dma_fetch_part(2, 2, 1);
-            dma_fetch_part(3, 3, 1);
-            dma_fetch_part(2, 2, 2);
-            dma_fetch_part(3, 3, 2);
-            dma_fetch_part(4, 4, 3);
+            if constexpr (KG == 2) { // step 0 reads K(1), K(2) and V(0) before its barrier
+                dma_fetch_part(0, 0, 3);
+                dma_fetch_part(1, 1, 1);
+                dma_fetch_part(2, 2, 1);
+                dma_fetch_part(1, 1, 2);
+                dma_fetch_part(3, 3, 1);
+            } else {
+                static_assert(KG == 2 || AHEAD == 5, "the prologue's load count assumes five blocks ahead");
+                dma_fetch_part(0, 0, 3);
+                dma_fetch_part(1, 1, 3);
+                dma_fetch_part(2, 2, 1);
+                dma_fetch_part(3, 3, 1);
+                dma_fetch_part(2, 2, 2);
+                dma_fetch_part(3, 3, 2);
+                dma_fetch_part(4, 4, 3);
+            }
             __builtin_amdgcn_s_waitcnt(0x0F74); // vmcnt(4)
             asm volatile("" ::: "memory");
+            if constexpr (KG == 2) __syncthreads(); // the other wave's half of the rows
             typedef const __attribute__((address_space(3))) bf16x8* lds_q_t;
 #pragma unroll
             for (int s = 0; s < 8; s++)
@@ -968,6 +1033,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
 #pragma unroll
                 for (int j = 0; j < 8; j++) p_a[qi][kb][j] = (bf16_t)0.0f;
         qk_block(0, s_a);
+        if constexpr (KG == 2) __syncthreads(); // step 0 sends K(4) and V(2) where K(0) and query rows were
         if constexpr (XSTEP) {
 #pragma unroll
             for (int g = 0; g < LA; g++) frag_read(1, NST - 1, g);
@@ -1010,6 +1076,61 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
         if constexpr (DMA) __builtin_amdgcn_s_waitcnt(0x0F70); // no direct load may outlive the workgroup's LDS
     }
 
+    if constexpr (KG == 2) {
+        // The second group's rows, reference points and denominators go through the idle ring to the
+        // first, which adds them to its own (weighted by the distance of the reference points) and
+        // stores: 64 KB in and out of LDS.
+        typedef __attribute__((address_space(3))) f32x4* lds_f32x4_t;
+        typedef __attribute__((address_space(3))) f32x2* lds_f32x2_t;
+        const unsigned xo = lds_address(Vs) + (unsigned)(gw * (64 * 64 * 4) + lane * 16); // 64 values a lane, 16 bytes at a time
+        const unsigned xm = lds_address(Ks) + (unsigned)(4 * (KSTAGE * 2) + gw * (64 * 8) + lane * 8);
+        __syncthreads(); // every wave is done with the ring
+        if (grp != 0) {
+            if constexpr (PV16) {
+#pragma unroll
+                for (int i = 0; i < 16; i++) *(lds_f32x4_t)(xo + (unsigned)(i * 1024)) = oacc16[i >> 1][i & 1];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    *(lds_f32x4_t)(xo + (unsigned)(i * 1024)) =
+                        f32x4{oacc[0][i >> 2][4 * (i & 3)], oacc[0][i >> 2][4 * (i & 3) + 1], oacc[0][i >> 2][4 * (i & 3) + 2], oacc[0][i >> 2][4 * (i & 3) + 3]};
+            }
+            *(lds_f32x2_t)xm = f32x2{m_run[0], l_run[0]};
+        }
+        __syncthreads();
+        if (grp != 0) return;
+        const f32x2 ml = *(lds_f32x2_t)xm;
+        float w0 = 1.f, w1 = 1.f;
+        if constexpr (!BOUNDED) {
+            const float m = fmaxf(m_run[0], ml[0]); // (a group without an admitted key has no reference: weight 0)
+            w0 = m_run[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[0] - m);
+            w1 = ml[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[0] - m);
+            m_run[0] = m;
+        }
+        l_run[0] = l_run[0] * w0 + ml[1] * w1;
+        float w0r[2] = {w0, w0}, w1r[2] = {w1, w1};
+        if constexpr (PV16 && !BOUNDED) { // the weights of query 16 r + c16 live with its scores
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                w0r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + c16), (int)__float_as_uint(w0)));
+                w1r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + c16), (int)__float_as_uint(w1)));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const f32x4 x = *(lds_f32x4_t)(xo + (unsigned)(i * 1024));
+            if constexpr (PV16) {
+                oacc16[i >> 1][i & 1] = BOUNDED ? oacc16[i >> 1][i & 1] + x : oacc16[i >> 1][i & 1] * w0r[i & 1] + x * w1r[i & 1];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int e = 4 * (i & 3) + j;
+                    oacc[0][i >> 2][e] = BOUNDED ? oacc[0][i >> 2][e] + x[j] : oacc[0][i >> 2][e] * w0 + x[j] * w1;
+                }
+            }
+        }
+    }
+
     // ---- epilogue: O = O^T / l
     if constexpr (PV16) {
         // The denominator lives with the scores (lane = query l32); the lane that holds query
@@ -1022,7 +1143,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             inv_r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + c16), (int)__float_as_uint(inv_l)));
         if (splits > 1) {
             // unnormalised rows, reference point and denominator of this part
-            const int64_t prow0 = (int64_t)blockIdx.x * BQ + wave * QR;
+            const int64_t prow0 = (int64_t)blockIdx.x * BQ + gw * QR;
 #pragma unroll
             for (int r = 0; r < 2; r++) {
                 float* op = a.part_o + (prow0 + 16 * r + c16) * D + 4 * g4;
@@ -1048,7 +1169,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             // 16 thirty-two-byte segments per store instruction. The wave turns its 32 x 128 tile
             // through 8 KB of LDS (its own stage of the idle K ring, K layout: chunk c of row r
             // at c ^ (r & 15)) and stores whole 256-byte rows, four per instruction.
-            __syncthreads(); // every wave is done with the ring
+            if constexpr (KG == 1) __syncthreads(); // every wave is done with the ring
             typedef __attribute__((address_space(3))) u32x2* lds_u32x2_t;
             typedef const __attribute__((address_space(3))) u32x4* lds_u32x4_t;
             typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -1082,7 +1203,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             const int qrow = q0 + 32 * qi + l32;
             if (splits > 1) {
                 // unnormalised rows, reference point and denominator of this part
-                const int64_t prow = ((int64_t)blockIdx.x * BQ + wave * QR + 32 * qi + l32);
+                const int64_t prow = ((int64_t)blockIdx.x * BQ + gw * QR + 32 * qi + l32);
                 float* op = a.part_o + prow * D;
 #pragma unroll
                 for (int blk = 0; blk < 4; blk++)
@@ -1115,7 +1236,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                 // 32 sixteen-byte segments per store instruction. The wave turns its 32 x 128 tile
                 // through 8 KB of LDS (its own stage of the idle K ring, K layout: chunk c of row r
                 // at c ^ (r & 15)) and stores whole 256-byte rows, four per instruction.
-                __syncthreads(); // every wave is done with the ring
+                if constexpr (KG == 1) __syncthreads(); // every wave is done with the ring
                 typedef __attribute__((address_space(3))) u32x2* lds_u32x2_t;
                 typedef const __attribute__((address_space(3))) u32x4* lds_u32x4_t;
                 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -1145,7 +1266,9 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
         }
     }
     // (whole tiles only: the parts carry no probe)
-    const int64_t probe_slot = (int64_t)blockIdx.x - a.part_wgs;
+    int64_t probe_slot = (int64_t)blockIdx.x - a.part_wgs;
+    // (a slot per 256 query rows in either shape: of two workgroups that share them, the first's)
+    if constexpr (KG == 2) probe_slot = (splits > 1 || (qb & 1)) ? -1 : (int64_t)bh * ((a.nqb + 1) >> 1) + (qb >> 1);
     if (a.clock_probe && tid == 0 && probe_slot >= 0 && probe_slot < a.clock_cap) {
         a.clock_probe[2 * probe_slot] = __builtin_readcyclecounter() - clk_c0;
         a.clock_probe[2 * probe_slot + 1] = __builtin_amdgcn_s_memrealtime() - clk_r0;
@@ -1211,20 +1334,20 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const AttnArgs a, int b
 }
 
 // One launch: the tiles of the last round in parts (tail.splits > 1), the whole tiles behind them; then the merge.
-template <typename TIn, int KMODE, bool MASKED, bool BOUNDED, int QB, int NW>
+template <typename TIn, int KMODE, bool MASKED, bool BOUNDED, int QB, int NW, int KG>
 static void launch_kernel(const AttnArgs& a, unsigned grid, hipStream_t stream) {
     if constexpr (std::is_same<TIn, bf16_t>::value && KMODE == kQkNone && QB == 1 && NW == 8) {
         if (a.score_f16) {
-            attn_fwd_kernel<TIn, KMODE, MASKED, BOUNDED, QB, NW, true>
+            attn_fwd_kernel<TIn, KMODE, MASKED, BOUNDED, QB, NW, true, KG>
                 <<<dim3(grid), dim3(NW * 64), lds_bytes(ring_stages(QB, NW)), stream>>>(a);
             return;
         }
     }
-    attn_fwd_kernel<TIn, KMODE, MASKED, BOUNDED, QB, NW>
+    attn_fwd_kernel<TIn, KMODE, MASKED, BOUNDED, QB, NW, false, KG>
         <<<dim3(grid), dim3(NW * 64), lds_bytes(ring_stages(QB, NW)), stream>>>(a);
 }
 
-template <typename TIn, int KMODE, bool MASKED, bool BOUNDED, int QB, int NW>
+template <typename TIn, int KMODE, bool MASKED, bool BOUNDED, int QB, int NW, int KG = 1>
 static hipError_t launch_one(const AttnArgs& a0, hipStream_t stream) {
     const int64_t nwg = (int64_t)a0.nqb * a0.heads * a0.batch;
     if (nwg <= 0 || nwg > 0x7fffffff) return hipErrorInvalidValue;
@@ -1235,17 +1358,17 @@ static hipError_t launch_one(const AttnArgs& a0, hipStream_t stream) {
     a.splits = tail > 0 ? a0.splits : 1;
     a.part_wgs = tail > 0 ? (int32_t)(((int64_t)tail * a0.splits + 7) & ~(int64_t)7) : 0;
     if (whole + a.part_wgs > 0x7fffffff) return hipErrorInvalidValue;
-    launch_kernel<TIn, KMODE, MASKED, BOUNDED, QB, NW>(a, (unsigned)(whole + a.part_wgs), stream);
+    launch_kernel<TIn, KMODE, MASKED, BOUNDED, QB, NW, KG>(a, (unsigned)(whole + a.part_wgs), stream);
     {
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     if (tail > 0) {
-        const int rows = tail * NW * 32 * QB;
+        const int rows = tail * (NW / KG * 32 * QB);
         const dim3 mgrid((unsigned)((rows + 7) / 8));
-        if (a.splits <= 4) attn_merge_kernel<4><<<mgrid, dim3(256), 0, stream>>>(a, NW * 32 * QB);
-        else if (a.splits <= 8) attn_merge_kernel<8><<<mgrid, dim3(256), 0, stream>>>(a, NW * 32 * QB);
-        else if (a.splits <= kMaxSplits) attn_merge_kernel<kMaxSplits><<<mgrid, dim3(256), 0, stream>>>(a, NW * 32 * QB);
+        if (a.splits <= 4) attn_merge_kernel<4><<<mgrid, dim3(256), 0, stream>>>(a, NW / KG * 32 * QB);
+        else if (a.splits <= 8) attn_merge_kernel<8><<<mgrid, dim3(256), 0, stream>>>(a, NW / KG * 32 * QB);
+        else if (a.splits <= kMaxSplits) attn_merge_kernel<kMaxSplits><<<mgrid, dim3(256), 0, stream>>>(a, NW / KG * 32 * QB);
         else return hipErrorInvalidValue;
         return hipGetLastError();
     }
@@ -1279,6 +1402,15 @@ static hipError_t launch_flags(const AttnArgs& a, int k_mode, hipStream_t stream
                    : launch_kmode<TIn, false, false, QB, NW>(a, k_mode, stream);
 }
 
+// The two-key-group build: prepared 16-bit operands only.
+static hipError_t launch_pair(const AttnArgs& a, int in_dtype, int k_mode, hipStream_t stream) {
+    if (in_dtype != kBF16 || k_mode != kQkNone || a.q_mode != kQkNone || (a.score_f16 && a.scale_log2 != 1.0f)) return hipErrorInvalidValue;
+    const bool masked = a.key_pad != nullptr || (a.key_limit % KB) != 0;
+    if (masked)
+        return a.bounded ? launch_one<bf16_t, kQkNone, true, true, 1, 8, 2>(a, stream) : launch_one<bf16_t, kQkNone, true, false, 1, 8, 2>(a, stream);
+    return a.bounded ? launch_one<bf16_t, kQkNone, false, true, 1, 8, 2>(a, stream) : launch_one<bf16_t, kQkNone, false, false, 1, 8, 2>(a, stream);
+}
+
 template <int QB, int NW>
 static hipError_t launch_shape(const AttnArgs& a, int in_dtype, int k_mode, hipStream_t stream) {
     if (in_dtype == kF32) return launch_flags<float, QB, NW>(a, k_mode, stream);
@@ -1288,13 +1420,15 @@ static hipError_t launch_shape(const AttnArgs& a, int in_dtype, int k_mode, hipS
 
 template <typename TIn, int KMODE, bool MASKED, bool BOUNDED, int QB, int NW>
 static hipError_t raise_lds() {
+    const int lds = (int)lds_bytes(ring_stages(QB, NW));
+    auto raise = [&](auto* kernel) { return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds); };
     if constexpr (std::is_same<TIn, bf16_t>::value && KMODE == kQkNone && QB == 1 && NW == 8) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_fwd_kernel<TIn, KMODE, MASKED, BOUNDED, QB, NW, true>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(ring_stages(QB, NW)));
+        hipError_t e = raise(&attn_fwd_kernel<TIn, KMODE, MASKED, BOUNDED, QB, NW, true>);
+        if (e == hipSuccess) e = raise(&attn_fwd_kernel<TIn, KMODE, MASKED, BOUNDED, QB, NW, true, 2>);
+        if (e == hipSuccess) e = raise(&attn_fwd_kernel<TIn, KMODE, MASKED, BOUNDED, QB, NW, false, 2>);
         if (e != hipSuccess) return e;
     }
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_fwd_kernel<TIn, KMODE, MASKED, BOUNDED, QB, NW>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(ring_stages(QB, NW)));
+    return raise(&attn_fwd_kernel<TIn, KMODE, MASKED, BOUNDED, QB, NW>);
 }
 
 template <int QB, int NW>
@@ -1313,7 +1447,7 @@ static hipError_t raise_shape() {
 
 } // namespace fwd
 
-int attention_block_rows(int shape) { return shape == 1 ? 128 : 256; }
+int attention_block_rows(int shape) { return shape == 0 ? 256 : 128; }
 
 void attention_tail_plan(int64_t tiles, int cus, int key_blocks, int* tail_tiles, int* splits) {
     *tail_tiles = 0;
@@ -1336,6 +1470,36 @@ size_t attention_part_o_bytes(int tail_tiles, int splits, int shape) {
 size_t attention_part_ml_bytes(int tail_tiles, int splits, int shape) {
     return (size_t)tail_tiles * splits * attention_block_rows(shape) * 2 * sizeof(float);
 }
+// Launches whose 128-row tiles fit the CUs once take the shape whose estimate is the smallest: 256-row
+// tiles or 128-row tiles with two key groups, each whole or with all tiles split along the keys
+// (attention_tail_plan), where the parts go to memory and back and a merge follows. Everything larger
+// stays on 256-row tiles: two key groups read K and V twice as often and sit at the power limit
+// sooner (24 heads, 1536 tokens, 288 tiles of 128 rows: call 56 us on 256-row tiles, 70 on 128). The
+// constants are a fit to 1 to 96 heads of 64 to 6144 tokens; the pick is the best of what was
+// measured or within 5 % of it in 104 of 106 launches. Fused call, us, 256-row tiles in parts
+// before: 24 heads 768 tokens 39.6 -> 33.4, 512 tokens 33.7 -> 27.1; 30 heads 1024 tokens 50.1 ->
+// 42.1; 8 heads 1536 tokens 45.4 -> 35.3.
+void attention_plan(int64_t heads, int tokens, int key_blocks, int cus, int* shape, int* tail_tiles, int* splits) {
+    constexpr float kBlockUs = 0.8f, kPairUs = 0.8f, kPairFixUs = 1.0f, kMergeUs = 3.0f, kShareBytesPerUs = 2.5e6f;
+    const int64_t pairs = heads * ((tokens + 127) / 128);
+    *shape = 0;
+    attention_tail_plan(heads * ((tokens + 255) / 256), cus, key_blocks, tail_tiles, splits);
+    if (pairs > cus) return;
+    // (fewer tiles than CUs: all of them are the tail)
+    auto estimate = [&](int sh, int tiles, int s) {
+        const int per = (key_blocks + s - 1) / s;
+        float us = sh == 0 ? (float)per * kBlockUs : (float)((per + 1) / 2) * kPairUs + kPairFixUs;
+        if (s > 1) us += kMergeUs + (float)(attention_part_o_bytes(tiles, s, sh)) / kShareBytesPerUs;
+        return us;
+    };
+    float best = estimate(0, *tail_tiles, *splits);
+    int tail = 0, s = 1;
+    attention_tail_plan(pairs, cus, key_blocks, &tail, &s);
+    const float split_us = s > 1 ? estimate(2, tail, s) : INFINITY;
+    const float whole_us = estimate(2, 0, 1);
+    if (whole_us < best) { best = whole_us; *shape = 2; *tail_tiles = 0; *splits = 1; }
+    if (split_us < best) { *shape = 2; *tail_tiles = tail; *splits = s; }
+}
 int attention_key_block() { return fwd::KB; }
 int attention_max_tokens() { return fwd::MAX_BLOCKS * fwd::KB; }
 
@@ -1343,6 +1507,7 @@ hipError_t launch_attention(const AttnArgs& a, int in_dtype, int k_mode, int sha
     switch (shape) {
     case 0: return fwd::launch_shape<1, 8>(a, in_dtype, k_mode, stream);
     case 1: return fwd::launch_shape<1, 4>(a, in_dtype, k_mode, stream);
+    case 2: return fwd::launch_pair(a, in_dtype, k_mode, stream);
     default: return hipErrorInvalidValue;
     }
 }

@@ -122,7 +122,8 @@ struct WeightStageArgs {
 hipError_t launch_weight_stage(const WeightStageArgs& args, hipStream_t stream);
 
 // Kernel shape: 0 = 8 waves x 32 query rows (one workgroup per CU, 8-stage LDS
-// ring), 1 = 4 waves x 32 query rows (two workgroups per CU, 4-stage rings).
+// ring), 1 = 4 waves x 32 query rows (two workgroups per CU, 4-stage rings), 2 = 4 x 32 query rows
+// by two groups of four waves, each over half of the keys (prepared 16-bit operands only).
 int attention_block_rows(int shape);
 int attention_key_block();
 int attention_max_tokens();
@@ -166,6 +167,9 @@ hipError_t launch_attention(const AttnArgs& args, int in_dtype, int k_mode, int 
 // the last, partly filled round are better split along the keys, and into how many parts
 // (0 tiles = run everything whole). key_blocks = 32-key blocks per tile.
 void attention_tail_plan(int64_t tiles, int cus, int key_blocks, int* tail_tiles, int* splits);
+// The kernel shape (0 or 2) and tail plan of a launch of prepared 16-bit operands over `heads`
+// (segment, head) pairs.
+void attention_plan(int64_t heads, int tokens, int key_blocks, int cus, int* shape, int* tail_tiles, int* splits);
 // Bytes of part_o and part_ml that `tail_tiles` x `splits` need for the kernel shape.
 size_t attention_part_o_bytes(int tail_tiles, int splits, int shape);
 size_t attention_part_ml_bytes(int tail_tiles, int splits, int shape);

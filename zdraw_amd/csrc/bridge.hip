@@ -240,6 +240,7 @@ struct FusedPlan {
     AttnArgs args;
     int in_dtype;
     int k_mode;
+    int shape;       // kernel shape (launch_attention)
     bool prepass;
     PrepArgs prep;   // K pre-pass
     PrepArgs prep_q; // Q pre-pass (same launch condition)
@@ -420,7 +421,15 @@ int plan_attention(Device* dev, void* q, void* k, void* v, void* out, const Zdra
     a.heads = (int32_t)p->heads;
     a.batch = (int32_t)x->batch;
     a.key_limit = (int32_t)((p->valid != 0 && p->valid < p->tokens) ? p->valid : p->tokens);
-    const int rows = attention_block_rows(g_variant & 1);
+    const int key_blocks = (a.key_limit + attention_key_block() - 1) / attention_key_block();
+    plan->shape = g_variant & 1;
+    int tail = 0, splits = 1;
+    // the kernel will read prepared 16-bit operands (or bf16 ones as given): its shape is a choice
+    const bool direct = x->qk_mode != ZDRAW_HIP_QK_NONE ? x->k_site == ZDRAW_HIP_K_PREPASS
+                                                         : x->in_dtype == ZDRAW_HIP_BF16 || stage_f16 || p->tokens >= kRoundPlainTokens;
+    if (direct && g_variant == 0)
+        attention_plan((int64_t)p->heads * x->batch, (int)p->tokens, key_blocks, dev->cus, &plan->shape, &tail, &splits);
+    const int rows = attention_block_rows(plan->shape);
     a.nqb = (int32_t)((p->tokens + rows - 1) / rows);
     a.q_mode = (int32_t)x->qk_mode;
     a.out_dtype = (int32_t)x->out_dtype;
@@ -537,12 +546,11 @@ int plan_attention(Device* dev, void* q, void* k, void* v, void* out, const Zdra
     // A last round of workgroups that fills at most half the CUs is split along the keys so
     // that it fills them all (its parts are merged by a small kernel, in a fixed order).
     if ((g_variant & 2) == 0) {
-        int tail = 0, splits = 1;
-        attention_tail_plan((int64_t)a.nqb * a.heads * a.batch, dev->cus, (a.key_limit + attention_key_block() - 1) / attention_key_block(),
-                            &tail, &splits);
+        if (!direct || g_variant != 0)
+            attention_tail_plan((int64_t)a.nqb * a.heads * a.batch, dev->cus, key_blocks, &tail, &splits);
         if (splits > 1) {
-            void* po = src->get(3, attention_part_o_bytes(tail, splits, g_variant & 1));
-            void* pm = src->get(4, attention_part_ml_bytes(tail, splits, g_variant & 1));
+            void* po = src->get(3, attention_part_o_bytes(tail, splits, plan->shape));
+            void* pm = src->get(4, attention_part_ml_bytes(tail, splits, plan->shape));
             if (!po || !pm) return scratch_failed(src);
             a.splits = splits;
             a.tile_base = tail; // launch_attention reads the tail size here
@@ -711,14 +719,15 @@ int enqueue(const FusedPlan& plan, hipStream_t stream, bool no_alloc = false) {
             args.clock_probe = g_clock_buf;
             args.clock_cap = kClockCap;
             // key-split tail tiles carry no probe
-            g_clock_wgs = (int64_t)args.nqb * args.heads * args.batch - (args.splits > 1 ? args.tile_base : 0);
+            const int64_t slots = (plan.shape == 2 ? (args.nqb + 1) / 2 : args.nqb) * (int64_t)args.heads * args.batch;
+            g_clock_wgs = plan.shape == 2 && args.splits > 1 ? 0 : slots - (args.splits > 1 ? args.tile_base : 0);
             g_clock_stream = stream;
         }
     }
     TracePair tp{nullptr, nullptr};
     if (g_trace && !no_alloc && hipEventCreate(&tp.a) == hipSuccess && hipEventCreate(&tp.b) == hipSuccess)
         (void)hipEventRecord(tp.a, stream);
-    hipError_t e = launch_attention(args, plan.in_dtype, plan.k_mode, g_variant & 1, stream);
+    hipError_t e = launch_attention(args, plan.in_dtype, plan.k_mode, plan.shape, stream);
     if (e != hipSuccess) {
         set_err("attention launch: %s", hipGetErrorString(e));
         return ZDRAW_HIP_ERR_HANDLE;
