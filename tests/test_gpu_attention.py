@@ -879,6 +879,21 @@ def test_two_key_groups_sampled_rows(ctx, tokens, heads, dead, in_dtype, out_dty
         b.release()
 
 
+# Plain attention on f32 rows either side of the length from which one launch rounds the operands
+# ahead of the kernel (160 tokens): one launch below, two from there on, with a key limit and ragged
+# last blocks, every row against the oracle. The copies keep the bits the tile load would have made.
+@pytest.mark.parametrize("tokens,valid,launches", [(128, None, 1), (159, 100, 1), (160, None, 2), (161, 33, 2), (447, None, 2), (1023, 1000, 2)])
+def test_plain_f32_rows_either_side_of_the_rounding_launch(ctx, tokens, valid, launches):
+    L = hip.lib()
+    rng = np.random.default_rng(tokens)
+    q, k, v = (rng.standard_normal((tokens, 2, 128), dtype=np.float32) * 0.5 for _ in range(3))
+    cfg = host.Config(tokens, 2, 2, 128) if valid is None else host.Config(tokens, 2, 2, 128, valid=valid)
+    d0 = L.zdraw_hip_dispatch_count()
+    got = ctx.run(q, k, v, cfg)
+    assert L.zdraw_hip_dispatch_count() - d0 == launches
+    refimpl.check_close(got, zo.attention_run(q, k, v, oracle_cfg(cfg)), f"plain {tokens} valid={valid}")
+
+
 # first, a middle and the last key block; rising, so that the reference moves at each of them
 PLANT_CASES = [
     # name, tokens, heads, in_dtype, valid, planted (key, nats), whole tiles only (knob 2)

@@ -234,7 +234,24 @@ struct ScratchSource {
     void* get(int slot, size_t bytes);
 };
 
-constexpr uint32_t kRoundPlainTokens = 1024; // plain f32 attention from this length on rounds its operands once, ahead of the kernel
+// Plain f32 attention from this length on rounds its operands once, ahead of the kernel, which then takes
+// two key groups and more: call on resident rows, two heads, 256 tokens 31.9 -> 31.3 us, 512 35.8 -> 33.9,
+// 24 heads 700 tokens 51.4 -> 44.5. At 128 tokens and below one launch is as fast as two (64 tokens, 24
+// heads: 25.5 against 26.5). Below kRoundAlwaysTokens only where the copies cost no one an allocation
+// that is not allowed (plain_may_round).
+constexpr uint32_t kRoundPlainTokens = 160, kRoundAlwaysTokens = 1024;
+
+// Whether a plain f32 call shorter than kRoundAlwaysTokens may take the three scratch slots of the
+// rounding launch: from a queue whose slots are large enough already or may grow now (a stream
+// under capture may not allocate), not from a caller's span.
+bool plain_may_round(const ScratchSource* src, size_t bytes) {
+    if (!src->queue || src->dry || src->span) return false;
+    bool ready = true;
+    for (int i = 0; i < 3; i++) ready = ready && src->queue->scratch[i] && src->queue->scratch[i]->len >= bytes;
+    if (ready) return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(src->queue->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
 
 struct FusedPlan {
     AttnArgs args;
@@ -425,8 +442,10 @@ int plan_attention(Device* dev, void* q, void* k, void* v, void* out, const Zdra
     plan->shape = g_variant & 1;
     int tail = 0, splits = 1;
     // the kernel will read prepared 16-bit operands (or bf16 ones as given): its shape is a choice
+    const bool round_plain = x->qk_mode == ZDRAW_HIP_QK_NONE && x->in_dtype == ZDRAW_HIP_F32 && p->tokens >= kRoundPlainTokens &&
+                             (p->tokens >= kRoundAlwaysTokens || plain_may_round(src, (size_t)x->batch * p->heads * p->tokens * kHeadDim * 2));
     const bool direct = x->qk_mode != ZDRAW_HIP_QK_NONE ? x->k_site == ZDRAW_HIP_K_PREPASS
-                                                         : x->in_dtype == ZDRAW_HIP_BF16 || stage_f16 || p->tokens >= kRoundPlainTokens;
+                                                         : x->in_dtype == ZDRAW_HIP_BF16 || stage_f16 || round_plain;
     if (direct && g_variant == 0)
         attention_plan((int64_t)p->heads * x->batch, (int)p->tokens, key_blocks, dev->cus, &plan->shape, &tail, &splits);
     const int rows = attention_block_rows(plan->shape);
@@ -633,8 +652,7 @@ int plan_attention(Device* dev, void* q, void* k, void* v, void* out, const Zdra
             plan->in_dtype = kBF16;
         }
     }
-    if (x->qk_mode == ZDRAW_HIP_QK_NONE &&
-        ((x->in_dtype == ZDRAW_HIP_F32 && p->tokens >= kRoundPlainTokens) || stage_f16)) {
+    if (x->qk_mode == ZDRAW_HIP_QK_NONE && (round_plain || stage_f16)) {
         // Plain attention on f32 rows (the reference's base entry, metal_c.zig:286-299, takes
         // them): Q (with the softmax scale), K and V are rounded to bf16 once, head-major, into
         // slots 0-2 by one launch, and the kernel is the direct-to-LDS build, as for prepared
