@@ -584,3 +584,55 @@ def test_every_tile_of_the_pipelined_kernel(ctx, tile, m, n, count, k, c_dtype):
         assert (np.abs(got[rows] - want) <= 2e-5 * s + 1e-6 + place).all(), f"product {i}: max {np.abs(got[rows] - want).max():.3e}"
     for b in [ab, wb] + cbs:
         b.release()
+
+
+# edges of the 64 x 64 tiles and of the 32-wide steps, the smallest product, a k of whole slabs
+@pytest.mark.parametrize("m,k,n,count", [(1, 8, 1, 1), (64, 64, 64, 2), (77, 200, 131, 3), (300, 264, 70, 1)])
+@pytest.mark.parametrize("wdt", [hip.W_BF16, hip.W_F16])
+@pytest.mark.parametrize("c16", [False, True])
+def test_f32_activations_on_a_queue_under_capture_that_has_no_scratch(ctx, m, k, n, count, wdt, c16):
+    # The rounded copy of A may not be allocated under capture: the product rounds its rows on the
+    # way instead. Same roundings and the same order of sums, so the bits are those of the call
+    # with scratch; every replay of the graph writes them.
+    L = hip.lib()
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    w_bits, _ = to16(rng.standard_normal((count, n, k), dtype=np.float32) * np.float32(k ** -0.5), wdt)
+    c_dtype = act_dtype(wdt) if c16 else hip.F32
+    nbytes = m * n * (2 if c16 else 4)
+    ab, wb = ctx.buffer(a), ctx.buffer(w_bits)
+    cbs = [ctx.buffer(np.full(nbytes, 0x5A, np.uint8)) for _ in range(count)]
+    ps = [hip.GemmParams(m, k, n, wdt, hip.GEMM_HALF, i * n * k * 2) for i in range(count)]
+    ext = hip.GemmExt(0, 0, 0, 0, 0, hip.F32, c_dtype)
+
+    def enqueue(batch):
+        return L.zdraw_hip_run_gemm_group_ext_enc(batch, ab.handle, (C.c_void_p * count)(*([wb.handle] * count)),
+                                                  (C.c_void_p * count)(*(b.handle for b in cbs)),
+                                                  (C.POINTER(hip.GemmParams) * count)(*(C.pointer(p) for p in ps)), count, C.byref(ext))
+
+    batch = L.zdraw_hip_batch_begin(ctx.queue)
+    assert enqueue(batch) == 0, hip.last_error()
+    assert L.zdraw_hip_batch_end(batch) == 0
+    want = [b.read(np.uint8, (nbytes,)) for b in cbs]
+
+    queue = L.zdraw_hip_create_queue(ctx.device)
+    stream = C.c_void_p((C.c_void_p * 2).from_address(queue)[1])  # a queue is a device and a stream
+    graph, run = C.c_void_p(), C.c_void_p()
+    batch = L.zdraw_hip_batch_begin(queue)
+    assert L.hipStreamBeginCapture(stream, C.c_int(2)) == 0
+    rc = enqueue(batch)
+    assert L.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert rc == 0, hip.last_error()
+    assert L.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    for replay in range(3):
+        for b in cbs:
+            b.write(np.full(nbytes, 0x5A, np.uint8))
+        assert L.hipGraphLaunch(run, stream) == 0
+        assert L.hipStreamSynchronize(stream) == 0
+        for i, b in enumerate(cbs):
+            assert np.array_equal(b.read(np.uint8, (nbytes,)), want[i]), f"replay {replay}, product {i}"
+    assert L.zdraw_hip_batch_end(batch) == 0
+    assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
+    for b in [ab, wb] + cbs:
+        b.release()
+    L.zdraw_hip_release_queue(queue)

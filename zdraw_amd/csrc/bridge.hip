@@ -220,6 +220,13 @@ Buffer* queue_scratch(Queue* q, int slot, size_t bytes) {
     return grow_slot(&q->scratch[slot], slot, bytes, [q] { (void)hipStreamSynchronize(q->stream); });
 }
 
+// Whether a slot of the queue has the room, or may be grown now (a stream under capture may not allocate).
+bool may_grow(const Queue* q, int slot, size_t bytes) {
+    if (q->scratch[slot] && q->scratch[slot]->len >= bytes) return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(q->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
+
 // Where a call's scratch comes from: the grow-only slots of the queue the call runs on,
 // or a caller-supplied span handed out piece by piece in 256-byte steps (the entry that
 // allocates nothing), or nowhere (a plan that is only validated).
@@ -246,11 +253,9 @@ constexpr uint32_t kRoundPlainTokens = 160, kRoundAlwaysTokens = 1024;
 // under capture may not allocate), not from a caller's span.
 bool plain_may_round(const ScratchSource* src, size_t bytes) {
     if (!src->queue || src->dry || src->span) return false;
-    bool ready = true;
-    for (int i = 0; i < 3; i++) ready = ready && src->queue->scratch[i] && src->queue->scratch[i]->len >= bytes;
-    if (ready) return true;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(src->queue->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+    for (int i = 0; i < 3; i++)
+        if (!may_grow(src->queue, i, bytes)) return false;
+    return true;
 }
 
 struct FusedPlan {
@@ -1002,12 +1007,14 @@ int enqueue_gemm_group(void* a, void* const* ws, void* const* cs, const uint64_t
     if (const size_t rb = gemm_round_bytes(g, (int)x->a_dtype)) {
         // f32 activations are rounded to the weight's type once, into scratch slot 6, and the
         // product then runs as for 16-bit activations
-        Buffer* a16 = queue_scratch(queue, 6, rb);
-        if (!a16) {
+        const bool in_place = gemm_rounds_in_place(g);
+        Buffer* a16 = in_place && !may_grow(queue, 6, rb) ? nullptr : queue_scratch(queue, 6, rb);
+        if (!a16 && !in_place) {
             set_err("scratch allocation failed");
             return ZDRAW_HIP_ERR_HANDLE;
         }
-        g.a16 = a16->ptr;
+        if (a16) g.a16 = a16->ptr;
+        else (void)hipGetLastError(); // or the launch would report the failed allocation
     }
     g.shape = gemm_shape(g, queue->dev->cus);
     if (g.shape < 0) {

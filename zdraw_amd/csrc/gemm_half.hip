@@ -892,6 +892,72 @@ __global__ void __launch_bounds__(256) gemm_round_kernel(const float* a, int64_t
     }
 }
 
+// f32 activations where there is no room for their rounded copy (a queue under capture that has not
+// grown its scratch yet): each 64 x 64 tile rounds the rows it reads on their way into LDS, one
+// 32-wide step in flight. Bound by the wait for memory in every step, so it is the way out and never
+// the choice. The MFMAs add k in the order of the other kernels: same bits.
+template <bool F16, typename TC>
+__global__ void __launch_bounds__(256) gemm_unstaged_kernel(const GemmArgs g) {
+    constexpr int T = 64, KS = 32, PITCH = KS * 2 + 16; // bytes per LDS row
+    __shared__ __attribute__((aligned(16))) unsigned char sa[T * PITCH], sw[T * PITCH];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c16 = lane & 15, q4 = lane >> 4;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int row_tiles = g.tiles_n * g.groups;
+    const int tm = (int)blockIdx.x / row_tiles;
+    int tn = (int)blockIdx.x - tm * row_tiles;
+    const int grp = tn / g.tiles_n;
+    tn -= grp * g.tiles_n;
+    const void* const wp = grp == 0 ? g.w : g.w_more[grp - 1];
+    void* const cp = grp == 0 ? g.c : g.c_more[grp - 1];
+    const int m0 = tm * T, n0 = tn * T;
+    // thread = 8 k of one row of either operand; rows past the edge re-read the last one, never stored
+    const int r = tid >> 2, c = (tid & 3) * 8;
+    const float* const arow = static_cast<const float*>(g.a) + (int64_t)min(m0 + r, g.m - 1) * g.lda;
+    const unsigned short* const wrow = static_cast<const unsigned short*>(wp) + (int64_t)min(n0 + r, g.n - 1) * g.ldw;
+    f32x4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < g.k; k0 += KS) {
+        const bool keep = k0 + c < g.k; // (k is a multiple of 8: a group is whole or past the end)
+        const int at = keep ? k0 + c : 0;
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(arow + at), hi = *reinterpret_cast<const f32x4*>(arow + at + 4);
+        u32x4 wv = *reinterpret_cast<const u32x4*>(wrow + at), av;
+        f32x8 v;
+#pragma unroll
+        for (int i = 0; i < 4; i++) { v[i] = lo[i]; v[4 + i] = hi[i]; }
+        if constexpr (F16) av = __builtin_bit_cast(u32x4, __builtin_convertvector(v, f16x8));
+        else av = __builtin_bit_cast(u32x4, __builtin_convertvector(v, bf16x8));
+        if (!keep) av = wv = u32x4{0u, 0u, 0u, 0u};
+        __syncthreads(); // the last step's fragments have been read
+        *reinterpret_cast<u32x4*>(sa + r * PITCH + c * 2) = av;
+        *reinterpret_cast<u32x4*>(sw + r * PITCH + c * 2) = wv;
+        __syncthreads();
+        u32x4 fa[2], fw[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            fa[i] = *reinterpret_cast<const u32x4*>(sa + (wm * 32 + i * 16 + c16) * PITCH + q4 * 16);
+            fw[i] = *reinterpret_cast<const u32x4*>(sw + (wn * 32 + i * 16 + c16) * PITCH + q4 * 16);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) mfma16<F16>(fw[j], fa[i], acc[i][j]);
+        mfma16_drain();
+    }
+    store_tile16<F16, TC, 2, 2>(g, cp, acc, m0 + wm * 32, n0 + wn * 32, lane);
+}
+template <bool F16, typename TC>
+static hipError_t launch_unstaged(GemmArgs g, hipStream_t stream) {
+    g.tiles_n = (g.n + 63) / 64;
+    const int64_t nwg = (int64_t)((g.m + 63) / 64) * g.tiles_n * g.groups;
+    if (nwg <= 0 || nwg > 0x7fffffff) return hipErrorInvalidValue;
+    gemm_unstaged_kernel<F16, TC><<<dim3((unsigned)nwg), dim3(256), 0, stream>>>(g);
+    return hipGetLastError();
+}
+
 // Measured on the Klein projections, same box, all with row-by-row stores and row-major tile
 // order: eight waves (two per SIMD, 64 x 128 each) 1048-1217 TFLOP/s; four waves with the
 // schedule above 1047-1248; four waves with the simple loop of the eight-wave build 960-1120.
@@ -1054,12 +1120,20 @@ void gemm_shape_tile(int shape, int* rows, int* cols) {
 // f32 activations are rounded to the weight's type once, ahead of the product.
 size_t gemm_round_bytes(const GemmArgs& g, int a_dtype) { return a_dtype == kF32 ? (size_t)g.m * (size_t)g.k * 2 : 0; }
 
+// Products of less than a 256-tile either way, or of a ragged k, must not fail for want of that copy's
+// room; larger ones report the failed allocation rather than run several times slower.
+bool gemm_rounds_in_place(const GemmArgs& g) { return g.k % gemm::BK != 0 || g.m < gemm::BM || g.n < gemm::BN; }
+
 hipError_t launch_gemm(const GemmArgs& g0, int a_dtype, int w_dtype, int c_dtype, hipStream_t stream) {
     using namespace gemm;
     typedef unsigned short h16; // a 16-bit operand in the compute type (bf16 or f16 per the weight)
     GemmArgs g = g0;
+    if (a_dtype == kF32 && g.a16 == nullptr) {
+        if (!gemm_rounds_in_place(g)) return hipErrorInvalidValue;
+        if (w_dtype == kBF16) return c_dtype == kF32 ? launch_unstaged<false, float>(g, stream) : launch_unstaged<false, h16>(g, stream);
+        return c_dtype == kF32 ? launch_unstaged<true, float>(g, stream) : launch_unstaged<true, h16>(g, stream);
+    }
     if (a_dtype == kF32) {
-        if (g.a16 == nullptr) return hipErrorInvalidValue;
         const dim3 grid((unsigned)g.m, (unsigned)((g.k + 4095) / 4096));
         if (w_dtype == kF16)
             gemm_round_kernel<true><<<grid, dim3(256), 0, stream>>>(static_cast<const float*>(g.a), g.lda, static_cast<h16*>(g.a16), g.m, g.k);

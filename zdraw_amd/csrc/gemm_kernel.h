@@ -31,7 +31,7 @@ struct GemmArgs {
     int32_t part_wgs; // set by the launcher
     int32_t pad1;
     // f32 activations: room for A rounded to the weight's type, [m][k] 16-bit (gemm_round_bytes
-    // says how much)
+    // says how much); null where gemm_rounds_in_place allows it
     void* a16;
 };
 
@@ -51,6 +51,8 @@ void gemm_tail_plan(const GemmArgs& args, int cus, int* tail_tiles, int* splits)
 size_t gemm_part_bytes(int tail_tiles, int splits);
 // Bytes of scratch launch_gemm needs for f32 activations rounded ahead of the product (0: none).
 size_t gemm_round_bytes(const GemmArgs& args, int a_dtype);
+// Whether launch_gemm takes f32 activations without that scratch (slower, same bits).
+bool gemm_rounds_in_place(const GemmArgs& args);
 void gemm_set_build(int build); // 256-tiles of 16-bit activations: 1 = four-wave build (default), 0 = eight-wave build
 
 } // namespace zdraw
