@@ -680,6 +680,34 @@ def test_qk_norm_rope_in_place_matches_oracle(ctx):
     kb.release()
 
 
+# heads at the edges of a wave's walk: 8 per pass in small launches, 24 or 32 in large ones; the line is
+# at 8192 tokens, the second length is one past it with a part of a workgroup left over
+@pytest.mark.parametrize("heads", [1, 8, 9, 25])
+@pytest.mark.parametrize("tokens", [1, 8192, 8193])
+def test_qk_norm_rope_by_head_groups_of_either_size(ctx, heads, tokens):
+    rng = np.random.default_rng(heads + tokens)
+    pos = np.stack([rng.integers(0, 1536, tokens), rng.integers(0, 512, tokens), rng.integers(0, 512, tokens)], 1)
+    q = rng.standard_normal((tokens, heads, 128), dtype=np.float32)
+    w = 1.0 + 0.2 * rng.standard_normal(128).astype(np.float32)
+    cfg = zo.RopeConfig(wl.ZIMAGE_DIMS, wl.ZIMAGE_LENS, wl.ZIMAGE_THETA)
+    vals = zo.zrope_fill(cfg)
+    qb, kb = ctx.buffer(q), ctx.buffer(q)
+    ctx.qk_run(qb, kb, w, w, pos, vals, wl.ZIMAGE_DIMS, wl.ZIMAGE_LENS, tokens=tokens, heads=heads,
+               kv_heads=heads, head_dim=128, norm_eps=wl.ZIMAGE_EPS)
+    gq, gk = qb.read(np.float32, q.shape), kb.read(np.float32, q.shape)
+    assert np.array_equal(gq, gk)
+    rows = sorted({0, tokens // 2, max(0, tokens - 4), tokens - 1})
+    want = zo.zimage_rotate(zo.zimage_norm_heads(np.ascontiguousarray(q[rows]), w, wl.ZIMAGE_EPS), vals, cfg, np.ascontiguousarray(pos[rows]))
+    # fp32 on both sides, as above
+    assert np.abs(gq[rows] - want).max() < 5e-6 * np.abs(want).max() + 2e-6
+    # every row against its norm: rotation keeps it, so none was left out or done twice
+    t64 = q.astype(np.float64)
+    normed = t64 / np.sqrt((t64 ** 2).mean(-1, keepdims=True) + wl.ZIMAGE_EPS) * w
+    assert np.allclose(np.sqrt((gq.astype(np.float64) ** 2).sum(-1)), np.sqrt((normed ** 2).sum(-1)), rtol=1e-5)
+    qb.release()
+    kb.release()
+
+
 # ------------------------------------------------ key-split tail tiles and their merge
 @pytest.mark.parametrize("tokens,valid,heads,bounded", [(700, 0, 2, True), (700, 650, 2, False), (1000, 0, 1, False),
                                                        (1500, 1300, 3, True)])

@@ -12,15 +12,24 @@ namespace zdraw {
 // 16 lanes per row (8 dims each). A wave covers one token: its four 16-lane
 // groups take four heads at a time (1 KB contiguous in a token-major operand)
 // and walk G such groups of heads, keeping the token's rope coefficients and
-// norm weights in registers, so the rope table is read once per token. All G
-// loads of a lane are issued before the first is used. Input and output are
+// norm weights in registers. All G loads of a lane are issued before the first
+// is used. Input and output are
 // addressed by strides, so the same kernel serves the 16-bit Q/K pre-pass and the
 // in-place f32 token-major form. A lane reads and writes only its own 8
 // elements, so the output may alias the input.
 constexpr int kPrepTokens = 4; // tokens (waves) per workgroup
 
-// G = groups of four heads walked by one lane: 6 (24 heads per pass: Klein) or 8 (32 heads
-// per pass: Z-Image's 30 heads in one pass instead of two)
+// G = groups of four heads walked by one wave: 2, or all of a token's heads (6: 24 heads per pass,
+// Klein; 8: 32 heads per pass, Z-Image's 30 heads in one pass instead of two) in large launches.
+// Bound by memory in those, by a wave's own chain in small ones: a round trip for the rope row, then
+// norm and rope of one group after the other, with too few waves on a CU to fill the gaps. Two
+// groups a wave cut that chain to a third and cost the rope row again, from L2. Fused call per
+// block, us, 6 or 8 -> 2 groups: 24 heads bf16 256 tokens 18.6 -> 17.0, 768 30.6 -> 28.1, 1040 38.2
+// -> 34.5, 4 x 1536 158.6 -> 154.8, 4608 240.2 -> 239.2; 30 heads 80 tokens 16.6 -> 14.5, 768 34.2
+// -> 30.3, 4608 301 -> 299.5; but 2 x 8704 tokens 1459 -> 1467, hence the line between 6144 and
+// 17408 tokens over all segments.
+constexpr int64_t kThinTokens = 8192;
+
 template <typename TIn, int MODE, int G>
 __global__ void __launch_bounds__(kPrepTokens * 64) qk_prepass_kernel(const PrepPair pair) {
     // grid z = operand * batch + segment; the choice is uniform over the workgroup
@@ -181,8 +190,9 @@ hipError_t launch_qk_prepass(const PrepArgs* ops, int count, int in_dtype, hipSt
     for (int i = 0; i < 3; i++) pair.op[i] = ops[i < count ? i : count - 1];
     pair.count = count;
     pair.pad0 = 0;
+    const bool thin = (int64_t)p.tokens * p.batch <= kThinTokens;
     const bool wide_pass = (p.heads + 31) / 32 < (p.heads + 23) / 24; // fewer passes over the heads with 32 per pass
-    const int per_pass = wide_pass ? 32 : 24;
+    const int per_pass = thin ? 8 : wide_pass ? 32 : 24;
     const dim3 grid((unsigned)((p.tokens + kPrepTokens - 1) / kPrepTokens), (unsigned)((p.heads + per_pass - 1) / per_pass),
                     (unsigned)(p.batch * count));
     const dim3 block(kPrepTokens * 64);
@@ -190,7 +200,8 @@ hipError_t launch_qk_prepass(const PrepArgs* ops, int count, int in_dtype, hipSt
     if (!klein && p.mode != kQkZimage) return hipErrorInvalidValue;
 #define ZD_PREP(T, M) \
     do { \
-        if (wide_pass) qk_prepass_kernel<T, M, 8><<<grid, block, 0, stream>>>(pair); \
+        if (thin) qk_prepass_kernel<T, M, 2><<<grid, block, 0, stream>>>(pair); \
+        else if (wide_pass) qk_prepass_kernel<T, M, 8><<<grid, block, 0, stream>>>(pair); \
         else qk_prepass_kernel<T, M, 6><<<grid, block, 0, stream>>>(pair); \
     } while (0)
     if (in_dtype == kF32) {
