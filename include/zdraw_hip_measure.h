@@ -33,12 +33,18 @@ size_t zdraw_hip_clock_probe_read(uint64_t* cycles, uint64_t* ref_ticks, size_t 
 void zdraw_hip_set_attention_variant(int variant);
 
 /* Which build multiplies 256 x 256 tiles of 16-bit activations. 1 = four waves, 128 x 128
- * each (default); 0 = eight waves, 64 x 128 each. */
+ * each (default); 0 = eight waves, 64 x 128 each. 2 = every product on the kernel that
+ * addresses A and W through pointers and takes no scratch. */
 void zdraw_hip_set_gemm_build(int build);
 
 /* The tile of C (rows x columns) that `groups` (1..3) side-by-side products C[m][n] =
  * A[m][k] x W[n][k]^T run on, on a device with `cus` compute units. Host arithmetic only. */
 void zdraw_hip_gemm_tile(uint32_t m, uint32_t k, uint32_t n, uint32_t groups, uint32_t cus, uint32_t* rows, uint32_t* cols);
+
+/* How many of `rows` rows of a 16-bit A or W (`ld` elements apart, k of them used) one launch of a
+ * product takes: all, unless they span all but 4 GiB; 0 where not even one row fits the kernels'
+ * 32-bit offsets. A product is cut accordingly. Host arithmetic only. */
+void zdraw_hip_gemm_launch_rows(uint32_t rows, uint64_t ld, uint32_t k, uint32_t* per_launch);
 
 /* How many query tiles (128 rows) of the last wide-head launch had a score outgrow its row's
  * fixed reference point and were formed again by the running-maximum kernel (waits for that

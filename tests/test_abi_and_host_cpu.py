@@ -108,6 +108,32 @@ def test_gemm_tile_of_the_projection_shapes():
     assert tile(0, 64, 64) == (0, 0) and tile(64, 64, 64, 4) == (0, 0)
 
 
+def test_gemm_rows_of_one_launch_stay_inside_32_bit_offsets():
+    # The kernels add 3 KB (where their descriptors start) and up to 112 bytes (the last slab of a
+    # ragged k) to an operand's span: formed here with unlimited integers for every piece of a cut
+    L = hip.lib()
+
+    def per_launch(rows, ld, k):
+        r = C.c_uint32(99)
+        L.zdraw_hip_gemm_launch_rows(rows, ld, k, C.byref(r))
+        return r.value
+
+    for rows, ld, k in [(4608, 3072, 3072), (4608, 12288, 12288), (1, 2 ** 40, 64), (65536, 32768, 32768 - 1664), (2 ** 28 - 256, 8, 8), (255, 8421504, 64)]:
+        assert per_launch(rows, ld, k) == rows          # whole up to the limit
+    cases = [(65536, 32768, k) for k in (32760, 32704, 32768 - 1536)] + [(2 ** 28 - 1, 8, 8), (2, 2 ** 30, 2 ** 30 - 8), (3, 2 ** 30 - 800, 64),
+             (256, 8421504, 64), (257, 8388600, 2040), (513, 4194296, 4000), (1, 2 ** 31 - 8, 2 ** 31 - 1640)]
+    for rows, ld, k in cases:
+        assert ((rows - 1) * ld + k) * 2 < 2 ** 32      # what the entry accepts
+        step = per_launch(rows, ld, k)
+        assert 0 < step <= rows and (step == rows or step < 256 or step % 256 == 0)
+        for r0 in range(0, rows, step):
+            n = min(step, rows - r0)
+            assert ((n - 1) * ld + k) * 2 + 3 * 1024 + 112 < 2 ** 32, (rows, ld, k, r0)
+    assert per_launch(65536, 32768, 32760) == 65280 and per_launch(257, 8388600, 2040) == 256
+    assert per_launch(1, 2 ** 31 - 8, 2 ** 31 - 8) == 0  # one row alone is too long
+    assert per_launch(0, 8, 8) == 0 and per_launch(8, 8, 0) == 0
+
+
 def test_tail_plan_of_the_baseline_shapes():
     # 256 CUs, one 256-row tile per workgroup: which last rounds are split along the keys
     L = hip.lib()

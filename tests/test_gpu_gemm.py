@@ -586,6 +586,67 @@ def test_every_tile_of_the_pipelined_kernel(ctx, tile, m, n, count, k, c_dtype):
         b.release()
 
 
+# A or W whose last row ends within 3 KB of 4 GiB: the kernels' descriptors cannot hold it together with
+# what they add to it, so the product runs as two launches. A ragged k and whole slabs, one
+# product and a group. Rows either side of the cut, the first and the last, against float64.
+@pytest.mark.parametrize("side", ["a", "w"])
+@pytest.mark.parametrize("k,count", [(32760, 1), (32704, 2)])
+def test_operand_that_spans_almost_4_gib(ctx, side, k, count):
+    import torch
+
+    L = hip.lib()
+    ld, many, few = 32768, 65536, 72
+    m, n = (many, few) if side == "a" else (few, many)
+    span = ((many - 1) * ld + k) * 2
+    assert 2 ** 32 - 3 * 1024 <= span < 2 ** 32
+    g = torch.Generator(device="cuda")
+    g.manual_seed(k)
+    big = torch.empty(span // 2, device="cuda", dtype=torch.bfloat16).normal_(generator=g)
+    small = torch.empty((count if side == "a" else 1, few, k), device="cuda", dtype=torch.bfloat16).normal_(generator=g)
+    outs = [torch.zeros((m, n), device="cuda") for _ in range(count)]
+    torch.cuda.synchronize()
+    wrap = lambda t: L.zdraw_hip_wrap_device_memory(ctx.device, t.data_ptr(), t.numel() * t.element_size())
+    bh, sh, cs = wrap(big), wrap(small), [wrap(o) for o in outs]
+    assert bh and sh and all(cs)
+    ah, wh = (bh, sh) if side == "a" else (sh, bh)
+    ps = [hip.GemmParams(m, k, n, hip.W_BF16, hip.GEMM_HALF, i * few * k * 2 if side == "a" else 0) for i in range(count)]
+    ext = hip.GemmExt(0, 0, ld if side == "a" else k, k if side == "a" else ld, 0, hip.BF16, hip.F32)
+    d0 = L.zdraw_hip_dispatch_count()
+    batch = L.zdraw_hip_batch_begin(ctx.queue)
+    rc = L.zdraw_hip_run_gemm_group_ext_enc(batch, ah, (C.c_void_p * count)(*([wh] * count)), (C.c_void_p * count)(*cs),
+                                            (C.POINTER(hip.GemmParams) * count)(*(C.pointer(p) for p in ps)), count, C.byref(ext))
+    assert L.zdraw_hip_batch_end(batch) == 0
+    assert rc == 0, hip.last_error()
+    assert L.zdraw_hip_dispatch_count() - d0 == 1
+    for r in (0, 1, 255, 32767, 65279, 65280, 65535):
+        row = big[r * ld:r * ld + k].double()
+        for i in range(count):
+            want = small[i if side == "a" else 0].double() @ row
+            got = (outs[i][r] if side == "a" else outs[i][:, r]).double()
+            assert float((got - want).abs().max()) <= 2e-5 * k ** 0.5, (r, i)  # 32-bit sums, the bar of `check`
+    for h in (bh, sh, *cs):
+        L.zdraw_hip_release_buffer(h)
+
+
+# The kernel without descriptors or scratch, which serves rows that no descriptor reaches the end of and
+# f32 activations under capture: 16-bit and f32 activations, edges of its tiles, against the oracle.
+@pytest.mark.parametrize("m,k,n", [(1, 8, 1), (64, 64, 64), (130, 200, 77)])
+@pytest.mark.parametrize("wdt", [hip.W_BF16, hip.W_F16])
+@pytest.mark.parametrize("a16", [False, True])
+def test_kernel_that_addresses_through_pointers(ctx, m, k, n, wdt, a16):
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    w_bits, wr = to16(rng.standard_normal((n, k), dtype=np.float32), wdt)
+    a_bits, ar = to16(a, wdt)
+    L = hip.lib()
+    try:
+        L.zdraw_hip_set_gemm_build(2)
+        got = run_ext(ctx, a_bits if a16 else a, w_bits, m, k, n, wdt, act_dtype(wdt) if a16 else hip.F32, hip.F32)
+    finally:
+        L.zdraw_hip_set_gemm_build(1)
+    check(got.view(np.float32).reshape(m, n), zo.linear_batch(ar, wr), zo.linear_batch(a, wr), k, a, wr, f"{m}x{k}x{n}")
+
+
 # edges of the 64 x 64 tiles and of the 32-wide steps, the smallest product, a k of whole slabs
 @pytest.mark.parametrize("m,k,n,count", [(1, 8, 1, 1), (64, 64, 64, 2), (77, 200, 131, 3), (300, 264, 70, 1)])
 @pytest.mark.parametrize("wdt", [hip.W_BF16, hip.W_F16])

@@ -14,6 +14,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -1004,7 +1005,9 @@ int enqueue_gemm_group(void* a, void* const* ws, void* const* cs, const uint64_t
     g.tiles_n = (int32_t)((p->n + (uint32_t)gemm_tile_cols() - 1) / (uint32_t)gemm_tile_cols());
     if ((uint64_t)g.tiles_n * (uint64_t)groups * ((p->m + (uint32_t)gemm_tile_rows() - 1) / (uint32_t)gemm_tile_rows()) > 0x7fffffffull)
         return unavailable("grid too large");
-    if (const size_t rb = gemm_round_bytes(g, (int)x->a_dtype)) {
+    bool unstaged = false;
+    int a_dtype = (int)x->a_dtype;
+    if (const size_t rb = gemm_round_bytes(g, a_dtype)) {
         // f32 activations are rounded to the weight's type once, into scratch slot 6, and the
         // product then runs as for 16-bit activations
         const bool in_place = gemm_rounds_in_place(g);
@@ -1015,29 +1018,55 @@ int enqueue_gemm_group(void* a, void* const* ws, void* const* cs, const uint64_t
         }
         if (a16) g.a16 = a16->ptr;
         else (void)hipGetLastError(); // or the launch would report the failed allocation
+        unstaged = !a16;
     }
-    g.shape = gemm_shape(g, queue->dev->cus);
-    if (g.shape < 0) {
-        // a last round of 256-tiles that fills at most half the CUs runs split along k; its fp32
-        // partial tiles go through scratch slot 5
-        int tail = 0, splits = 1;
-        gemm_tail_plan(g, queue->dev->cus, &tail, &splits);
-        if (splits > 1) {
-            Buffer* part = queue_scratch(queue, 5, gemm_part_bytes(tail, splits));
-            if (!part) {
-                set_err("scratch allocation failed");
+    // Pieces of C that one launch can address: the whole but where A or W spans all but 4 GiB (the rounded
+    // copy of f32 rows spans at most half of that)
+    int64_t m_step = a_dtype == ZDRAW_HIP_F32 ? g.m : gemm_launch_rows(g.m, g.lda, g.k), n_step = gemm_launch_rows(g.n, g.ldw, g.k);
+    if (m_step == 0 || n_step == 0) unstaged = true;
+    if (unstaged) m_step = g.m, n_step = g.n;
+    for (int64_t m0 = 0; m0 < g.m; m0 += m_step)
+        for (int64_t n0 = 0; n0 < g.n; n0 += n_step) {
+            GemmArgs piece = g;
+            piece.m = (int32_t)std::min<int64_t>(m_step, g.m - m0);
+            piece.n = (int32_t)std::min<int64_t>(n_step, g.n - n0);
+            piece.a = static_cast<const char*>(g.a) + m0 * g.lda * (int64_t)ea;
+            auto w_at = [&](const void* w) { return static_cast<const char*>(w) + n0 * g.ldw * 2; };
+            auto c_at = [&](void* c) { return static_cast<char*>(c) + (m0 * g.ldc + n0) * (int64_t)ec; };
+            piece.w = w_at(g.w);
+            piece.c = c_at(g.c);
+            for (int i = 1; i < groups; i++) {
+                piece.w_more[i - 1] = w_at(g.w_more[i - 1]);
+                piece.c_more[i - 1] = c_at(g.c_more[i - 1]);
+            }
+            piece.shape = unstaged ? kGemmUnstaged : gemm_shape(piece, queue->dev->cus);
+            if (piece.shape == -1) {
+                // a last round of 256-tiles that fills at most half the CUs runs split along k; its fp32
+                // partial tiles go through scratch slot 5
+                int tail = 0, splits = 1;
+                gemm_tail_plan(piece, queue->dev->cus, &tail, &splits);
+                if (splits > 1) {
+                    Buffer* part = queue_scratch(queue, 5, gemm_part_bytes(tail, splits));
+                    if (!part) {
+                        set_err("scratch allocation failed");
+                        return ZDRAW_HIP_ERR_HANDLE;
+                    }
+                    piece.splits = splits;
+                    piece.tile_base = tail; // launch_gemm reads the tail size here
+                    piece.part = static_cast<float*>(part->ptr);
+                }
+            }
+            hipError_t e = launch_gemm(piece, a_dtype, (int)wt, (int)x->c_dtype, queue->stream);
+            if (e != hipSuccess) {
+                set_err("gemm launch: %s", hipGetErrorString(e));
                 return ZDRAW_HIP_ERR_HANDLE;
             }
-            g.splits = splits;
-            g.tile_base = tail; // launch_gemm reads the tail size here
-            g.part = static_cast<float*>(part->ptr);
+            if (a_dtype == ZDRAW_HIP_F32 && !unstaged && piece.shape != kGemmUnstaged) { // rounded once; the next piece reads the copy
+                g.a = g.a16;
+                g.lda = g.k;
+                a_dtype = (int)wt;
+            }
         }
-    }
-    hipError_t e = launch_gemm(g, (int)x->a_dtype, (int)wt, (int)x->c_dtype, queue->stream);
-    if (e != hipSuccess) {
-        set_err("gemm launch: %s", hipGetErrorString(e));
-        return ZDRAW_HIP_ERR_HANDLE;
-    }
     g_dispatch++;
     return ZDRAW_HIP_OK;
 }
@@ -1861,6 +1890,11 @@ void zdraw_hip_gemm_tail_plan(uint32_t m, uint32_t k, uint32_t n, uint32_t group
         gemm_tail_plan(g, (int)cus, &t, &s);
     if (tail_tiles) *tail_tiles = (uint32_t)t;
     if (splits) *splits = (uint32_t)s;
+}
+
+void zdraw_hip_gemm_launch_rows(uint32_t rows, uint64_t ld, uint32_t k, uint32_t* per_launch) {
+    const bool ok = rows && k && rows <= 0x7fffffffu && k <= 0x7fffffffu && ld <= 0x7fffffffffffffffull / rows;
+    if (per_launch) *per_launch = ok ? (uint32_t)gemm_launch_rows((int32_t)rows, (int64_t)ld, (int32_t)k) : 0;
 }
 
 void zdraw_hip_gemm_tile(uint32_t m, uint32_t k, uint32_t n, uint32_t groups, uint32_t cus, uint32_t* rows, uint32_t* cols) {

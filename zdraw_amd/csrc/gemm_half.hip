@@ -16,6 +16,7 @@
 //   * gemm_pipe_kernel: nine tiles from 64 x 64 to 256 x 160 with three or four slabs in LDS, for
 //     problems that do not fill the chip with 256-tiles, and for any k that is not a multiple of 64;
 //   * f32 activations are rounded to the weight's type by a launch of their own;
+//   * gemm_unstaged_kernel: what neither can take (no room for that rounded copy, rows of 4 GiB);
 //   * two or three products of one A with equal shapes (q/k/v, gate/up) run as one launch
 //     whose tiles cover all of them;
 //   * fixed summation order and no atomics (a thinly filled last round is cut along k and
@@ -455,7 +456,7 @@ __global__ void __launch_bounds__(256, 1) gemm_ring_kernel(const GemmArgs g) {
     // once per run and the other three use the instruction's offset field, which also moves the
     // address in memory; that is taken off the lane's offset, and the descriptors start 3 KB
     // below the operands so that the offset stays positive.
-    constexpr unsigned kBias = 3 * 1024;
+    constexpr unsigned kBias = kGemmDescBias;
     const u32x4 a_rsrc = make_rsrc_words(reinterpret_cast<const unsigned char*>(g.a) - kBias, a_span + kBias);
     const u32x4 w_rsrc = make_rsrc_words(reinterpret_cast<const unsigned char*>(wp) - kBias, w_span + kBias);
     const unsigned lds0 = lds_address(smem);
@@ -656,7 +657,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pipe_kernel(const GemmArgs g) {
     const unsigned a_span = ((unsigned)(g.m - 1) * (unsigned)g.lda + (unsigned)g.k) * 2u;
     const unsigned w_span = ((unsigned)(g.n - 1) * (unsigned)g.ldw + (unsigned)g.k) * 2u;
     // loads in runs of four under one M0, as in gemm_ring_kernel
-    constexpr unsigned kBias = 3 * 1024;
+    constexpr unsigned kBias = kGemmDescBias;
     const u32x4 a_rsrc = make_rsrc_words(reinterpret_cast<const unsigned char*>(g.a) - kBias, a_span + kBias);
     const u32x4 w_rsrc = make_rsrc_words(reinterpret_cast<const unsigned char*>(wp) - kBias, w_span + kBias);
     const unsigned lds0 = lds_address(smem);
@@ -893,10 +894,11 @@ __global__ void __launch_bounds__(256) gemm_round_kernel(const float* a, int64_t
 }
 
 // f32 activations where there is no room for their rounded copy (a queue under capture that has not
-// grown its scratch yet): each 64 x 64 tile rounds the rows it reads on their way into LDS, one
+// grown its scratch yet), and rows so long that a descriptor does not reach their end: each 64 x 64
+// tile reads its rows through pointers and rounds them on their way into LDS, one
 // 32-wide step in flight. Bound by the wait for memory in every step, so it is the way out and never
 // the choice. The MFMAs add k in the order of the other kernels: same bits.
-template <bool F16, typename TC>
+template <typename TA, bool F16, typename TC>
 __global__ void __launch_bounds__(256) gemm_unstaged_kernel(const GemmArgs g) {
     constexpr int T = 64, KS = 32, PITCH = KS * 2 + 16; // bytes per LDS row
     __shared__ __attribute__((aligned(16))) unsigned char sa[T * PITCH], sw[T * PITCH];
@@ -913,23 +915,27 @@ __global__ void __launch_bounds__(256) gemm_unstaged_kernel(const GemmArgs g) {
     const int m0 = tm * T, n0 = tn * T;
     // thread = 8 k of one row of either operand; rows past the edge re-read the last one, never stored
     const int r = tid >> 2, c = (tid & 3) * 8;
-    const float* const arow = static_cast<const float*>(g.a) + (int64_t)min(m0 + r, g.m - 1) * g.lda;
+    const TA* const arow = static_cast<const TA*>(g.a) + (int64_t)min(m0 + r, g.m - 1) * g.lda;
     const unsigned short* const wrow = static_cast<const unsigned short*>(wp) + (int64_t)min(n0 + r, g.n - 1) * g.ldw;
     f32x4 acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
         for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < g.k; k0 += KS) {
-        const bool keep = k0 + c < g.k; // (k is a multiple of 8: a group is whole or past the end)
-        const int at = keep ? k0 + c : 0;
-        const f32x4 lo = *reinterpret_cast<const f32x4*>(arow + at), hi = *reinterpret_cast<const f32x4*>(arow + at + 4);
+    for (unsigned k0 = 0; k0 < (unsigned)g.k; k0 += KS) { // (k may be just short of 2^31)
+        const bool keep = k0 + c < (unsigned)g.k; // (k is a multiple of 8: a group is whole or past the end)
+        const unsigned at = keep ? k0 + c : 0;
         u32x4 wv = *reinterpret_cast<const u32x4*>(wrow + at), av;
-        f32x8 v;
+        if constexpr (std::is_same<TA, float>::value) {
+            const f32x4 lo = *reinterpret_cast<const f32x4*>(arow + at), hi = *reinterpret_cast<const f32x4*>(arow + at + 4);
+            f32x8 v;
 #pragma unroll
-        for (int i = 0; i < 4; i++) { v[i] = lo[i]; v[4 + i] = hi[i]; }
-        if constexpr (F16) av = __builtin_bit_cast(u32x4, __builtin_convertvector(v, f16x8));
-        else av = __builtin_bit_cast(u32x4, __builtin_convertvector(v, bf16x8));
+            for (int i = 0; i < 4; i++) { v[i] = lo[i]; v[4 + i] = hi[i]; }
+            if constexpr (F16) av = __builtin_bit_cast(u32x4, __builtin_convertvector(v, f16x8));
+            else av = __builtin_bit_cast(u32x4, __builtin_convertvector(v, bf16x8));
+        } else {
+            av = *reinterpret_cast<const u32x4*>(arow + at);
+        }
         if (!keep) av = wv = u32x4{0u, 0u, 0u, 0u};
         __syncthreads(); // the last step's fragments have been read
         *reinterpret_cast<u32x4*>(sa + r * PITCH + c * 2) = av;
@@ -949,12 +955,12 @@ __global__ void __launch_bounds__(256) gemm_unstaged_kernel(const GemmArgs g) {
     }
     store_tile16<F16, TC, 2, 2>(g, cp, acc, m0 + wm * 32, n0 + wn * 32, lane);
 }
-template <bool F16, typename TC>
+template <typename TA, bool F16, typename TC>
 static hipError_t launch_unstaged(GemmArgs g, hipStream_t stream) {
     g.tiles_n = (g.n + 63) / 64;
     const int64_t nwg = (int64_t)((g.m + 63) / 64) * g.tiles_n * g.groups;
     if (nwg <= 0 || nwg > 0x7fffffff) return hipErrorInvalidValue;
-    gemm_unstaged_kernel<F16, TC><<<dim3((unsigned)nwg), dim3(256), 0, stream>>>(g);
+    gemm_unstaged_kernel<TA, F16, TC><<<dim3((unsigned)nwg), dim3(256), 0, stream>>>(g);
     return hipGetLastError();
 }
 
@@ -963,7 +969,7 @@ static hipError_t launch_unstaged(GemmArgs g, hipStream_t stream) {
 // schedule above 1047-1248; four waves with the simple loop of the eight-wave build 960-1120.
 constexpr int DMA_WM = 4, DMA_WN = 2;
 
-static int g_gemm_build = 1; // 256-tiles: 1 = four-wave build (default), 0 = eight-wave build (measurement knob)
+static int g_gemm_build = 1; // measurement knob (gemm_set_build)
 
 // The tiles gemm_pipe_kernel is built for: (32 ti) x (32 tj) with st slabs in LDS, what one slab of
 // it takes when weights come from memory (us, every CU busy) and what a tile costs beside its slabs.
@@ -1091,6 +1097,7 @@ size_t gemm_part_bytes(int tail_tiles, int splits) {
 // 3 x 3072 64 x 96 20 (48), 2816 x 12288 x 3072 192 x 192 164 (238), 2304 x 3840 x 3840 192 x 192 61 (95).
 int gemm_shape(const GemmArgs& g, int cus) {
     using namespace gemm;
+    if (g_gemm_build == 2) return kGemmUnstaged;
     if (cus <= 0) return 0;
     auto count = [&](int rows, int cols) { return (int64_t)((g.m + rows - 1) / rows) * ((g.n + cols - 1) / cols) * g.groups; };
     const int nslab = (g.k + BK - 1) / BK;
@@ -1113,8 +1120,16 @@ int gemm_shape(const GemmArgs& g, int cus) {
     return best;
 }
 void gemm_shape_tile(int shape, int* rows, int* cols) {
-    *rows = shape < 0 ? gemm::BM : 32 * gemm::kPipe[shape].ti;
-    *cols = shape < 0 ? gemm::BN : 32 * gemm::kPipe[shape].tj;
+    *rows = shape == kGemmUnstaged ? 64 : shape < 0 ? gemm::BM : 32 * gemm::kPipe[shape].ti;
+    *cols = shape == kGemmUnstaged ? 64 : shape < 0 ? gemm::BN : 32 * gemm::kPipe[shape].tj;
+}
+
+int32_t gemm_launch_rows(int32_t rows, int64_t ld, int32_t k) {
+    const uint64_t most = kGemmSpanLimit / 2; // elements
+    if ((uint64_t)k > most) return 0;
+    if (rows == 1 || (uint64_t)(rows - 1) * (uint64_t)ld + (uint64_t)k <= most) return rows;
+    const uint64_t fit = (most - (uint64_t)k) / (uint64_t)ld + 1; // < rows
+    return (int32_t)(fit >= 256 ? fit & ~uint64_t{255} : fit);
 }
 
 // f32 activations are rounded to the weight's type once, ahead of the product.
@@ -1128,12 +1143,16 @@ hipError_t launch_gemm(const GemmArgs& g0, int a_dtype, int w_dtype, int c_dtype
     using namespace gemm;
     typedef unsigned short h16; // a 16-bit operand in the compute type (bf16 or f16 per the weight)
     GemmArgs g = g0;
-    if (a_dtype == kF32 && g.a16 == nullptr) {
-        if (!gemm_rounds_in_place(g)) return hipErrorInvalidValue;
-        if (w_dtype == kBF16) return c_dtype == kF32 ? launch_unstaged<false, float>(g, stream) : launch_unstaged<false, h16>(g, stream);
-        return c_dtype == kF32 ? launch_unstaged<true, float>(g, stream) : launch_unstaged<true, h16>(g, stream);
+    if (a_dtype != kF32 && a_dtype != w_dtype) return hipErrorInvalidValue;
+    if (g.shape == kGemmUnstaged) {
+#define ZD_UNSTAGED(TA) \
+    (w_dtype == kBF16 ? (c_dtype == kF32 ? launch_unstaged<TA, false, float>(g, stream) : launch_unstaged<TA, false, h16>(g, stream)) \
+                      : (c_dtype == kF32 ? launch_unstaged<TA, true, float>(g, stream) : launch_unstaged<TA, true, h16>(g, stream)))
+        return a_dtype == kF32 ? ZD_UNSTAGED(float) : ZD_UNSTAGED(h16);
+#undef ZD_UNSTAGED
     }
     if (a_dtype == kF32) {
+        if (g.a16 == nullptr) return hipErrorInvalidValue;
         const dim3 grid((unsigned)g.m, (unsigned)((g.k + 4095) / 4096));
         if (w_dtype == kF16)
             gemm_round_kernel<true><<<grid, dim3(256), 0, stream>>>(static_cast<const float*>(g.a), g.lda, static_cast<h16*>(g.a16), g.m, g.k);
@@ -1143,8 +1162,6 @@ hipError_t launch_gemm(const GemmArgs& g0, int a_dtype, int w_dtype, int c_dtype
         if (e != hipSuccess) return e;
         g.a = g.a16;
         g.lda = g.k;
-    } else if (a_dtype != w_dtype) {
-        return hipErrorInvalidValue;
     }
     if (w_dtype == kBF16) {
         if (c_dtype == kF32) return launch_one<false, float>(g, stream);
@@ -1156,7 +1173,7 @@ hipError_t launch_gemm(const GemmArgs& g0, int a_dtype, int w_dtype, int c_dtype
     return hipErrorInvalidValue;
 }
 
-void gemm_set_build(int build) { gemm::g_gemm_build = build == 1 ? 1 : 0; }
+void gemm_set_build(int build) { gemm::g_gemm_build = build == 1 || build == 2 ? build : 0; }
 
 hipError_t gemm_setup() {
     using namespace gemm;

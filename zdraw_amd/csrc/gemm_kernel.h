@@ -31,12 +31,23 @@ struct GemmArgs {
     int32_t part_wgs; // set by the launcher
     int32_t pad1;
     // f32 activations: room for A rounded to the weight's type, [m][k] 16-bit (gemm_round_bytes
-    // says how much); null where gemm_rounds_in_place allows it
+    // says how much); unused by kGemmUnstaged
     void* a16;
 };
 
+// The kernels address A and W through buffer descriptors, with 32-bit byte offsets. Those of the four-wave
+// kernels start kGemmDescBias below the operand, and the last slab of a k that is not a multiple of
+// 64 reaches up to 112 bytes past the last row: an operand may span no more than kGemmSpanLimit in one launch.
+constexpr unsigned kGemmDescBias = 3 * 1024;
+constexpr uint64_t kGemmSpanLimit = (1ull << 32) - 1 - kGemmDescBias - 128;
+// How many of `rows` rows of 16-bit elements (`ld` apart, k used) one launch can take: all of them, or
+// what fits (a multiple of 256 where that many do). 0: not even one.
+int32_t gemm_launch_rows(int32_t rows, int64_t ld, int32_t k);
+
 // Kernel and tile for this product on a device with `cus` compute units (GemmArgs::shape): -1 the
 // 256-tiles of gemm_ring_kernel, otherwise an entry of gemm_pipe_kernel's table of tiles.
+// kGemmUnstaged: the kernel that needs neither descriptors nor a rounded copy of f32 activations.
+constexpr int kGemmUnstaged = -2;
 int gemm_shape(const GemmArgs& args, int cus);
 void gemm_shape_tile(int shape, int* rows, int* cols);
 int gemm_tile_rows();
@@ -51,8 +62,8 @@ void gemm_tail_plan(const GemmArgs& args, int cus, int* tail_tiles, int* splits)
 size_t gemm_part_bytes(int tail_tiles, int splits);
 // Bytes of scratch launch_gemm needs for f32 activations rounded ahead of the product (0: none).
 size_t gemm_round_bytes(const GemmArgs& args, int a_dtype);
-// Whether launch_gemm takes f32 activations without that scratch (slower, same bits).
+// Whether f32 activations may run without that scratch, as kGemmUnstaged (slower, same bits).
 bool gemm_rounds_in_place(const GemmArgs& args);
-void gemm_set_build(int build); // 256-tiles of 16-bit activations: 1 = four-wave build (default), 0 = eight-wave build
+void gemm_set_build(int build); // 256-tiles of 16-bit activations: 1 = four-wave build (default), 0 = eight-wave build; 2 = every product as kGemmUnstaged
 
 } // namespace zdraw
