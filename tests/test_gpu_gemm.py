@@ -630,7 +630,7 @@ def test_operand_that_spans_almost_4_gib(ctx, side, k, count):
 
 # The kernel without descriptors or scratch, which serves rows that no descriptor reaches the end of and
 # f32 activations under capture: 16-bit and f32 activations, edges of its tiles, against the oracle.
-@pytest.mark.parametrize("m,k,n", [(1, 8, 1), (64, 64, 64), (130, 200, 77)])
+@pytest.mark.parametrize("m,k,n", [(1, 8, 1), (64, 64, 64), (130, 200, 77), (1930, 136, 1931)])  # the last: 128-tiles
 @pytest.mark.parametrize("wdt", [hip.W_BF16, hip.W_F16])
 @pytest.mark.parametrize("a16", [False, True])
 def test_kernel_that_addresses_through_pointers(ctx, m, k, n, wdt, a16):
@@ -647,14 +647,17 @@ def test_kernel_that_addresses_through_pointers(ctx, m, k, n, wdt, a16):
     check(got.view(np.float32).reshape(m, n), zo.linear_batch(ar, wr), zo.linear_batch(a, wr), k, a, wr, f"{m}x{k}x{n}")
 
 
-# edges of the 64 x 64 tiles and of the 32-wide steps, the smallest product, a k of whole slabs
+# edges of the 64 x 64 tiles and of the 32-wide steps, the smallest product, a k of whole slabs; under
+# capture on a queue that has no scratch yet, and on one whose scratch has room for the copy of A
 @pytest.mark.parametrize("m,k,n,count", [(1, 8, 1, 1), (64, 64, 64, 2), (77, 200, 131, 3), (300, 264, 70, 1)])
 @pytest.mark.parametrize("wdt", [hip.W_BF16, hip.W_F16])
 @pytest.mark.parametrize("c16", [False, True])
-def test_f32_activations_on_a_queue_under_capture_that_has_no_scratch(ctx, m, k, n, count, wdt, c16):
-    # The rounded copy of A may not be allocated under capture: the product rounds its rows on the
-    # way instead. Same roundings and the same order of sums, so the bits are those of the call
-    # with scratch; every replay of the graph writes them.
+@pytest.mark.parametrize("warm", [False, True])
+def test_f32_activations_under_capture_take_no_scratch(ctx, m, k, n, count, wdt, c16, warm):
+    # The rounded copy of A may not be allocated under capture, and a graph must not hold the address of
+    # a slot that a larger call replaces: the product rounds its rows on the way instead, in one
+    # kernel. Same roundings and the same order of sums, so the bits are those of the call with
+    # scratch; every replay of the graph writes them, also after the slot has grown.
     L = hip.lib()
     rng = np.random.default_rng(m + n + k)
     a = rng.standard_normal((m, k), dtype=np.float32)
@@ -679,11 +682,21 @@ def test_f32_activations_on_a_queue_under_capture_that_has_no_scratch(ctx, m, k,
     queue = L.zdraw_hip_create_queue(ctx.device)
     stream = C.c_void_p((C.c_void_p * 2).from_address(queue)[1])  # a queue is a device and a stream
     graph, run = C.c_void_p(), C.c_void_p()
+    big_m, big_k, big_n = 700, 512, 64
+    big = [ctx.buffer(np.ones((big_m, big_k), np.float32)), ctx.buffer(np.zeros((big_n, big_k), np.uint16)), ctx.buffer(nbytes=big_m * big_n * 4)]
+    big_p, big_x = hip.GemmParams(big_m, big_k, big_n, wdt, hip.GEMM_HALF, 0), hip.GemmExt(0, 0, 0, 0, 0, hip.F32, hip.F32)
+    if warm:
+        batch = L.zdraw_hip_batch_begin(queue)
+        assert enqueue(batch) == 0, hip.last_error()
+        assert L.zdraw_hip_batch_end(batch) == 0
     batch = L.zdraw_hip_batch_begin(queue)
     assert L.hipStreamBeginCapture(stream, C.c_int(2)) == 0
     rc = enqueue(batch)
     assert L.hipStreamEndCapture(stream, C.byref(graph)) == 0
     assert rc == 0, hip.last_error()
+    nodes = C.c_size_t(0)
+    assert L.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0
+    assert nodes.value == 1  # the product alone: no launch that writes a copy of A
     assert L.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
     for replay in range(3):
         for b in cbs:
@@ -692,8 +705,10 @@ def test_f32_activations_on_a_queue_under_capture_that_has_no_scratch(ctx, m, k,
         assert L.hipStreamSynchronize(stream) == 0
         for i, b in enumerate(cbs):
             assert np.array_equal(b.read(np.uint8, (nbytes,)), want[i]), f"replay {replay}, product {i}"
+        if replay == 0:  # a larger product of the same queue replaces the slot
+            assert L.zdraw_hip_run_gemm_ext_enc(batch, *(b.handle for b in big), C.byref(big_p), C.byref(big_x)) == 0, hip.last_error()
     assert L.zdraw_hip_batch_end(batch) == 0
     assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
-    for b in [ab, wb] + cbs:
+    for b in [ab, wb] + cbs + big:
         b.release()
     L.zdraw_hip_release_queue(queue)

@@ -221,11 +221,15 @@ Buffer* queue_scratch(Queue* q, int slot, size_t bytes) {
     return grow_slot(&q->scratch[slot], slot, bytes, [q] { (void)hipStreamSynchronize(q->stream); });
 }
 
+// Whether what is enqueued now becomes part of a graph.
+bool capturing(const Queue* q) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(q->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
 // Whether a slot of the queue has the room, or may be grown now (a stream under capture may not allocate).
 bool may_grow(const Queue* q, int slot, size_t bytes) {
-    if (q->scratch[slot] && q->scratch[slot]->len >= bytes) return true;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(q->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+    return (q->scratch[slot] && q->scratch[slot]->len >= bytes) || !capturing(q);
 }
 
 // Where a call's scratch comes from: the grow-only slots of the queue the call runs on,
@@ -1005,13 +1009,15 @@ int enqueue_gemm_group(void* a, void* const* ws, void* const* cs, const uint64_t
     g.tiles_n = (int32_t)((p->n + (uint32_t)gemm_tile_cols() - 1) / (uint32_t)gemm_tile_cols());
     if ((uint64_t)g.tiles_n * (uint64_t)groups * ((p->m + (uint32_t)gemm_tile_rows() - 1) / (uint32_t)gemm_tile_rows()) > 0x7fffffffull)
         return unavailable("grid too large");
-    bool unstaged = false;
+    bool unstaged = false, in_place = false;
     int a_dtype = (int)x->a_dtype;
     if (const size_t rb = gemm_round_bytes(g, a_dtype)) {
         // f32 activations are rounded to the weight's type once, into scratch slot 6, and the
         // product then runs as for 16-bit activations
-        const bool in_place = gemm_rounds_in_place(g);
-        Buffer* a16 = in_place && !may_grow(queue, 6, rb) ? nullptr : queue_scratch(queue, 6, rb);
+        // (a product that can run without the copy keeps its address out of a graph: the slot may be
+        // replaced by a larger one, and another stream may replay the graph while this queue works)
+        in_place = gemm_rounds_in_place(g);
+        Buffer* a16 = in_place && capturing(queue) ? nullptr : queue_scratch(queue, 6, rb);
         if (!a16 && !in_place) {
             set_err("scratch allocation failed");
             return ZDRAW_HIP_ERR_HANDLE;
@@ -1047,13 +1053,17 @@ int enqueue_gemm_group(void* a, void* const* ws, void* const* cs, const uint64_t
                 gemm_tail_plan(piece, queue->dev->cus, &tail, &splits);
                 if (splits > 1) {
                     Buffer* part = queue_scratch(queue, 5, gemm_part_bytes(tail, splits));
-                    if (!part) {
+                    if (!part && !in_place) {
                         set_err("scratch allocation failed");
                         return ZDRAW_HIP_ERR_HANDLE;
                     }
-                    piece.splits = splits;
-                    piece.tile_base = tail; // launch_gemm reads the tail size here
-                    piece.part = static_cast<float*>(part->ptr);
+                    if (part) {
+                        piece.splits = splits;
+                        piece.tile_base = tail; // launch_gemm reads the tail size here
+                        piece.part = static_cast<float*>(part->ptr);
+                    } else {
+                        (void)hipGetLastError(); // as above; the last round stays whole
+                    }
                 }
             }
             hipError_t e = launch_gemm(piece, a_dtype, (int)wt, (int)x->c_dtype, queue->stream);

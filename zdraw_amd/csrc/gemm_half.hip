@@ -16,7 +16,7 @@
 //   * gemm_pipe_kernel: nine tiles from 64 x 64 to 256 x 160 with three or four slabs in LDS, for
 //     problems that do not fill the chip with 256-tiles, and for any k that is not a multiple of 64;
 //   * f32 activations are rounded to the weight's type by a launch of their own;
-//   * gemm_unstaged_kernel: what neither can take (no room for that rounded copy, rows of 4 GiB);
+//   * gemm_unstaged_kernel: what neither can take (no rounded copy under capture, rows of 4 GiB);
 //   * two or three products of one A with equal shapes (q/k/v, gate/up) run as one launch
 //     whose tiles cover all of them;
 //   * fixed summation order and no atomics (a thinly filled last round is cut along k and
@@ -893,74 +893,108 @@ __global__ void __launch_bounds__(256) gemm_round_kernel(const float* a, int64_t
     }
 }
 
-// f32 activations where there is no room for their rounded copy (a queue under capture that has not
-// grown its scratch yet), and rows so long that a descriptor does not reach their end: each 64 x 64
-// tile reads its rows through pointers and rounds them on their way into LDS, one
-// 32-wide step in flight. Bound by the wait for memory in every step, so it is the way out and never
-// the choice. The MFMAs add k in the order of the other kernels: same bits.
-template <typename TA, bool F16, typename TC>
+// f32 activations where there is no room for their rounded copy or none may be taken (a queue under
+// capture), and rows so long that a descriptor does not reach their end: each (32 TI) x (32 TI)
+// tile reads its rows through pointers and rounds them on their way into LDS, the next
+// 64-wide slab on its way in registers. Bound by that slab's wait for memory, or (many tiles) by what the
+// tiles read from L2: the way out and never the choice (f32 A, us: 77 x 3072 x 3 x 3072 39, 600 x 3000 x 3 x
+// 3000 91, 4096 x 3000 x 3000 146). The MFMAs add k in the order of the other kernels: same bits.
+template <typename TA, bool F16, typename TC, int TI>
 __global__ void __launch_bounds__(256) gemm_unstaged_kernel(const GemmArgs g) {
-    constexpr int T = 64, KS = 32, PITCH = KS * 2 + 16; // bytes per LDS row
+    constexpr bool F32 = std::is_same<TA, float>::value;
+    constexpr int T = 32 * TI, PITCH = BK * 2 + 16; // bytes per LDS row
+    constexpr int CPT = T * BK / (256 * 8);         // 8-element chunks of a slab per thread and operand
     __shared__ __attribute__((aligned(16))) unsigned char sa[T * PITCH], sw[T * PITCH];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c16 = lane & 15, q4 = lane >> 4;
     const int wm = wave >> 1, wn = wave & 1;
-    const int row_tiles = g.tiles_n * g.groups;
-    const int tm = (int)blockIdx.x / row_tiles;
-    int tn = (int)blockIdx.x - tm * row_tiles;
+    int tm, tn;
+    tile_coords(logical_tile((int)blockIdx.x, (int)gridDim.x), (g.m + T - 1) / T, g.tiles_n * g.groups, tm, tn);
     const int grp = tn / g.tiles_n;
     tn -= grp * g.tiles_n;
     const void* const wp = grp == 0 ? g.w : g.w_more[grp - 1];
     void* const cp = grp == 0 ? g.c : g.c_more[grp - 1];
     const int m0 = tm * T, n0 = tn * T;
-    // thread = 8 k of one row of either operand; rows past the edge re-read the last one, never stored
-    const int r = tid >> 2, c = (tid & 3) * 8;
-    const TA* const arow = static_cast<const TA*>(g.a) + (int64_t)min(m0 + r, g.m - 1) * g.lda;
-    const unsigned short* const wrow = static_cast<const unsigned short*>(wp) + (int64_t)min(n0 + r, g.n - 1) * g.ldw;
-    f32x4 acc[2][2];
+    // thread = chunk c of rows r, r + 32, .. of either operand; rows past the edge re-read the last one, never stored
+    const int r = tid >> 3, c = (tid & 7) * 8;
+    const TA* arow[CPT];
+    const unsigned short* wrow[CPT];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (unsigned k0 = 0; k0 < (unsigned)g.k; k0 += KS) { // (k may be just short of 2^31)
-        const bool keep = k0 + c < (unsigned)g.k; // (k is a multiple of 8: a group is whole or past the end)
-        const unsigned at = keep ? k0 + c : 0;
-        u32x4 wv = *reinterpret_cast<const u32x4*>(wrow + at), av;
-        if constexpr (std::is_same<TA, float>::value) {
-            const f32x4 lo = *reinterpret_cast<const f32x4*>(arow + at), hi = *reinterpret_cast<const f32x4*>(arow + at + 4);
-            f32x8 v;
-#pragma unroll
-            for (int i = 0; i < 4; i++) { v[i] = lo[i]; v[4 + i] = hi[i]; }
-            if constexpr (F16) av = __builtin_bit_cast(u32x4, __builtin_convertvector(v, f16x8));
-            else av = __builtin_bit_cast(u32x4, __builtin_convertvector(v, bf16x8));
-        } else {
-            av = *reinterpret_cast<const u32x4*>(arow + at);
-        }
-        if (!keep) av = wv = u32x4{0u, 0u, 0u, 0u};
-        __syncthreads(); // the last step's fragments have been read
-        *reinterpret_cast<u32x4*>(sa + r * PITCH + c * 2) = av;
-        *reinterpret_cast<u32x4*>(sw + r * PITCH + c * 2) = wv;
-        __syncthreads();
-        u32x4 fa[2], fw[2];
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            fa[i] = *reinterpret_cast<const u32x4*>(sa + (wm * 32 + i * 16 + c16) * PITCH + q4 * 16);
-            fw[i] = *reinterpret_cast<const u32x4*>(sw + (wn * 32 + i * 16 + c16) * PITCH + q4 * 16);
-        }
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) mfma16<F16>(fw[j], fa[i], acc[i][j]);
-        mfma16_drain();
+    for (int u = 0; u < CPT; u++) {
+        arow[u] = static_cast<const TA*>(g.a) + (int64_t)min(m0 + r + 32 * u, g.m - 1) * g.lda;
+        wrow[u] = static_cast<const unsigned short*>(wp) + (int64_t)min(n0 + r + 32 * u, g.n - 1) * g.ldw;
     }
-    store_tile16<F16, TC, 2, 2>(g, cp, acc, m0 + wm * 32, n0 + wn * 32, lane);
+    f32x4 acc[TI][TI];
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < TI; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const unsigned k = (unsigned)g.k; // (may be just short of 2^31)
+    constexpr int AV = F32 ? 2 : 1;   // 16-byte loads per chunk of A
+    u32x4 av[CPT * AV], wv[CPT];
+    auto load = [&](unsigned k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < CPT; u++) {
+            const unsigned at = k0 + c < k ? k0 + c : 0; // (k is a multiple of 8: a chunk is whole or past the end)
+#pragma unroll
+            for (int x = 0; x < AV; x++) av[u * AV + x] = *reinterpret_cast<const u32x4*>(arow[u] + at + 4 * x);
+            wv[u] = *reinterpret_cast<const u32x4*>(wrow[u] + at);
+        }
+    };
+    load(0);
+    for (unsigned k0 = 0; k0 < k; k0 += BK) {
+        u32x4 ah[CPT], wh[CPT];
+#pragma unroll
+        for (int u = 0; u < CPT; u++) {
+            if constexpr (F32) {
+                f32x8 v;
+#pragma unroll
+                for (int i = 0; i < 8; i++) v[i] = __uint_as_float(av[2 * u + (i >> 2)][i & 3]);
+                if constexpr (F16) ah[u] = __builtin_bit_cast(u32x4, __builtin_convertvector(v, f16x8));
+                else ah[u] = __builtin_bit_cast(u32x4, __builtin_convertvector(v, bf16x8));
+            } else {
+                ah[u] = av[u];
+            }
+            wh[u] = wv[u];
+            if (k0 + c >= k) ah[u] = wh[u] = u32x4{0u, 0u, 0u, 0u};
+        }
+        __syncthreads(); // the last slab's fragments have been read
+#pragma unroll
+        for (int u = 0; u < CPT; u++) {
+            *reinterpret_cast<u32x4*>(sa + (r + 32 * u) * PITCH + c * 2) = ah[u];
+            *reinterpret_cast<u32x4*>(sw + (r + 32 * u) * PITCH + c * 2) = wh[u];
+        }
+        __syncthreads();
+        if (k - k0 > BK) load(k0 + BK);
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+            u32x4 fa[TI], fw[TI];
+#pragma unroll
+            for (int i = 0; i < TI; i++) {
+                fa[i] = *reinterpret_cast<const u32x4*>(sa + ((wm * TI + i) * 16 + c16) * PITCH + ks * 64 + q4 * 16);
+                fw[i] = *reinterpret_cast<const u32x4*>(sw + ((wn * TI + i) * 16 + c16) * PITCH + ks * 64 + q4 * 16);
+            }
+#pragma unroll
+            for (int i = 0; i < TI; i++)
+#pragma unroll
+                for (int j = 0; j < TI; j++) mfma16<F16>(fw[j], fa[i], acc[i][j]);
+            mfma16_drain();
+        }
+    }
+    store_tile16<F16, TC, TI, TI>(g, cp, acc, m0 + wm * (16 * TI), n0 + wn * (16 * TI), lane);
 }
+// From this many 128-tiles on they are taken instead of 64-tiles (us, 64 against 128: 192 tiles 46 / 65, 240
+// 71 / 72, 360 111 / 91, 768 215 / 146).
+constexpr int kUnstagedLargeTiles = 240;
 template <typename TA, bool F16, typename TC>
 static hipError_t launch_unstaged(GemmArgs g, hipStream_t stream) {
-    g.tiles_n = (g.n + 63) / 64;
-    const int64_t nwg = (int64_t)((g.m + 63) / 64) * g.tiles_n * g.groups;
+    auto count = [&](int t) { return (int64_t)((g.m + t - 1) / t) * ((g.n + t - 1) / t) * g.groups; };
+    const int t = count(128) >= kUnstagedLargeTiles ? 128 : 64;
+    g.tiles_n = (g.n + t - 1) / t;
+    const int64_t nwg = count(t);
     if (nwg <= 0 || nwg > 0x7fffffff) return hipErrorInvalidValue;
-    gemm_unstaged_kernel<TA, F16, TC><<<dim3((unsigned)nwg), dim3(256), 0, stream>>>(g);
+    if (t == 128) gemm_unstaged_kernel<TA, F16, TC, 4><<<dim3((unsigned)nwg), dim3(256), 0, stream>>>(g);
+    else gemm_unstaged_kernel<TA, F16, TC, 2><<<dim3((unsigned)nwg), dim3(256), 0, stream>>>(g);
     return hipGetLastError();
 }
 
