@@ -922,6 +922,58 @@ def test_plain_f32_rows_either_side_of_the_rounding_launch(ctx, tokens, valid, l
     refimpl.check_close(got, zo.attention_run(q, k, v, oracle_cfg(cfg)), f"plain {tokens} valid={valid}")
 
 
+# A captured plain f32 call of 160 to 1023 tokens holds no scratch address (it can run without the rounded
+# copies): one kernel in the graph, on a queue without scratch and on one whose slots have room. A
+# longer call replaces the slots between the replays; every row of every replay against the oracle.
+@pytest.mark.parametrize("warm", [False, True])
+@pytest.mark.parametrize("tokens,heads", [(160, 3), (239, 2)])
+def test_short_plain_f32_rows_under_capture_take_no_scratch(ctx, tokens, heads, warm):
+    L = hip.lib()
+    rng = np.random.default_rng(tokens)
+    shape = (tokens, heads, 128)
+    q, k, v = (rng.standard_normal(shape, dtype=np.float32) * 0.5 for _ in range(3))
+    want = zo.attention_run(q, k, v, zo.Config(tokens, heads, heads, 128))
+    bufs = [ctx.buffer(a) for a in (q, k, v)] + [ctx.buffer(nbytes=q.size * 4)]
+    big = [ctx.buffer(np.zeros((1024, heads, 128), np.float32)) for _ in range(4)]
+
+    def enqueue(batch, b, n):
+        p, x = hip.AttnParams(n, heads, heads, 128, 0, 0), hip.AttnExt()
+        for s_ in (x.q_stride, x.k_stride, x.v_stride, x.out_stride):
+            s_[0], s_[1], s_[2] = 0, heads * 128, 128
+        x.batch, x.in_dtype, x.out_dtype, x.qk_mode = 1, hip.F32, hip.F32, hip.QK_NONE
+        return L.zdraw_hip_run_attention_fused_enc(batch, *(i.handle for i in b), C.byref(p), C.byref(x), None)
+
+    queue = L.zdraw_hip_create_queue(ctx.device)
+    stream = C.c_void_p((C.c_void_p * 2).from_address(queue)[1])  # a queue is a device and a stream
+    if warm:
+        batch = L.zdraw_hip_batch_begin(queue)
+        d0 = L.zdraw_hip_dispatch_count()
+        assert enqueue(batch, bufs, tokens) == 0, hip.last_error()
+        assert L.zdraw_hip_dispatch_count() - d0 == 2  # not under capture: the copies, then the kernel
+        assert L.zdraw_hip_batch_end(batch) == 0
+    graph, run, nodes = C.c_void_p(), C.c_void_p(), C.c_size_t(0)
+    batch = L.zdraw_hip_batch_begin(queue)
+    assert L.hipStreamBeginCapture(stream, C.c_int(2)) == 0
+    rc = enqueue(batch, bufs, tokens)
+    assert L.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert rc == 0, hip.last_error()
+    assert L.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0
+    assert nodes.value == 1
+    assert L.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    for replay in range(3):
+        bufs[3].write(np.full(q.size * 4, 0x7B, np.uint8))
+        assert L.hipGraphLaunch(run, stream) == 0
+        assert L.hipStreamSynchronize(stream) == 0
+        refimpl.check_close(bufs[3].read(np.float32, shape), want, f"replay {replay}")
+        if replay == 0:
+            assert enqueue(batch, big, 1024) == 0, hip.last_error()
+    assert L.zdraw_hip_batch_end(batch) == 0
+    assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
+    for b in bufs + big:
+        b.release()
+    L.zdraw_hip_release_queue(queue)
+
+
 # first, a middle and the last key block; rising, so that the reference moves at each of them
 PLANT_CASES = [
     # name, tokens, heads, in_dtype, valid, planted (key, nats), whole tiles only (knob 2)

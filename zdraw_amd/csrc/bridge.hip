@@ -227,11 +227,6 @@ bool capturing(const Queue* q) {
     return hipStreamIsCapturing(q->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
 
-// Whether a slot of the queue has the room, or may be grown now (a stream under capture may not allocate).
-bool may_grow(const Queue* q, int slot, size_t bytes) {
-    return (q->scratch[slot] && q->scratch[slot]->len >= bytes) || !capturing(q);
-}
-
 // Where a call's scratch comes from: the grow-only slots of the queue the call runs on,
 // or a caller-supplied span handed out piece by piece in 256-byte steps (the entry that
 // allocates nothing), or nowhere (a plan that is only validated).
@@ -249,18 +244,14 @@ struct ScratchSource {
 // Plain f32 attention from this length on rounds its operands once, ahead of the kernel, which then takes
 // two key groups and more: call on resident rows, two heads, 256 tokens 31.9 -> 31.3 us, 512 35.8 -> 33.9,
 // 24 heads 700 tokens 51.4 -> 44.5. At 128 tokens and below one launch is as fast as two (64 tokens, 24
-// heads: 25.5 against 26.5). Below kRoundAlwaysTokens only where the copies cost no one an allocation
-// that is not allowed (plain_may_round).
+// heads: 25.5 against 26.5). Below kRoundAlwaysTokens only where plain_may_round allows it.
 constexpr uint32_t kRoundPlainTokens = 160, kRoundAlwaysTokens = 1024;
 
 // Whether a plain f32 call shorter than kRoundAlwaysTokens may take the three scratch slots of the
-// rounding launch: from a queue whose slots are large enough already or may grow now (a stream
-// under capture may not allocate), not from a caller's span.
-bool plain_may_round(const ScratchSource* src, size_t bytes) {
-    if (!src->queue || src->dry || src->span) return false;
-    for (int i = 0; i < 3; i++)
-        if (!may_grow(src->queue, i, bytes)) return false;
-    return true;
+// rounding launch: not under capture, whatever the slots hold (it can run without, and its graph then
+// holds no address of a slot that a larger call replaces), and not from a caller's span.
+bool plain_may_round(const ScratchSource* src) {
+    return src->queue && !src->dry && !src->span && !capturing(src->queue);
 }
 
 struct FusedPlan {
@@ -453,7 +444,7 @@ int plan_attention(Device* dev, void* q, void* k, void* v, void* out, const Zdra
     int tail = 0, splits = 1;
     // the kernel will read prepared 16-bit operands (or bf16 ones as given): its shape is a choice
     const bool round_plain = x->qk_mode == ZDRAW_HIP_QK_NONE && x->in_dtype == ZDRAW_HIP_F32 && p->tokens >= kRoundPlainTokens &&
-                             (p->tokens >= kRoundAlwaysTokens || plain_may_round(src, (size_t)x->batch * p->heads * p->tokens * kHeadDim * 2));
+                             (p->tokens >= kRoundAlwaysTokens || plain_may_round(src));
     const bool direct = x->qk_mode != ZDRAW_HIP_QK_NONE ? x->k_site == ZDRAW_HIP_K_PREPASS
                                                          : x->in_dtype == ZDRAW_HIP_BF16 || stage_f16 || round_plain;
     if (direct && g_variant == 0)
