@@ -46,6 +46,10 @@ void zdraw_hip_gemm_tile(uint32_t m, uint32_t k, uint32_t n, uint32_t groups, ui
  * 32-bit offsets. A product is cut accordingly. Host arithmetic only. */
 void zdraw_hip_gemm_launch_rows(uint32_t rows, uint64_t ld, uint32_t k, uint32_t* per_launch);
 
+/* From here on a scratch slot may not grow past `bytes`: what a call does when the device has no
+ * more memory. 0 = no limit (default). */
+void zdraw_hip_set_scratch_limit(size_t bytes);
+
 /* How many query tiles (128 rows) of the last wide-head launch had a score outgrow its row's
  * fixed reference point and were formed again by the running-maximum kernel (waits for that
  * launch). 0 on ordinary data; -1 if no wide-head launch has been made or the read failed. */

@@ -922,6 +922,39 @@ def test_plain_f32_rows_either_side_of_the_rounding_launch(ctx, tokens, valid, l
     refimpl.check_close(got, zo.attention_run(q, k, v, oracle_cfg(cfg)), f"plain {tokens} valid={valid}")
 
 
+# Without memory for the rounded copies a plain f32 call of 160 to 1023 tokens still runs, in one kernel that
+# needs none; one of 1024 tokens, which always needed them, reports it; and the queue goes on.
+def test_plain_f32_rows_without_memory_for_their_rounded_copies(ctx):
+    L = hip.lib()
+    rng = np.random.default_rng(7)
+    queue = L.zdraw_hip_create_queue(ctx.device)
+
+    def run(tokens):
+        q, k, v = (rng.standard_normal((tokens, 2, 128), dtype=np.float32) * 0.5 for _ in range(3))
+        bufs = [ctx.buffer(a) for a in (q, k, v)] + [ctx.buffer(nbytes=q.size * 4)]
+        p, x = hip.AttnParams(tokens, 2, 2, 128, 0, 0), hip.AttnExt()
+        for s_ in (x.q_stride, x.k_stride, x.v_stride, x.out_stride):
+            s_[0], s_[1], s_[2] = 0, 256, 128
+        x.batch, x.in_dtype, x.out_dtype, x.qk_mode = 1, hip.F32, hip.F32, hip.QK_NONE
+        d0 = L.zdraw_hip_dispatch_count()
+        rc = L.zdraw_hip_run_attention_fused(queue, *(b.handle for b in bufs), C.byref(p), C.byref(x), None)
+        if rc == 0:
+            refimpl.check_close(bufs[3].read(np.float32, q.shape), zo.attention_run(q, k, v, zo.Config(tokens, 2, 2, 128)), f"{tokens} tokens")
+        for b in bufs:
+            b.release()
+        return rc, L.zdraw_hip_dispatch_count() - d0
+
+    try:
+        L.zdraw_hip_set_scratch_limit(1)
+        assert run(239) == (0, 1)
+        assert run(1024) == (hip.ERR_HANDLE, 0)
+        assert "scratch" in hip.last_error()
+    finally:
+        L.zdraw_hip_set_scratch_limit(0)
+    assert run(239) == (0, 2)
+    L.zdraw_hip_release_queue(queue)
+
+
 # A captured plain f32 call of 160 to 1023 tokens holds no scratch address (it can run without the rounded
 # copies): one kernel in the graph, on a queue without scratch and on one whose slots have room. A
 # longer call replaces the slots between the replays; every row of every replay against the oracle.

@@ -712,3 +712,31 @@ def test_f32_activations_under_capture_take_no_scratch(ctx, m, k, n, count, wdt,
     for b in [ab, wb] + cbs + big:
         b.release()
     L.zdraw_hip_release_queue(queue)
+
+
+def test_f32_activations_without_memory_for_their_rounded_copy(ctx):
+    # a product of less than a 256-tile runs without the copy, with the same bits; a larger one reports it
+    L = hip.lib()
+    rng = np.random.default_rng(8)
+    m, k, n = 77, 200, 131
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    w_bits, _ = to16(rng.standard_normal((n, k), dtype=np.float32), hip.W_BF16)
+    want = run_ext(ctx, a, w_bits, m, k, n, hip.W_BF16, hip.F32, hip.F32)
+    queue = L.zdraw_hip_create_queue(ctx.device)
+    bufs = [ctx.buffer(a), ctx.buffer(w_bits), ctx.buffer(nbytes=m * n * 4)]
+    big = [ctx.buffer(nbytes=256 * 64 * 4), ctx.buffer(nbytes=256 * 64 * 2), ctx.buffer(nbytes=256 * 256 * 4)]
+    ext = hip.GemmExt(0, 0, 0, 0, 0, hip.F32, hip.F32)
+    batch = L.zdraw_hip_batch_begin(queue)
+    try:
+        L.zdraw_hip_set_scratch_limit(1)
+        assert L.zdraw_hip_run_gemm_ext_enc(batch, *(b.handle for b in bufs), C.byref(hip.GemmParams(m, k, n, hip.W_BF16, hip.GEMM_HALF, 0)),
+                                            C.byref(ext)) == 0, hip.last_error()
+        assert L.zdraw_hip_run_gemm_ext_enc(batch, *(b.handle for b in big), C.byref(hip.GemmParams(256, 64, 256, hip.W_BF16, hip.GEMM_HALF, 0)),
+                                            C.byref(ext)) == hip.ERR_HANDLE
+    finally:
+        L.zdraw_hip_set_scratch_limit(0)
+        assert L.zdraw_hip_batch_end(batch) == 0
+    assert np.array_equal(bufs[2].read(np.uint8, (m * n * 4,)), want)
+    for b in bufs + big:
+        b.release()
+    L.zdraw_hip_release_queue(queue)

@@ -188,6 +188,7 @@ bool need(const void* handle, size_t bytes) {
 }
 
 bool scratch_poisoned(int slot);
+size_t g_scratch_limit = 0; // measurement header: slots larger than this cannot be had (0: no limit)
 
 // (Re)allocation of a grow-only scratch slot. `wait` drains whatever may still read the old
 // allocation before it is freed; the new one is filled (0x00, or 0xFF under
@@ -199,7 +200,8 @@ Buffer* grow_slot(Buffer** slot_ptr, int slot, size_t bytes, Wait wait) {
     if (cur && cur->len >= bytes) return cur;
     wait();
     void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
+    if ((g_scratch_limit != 0 && bytes > g_scratch_limit) || hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError(); // or the next launch would report the failed allocation
         set_err("scratch hipMalloc(%zu) failed", bytes);
         return nullptr;
     }
@@ -248,10 +250,14 @@ struct ScratchSource {
 constexpr uint32_t kRoundPlainTokens = 160, kRoundAlwaysTokens = 1024;
 
 // Whether a plain f32 call shorter than kRoundAlwaysTokens may take the three scratch slots of the
-// rounding launch: not under capture, whatever the slots hold (it can run without, and its graph then
-// holds no address of a slot that a larger call replaces), and not from a caller's span.
-bool plain_may_round(const ScratchSource* src) {
-    return src->queue && !src->dry && !src->span && !capturing(src->queue);
+// rounding launch, of `bytes` each: not under capture, whatever the slots hold (it can run without, and its
+// graph then holds no address of a slot that a larger call replaces), not from a caller's span, and
+// not where there is no memory for them.
+bool plain_may_round(ScratchSource* src, size_t bytes) {
+    if (!src->queue || src->dry || src->span || capturing(src->queue)) return false;
+    for (int i = 0; i < 3; i++)
+        if (!src->get(i, bytes)) return false;
+    return true;
 }
 
 struct FusedPlan {
@@ -444,7 +450,7 @@ int plan_attention(Device* dev, void* q, void* k, void* v, void* out, const Zdra
     int tail = 0, splits = 1;
     // the kernel will read prepared 16-bit operands (or bf16 ones as given): its shape is a choice
     const bool round_plain = x->qk_mode == ZDRAW_HIP_QK_NONE && x->in_dtype == ZDRAW_HIP_F32 && p->tokens >= kRoundPlainTokens &&
-                             (p->tokens >= kRoundAlwaysTokens || plain_may_round(src));
+                             (p->tokens >= kRoundAlwaysTokens || plain_may_round(src, (size_t)x->batch * p->heads * p->tokens * kHeadDim * 2));
     const bool direct = x->qk_mode != ZDRAW_HIP_QK_NONE ? x->k_site == ZDRAW_HIP_K_PREPASS
                                                          : x->in_dtype == ZDRAW_HIP_BF16 || stage_f16 || round_plain;
     if (direct && g_variant == 0)
@@ -872,7 +878,6 @@ int enqueue_wide(Queue* queue, void* q, void* k, void* v, void* out, const Zdraw
         // key ranges leave their shares in scratch slot 3; without room for them the keys stay whole
         Buffer* part = queue_scratch(queue, 3, wide_part_bytes(a.tokens, a.splits));
         if (!part) {
-            (void)hipGetLastError(); // or the next launch would report the failed allocation
             a.splits = 1;
         } else {
             a.part_o = static_cast<float*>(part->ptr);
@@ -1014,7 +1019,6 @@ int enqueue_gemm_group(void* a, void* const* ws, void* const* cs, const uint64_t
             return ZDRAW_HIP_ERR_HANDLE;
         }
         if (a16) g.a16 = a16->ptr;
-        else (void)hipGetLastError(); // or the launch would report the failed allocation
         unstaged = !a16;
     }
     // Pieces of C that one launch can address: the whole but where A or W spans all but 4 GiB (the rounded
@@ -1048,12 +1052,10 @@ int enqueue_gemm_group(void* a, void* const* ws, void* const* cs, const uint64_t
                         set_err("scratch allocation failed");
                         return ZDRAW_HIP_ERR_HANDLE;
                     }
-                    if (part) {
+                    if (part) { // (or the last round stays whole)
                         piece.splits = splits;
                         piece.tile_base = tail; // launch_gemm reads the tail size here
                         piece.part = static_cast<float*>(part->ptr);
-                    } else {
-                        (void)hipGetLastError(); // as above; the last round stays whole
                     }
                 }
             }
@@ -1867,6 +1869,8 @@ size_t zdraw_hip_clock_probe_read(uint64_t* cycles, uint64_t* ref_ticks, size_t 
 }
 
 void zdraw_hip_set_attention_variant(int variant) { g_variant = variant & 3; }
+
+void zdraw_hip_set_scratch_limit(size_t bytes) { g_scratch_limit = bytes; }
 
 void zdraw_hip_set_gemm_build(int build) { gemm_set_build(build); }
 
