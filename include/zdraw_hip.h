@@ -233,7 +233,9 @@ int zdraw_hip_reserve_attention_fused(void* queue, void* q, void* k, void* v, vo
 
 /* The fused entry for callers that cannot allocate (no counterpart in the reference: it is
  * for code under HIP graph capture, tight serving loops and harnesses that forbid hipMalloc).
- * Same arguments, results bit-identical to zdraw_hip_run_attention_fused_enc, but the prepared
+ * Same arguments, results bit-identical to zdraw_hip_run_attention_fused_enc (which keeps plain
+ * f32 rows of 160 to 1023 tokens out of its slots, and rounds them elsewhere, where its stream is
+ * under capture or no memory is left), but the prepared
  * Q and K (the bf16 copy of an f32 V, the parts of key-split tiles) live in an array inside the
  * library's device code instead of the grow-only slots: ZDRAW_HIP_NOALLOC_SCRATCH_BYTES per GPU,
  * held until the process ends. A call that needs more (with bf16 operands:

@@ -66,6 +66,40 @@ def test_noalloc_entry_matches_the_allocating_entry_on_shrinking_calls(ctx):
         assert np.array_equal(got.view(np.uint32), again.view(np.uint32)), name
 
 
+# Plain f32 rows either side of the lengths from which they are rounded ahead of the kernel (160, and
+# 1024 whatever the size), with key-split parts (901 tokens and up), a key limit, both softmax forms,
+# and a batch whose copies do not fit the array (rounded in the tile load by either entry)
+@pytest.mark.parametrize("bounded", [False, True])
+@pytest.mark.parametrize("tokens,heads,batch,valid", [(159, 2, 1, 0), (160, 3, 1, 0), (200, 2, 2, 131), (447, 24, 1, 0), (901, 2, 1, 0),
+                                                      (1023, 5, 1, 1000), (700, 32, 4, 0), (1024, 2, 1, 0)])
+def test_noalloc_entry_gives_the_same_bits_on_plain_f32_rows(ctx, tokens, heads, batch, valid, bounded):
+    L = hip.lib()
+    fits = 3 * batch * heads * tokens * 256 <= hip.NOALLOC_SCRATCH_BYTES
+    assert fits == (batch < 4)
+    rng = np.random.default_rng(tokens)
+    shape = (batch, tokens, heads, 128)
+    bufs = [ctx.buffer(rng.standard_normal(shape, dtype=np.float32) * np.float32(0.5)) for _ in range(3)]
+    bufs.append(ctx.buffer(nbytes=4 * batch * tokens * heads * 128))
+    p, x = hip.AttnParams(tokens, heads, heads, 128, 0, valid), hip.AttnExt()
+    for s in (x.q_stride, x.k_stride, x.v_stride, x.out_stride):
+        s[0], s[1], s[2] = tokens * heads * 128, heads * 128, 128
+    x.batch, x.in_dtype, x.out_dtype, x.qk_mode, x.score_bound = batch, hip.F32, hip.F32, hip.QK_NONE, 40.0 if bounded else 0.0
+    outs = []
+    for fn in (L.zdraw_hip_run_attention_fused_enc, L.zdraw_hip_run_attention_fused_noalloc_enc):
+        bufs[3].write(np.full(bufs[3].nbytes, 0x7B, np.uint8))
+        d0 = L.zdraw_hip_dispatch_count()
+        b = L.zdraw_hip_batch_begin(ctx.queue)
+        rc = fn(b, *(h.handle for h in bufs), C.byref(p), C.byref(x), None)
+        assert L.zdraw_hip_batch_end(b) == 0
+        assert rc == 0, hip.last_error()
+        assert L.zdraw_hip_dispatch_count() - d0 == (2 if tokens >= 160 and fits else 1)
+        outs.append(bufs[3].read(np.uint32, shape))
+    assert np.isfinite(outs[0].view(np.float32)).all() and (outs[0] != 0x7B7B7B7B).all()
+    assert np.array_equal(outs[0], outs[1])
+    for h in bufs:
+        h.release()
+
+
 def test_noalloc_entry_takes_no_device_memory_on_a_new_queue_with_weights_it_sees_first(ctx):
     import torch
 

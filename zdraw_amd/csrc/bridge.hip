@@ -249,14 +249,24 @@ struct ScratchSource {
 // heads: 25.5 against 26.5). Below kRoundAlwaysTokens only where plain_may_round allows it.
 constexpr uint32_t kRoundPlainTokens = 160, kRoundAlwaysTokens = 1024;
 
-// Whether a plain f32 call shorter than kRoundAlwaysTokens may take the three scratch slots of the
-// rounding launch, of `bytes` each: not under capture, whatever the slots hold (it can run without, and its
-// graph then holds no address of a slot that a larger call replaces), not from a caller's span, and
-// not where there is no memory for them.
-bool plain_may_round(ScratchSource* src, size_t bytes) {
-    if (!src->queue || src->dry || src->span || capturing(src->queue)) return false;
+// Whether a plain f32 call shorter than kRoundAlwaysTokens takes the rounding launch: where its three
+// copies and the parts of its key-split tiles fit the array of the entry that allocates nothing, whichever
+// entry is called, so that both give the same bits (with batch 1 they do: 1023 tokens of 30 heads take
+// 24 MB, the parts never more than 34). A queue's slots are not taken under capture, whatever they
+// hold (the call can run without, and its graph then holds no address of a slot that a larger call
+// replaces), and not where there is no memory for them.
+bool plain_may_round(ScratchSource* src, const ZdrawAttnParams* p, uint32_t batch, int key_blocks, int cus) {
+    const size_t copy = (size_t)batch * p->heads * p->tokens * kHeadDim * 2;
+    int shape = 0, tail = 0, splits = 1;
+    attention_plan((int64_t)p->heads * batch, (int)p->tokens, key_blocks, cus, &shape, &tail, &splits);
+    size_t all = 3 * ((copy + 255) & ~size_t{255});
+    if (splits > 1)
+        all += ((attention_part_o_bytes(tail, splits, shape) + 255) & ~size_t{255}) + attention_part_ml_bytes(tail, splits, shape);
+    if (all > kNoallocScratchBytes || src->dry) return false;
+    if (src->span) return true;
+    if (!src->queue || capturing(src->queue)) return false;
     for (int i = 0; i < 3; i++)
-        if (!src->get(i, bytes)) return false;
+        if (!src->get(i, copy)) return false;
     return true;
 }
 
@@ -450,7 +460,7 @@ int plan_attention(Device* dev, void* q, void* k, void* v, void* out, const Zdra
     int tail = 0, splits = 1;
     // the kernel will read prepared 16-bit operands (or bf16 ones as given): its shape is a choice
     const bool round_plain = x->qk_mode == ZDRAW_HIP_QK_NONE && x->in_dtype == ZDRAW_HIP_F32 && p->tokens >= kRoundPlainTokens &&
-                             (p->tokens >= kRoundAlwaysTokens || plain_may_round(src, (size_t)x->batch * p->heads * p->tokens * kHeadDim * 2));
+                             (p->tokens >= kRoundAlwaysTokens || plain_may_round(src, p, x->batch, key_blocks, dev->cus));
     const bool direct = x->qk_mode != ZDRAW_HIP_QK_NONE ? x->k_site == ZDRAW_HIP_K_PREPASS
                                                          : x->in_dtype == ZDRAW_HIP_BF16 || stage_f16 || round_plain;
     if (direct && g_variant == 0)
