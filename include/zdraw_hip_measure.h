@@ -46,6 +46,10 @@ void zdraw_hip_gemm_tile(uint32_t m, uint32_t k, uint32_t n, uint32_t groups, ui
  * 32-bit offsets. A product is cut accordingly. Host arithmetic only. */
 void zdraw_hip_gemm_launch_rows(uint32_t rows, uint64_t ld, uint32_t k, uint32_t* per_launch);
 
+/* Key ranges per query tile of a wide head of `tokens` tokens on a device with `cus` compute units,
+ * and the bytes of scratch that their shares take. Host arithmetic only. */
+void zdraw_hip_wide_ranges(uint32_t tokens, uint32_t cus, uint32_t* ranges, uint64_t* share_bytes);
+
 /* From here on a scratch slot may not grow past `bytes`: what a call does when the device has no
  * more memory. 0 = no limit (default). */
 void zdraw_hip_set_scratch_limit(size_t bytes);

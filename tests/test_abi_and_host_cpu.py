@@ -134,6 +134,26 @@ def test_gemm_rows_of_one_launch_stay_inside_32_bit_offsets():
     assert per_launch(0, 8, 8) == 0 and per_launch(8, 8, 0) == 0
 
 
+def test_wide_head_key_ranges_of_every_length():
+    # no empty range, at least eight blocks in each, and a ceiling on the scratch of their shares
+    L = hip.lib()
+
+    def ranges(tokens, cus=256):
+        n, b = C.c_uint32(99), C.c_uint64(99)
+        L.zdraw_hip_wide_ranges(tokens, cus, C.byref(n), C.byref(b))
+        return n.value, b.value
+
+    for tokens in range(64, 2 ** 20 + 1, 64):
+        n, share = ranges(tokens)
+        assert 1 <= n <= 8 and share == (n * tokens * 514 * 4 if n > 1 else 0) and share <= 512 << 20, tokens
+        blocks = tokens // 32
+        per = -(-blocks // n)
+        assert n == 1 or (per >= 8 and (n - 1) * per < blocks), tokens
+    assert [ranges(t)[0] for t in (256, 448, 4096, 6208, 9600, 16384, 16448, 18432)] == [1, 1, 5, 4, 3, 2, 3, 3]
+    assert ranges(33024)[0] == 6 and ranges(65536)[0] == ranges(1019904)[0] == 1
+    assert ranges(0) == ranges(65) == ranges(2 ** 20 + 64) == (0, 0) and ranges(4096, 0)[0] == 1
+
+
 def test_tail_plan_of_the_baseline_shapes():
     # 256 CUs, one 256-row tile per workgroup: which last rounds are split along the keys
     L = hip.lib()

@@ -173,6 +173,30 @@ def test_wide_head_scores_that_outgrow_the_fixed_reference_take_the_safe_kernel(
     assert got.tobytes() == again.tobytes()
 
 
+def test_wide_head_without_memory_for_the_shares_of_its_key_ranges(ctx):
+    # the keys stay whole
+    L = hip.lib()
+    tokens = 3008
+    n, share = C.c_uint32(), C.c_uint64()
+    L.zdraw_hip_wide_ranges(tokens, 256, C.byref(n), C.byref(share))
+    assert n.value > 1
+    q, k, v = draw(np.random.default_rng(11), tokens)
+    c2 = host.Context.init()  # a queue without scratch
+    try:
+        L.zdraw_hip_set_scratch_limit(tokens * 512 * 2)
+        assert tokens * 512 * 2 < share.value
+        got = c2.run(q, k, v, host.Config(tokens, 1, 1, 512)).reshape(tokens, 1, 512)
+    finally:
+        L.zdraw_hip_set_scratch_limit(0)
+        c2.deinit()
+    rows = [0, 127, tokens // 2, tokens - 65, tokens - 1]
+    want = zo.attention_token_list(q, k, v, zo.Config(tokens, 1, 1, 512), rows)
+    refimpl.check_close(got[rows], want.reshape(len(rows), 1, 512), "whole keys")
+    ranges = ctx.run(q, k, v, host.Config(tokens, 1, 1, 512)).reshape(tokens, 1, 512)
+    refimpl.check_close(got, ranges, "whole keys against key ranges")
+    assert not np.array_equal(got, ranges)  # (the sums run in another order: it was the other form)
+
+
 def test_wide_head_refusals_leave_nothing_enqueued(ctx):
     L = hip.lib()
     d0 = L.zdraw_hip_dispatch_count()

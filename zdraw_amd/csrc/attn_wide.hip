@@ -660,34 +660,41 @@ hipError_t launch_wide_round(const WidePrepArgs& p, hipStream_t stream) {
     return hipGetLastError();
 }
 
+size_t wide_part_bytes(int tokens, int splits) {
+    return splits > 1 ? (size_t)splits * (size_t)tokens * (wide::WD + 2) * sizeof(float) : 0;
+}
 // Key ranges per query tile (one workgroup each, of equal length but for the last, at least eight
 // blocks): the number whose estimate is the smallest. A full round over the CUs takes kFullUs per
 // block of a range (the power limit), a thinly filled one kThinUs (a wave's own chain), in between
 // in proportion; every range's share of O goes to memory and back once. The constants are a fit to
-// 1 to 8 ranges of 256 to 18432 tokens; the rule's pick is the measured best or within 4 % of it.
+// 1 to 8 ranges of 256 to 18432 tokens; the rule's pick is the measured best or within 4 % of it, so
+// ranges that save less than 3 % are not worth their shares (1019904 tokens would take six ranges and 12 GB
+// for 1.5 %), and neither are shares of more than kMaxShareBytes, which the queue keeps (33024 tokens: six
+// ranges, 389 MB, a quarter of the time by the estimate; 18432: three, 108 MB, 11 %).
 // (A power of two that divides the blocks, which this was before, left 6208 tokens, 194 blocks, at
 // two ranges and 98 workgroups: call 163 us against 118 with four; 18432 tokens at one range:
 // 678 against 610 with three.)
 int wide_splits(int tokens, int cus) {
+    constexpr size_t kMaxShareBytes = (size_t)512 << 20;
+    constexpr float kMinGain = 0.03f;
     constexpr float kFullUs = 1.6f, kThinUs = 1.16f, kRoundUs = 4.0f, kMergeUs = 3.0f, kShareBytesPerUs = 2.0e6f;
     if (cus <= 0) return 1;
     const int tiles = (tokens + wide::BQ - 1) / wide::BQ;
     const int nblk = tokens / wide::KB;
     int best = 1;
-    float best_us = INFINITY;
+    float best_us = INFINITY, whole_us = INFINITY;
     for (int s = 1; s <= wide::kMaxSplits; s++) {
+        if (wide_part_bytes(tokens, s) > kMaxShareBytes) break;
         const int per = (nblk + s - 1) / s;
         if (s > 1 && (per < 8 || (s - 1) * per >= nblk)) continue; // (no empty range)
         const int rounds = tiles * s / cus, last = tiles * s % cus;
         float us = (float)rounds * ((float)per * kFullUs + kRoundUs);
         if (last) us += (float)per * fmaxf(kThinUs, kFullUs * (float)last / (float)cus) + kRoundUs;
         if (s > 1) us += kMergeUs + (float)s * (float)tokens * (float)(wide::WD * sizeof(float)) / kShareBytesPerUs;
+        if (s == 1) whole_us = us;
         if (us < best_us) { best_us = us; best = s; }
     }
-    return best;
-}
-size_t wide_part_bytes(int tokens, int splits) {
-    return splits > 1 ? (size_t)splits * (size_t)tokens * (wide::WD + 2) * sizeof(float) : 0;
+    return best_us < whole_us * (1.f - kMinGain) ? best : 1;
 }
 
 hipError_t launch_wide_attention(const WideArgs& a, hipStream_t stream) {

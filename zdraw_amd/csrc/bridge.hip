@@ -1880,6 +1880,13 @@ size_t zdraw_hip_clock_probe_read(uint64_t* cycles, uint64_t* ref_ticks, size_t 
 
 void zdraw_hip_set_attention_variant(int variant) { g_variant = variant & 3; }
 
+void zdraw_hip_wide_ranges(uint32_t tokens, uint32_t cus, uint32_t* ranges, uint64_t* share_bytes) {
+    const bool ok = tokens != 0 && tokens <= (1u << 20) && tokens % (uint32_t)wide_block_rows() == 0;
+    const int n = ok ? wide_splits((int)tokens, (int)cus) : 0;
+    if (ranges) *ranges = (uint32_t)n;
+    if (share_bytes) *share_bytes = ok ? wide_part_bytes((int)tokens, n) : 0;
+}
+
 void zdraw_hip_set_scratch_limit(size_t bytes) { g_scratch_limit = bytes; }
 
 void zdraw_hip_set_gemm_build(int build) { gemm_set_build(build); }
