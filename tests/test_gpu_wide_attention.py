@@ -197,6 +197,50 @@ def test_wide_head_without_memory_for_the_shares_of_its_key_ranges(ctx):
     assert not np.array_equal(got, ranges)  # (the sums run in another order: it was the other form)
 
 
+def test_wide_head_under_capture_does_not_grow_the_slot_of_its_shares(ctx):
+    # a queue whose operand slots have room and whose share slot does not: the capture goes through with
+    # whole keys, and every replay gives the bits of the call without memory for the shares
+    L = hip.lib()
+    tokens = 3008
+    q, k, v = draw(np.random.default_rng(12), tokens)
+    bufs = [ctx.buffer(a) for a in (q, k, v)] + [ctx.buffer(nbytes=q.nbytes)]
+    err = C.create_string_buffer(128)
+    wide = L.zdraw_hip_compile(ctx.device, None, b"attention_wide_mfma", err, 128)
+    p = hip.AttnParams(tokens, 1, 1, 512, 0, 0)
+    queue = L.zdraw_hip_create_queue(ctx.device)
+    stream = C.c_void_p((C.c_void_p * 2).from_address(queue)[1])  # a queue is a device and a stream
+
+    def enqueue(batch):
+        return L.zdraw_hip_run_attention_enc_off(batch, wide, *(b.handle for b in bufs), C.byref(p), hip.K_WIDE, 512, 0, 0)
+
+    batch = L.zdraw_hip_batch_begin(queue)
+    try:
+        L.zdraw_hip_set_scratch_limit(tokens * 512 * 2)
+        assert enqueue(batch) == 0, hip.last_error()
+        assert L.zdraw_hip_batch_end(batch) == 0
+    finally:
+        L.zdraw_hip_set_scratch_limit(0)
+    want = bufs[3].read(np.uint32, q.shape)
+    graph, run = C.c_void_p(), C.c_void_p()
+    batch = L.zdraw_hip_batch_begin(queue)
+    assert L.hipStreamBeginCapture(stream, C.c_int(2)) == 0
+    rc = enqueue(batch)
+    assert L.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert rc == 0, hip.last_error()
+    assert L.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    for replay in range(3):
+        bufs[3].write(np.full(q.nbytes, 0x7B, np.uint8))
+        assert L.hipGraphLaunch(run, stream) == 0
+        assert L.hipStreamSynchronize(stream) == 0
+        assert np.array_equal(bufs[3].read(np.uint32, q.shape), want), f"replay {replay}"
+    assert L.zdraw_hip_batch_end(batch) == 0
+    assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0
+    L.zdraw_hip_release_pipeline(wide)
+    L.zdraw_hip_release_queue(queue)
+    for b in bufs:
+        b.release()
+
+
 def test_wide_head_refusals_leave_nothing_enqueued(ctx):
     L = hip.lib()
     d0 = L.zdraw_hip_dispatch_count()

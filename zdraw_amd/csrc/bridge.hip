@@ -885,8 +885,11 @@ int enqueue_wide(Queue* queue, void* q, void* k, void* v, void* out, const Zdraw
     a.redo = static_cast<int*>(redo->ptr);
     a.splits = wide_splits(a.tokens, queue->dev->cus);
     if (a.splits > 1) {
-        // key ranges leave their shares in scratch slot 3; without room for them the keys stay whole
-        Buffer* part = queue_scratch(queue, 3, wide_part_bytes(a.tokens, a.splits));
+        // key ranges leave their shares in scratch slot 3; without room for them (a stream under capture may
+        // not allocate, and the attempt would end the capture) the keys stay whole
+        const size_t bytes = wide_part_bytes(a.tokens, a.splits);
+        const bool room = queue->scratch[3] && queue->scratch[3]->len >= bytes;
+        Buffer* part = room || !capturing(queue) ? queue_scratch(queue, 3, bytes) : nullptr;
         if (!part) {
             a.splits = 1;
         } else {
