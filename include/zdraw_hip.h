@@ -431,7 +431,9 @@ int zdraw_hip_queue_sync(void* queue);
  * compute units (no reference counterpart: scheduling, exposed so that it can be checked
  * without a device). A last round that fills at most half the CUs is split along the keys:
  * *tail_tiles tiles (the last ones) run as *splits parts each, at least 8 key blocks per part,
- * at most 16 parts; *tail_tiles = 0 and *splits = 1 when everything runs whole. */
+ * at most 16 parts; *tail_tiles = 0 and *splits = 1 when everything runs whole. (A launch of
+ * prepared operands whose 128-row tiles fit the CUs once may take those instead, whole or all of
+ * them in parts; zdraw_hip_attention_plan in the measurement header says which.) */
 void zdraw_hip_attention_tail_plan(uint64_t tiles, uint32_t cus, uint32_t key_blocks, uint32_t* tail_tiles,
                                    uint32_t* splits);
 

@@ -29,8 +29,16 @@ size_t zdraw_hip_clock_probe_read(uint64_t* cycles, uint64_t* ref_ticks, size_t 
 /* Which build of the attention kernel runs. Bit 0: 0 = 8 waves x 32 query rows per
  * workgroup, one workgroup per CU (default); 1 = 4 waves x 32 query rows, two workgroups
  * per CU. Bit 1: 2 = never split the tiles of a thinly filled last round along the keys
- * (by default they are). */
+ * (by default they are). Bit 2: 4 = 256-row tiles also where a small launch would take
+ * 128-row tiles with two key groups. */
 void zdraw_hip_set_attention_variant(int variant);
+
+/* The tiles that a launch of prepared (or bf16) operands takes by default on a device with `cus`
+ * compute units: `heads` = segments x heads, `keys` = tokens or the key limit. *rows = query rows per
+ * tile (256, or 128 with two key groups); *tail_tiles and *splits as zdraw_hip_attention_tail_plan
+ * gives them. Host arithmetic only. */
+void zdraw_hip_attention_plan(uint64_t heads, uint32_t tokens, uint32_t keys, uint32_t cus, uint32_t* rows, uint32_t* tail_tiles,
+                              uint32_t* splits);
 
 /* Which build multiplies 256 x 256 tiles of 16-bit activations. 1 = four waves, 128 x 128
  * each (default); 0 = eight waves, 64 x 128 each. 2 = every product on the kernel that

@@ -179,6 +179,29 @@ def test_tail_plan_of_the_baseline_shapes():
         assert (t == 0 and s == 1) or (t == tiles % 256 and 2 <= s <= 16 and t * s <= 256 and 144 // s >= 8)
 
 
+def test_attention_tiles_of_small_and_large_launches():
+    # 256 CUs: launches whose 128-row tiles fit the CUs once may take two key groups, others never do
+    L = hip.lib()
+
+    def plan(heads, tokens, keys=0, cus=256):
+        r, t, s = C.c_uint32(99), C.c_uint32(99), C.c_uint32(99)
+        L.zdraw_hip_attention_plan(heads, tokens, keys or tokens, cus, C.byref(r), C.byref(t), C.byref(s))
+        return r.value, t.value, s.value
+
+    assert plan(24, 4608) == (256, 0, 1) and plan(96, 1536) == (256, 64, 4)  # Klein 1024^2, 512^2 x 4
+    assert plan(24, 768) == (128, 0, 1)             # Klein 256^2: 144 tiles of 128 rows
+    assert plan(2, 96) == (256, 0, 1) and plan(2, 97) == (128, 0, 1)  # up to three key blocks there is nothing to share out
+    assert plan(2, 700) == (128, 12, 2) and plan(3, 1500) == (128, 36, 5)    # every tile in parts of two groups
+    assert plan(24, 1280) == (128, 0, 1) and plan(24, 1281) == (256, 0, 1)   # 264 tiles: more than the CUs
+    assert plan(0, 64) == (0, 0, 1) and plan(1, 64, 65) == (0, 0, 1)
+    for heads in (1, 5, 24, 30, 96):
+        for tokens in range(32, 6000, 97):
+            r, t, s = plan(heads, tokens)
+            tiles = heads * -(-tokens // r)
+            assert r == 256 or tiles <= 256
+            assert (t == 0 and s == 1) or (t == tiles % 256 and 2 <= s <= 16 and t * s <= 256 and -(-tokens // 32) // s >= 8), (heads, tokens)
+
+
 def test_zimage_axis_lens_are_the_positions_the_pair_table_holds():
     # what the kernels hold device-resident positions to (the reference refuses pos >= len
     # on the host, zimage/zrope.zig:48): for zrope.Cache's layout the counts are its lens

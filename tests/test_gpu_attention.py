@@ -709,25 +709,37 @@ def test_qk_norm_rope_by_head_groups_of_either_size(ctx, heads, tokens):
 
 
 # ------------------------------------------------ key-split tail tiles and their merge
+def _plan(tokens, valid, heads, knob=0):
+    """(query rows per tile, tail tiles, parts) of a launch of prepared operands on 256 CUs"""
+    L = hip.lib()
+    rows, tail, splits = C.c_uint32(256), C.c_uint32(0), C.c_uint32(1)
+    if knob == 0:
+        L.zdraw_hip_attention_plan(heads, tokens, valid or tokens, 256, C.byref(rows), C.byref(tail), C.byref(splits))
+    else:
+        L.zdraw_hip_attention_tail_plan(-(-tokens // 256) * heads, 256, -(-(valid or tokens) // 32), C.byref(tail), C.byref(splits))
+    return rows.value, tail.value, splits.value
+
+
+@pytest.mark.parametrize("parts_knob", [0, 4])
 @pytest.mark.parametrize("tokens,valid,heads,bounded", [(700, 0, 2, True), (700, 650, 2, False), (1000, 0, 1, False),
                                                        (1500, 1300, 3, True)])
-def test_key_split_tail_matches_whole_tiles_and_oracle(ctx, tokens, valid, heads, bounded):
+def test_key_split_tail_matches_whole_tiles_and_oracle(ctx, tokens, valid, heads, bounded, parts_knob):
     # A launch far smaller than the chip is all tail: its tiles are split along the keys
     # (at least 8 key blocks per part) and merged. Shapes with a ragged last block, a key
-    # limit, and both softmax forms; compared with the same call made whole (knob 2) and
-    # with the oracle on every row.
+    # limit, and both softmax forms; 128-row tiles with two key groups (what such launches take) and
+    # 256-row tiles (what larger ones split their last round of; knob 4). Compared with the same call
+    # made whole (knob 2: 256-row tiles) and with the oracle on every row.
     L = hip.lib()
     rng = np.random.default_rng(tokens + heads)
     shape = (tokens, heads, 128)
     scale = 0.35 if bounded else 1.0
     q, k, v = (rng.standard_normal(shape, dtype=np.float32) * np.float32(scale) for _ in range(3))
-    tail, splits = C.c_uint32(0), C.c_uint32(0)
-    key_blocks = ((valid or tokens) + 31) // 32
-    L.zdraw_hip_attention_tail_plan(((tokens + 255) // 256) * heads, 256, key_blocks, C.byref(tail), C.byref(splits))
-    assert splits.value >= 2 and tail.value == ((tokens + 255) // 256) * heads  # this test is about the split path
+    rows, tail, splits = _plan(tokens, valid, heads, parts_knob)
+    assert rows == (256 if parts_knob else 128)
+    assert splits >= 2 and tail == -(-tokens // rows) * heads  # this test is about the split path
     bufs = [ctx.buffer(host.f32_to_bf16_bits(a)) for a in (q, k, v)]
     outs = []
-    for knob in (0, 2):
+    for knob in (parts_knob, 2):
         L.zdraw_hip_set_attention_variant(knob)
         o = ctx.buffer(nbytes=q.size * 4)
         p = hip.AttnParams(tokens, heads, heads, 128, 0, valid)
@@ -849,18 +861,22 @@ def test_masked_key_lists_sampled_rows(ctx, tokens, valid, heads, bounded):
         b.release()
 
 
-# Launches of few tiles run 128 query rows per workgroup and two groups of waves over half of the
-# keys each: one key block (the second group has none), an odd number of blocks (an idle last step),
-# fewer blocks than ring stages and a whole turn of the ring more, half a tile left over, a half
-# whose keys are all masked, parts of a split tile on top (two heads from 640 tokens on); both
-# softmax forms, both score types, every type of output. Sampled rows against float64 on the
-# operands as given; the bf16 attention bar.
+# Launches of few tiles of more than 96 keys run 128 query rows per workgroup and two groups of waves over
+# half of the keys each: an odd number of blocks (an idle last step), fewer blocks than ring stages
+# and a whole turn of the ring more, half a tile left over, a half whose keys are all masked, masks
+# that admit no block, one (the second group has none), two and three, parts of a split tile on top
+# (two heads from 640 tokens on); both softmax forms, both score types, every type of output. Up to 96
+# keys they stay on one group. Sampled rows against float64 on the operands as given; the bf16
+# attention bar.
 @pytest.mark.parametrize("bounded", [True, False])
 @pytest.mark.parametrize("tokens,heads,dead,in_dtype,out_dtype", [
     (1, 1, None, hip.BF16, hip.F32), (32, 2, None, hip.BF16, hip.BF16), (33, 3, None, hip.BF16, hip.F16), (96, 2, None, hip.F16, hip.F32),
     (128, 24, None, hip.BF16, hip.BF16), (129, 5, (0, 64), hip.BF16, hip.F32), (160, 2, (64, 159), hip.F16, hip.F16),
     (257, 3, (0, 257), hip.BF16, hip.F32), (288, 30, None, hip.BF16, hip.BF16), (320, 2, (0, 200), hip.BF16, hip.BF16),
-    (1024, 2, None, hip.BF16, hip.F32), (1501, 2, (700, 1500), hip.BF16, hip.BF16)])
+    (1024, 2, None, hip.BF16, hip.F32), (1501, 2, (700, 1500), hip.BF16, hip.BF16),
+    (129, 3, ((0, 129),), hip.BF16, hip.BF16), (129, 3, ((0, 64), (96, 129)), hip.BF16, hip.F32), (129, 2, ((0, 128),), hip.F16, hip.F32),
+    (257, 2, ((0, 40), (41, 257)), hip.BF16, hip.BF16), (161, 3, ((1, 160),), hip.BF16, hip.F32), (257, 5, ((0, 70), (100, 230)), hip.BF16, hip.F16),
+    (289, 2, ((30, 63), (64, 250), (256, 288)), hip.F16, hip.F32), (901, 2, ((0, 450), (482, 901)), hip.BF16, hip.F32)])
 def test_two_key_groups_sampled_rows(ctx, tokens, heads, dead, in_dtype, out_dtype, bounded):
     L = hip.lib()
     rng = np.random.default_rng(tokens + heads)
@@ -876,8 +892,11 @@ def test_two_key_groups_sampled_rows(ctx, tokens, heads, dead, in_dtype, out_dty
     keep = np.ones(tokens, bool)
     ops = hip.QkOperands()
     bufs = [ctx.buffer(b) for b in raw] + [ctx.buffer(nbytes=q.size * (4 if out_dtype == hip.F32 else 2))]
+    rows_per_tile, _, splits = _plan(tokens, 0, heads)
+    assert rows_per_tile == (128 if tokens > 96 else 256) and (splits > 1) == (tokens >= 640)
     if dead:
-        keep[dead[0]:dead[1]] = False
+        for lo, hi in dead if isinstance(dead[0], tuple) else (dead,):
+            keep[lo:hi] = False
         bufs.append(ctx.buffer((~keep).astype(np.uint8)))
         ops.key_pad = bufs[4].handle
     p = hip.AttnParams(tokens, heads, heads, 128, 0, 0)
@@ -1009,15 +1028,20 @@ def test_short_plain_f32_rows_under_capture_take_no_scratch(ctx, tokens, heads, 
 
 # first, a middle and the last key block; rising, so that the reference moves at each of them
 PLANT_CASES = [
-    # name, tokens, heads, in_dtype, valid, planted (key, nats), whole tiles only (knob 2)
+    # name, tokens, heads, in_dtype, valid, planted (key, nats), knob: 2 = whole 256-row tiles, 4 = 256-row
+    # tiles in parts, 0 = what the launch takes (here 128-row tiles with two key groups)
     ("bf16 direct-to-LDS", 1024, 2, hip.BF16, 0, [(5, 21.0), (500, 28.0), (1023, 35.0)], 2),
     ("bf16 direct-to-LDS, last block only", 2048, 1, hip.BF16, 0, [(2047, 33.0)], 2),
     ("f32 rows rounded in the tile load", 640, 2, hip.F32, 0, [(3, 21.0), (333, 28.0), (639, 35.0)], 2),
     ("bf16 masked by a key limit", 1100, 2, hip.BF16, 1000, [(7, 21.0), (480, 28.0), (999, 35.0), (1050, 60.0)], 2),
     ("bf16 ragged last block", 1001, 2, hip.BF16, 0, [(40, 24.0), (1000, 34.0)], 2),
     ("f32 masked by a key limit", 700, 1, hip.F32, 650, [(600, 30.0), (649, 36.0), (660, 60.0)], 2),
-    ("key-split parts", 1500, 3, hip.BF16, 0, [(30, 21.0), (820, 28.0), (1310, 35.0)], 0),
-    ("key-split parts, masked", 1500, 3, hip.BF16, 1400, [(700, 25.0), (1399, 35.0), (1450, 60.0)], 0),
+    ("key-split parts", 1500, 3, hip.BF16, 0, [(30, 21.0), (820, 28.0), (1310, 35.0)], 4),
+    ("key-split parts, masked", 1500, 3, hip.BF16, 1400, [(700, 25.0), (1399, 35.0), (1450, 60.0)], 4),
+    ("two key groups", 700, 24, hip.BF16, 0, [(5, 21.0), (300, 28.0), (699, 35.0)], 0),
+    ("two key groups, masked", 500, 8, hip.BF16, 470, [(5, 21.0), (250, 28.0), (469, 35.0), (480, 60.0)], 0),
+    ("two key groups in key-split parts", 1500, 3, hip.BF16, 0, [(30, 21.0), (820, 28.0), (1310, 35.0)], 0),
+    ("two key groups in key-split parts, masked", 1500, 3, hip.BF16, 1400, [(700, 25.0), (1399, 35.0), (1450, 60.0)], 0),
 ]
 
 
@@ -1030,14 +1054,14 @@ def test_running_maximum_moves_its_reference_point_late(ctx, name, tokens, heads
     # already formed. Keys past a key limit score higher still and must stay out. Every row
     # against the oracle on the same bf16-rounded operands; bit-identical rerun.
     say(f"planted keys: {name}")
-    if knob == 0:
-        tail, splits = C.c_uint32(0), C.c_uint32(0)
-        hip.lib().zdraw_hip_attention_tail_plan(((tokens + 255) // 256) * heads, 256, ((valid or tokens) + 31) // 32,
-                                                C.byref(tail), C.byref(splits))
-        assert splits.value >= 3
-        per = -(-(((valid or tokens) + 31) // 32) // splits.value)  # key blocks per part
+    if knob != 2:
+        rows, _, splits = _plan(tokens, valid, heads, knob)
+        assert rows == (256 if knob else 128) and (splits > 1) == ("parts" in name)
+        per = -(-(((valid or tokens) + 31) // 32) // splits)  # key blocks per part
+        if rows == 128:
+            per = (per + 1) // 2  # and per key group
         parts = {key // 32 // per for key, _ in plant if not valid or key < valid}
-        assert len(parts) >= 2 and max(parts) >= 2  # a later part than the first carries a planted key
+        assert len(parts) >= 2 and (splits == 1 or max(parts) >= 2)  # a later part than the first carries a planted key
     q, k, v = _planted(tokens, heads, plant, seed=tokens + heads)
     got = _plain_fused(ctx, q, k, v, valid=valid, in_dtype=in_dtype, knob=knob)
     want = zo.attention_run(q, k, v, zo.Config(tokens, heads, heads, 128, False, valid))

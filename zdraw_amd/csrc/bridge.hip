@@ -85,7 +85,7 @@ uint64_t g_dispatch = 0;
 uint64_t g_command = 0;
 uint64_t g_fallback = 0;
 uint64_t g_gpu_ns = 0;
-int g_variant = 0; // bit 0: kernel shape, 0 = 8 waves per workgroup, 1 = 4 waves (two workgroups per CU); bit 1: never split tail tiles
+int g_variant = 0; // bit 0: kernel shape, 0 = 8 waves per workgroup, 1 = 4 waves (two workgroups per CU); bit 1: never split tail tiles; bit 2: no 128-row tiles
 bool g_setup_done = false;
 bool g_gemm_setup_done = false;
 
@@ -1881,7 +1881,16 @@ size_t zdraw_hip_clock_probe_read(uint64_t* cycles, uint64_t* ref_ticks, size_t 
     return m;
 }
 
-void zdraw_hip_set_attention_variant(int variant) { g_variant = variant & 3; }
+void zdraw_hip_set_attention_variant(int variant) { g_variant = variant & 7; }
+
+void zdraw_hip_attention_plan(uint64_t heads, uint32_t tokens, uint32_t keys, uint32_t cus, uint32_t* rows, uint32_t* tail_tiles, uint32_t* splits) {
+    int shape = 0, t = 0, s = 1;
+    const bool ok = heads && heads <= 0x7fffffffull && tokens && keys && keys <= tokens && tokens <= (uint32_t)attention_max_tokens();
+    if (ok) attention_plan((int64_t)heads, (int)tokens, ((int)keys + attention_key_block() - 1) / attention_key_block(), (int)cus, &shape, &t, &s);
+    if (rows) *rows = ok ? (uint32_t)attention_block_rows(shape) : 0;
+    if (tail_tiles) *tail_tiles = (uint32_t)t;
+    if (splits) *splits = (uint32_t)s;
+}
 
 void zdraw_hip_wide_ranges(uint32_t tokens, uint32_t cus, uint32_t* ranges, uint64_t* share_bytes) {
     const bool ok = tokens != 0 && tokens <= (1u << 20) && tokens % (uint32_t)wide_block_rows() == 0;

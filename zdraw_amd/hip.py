@@ -152,6 +152,7 @@ SYMBOLS = {
     "zdraw_hip_gemm_launch_rows": (None, [_u32, _u64, _u32, C.POINTER(C.c_uint32)]),
     "zdraw_hip_set_scratch_limit": (None, [_sz]),
     "zdraw_hip_wide_ranges": (None, [_u32, _u32, C.POINTER(C.c_uint32), C.POINTER(C.c_uint64)]),
+    "zdraw_hip_attention_plan": (None, [_u64, _u32, _u32, _u32, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32), C.POINTER(C.c_uint32)]),
     "zdraw_hip_gemm_tile": (None, [_u32, _u32, _u32, _u32, _u32, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32)]),
     "zdraw_hip_zimage_axis_lens": (_int, [_u64, C.POINTER(C.c_uint64), C.POINTER(C.c_uint32), C.POINTER(C.c_uint32)]),
     "zdraw_hip_abi_sizeof": (_sz, [_int]),
