@@ -926,6 +926,36 @@ def test_two_key_groups_sampled_rows(ctx, tokens, heads, dead, in_dtype, out_dty
         b.release()
 
 
+# An infinite value reaches every row that attends to its key, as infinity, and no other column: the second
+# group's idle last step (an odd number of blocks, or none of its own) adds nothing, 0 x inf included.
+@pytest.mark.parametrize("bounded", [True, False])
+@pytest.mark.parametrize("tokens,key,admitted", [(160, 150, None), (160, 3, None), (129, 70, (64, 96)), (192, 191, None), (416, 400, None)])
+def test_two_key_groups_pass_infinite_values_on(ctx, tokens, key, admitted, bounded):
+    L = hip.lib()
+    assert _plan(tokens, 0, 2)[0] == 128
+    rng = np.random.default_rng(tokens + key)
+    q, k, v = (rng.standard_normal((tokens, 2, 128), dtype=np.float32) * np.float32(0.35) for _ in range(3))
+    v[key, 0, 5], v[key, 1, 77] = np.inf, -np.inf
+    bufs = [ctx.buffer(host.f32_to_bf16_bits(a)) for a in (q, k, v)] + [ctx.buffer(nbytes=q.size * 4)]
+    p, x, ops = hip.AttnParams(tokens, 2, 2, 128, 0, 0), hip.AttnExt(), hip.QkOperands()
+    if admitted:
+        pad = np.ones(tokens, np.uint8)
+        pad[admitted[0]:admitted[1]] = 0
+        bufs.append(ctx.buffer(pad))
+        ops.key_pad = bufs[4].handle
+    for s_ in (x.q_stride, x.k_stride, x.v_stride, x.out_stride):
+        s_[0], s_[1], s_[2] = 0, 256, 128
+    x.batch, x.in_dtype, x.out_dtype, x.qk_mode, x.score_bound = 1, hip.BF16, hip.F32, hip.QK_NONE, 40.0 if bounded else 0.0
+    rc = L.zdraw_hip_run_attention_fused(ctx.queue, *(b.handle for b in bufs[:4]), C.byref(p), C.byref(x), C.byref(ops))
+    assert rc == 0, hip.last_error()
+    got = bufs[3].read(np.float32, q.shape)
+    assert (got[:, 0, 5] == np.inf).all() and (got[:, 1, 77] == -np.inf).all()
+    got[:, 0, 5] = got[:, 1, 77] = 0
+    assert np.isfinite(got).all()
+    for b in bufs:
+        b.release()
+
+
 # Plain attention on f32 rows either side of the length from which one launch rounds the operands
 # ahead of the kernel (160 tokens): one launch below, two from there on, with a key limit and ragged
 # last blocks, every row against the oracle. The copies keep the bits the tile load would have made.

@@ -1067,11 +1067,12 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             step(Dyn{}, b, sets[0], NST != 8, s_a, s_b, p_a, p_b);
             step(Dyn{}, b + 1, sets[1], true, s_b, s_a, p_b, p_a);
         }
+        // (a group's idle last step has nothing to add: its probabilities are zero, but a value may be infinite)
         if (b < nblk) {
             step(Dyn{}, b, sets[0], true, s_a, s_b, p_a, p_b);
-            pv_block((nblk - 1) & (NST - 1), p_b);
+            if (KG == 1 || nown == nblk) pv_block((nblk - 1) & (NST - 1), p_b);
         } else {
-            pv_block((nblk - 1) & (NST - 1), p_a);
+            if (KG == 1 || nown == nblk) pv_block((nblk - 1) & (NST - 1), p_a);
         }
         if constexpr (DMA) __builtin_amdgcn_s_waitcnt(0x0F70); // no direct load may outlive the workgroup's LDS
     }
