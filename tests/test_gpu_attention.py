@@ -1008,8 +1008,12 @@ def test_plain_f32_rows_without_memory_for_their_rounded_copies(ctx):
 # copies): one kernel in the graph, on a queue without scratch and on one whose slots have room. A
 # longer call replaces the slots between the replays; every row of every replay against the oracle.
 @pytest.mark.parametrize("warm", [False, True])
-@pytest.mark.parametrize("tokens,heads", [(160, 3), (239, 2)])
+# (Launches whose tiles are split along the keys, 700 tokens here, keep their parts in slots 3 and 4, as before
+# they were rounded: capturable once the call, or its reservation, has made room.)
+@pytest.mark.parametrize("tokens,heads", [(160, 3), (239, 2), (700, 24)])
 def test_short_plain_f32_rows_under_capture_take_no_scratch(ctx, tokens, heads, warm):
+    parts = _plan(tokens, 0, heads, knob=4)[2] > 1
+    assert parts == (tokens == 700)
     L = hip.lib()
     rng = np.random.default_rng(tokens)
     shape = (tokens, heads, 128)
@@ -1018,15 +1022,17 @@ def test_short_plain_f32_rows_under_capture_take_no_scratch(ctx, tokens, heads, 
     bufs = [ctx.buffer(a) for a in (q, k, v)] + [ctx.buffer(nbytes=q.size * 4)]
     big = [ctx.buffer(np.zeros((1024, heads, 128), np.float32)) for _ in range(4)]
 
-    def enqueue(batch, b, n):
+    def enqueue(batch, b, n, fn=L.zdraw_hip_run_attention_fused_enc):
         p, x = hip.AttnParams(n, heads, heads, 128, 0, 0), hip.AttnExt()
         for s_ in (x.q_stride, x.k_stride, x.v_stride, x.out_stride):
             s_[0], s_[1], s_[2] = 0, heads * 128, 128
         x.batch, x.in_dtype, x.out_dtype, x.qk_mode = 1, hip.F32, hip.F32, hip.QK_NONE
-        return L.zdraw_hip_run_attention_fused_enc(batch, *(i.handle for i in b), C.byref(p), C.byref(x), None)
+        return fn(batch, *(i.handle for i in b), C.byref(p), C.byref(x), None)
 
     queue = L.zdraw_hip_create_queue(ctx.device)
     stream = C.c_void_p((C.c_void_p * 2).from_address(queue)[1])  # a queue is a device and a stream
+    if parts and not warm:
+        assert enqueue(queue, bufs, tokens, L.zdraw_hip_reserve_attention_fused) == 0, hip.last_error()
     if warm:
         batch = L.zdraw_hip_batch_begin(queue)
         d0 = L.zdraw_hip_dispatch_count()
@@ -1040,14 +1046,14 @@ def test_short_plain_f32_rows_under_capture_take_no_scratch(ctx, tokens, heads, 
     assert L.hipStreamEndCapture(stream, C.byref(graph)) == 0
     assert rc == 0, hip.last_error()
     assert L.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0
-    assert nodes.value == 1
+    assert nodes.value == (2 if parts else 1)  # the kernel, and the merge of its parts
     assert L.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
     for replay in range(3):
         bufs[3].write(np.full(q.size * 4, 0x7B, np.uint8))
         assert L.hipGraphLaunch(run, stream) == 0
         assert L.hipStreamSynchronize(stream) == 0
         refimpl.check_close(bufs[3].read(np.float32, shape), want, f"replay {replay}")
-        if replay == 0:
+        if replay == 0 and not parts:
             assert enqueue(batch, big, 1024) == 0, hip.last_error()
     assert L.zdraw_hip_batch_end(batch) == 0
     assert L.hipGraphExecDestroy(run) == 0 and L.hipGraphDestroy(graph) == 0

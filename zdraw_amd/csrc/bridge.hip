@@ -254,7 +254,8 @@ constexpr uint32_t kRoundPlainTokens = 160, kRoundAlwaysTokens = 1024;
 // entry is called, so that both give the same bits (with batch 1 they do: 1023 tokens of 30 heads take
 // 24 MB, the parts never more than 34). A queue's slots are not taken under capture, whatever they
 // hold (the call can run without, and its graph then holds no address of a slot that a larger call
-// replaces), and not where there is no memory for them.
+// replaces), and not where there is no memory for them. A call that takes them also makes room for the parts
+// that the unrounded form would split its tiles into: a capture of the same call finds it there.
 bool plain_may_round(ScratchSource* src, const ZdrawAttnParams* p, uint32_t batch, int key_blocks, int cus) {
     const size_t copy = (size_t)batch * p->heads * p->tokens * kHeadDim * 2;
     int shape = 0, tail = 0, splits = 1;
@@ -267,6 +268,11 @@ bool plain_may_round(ScratchSource* src, const ZdrawAttnParams* p, uint32_t batc
     if (!src->queue || capturing(src->queue)) return false;
     for (int i = 0; i < 3; i++)
         if (!src->get(i, copy)) return false;
+    attention_tail_plan((int64_t)batch * p->heads * ((p->tokens + 255) / 256), cus, key_blocks, &tail, &splits);
+    if (splits > 1) {
+        (void)src->get(3, attention_part_o_bytes(tail, splits, 0));
+        (void)src->get(4, attention_part_ml_bytes(tail, splits, 0));
+    }
     return true;
 }
 
