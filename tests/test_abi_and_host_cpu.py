@@ -79,7 +79,7 @@ def test_gemm_tail_plan_of_the_projection_shapes():
     assert plan(4608, 3840, 3840, 3) == (42, 6)      # Z-Image q/k/v group: 810 tiles = 3 rounds + 42
     assert plan(4608, 3840, 3840) == (14, 8)         # Z-Image out projection: 270 tiles, never more than 8 parts
     assert plan(4608, 12288, 3072) == (0, 1)         # 216 tiles: one partly filled round, nothing before it to balance
-    assert plan(512, 3072, 9216) == (0, 1)           # fewer than 160 tiles: the 128-tile build
+    assert plan(512, 3072, 9216) == (0, 1)           # fewer than 160 tiles: smaller ones
     assert plan(4322, 1216, 4090) == (16, 4)         # 272 tiles, 19 slabs: at least four slabs per part
     assert plan(4322, 128, 4090) == (0, 1)           # two slabs: too short to split
     assert plan(4322, 1220, 4090) == (0, 1)          # k not a multiple of 64: another build

@@ -406,7 +406,7 @@ def test_256_tile_builds_16_bit_output_with_unaligned_rows(ctx, build):
 @pytest.mark.parametrize("wdt", [hip.W_BF16, hip.W_F16])
 @pytest.mark.parametrize("ldc", [256, 251])
 def test_small_tile_build_16_bit_output_edges_and_pitch(ctx, wdt, ldc):
-    # Few tiles, 16-bit activations, k a multiple of 64: the 128-tile build. With rows of C on
+    # Few tiles, 16-bit activations, k a multiple of 64: a small tile of the pipelined kernel. With rows of C on
     # 16 bytes (ldc 256) its 16-bit output leaves through LDS as whole rows: the last rows
     # (m = 200 of 256) must not be stored, the last column chunk (n = 250: two of eight
     # columns) goes element by element, and the pad columns of the pitch stay untouched. With
@@ -533,7 +533,8 @@ def test_k_split_last_round_of_a_group(ctx):
 
 
 # one problem per tile of the pipelined kernel: more than one tile each way, a ragged last row and
-# column of tiles, and a k of three slabs (fewer than the LDS holds) or of 3.125 (the last slab
+# column of tiles, and a k of three slabs (no turn of a four-slab ring), of nine, ten and eleven
+# (turns of either ring with every remainder), or of 3.125 and 8.125 (the last slab
 # keeps one of its eight chunks)
 TILE_CASES = [((64, 64), 72, 73, 1), ((64, 96), 199, 1349, 3), ((128, 64), 1797, 202, 3), ((128, 96), 259, 1794, 3),
               ((128, 128), 522, 1636, 3), ((128, 160), 899, 1304, 3), ((128, 192), 902, 1601, 3),
@@ -541,7 +542,7 @@ TILE_CASES = [((64, 64), 72, 73, 1), ((64, 96), 199, 1349, 3), ((128, 64), 1797,
 
 
 @pytest.mark.parametrize("tile,m,n,count", TILE_CASES, ids=[f"{t[0]}x{t[1]}" for t, *_ in TILE_CASES])
-@pytest.mark.parametrize("k", [192, 200, 520])
+@pytest.mark.parametrize("k", [192, 200, 520, 576, 640, 704])
 @pytest.mark.parametrize("c_dtype", [hip.F32, hip.BF16])
 def test_every_tile_of_the_pipelined_kernel(ctx, tile, m, n, count, k, c_dtype):
     # Every product of the group on sampled rows (first, last, the edges of tiles and of their waves)
@@ -551,8 +552,7 @@ def test_every_tile_of_the_pipelined_kernel(ctx, tile, m, n, count, k, c_dtype):
     L = hip.lib()
     r, c = C.c_uint32(), C.c_uint32()
     L.zdraw_hip_gemm_tile(m, k, n, count, 256, C.byref(r), C.byref(c))
-    if k < 512:
-        assert (r.value, c.value) == tile
+    assert (r.value, c.value) == tile
     rng = np.random.default_rng(m + n + k)
     lda = ldw = k + 8
     ldc = n + (3 if c_dtype == hip.F32 else 5)
