@@ -672,7 +672,7 @@ size_t wide_part_bytes(int tokens, int splits) {
 // for 1.5 %), and neither are shares of more than kMaxShareBytes, which the queue keeps (33024 tokens: six
 // ranges, 389 MB, a quarter of the time by the estimate; 18432: three, 108 MB, 11 %).
 // (A power of two that divides the blocks, which this was before, left 6208 tokens, 194 blocks, at
-// two ranges and 98 workgroups: call 163 us against 118 with four; 18432 tokens at one range:
+// two ranges and 98 workgroups: call 152 us against 119 with four; 18432 tokens at one range:
 // 678 against 610 with three.)
 int wide_splits(int tokens, int cus) {
     constexpr size_t kMaxShareBytes = (size_t)512 << 20;

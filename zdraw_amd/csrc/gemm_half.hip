@@ -1007,9 +1007,9 @@ static int g_gemm_build = 1; // measurement knob (gemm_set_build)
 
 // The tiles gemm_pipe_kernel is built for: (32 ti) x (32 tj) with st slabs in LDS, what one slab of
 // it takes when weights come from memory (us, every CU busy) and what a tile costs beside its slabs.
-// A slab's time is close to its bytes (A and W rows of 128 bytes) at 55-60 GB/s: a CU has at most
-// 32 KB of loads in flight, in order, and memory answers after 600 ns (350 ns from the last-level
-// cache, 190 ns from L2: 93 and 173 GB/s). So a tile's bytes per FLOP decide, and they fall with its
+// A slab's time is its bytes (A and W rows of 128 bytes) at 55 to 66 GB/s: a CU has at most 32 KB of
+// loads in flight, in order, and memory answers after 600 ns, 55 GB/s (350 ns from the last-level
+// cache, 190 ns from L2: 93 and 173 GB/s; part of A comes from there). So a tile's bytes per FLOP decide, and they fall with its
 // size, until there are fewer tiles than CUs.
 struct PipeShape { int ti, tj, st; float slab_us, fix_us; };
 constexpr PipeShape kPipe[] = {
@@ -1022,6 +1022,8 @@ constexpr int kRingShape = -1;
 // partial tiles' way through memory and for the merge.
 constexpr float kRingSlabUs = 1.28f, kRingFixUs = 8.0f, kRingSplitUs = 28.0f;
 
+// A ragged k (RAG) is built for every tile too: its products have the rows and columns of the others (a
+// hidden width of 2568 is 40 slabs and an eighth), and the estimates hold for them.
 template <bool F16, typename TC, int I, bool RAG>
 static const void* pipe_entry() {
     return reinterpret_cast<const void*>(&gemm_pipe_kernel<F16, TC, kPipe[I].ti, kPipe[I].tj, kPipe[I].st, RAG>);

@@ -27,7 +27,8 @@ constexpr int kPrepTokens = 4; // tokens (waves) per workgroup
 // block, us, 6 or 8 -> 2 groups: 24 heads bf16 256 tokens 18.6 -> 17.0, 768 30.6 -> 28.1, 1040 38.2
 // -> 34.5, 4 x 1536 158.6 -> 154.8, 4608 240.2 -> 239.2; 30 heads 80 tokens 16.6 -> 14.5, 768 34.2
 // -> 30.3, 4608 301 -> 299.5; but 2 x 8704 tokens 1459 -> 1467, hence the line between 6144 and
-// 17408 tokens over all segments.
+// 17408 tokens over all segments. It was drawn with 24 and 30 heads: with eight or fewer, longer launches
+// still walk six groups, most of which repeat the last head (not measured).
 constexpr int64_t kThinTokens = 8192;
 
 template <typename TIn, int MODE, int G>
