@@ -226,7 +226,11 @@ Buffer* queue_scratch(Queue* q, int slot, size_t bytes) {
 // Whether what is enqueued now becomes part of a graph.
 bool capturing(const Queue* q) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(q->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(q->stream, &st) != hipSuccess) {
+        (void)hipGetLastError(); // or the next launch would report it
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
 }
 
 // Where a call's scratch comes from: the grow-only slots of the queue the call runs on,
