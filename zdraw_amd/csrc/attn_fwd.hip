@@ -1067,12 +1067,27 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             step(Dyn{}, b, sets[0], NST != 8, s_a, s_b, p_a, p_b);
             step(Dyn{}, b + 1, sets[1], true, s_b, s_a, p_b, p_a);
         }
-        // (a group's idle last step has nothing to add: its probabilities are zero, but a value may be infinite)
+        // A group's idle last step has nothing to add: its probabilities are zero, but a value of the block it
+        // fetched again may be infinite. Each wave clears the stage (8 KB) itself before it reads it, so no
+        // barrier is needed: the block has landed, and the others write zeros too. (A branch around the
+        // product instead costs every launch 0.3 us: the accumulators move at its join.)
+        auto clear_idle = [&]() __attribute__((always_inline)) {
+            if constexpr (KG == 2) {
+                typedef __attribute__((address_space(3))) u32x4* lds_clear_t;
+                const unsigned at = lds_address(Vs + (grp * NST + ((nblk - 1) & (NST - 1))) * VSTAGE) + (unsigned)(lane * 16);
+                if (nown < nblk) {
+#pragma unroll
+                    for (int i = 0; i < (int)(VSTAGE * sizeof(bf16_t)) / 1024; i++) *(lds_clear_t)(at + (unsigned)(i * 1024)) = u32x4{0u, 0u, 0u, 0u};
+                }
+            }
+        };
         if (b < nblk) {
             step(Dyn{}, b, sets[0], true, s_a, s_b, p_a, p_b);
-            if (KG == 1 || nown == nblk) pv_block((nblk - 1) & (NST - 1), p_b);
+            clear_idle();
+            pv_block((nblk - 1) & (NST - 1), p_b);
         } else {
-            if (KG == 1 || nown == nblk) pv_block((nblk - 1) & (NST - 1), p_a);
+            clear_idle();
+            pv_block((nblk - 1) & (NST - 1), p_a);
         }
         if constexpr (DMA) __builtin_amdgcn_s_waitcnt(0x0F70); // no direct load may outlive the workgroup's LDS
     }
