@@ -44,6 +44,18 @@ def test_wide_head_matches_oracle_on_every_row(ctx, tokens):
     assert np.array_equal(got, again)
 
 
+# The key loop walks two blocks a trip and the two waves of a pair swap their blocks' probabilities through two
+# slots in turn: few blocks and no range, two ranges of nine blocks, ranges of nine and a last one of seven with
+# half a query tile left over; every row, so that each wave's half of the dims counts.
+@pytest.mark.parametrize("tokens", [192, 576, 1088])
+def test_wide_head_odd_numbers_of_blocks_on_every_row(ctx, tokens):
+    rng = np.random.default_rng(60 + tokens)
+    q, k, v = draw(rng, tokens)
+    got = ctx.run(q, k, v, host.Config(tokens, 1, 1, 512)).reshape(tokens, 1, 512)
+    want = zo.attention_run(q, k, v, zo.Config(tokens, 1, 1, 512))
+    refimpl.check_close(got, want, f"wide head, {tokens} tokens")
+
+
 # Numbers of key blocks that the number of ranges does not divide (the last range is shorter),
 # half a query tile left over, three to seven ranges, and both sides of the length
 # where two ranges a tile outgrow one round; rows of the first, a middle and the last tile.

@@ -36,3 +36,12 @@ def test_wide_head_kernel_keeps_its_accumulators_in_place_and_its_loop_free_of_s
     # step, and the blocks that hold the MFMAs may not use scratch memory
     bad = build.wide_mfma_hazards()
     assert not bad, "\n".join(bad[:20])
+
+
+@pytest.mark.skipif(not (os.path.exists("/opt/rocm/bin/hipcc") or shutil.which("hipcc")), reason="needs hipcc")
+def test_wide_head_kernel_leaves_m0_alone_and_no_load_reads_a_scalar_register_too_early():
+    # its blocks come in runs of four loads that share one M0; and the compiler knows of no load in the
+    # assembly statements, so it keeps no distance between them and a scalar register it restores
+    src = os.path.join(build.CSRC, "attn_wide.hip")
+    bad = build.m0_writes(src, "attn_wide_kernel") + build.vmem_sgpr_hazards(src) + build.vmem_sgpr_hazards(os.path.join(build.CSRC, "gemm_half.hip"))
+    assert not bad, "\n".join(bad[:20])

@@ -128,6 +128,39 @@ def tied_mfma_hazards(src: str = os.path.join(CSRC, "gemm_half.hip"), extra_flag
     return bad
 
 
+def vmem_sgpr_hazards(src: str, extra_flags=()) -> list[str]:
+    """Compiles `src` to gfx950 assembly and lists every memory instruction that reads a scalar register
+    which a vector instruction (v_readlane, v_readfirstlane) wrote fewer than five wait states before. The
+    hardware does not wait for such a write; the compiler keeps the distance for its own loads, not for the
+    direct-to-LDS loads, which are assembly statements: with a stale descriptor or offset they would reach
+    anywhere. Scalar registers restored from a spill ahead of such a load are the usual way to get there."""
+    import re
+    lines = [l.split(";")[0].strip() for l in _device_asm(src, extra_flags)]
+    lines = [l for l in lines if l and (not l.startswith(".") or l.endswith(":"))]
+    write = re.compile(r"^v_read(?:first)?lane_b32(?:_e32|_e64)?\s+s(\d+)\b")
+    bad, kernel = [], ""
+    for i, text in enumerate(lines):
+        if text.endswith(":") and not text.startswith("."):
+            kernel = text[:-1]
+        m = write.match(text)
+        if not m:
+            continue
+        reg, states = int(m.group(1)), 0
+        for later in lines[i + 1:i + 12]:
+            if states >= 5 or re.match(rf"^s_\S+\s+s{reg}\b", later):
+                break  # far enough, or written again by the scalar unit
+            if re.match(r"^(buffer|global|flat|scratch)_", later):
+                read = {int(x) for x in re.findall(r"\bs(\d+)\b", later)}
+                for lo, hi in re.findall(r"\bs\[(\d+):(\d+)\]", later):
+                    read |= set(range(int(lo), int(hi) + 1))
+                if reg in read:
+                    bad.append(f"{kernel}: {text} | {states} wait states | {later}")
+                    break
+            nop = re.match(r"^s_nop\s+(\d+)", later)
+            states += int(nop.group(1)) + 1 if nop else 0 if later.endswith(":") else 1
+    return bad
+
+
 def wide_mfma_hazards(extra_flags=()) -> list[str]:
     """The same check for the wide-head kernel (attn_wide.hip, attn_wide_kernel): all of its MFMAs
     are assembly statements, its 256 accumulation registers hold O^T for the whole walk, and every
@@ -136,7 +169,7 @@ def wide_mfma_hazards(extra_flags=()) -> list[str]:
     register file exactly, and a spill there waits on every load in flight."""
     import re
     src = os.path.join(CSRC, "attn_wide.hip")
-    bad = tied_mfma_hazards(src, extra_flags, mfma_prefix="v_mfma_f32_32x32x16", kernel_substr="attn_wide_kernel")
+    bad = tied_mfma_hazards(src, extra_flags, mfma_prefix="v_mfma_f32_16x16x32", kernel_substr="attn_wide_kernel")
     lines = _device_asm(src, extra_flags)
     kernel, block, mfmas, scratch = "", "", 0, []
     label = re.compile(r"^([.\w$]+):")
@@ -178,11 +211,17 @@ def build_host(verbose: bool = False) -> str:
 def check_hand_scheduled_kernels(verbose: bool = False):
     """The GEMM's hand-placed MFMAs and its M0 held across loads are safe only as long as the
     compiler puts nothing of its own in between: a toolchain that does fails the build here."""
-    bad = m0_writes() + tied_mfma_hazards() + wide_mfma_hazards()
+    files = [os.path.join(CSRC, f) for f in ("attn_fwd.hip", "attn_wide.hip", "gemm_half.hip")]
+    from concurrent.futures import ThreadPoolExecutor
+    with ThreadPoolExecutor(max_workers=len(files)) as pool:  # one compilation per file, kept for all checks
+        list(pool.map(_device_asm, files))
+    bad = m0_writes() + m0_writes(files[1], "attn_wide_kernel") + tied_mfma_hazards() + wide_mfma_hazards()
+    for f in files:
+        bad += vmem_sgpr_hazards(f)
     if bad:
         raise RuntimeError("a kernel compiled to code that breaks its hand-written schedule:\n  " + "\n  ".join(bad))
     if verbose:
-        print("hand-scheduled kernels: no foreign M0 write, no accumulator touched inside an MFMA run")
+        print("hand-scheduled kernels: no foreign M0 write, no accumulator touched inside an MFMA run, no load on a scalar register just written")
 
 
 def build_all(verbose: bool = False):
