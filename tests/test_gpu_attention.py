@@ -1111,6 +1111,29 @@ def test_running_maximum_moves_its_reference_point_late(ctx, name, tokens, heads
     assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
 
 
+# A masked row's reference point stays at 0 while its first block's maximum lies within 16 (log2, 11.1 nats)
+# of it: first admitted blocks inside and outside that band on both sides of 0, close to its edges, and
+# later keys that leave the scores' start at 0, move it, or follow a move
+@pytest.mark.parametrize("knob", [2, 4, 0], ids=["whole", "parts", "default"])
+@pytest.mark.parametrize("first", [-30.0, -12.0, -10.0, 0.0, 10.0, 12.0, 30.0])
+@pytest.mark.parametrize("late", [0.0, 14.0, 45.0])
+def test_masked_first_blocks_about_the_zero_reference(ctx, first, late, knob):
+    tokens, heads, dead = 1490, 2, 64
+    say(f"first block {first} nats, late key {late} nats, knob {knob}")
+    rng = np.random.default_rng(int(first + 2 * late) + 100)
+    q, k, v = _planted(tokens, heads, [(900, late)] if late else [], seed=int(first + late) + 200)
+    u = np.full(128, 1.0 / np.sqrt(128.0), np.float32)
+    k[dead:dead + 32] = np.float32(first * np.sqrt(128.0) / 4.0) * u + np.float32(0.1) * rng.standard_normal((32, heads, 128), dtype=np.float32)
+    k[dead // 2] = np.float32(80.0) * u  # a key of the masked blocks ahead of it
+    k = host.bf16_bits_to_f32(host.f32_to_bf16_bits(k))
+    pad = np.zeros(tokens, np.uint8)
+    pad[:dead] = 1
+    pad[500:640] = 1
+    got = _plain_fused(ctx, q, k, v, in_dtype=hip.BF16, key_pad=pad, knob=knob)
+    want = zo.attention_token_list(q, k, v, zo.Config(tokens, heads, heads, 128), list(range(tokens)), key_pad=pad)
+    refimpl.check_close(got, want, "first block about the zero reference")
+
+
 def test_running_maximum_with_a_key_padding_mask_and_planted_keys(ctx):
     # the boolean key mask build (block list compacted, mask words in LDS): whole blocks are
     # dropped, planted keys sit right after a dropped stretch and inside a partly masked block
