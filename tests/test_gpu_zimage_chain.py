@@ -137,6 +137,61 @@ def test_chain_attention_segment_matches_oracle_chain(ctx, act, wdt, ndt):
         b.release()
 
 
+# f32 activations: the attention launch (or the merge of its parts) also writes the mixed heads rounded to the
+# projection's weight type, and the projection reads that copy. It has to be the copy that a product of
+# the f32 rows makes for itself: same bits out. 128- and 256-row tiles, whole and in parts, ragged last
+# blocks (masked builds) and rows past the last tile, with and without a score bound, either weight type.
+@pytest.mark.parametrize("wdt", [hip.W_F16, hip.W_BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("bounded", [True, False])
+@pytest.mark.parametrize("tokens,heads,knob", [(1, 1, 0), (33, 2, 0), (96, 2, 1), (320, 2, 0), (330, 2, 0), (288, 2, 2), (300, 2, 2),
+                                               (1100, 3, 4), (1088, 3, 4), (1504, 3, 0), (1500, 3, 0), (2304, 30, 0)])
+def test_projection_of_the_rounded_copy_equals_the_product_of_the_f32_rows(ctx, tokens, heads, knob, bounded, wdt):
+    L = hip.lib()
+    say = f"tokens {tokens} heads {heads} knob {knob} bounded {bounded}"
+    print(say, flush=True)
+    rng = np.random.default_rng(tokens + heads)
+    hidden, inner = 136, heads * 128
+    cfg = zo.RopeConfig(wl.ZIMAGE_DIMS, wl.ZIMAGE_LENS, wl.ZIMAGE_THETA)
+    bases = zo.zrope_axis_bases(cfg)
+    ones = np.ones(128, np.float32)
+    ropeb, normb = ctx.buffer(zo.zrope_fill(cfg)), ctx.buffer(ones)
+    posb = ctx.buffer(rng.integers(0, 32, (tokens, 3)).astype(np.uint64))
+    wbuf = ctx.buffer(to16(rng.standard_normal((4 * inner, hidden), dtype=np.float32) * np.float32(hidden ** -0.5), wdt)[0])
+    nb = ctx.buffer(rng.standard_normal((tokens, hidden), dtype=np.float32))
+    qb, kb, vb, mixb = (ctx.buffer(nbytes=tokens * inner * 4) for _ in range(4))
+    ob, ob2 = (ctx.buffer(nbytes=tokens * hidden * 4) for _ in range(2))
+    p = hip.ChainAttnParams()
+    for i, name in enumerate(("q", "k", "v")):
+        setattr(p, name, hip.GemmParams(tokens, hidden, inner, wdt, hip.GEMM_HALF, i * inner * hidden * 2))
+    p.proj = hip.GemmParams(tokens, inner, hidden, wdt, hip.GEMM_HALF, 3 * inner * hidden * 2)
+    p.qk = hip.QkNormParams(tokens, heads, heads, 128, hip.W_F32, hip.W_F32, *wl.ZIMAGE_DIMS, wl.ZIMAGE_EPS, 0, 0, *bases)
+    p.attn = hip.AttnParams(tokens, heads, heads, 128, 0, 0)
+    p.act_dtype = hip.F32
+    p.score_bound = host.score_bound(ones, ones, None, None) if bounded else 0.0
+    bufs = hip.ChainAttnBuffers(nb.handle, qb.handle, kb.handle, vb.handle, mixb.handle, ob.handle)
+    wts = hip.ChainAttnWeights(wbuf.handle, wbuf.handle, wbuf.handle, normb.handle, normb.handle, posb.handle, ropeb.handle, wbuf.handle)
+    x = hip.GemmExt()
+    x.a_dtype = x.c_dtype = hip.F32
+    for b in (mixb, ob, ob2):
+        b.write(np.full(b.nbytes, 0x7B, np.uint8))
+    L.zdraw_hip_set_attention_variant(knob)
+    try:
+        batch = L.zdraw_hip_batch_begin(ctx.queue)
+        rc = L.zdraw_hip_run_chain_attn_enc(batch, C.byref(bufs), C.byref(wts), C.byref(p))
+        assert L.zdraw_hip_batch_end(batch) == 0
+    finally:
+        L.zdraw_hip_set_attention_variant(0)
+    assert rc == 0, hip.last_error()
+    batch = L.zdraw_hip_batch_begin(ctx.queue)
+    assert L.zdraw_hip_run_gemm_ext_enc(batch, mixb.handle, wbuf.handle, ob2.handle, C.byref(p.proj), C.byref(x)) == 0, hip.last_error()
+    assert L.zdraw_hip_batch_end(batch) == 0
+    got, want = ob.read(np.uint32, (tokens, hidden)), ob2.read(np.uint32, (tokens, hidden))
+    assert np.array_equal(got, want), say
+    assert np.isfinite(got.view(np.float32)).all() and np.abs(got.view(np.float32)).max() > 0
+    for b in (nb, qb, kb, vb, mixb, ob, ob2, posb, ropeb, wbuf, normb):
+        b.release()
+
+
 def test_chain_attention_segment_refuses_what_it_cannot_run(ctx):
     # 1 = unavailable with nothing enqueued (the caller keeps its own path), negative = invalid
     L = hip.lib()

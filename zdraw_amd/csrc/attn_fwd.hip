@@ -95,6 +95,13 @@ __device__ __forceinline__ void pin(T& v) {
 // (i>>2)+4j, column i&3 of that lane's 4-element chunk); a lane's address must point at
 // row (lane&15)>>2, chunk lane&3 of the 4 x 16 patch.
 
+// Four f32 values rounded to 16 bits (kF16, or else bf16).
+__device__ __forceinline__ u32x2 round4(const f32x4& v, int dtype) {
+    typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+    return dtype == kF16 ? __builtin_bit_cast(u32x2, __builtin_convertvector(v, f16x4))
+                         : __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
+}
+
 // QB = 32-query blocks per wave, NW = waves per workgroup. Built shapes:
 //   QB=1, NW=8: two waves per SIMD, 256 registers each (default);
 //   QB=1, NW=4: two workgroups per CU, each with its own LDS ring.
@@ -1197,28 +1204,40 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
 #pragma unroll
         for (int r = 0; r < 2; r++)
             inv_r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + c16), (int)__float_as_uint(inv_l)));
-        if (splits > 1) {
-            // unnormalised rows, reference point and denominator of this part
+        const bool part = splits > 1; // unnormalised rows, reference point and denominator of a part of the keys
+        if (part || a.out_dtype == kF32) {
+            // f32 rows leave as the 16-bit ones below do, through 16 KB of LDS of the wave's own (16-byte
+            // chunk c of row r at c ^ (r & 15)) as whole 512-byte rows, two per instruction: straight from
+            // the lanes they are 64-byte pieces, which the CU's address unit takes one by one. (24 heads, 1024
+            // tokens in two parts 24.7 -> 24.2 us; 30 heads, 4224 tokens, f32 rows 267.5 -> 266.)
+            if constexpr (KG == 1) __syncthreads(); // every wave is done with the ring
+            typedef __attribute__((address_space(3))) f32x4* lds_turn_t;
+            const unsigned turn = KG == 2 ? lds_address(Vs) + (unsigned)(gw * (64 * 64 * 4)) : lds_address(smem) + (unsigned)(wave * (QR * D * 4));
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+#pragma unroll
+                for (int dt = 0; dt < 8; dt++)
+                    *(lds_turn_t)(turn + (unsigned)((16 * r + c16) * (D * 4) + (((4 * dt + g4) ^ c16) * 16))) = part ? oacc16[dt][r] : oacc16[dt][r] * inv_r[r];
             const int64_t prow0 = (int64_t)blockIdx.x * BQ + gw * QR;
+            float* const base = part ? a.part_o + prow0 * D
+                                     : reinterpret_cast<float*>(a.o) + (int64_t)seg * a.o_bs + (int64_t)q0 * a.o_ts + (int64_t)head * a.o_hs;
+            const int64_t stride = part ? (int64_t)D : a.o_ts;
+            const int rows = part ? QR : a.tokens - q0;
+            // (uniform) the rounded rows that the product behind this launch reads
+            unsigned short* const row16 = part || !a.o16 ? nullptr : static_cast<unsigned short*>(a.o16) + (((int64_t)seg * a.tokens + q0) * a.heads + head) * D;
 #pragma unroll
-            for (int r = 0; r < 2; r++) {
-                float* op = a.part_o + (prow0 + 16 * r + c16) * D + 4 * g4;
-#pragma unroll
-                for (int dt = 0; dt < 8; dt++) *reinterpret_cast<f32x4*>(op + 16 * dt) = oacc16[dt][r];
+            for (int i = 0; i < 16; i++) {
+                const int r = 2 * i + h;
+                const f32x4 v = *(lds_turn_t)(turn + (unsigned)(i * 1024 + lane * 16));
+                if (r < rows) {
+                    const int d = (l32 ^ (r & 15)) * 4;
+                    *reinterpret_cast<f32x4*>(base + r * stride + d) = v;
+                    if (row16) *reinterpret_cast<u32x2*>(row16 + (int64_t)r * (a.heads * D) + d) = round4(v, a.o16_dtype);
+                }
             }
-            if (h == 0) {
+            if (part && h == 0) {
                 a.part_ml[(prow0 + l32) * 2] = BOUNDED ? 0.f : m_run[0];
                 a.part_ml[(prow0 + l32) * 2 + 1] = l_tot;
-            }
-        } else if (a.out_dtype == kF32) {
-#pragma unroll
-            for (int r = 0; r < 2; r++) {
-                const int qrow = q0 + 16 * r + c16;
-                if (qrow < a.tokens) {
-                    float* op = reinterpret_cast<float*>(a.o) + (int64_t)seg * a.o_bs + (int64_t)qrow * a.o_ts + (int64_t)head * a.o_hs + 4 * g4;
-#pragma unroll
-                    for (int dt = 0; dt < 8; dt++) *reinterpret_cast<f32x4*>(op + 16 * dt) = oacc16[dt][r] * inv_r[r];
-                }
             }
         } else {
             // 16-bit output: a lane holds 8-byte pieces of two rows, which would leave the chip as
@@ -1285,6 +1304,10 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
 #pragma unroll
                             for (int j = 0; j < 4; j++) v[j] = oacc[qi][blk][4 * i + j] * inv_l;
                             *reinterpret_cast<f32x4*>(op + 32 * blk + 8 * i + 4 * h) = v;
+                            if constexpr (DMA)
+                                if (a.o16)
+                                    *reinterpret_cast<u32x2*>(static_cast<unsigned short*>(a.o16) + (((int64_t)seg * a.tokens + qrow) * a.heads + head) * D +
+                                                              32 * blk + 8 * i + 4 * h) = round4(v, a.o16_dtype);
                         }
                 }
             } else {
@@ -1381,6 +1404,8 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const AttnArgs a, int b
     const int64_t off = (int64_t)seg * a.o_bs + (int64_t)qrow * a.o_ts + (int64_t)head * a.o_hs + d0;
     if (a.out_dtype == kF32) {
         *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.o) + off) = acc;
+        if (a.o16)
+            *reinterpret_cast<u32x2*>(static_cast<unsigned short*>(a.o16) + (((int64_t)seg * a.tokens + qrow) * a.heads + head) * D + d0) = round4(acc, a.o16_dtype);
     } else if (a.out_dtype == kF16) {
         typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
         *reinterpret_cast<f16x4*>(reinterpret_cast<_Float16*>(a.o) + off) = __builtin_convertvector(acc, f16x4);

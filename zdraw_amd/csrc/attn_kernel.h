@@ -81,7 +81,8 @@ struct AttnArgs {
     int32_t tile_base;  // first logical tile (segment, head, query block) that is split
     int32_t splits;     // 0 or 1 = none
     int32_t part_wgs;   // workgroups at the head of the grid that are parts (a multiple of 8), or 0
-    int32_t pad2;
+    int32_t o16_dtype;  // kBF16 or kF16
+    void* o16;          // f32 results, prepared 16-bit operands only: the same rows rounded, dense [segment][tokens][heads][128], or null
     float* part_o;      // f32 [tile - tile_base][splits][block rows][128]
     float* part_ml;     // f32 [tile - tile_base][splits][block rows][2]
 };

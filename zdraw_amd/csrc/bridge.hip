@@ -966,11 +966,21 @@ bool scratch_poisoned(int slot) {
     return false;
 }
 
+// Scratch slot 6 as room for `bytes` of f32 activations rounded to the weight's type; null where there is none, or
+// none may be taken. A product that can run without the copy keeps its address out of a graph: the slot may be
+// replaced by a larger one, and another stream may replay the graph while this queue works.
+void* gemm_rounded_rows(const GemmArgs& g, size_t bytes, Queue* queue) {
+    if (gemm_rounds_in_place(g) && capturing(queue)) return nullptr;
+    Buffer* b = queue_scratch(queue, 6, bytes);
+    return b ? b->ptr : nullptr;
+}
+
 // C = A x W^T (metal_api.m gemm encode paths). Validates, then launches on `stream`.
 // One launch for `groups` (1..3) products that share A, every dimension and the
 // extension block: group i multiplies by ws[i] at byte offset w_offs[i] into cs[i].
+// a_rounded: a launch ahead has already written the rounded copy of dense f32 rows into gemm_rounded_rows(...).
 int enqueue_gemm_group(void* a, void* const* ws, void* const* cs, const uint64_t* w_offs, int groups,
-                       const ZdrawGemmParams* p, const ZdrawHipGemmExt* x, Queue* queue) {
+                       const ZdrawGemmParams* p, const ZdrawHipGemmExt* x, Queue* queue, bool a_rounded = false) {
     if (!p || !x || !queue || groups < 1 || groups > 3) {
         set_err("null params");
         return ZDRAW_HIP_ERR_HANDLE;
@@ -1033,22 +1043,24 @@ int enqueue_gemm_group(void* a, void* const* ws, void* const* cs, const uint64_t
     if (const size_t rb = gemm_round_bytes(g, a_dtype)) {
         // f32 activations are rounded to the weight's type once, into scratch slot 6, and the
         // product then runs as for 16-bit activations
-        // (a product that can run without the copy keeps its address out of a graph: the slot may be
-        // replaced by a larger one, and another stream may replay the graph while this queue works)
         in_place = gemm_rounds_in_place(g);
-        Buffer* a16 = in_place && capturing(queue) ? nullptr : queue_scratch(queue, 6, rb);
-        if (!a16 && !in_place) {
+        g.a16 = gemm_rounded_rows(g, rb, queue);
+        if (!g.a16 && !in_place) {
             set_err("scratch allocation failed");
             return ZDRAW_HIP_ERR_HANDLE;
         }
-        if (a16) g.a16 = a16->ptr;
-        unstaged = !a16;
+        unstaged = !g.a16;
     }
     // Pieces of C that one launch can address: the whole but where A or W spans all but 4 GiB (the rounded
     // copy of f32 rows spans at most half of that)
     int64_t m_step = a_dtype == ZDRAW_HIP_F32 ? g.m : gemm_launch_rows(g.m, g.lda, g.k), n_step = gemm_launch_rows(g.n, g.ldw, g.k);
     if (m_step == 0 || n_step == 0) unstaged = true;
     if (unstaged) m_step = g.m, n_step = g.n;
+    if (a_rounded && !unstaged && a_dtype == ZDRAW_HIP_F32) {
+        g.a = g.a16;
+        g.lda = g.k;
+        a_dtype = (int)wt;
+    }
     for (int64_t m0 = 0; m0 < g.m; m0 += m_step)
         for (int64_t n0 = 0; n0 < g.n; n0 += n_step) {
             GemmArgs piece = g;
@@ -1097,12 +1109,12 @@ int enqueue_gemm_group(void* a, void* const* ws, void* const* cs, const uint64_t
     return ZDRAW_HIP_OK;
 }
 
-int enqueue_gemm(void* a, void* w, void* c, const ZdrawGemmParams* p, const ZdrawHipGemmExt* x, Queue* queue) {
+int enqueue_gemm(void* a, void* w, void* c, const ZdrawGemmParams* p, const ZdrawHipGemmExt* x, Queue* queue, bool a_rounded = false) {
     if (!p) {
         set_err("null params");
         return ZDRAW_HIP_ERR_HANDLE;
     }
-    return enqueue_gemm_group(a, &w, &c, &p->weight_offset, 1, p, x, queue);
+    return enqueue_gemm_group(a, &w, &c, &p->weight_offset, 1, p, x, queue, a_rounded);
 }
 
 } // namespace
@@ -1798,8 +1810,18 @@ int zdraw_hip_run_chain_attn_enc(void* batch, const ZdrawHipChainAttnBuffers* bu
         if ((rc = enqueue_gemm(bufs->norm, w->k, bufs->k, &p->k, &gx, b->queue)) != ZDRAW_HIP_OK) return rc;
         if ((rc = enqueue_gemm(bufs->norm, w->v, bufs->v, &p->v, &gx, b->queue)) != ZDRAW_HIP_OK) return rc;
     }
+    // f32 rows: the output projection reads the mixed heads rounded to its weight's type. The attention launch
+    // (or its merge) holds every row whole and writes that copy beside the f32 one, instead of a launch
+    // that reads the rows back for it: 30 heads, 1536 tokens, 8 us and a gap a layer.
+    if (p->act_dtype == ZDRAW_HIP_F32 && plan.in_dtype == kBF16 && plan.k_mode == kQkNone && plan.shape != 1) {
+        GemmArgs g;
+        memset(&g, 0, sizeof(g));
+        g.m = (int32_t)p->proj.m; g.n = (int32_t)p->proj.n; g.k = (int32_t)p->proj.k;
+        plan.args.o16 = gemm_rounded_rows(g, gemm_round_bytes(g, ZDRAW_HIP_F32), b->queue);
+        plan.args.o16_dtype = p->proj.dtype == ZDRAW_HIP_W_F16 ? kF16 : kBF16;
+    }
     if ((rc = enqueue(plan, st)) != ZDRAW_HIP_OK) return rc;
-    return enqueue_gemm(bufs->mix, w->proj, bufs->attn, &p->proj, &gx, b->queue);
+    return enqueue_gemm(bufs->mix, w->proj, bufs->attn, &p->proj, &gx, b->queue, plan.args.o16 != nullptr);
 }
 
 // ------------------------------------------------------------------ scratch
