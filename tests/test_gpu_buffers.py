@@ -251,3 +251,59 @@ def test_read_buffer_any_is_ordered_after_the_queue(ctx):
     assert L.zdraw_hip_read_buffer_any(ctx.queue, res.o.handle, raw.ctypes.data_as(C.c_void_p), res.o.nbytes + 1) == hip.ERR_HANDLE
     assert L.zdraw_hip_read_buffer_any(None, res.o.handle, raw.ctypes.data_as(C.c_void_p), 16) == hip.ERR_HANDLE
     res.release()
+
+
+# ------------------------------------------------------ operands in host memory, read and written in place
+# Context.run takes them through the queue's pinned memory where it can and through device buffers of its own
+# where it cannot (more than 16 MB in all): the bits of run_pooled, which always takes device buffers. Sizes
+# around the bound and its growth, either side of the rounding launch, a key limit, the wide head; poisoned by
+# a larger call in between.
+@pytest.mark.parametrize("tokens,heads,dim,valid", [(1, 1, 128, 0), (159, 3, 128, 100), (160, 3, 128, 0), (257, 2, 128, 250), (700, 3, 128, 0),
+                                                    (1024, 8, 128, 0), (1025, 8, 128, 0), (64, 1, 512, 0), (2048, 1, 512, 0), (2112, 1, 512, 0)])
+def test_host_operands_in_place_equal_device_buffers(ctx, tokens, heads, dim, valid):
+    say(f"tokens {tokens} heads {heads} dim {dim}")
+    rng = np.random.default_rng(tokens + dim)
+    q, k, v = (rng.standard_normal((tokens, heads, dim), dtype=np.float32) for _ in range(3))
+    cfg = host.Config(tokens, heads, heads, dim, False, valid)
+    want = ctx.run_pooled(q, k, v, cfg)
+    other = rng.standard_normal((300, 2, 128), dtype=np.float32)
+    for _ in range(2):
+        assert np.array_equal(ctx.run(q, k, v, cfg).view(np.uint32), want.view(np.uint32))
+        ctx.run(other, other, other, host.Config(300, 2, 2, 128, False, 0))
+
+
+def test_host_operands_belong_to_one_call_at_a_time(ctx):
+    L = hip.lib()
+    sizes = lambda *n: (C.c_size_t * 4)(*n)
+    handles, memory = (C.c_void_p * 4)(), (C.c_void_p * 4)()
+    begin = lambda q, n: L.zdraw_hip_host_operands_begin(q, sizes(*n), handles, memory)
+    queue = L.zdraw_hip_create_queue(ctx.device)
+    assert begin(queue, (0, 4, 4, 4)) == hip.UNAVAILABLE
+    assert begin(queue, (1 << 24, 4, 4, 4)) == hip.UNAVAILABLE  # 16 MB and a little
+    assert begin(queue, ((1 << 64) - 1, 1, 1, 1)) == hip.UNAVAILABLE  # no sum that wraps
+    stream, graph = C.c_void_p((C.c_void_p * 2).from_address(queue)[1]), C.c_void_p()
+    assert L.hipStreamBeginCapture(stream, C.c_int(2)) == 0
+    rc = begin(queue, (512, 512, 512, 512))
+    assert L.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert rc == hip.UNAVAILABLE
+    if graph.value:
+        assert L.hipGraphDestroy(graph) == 0
+    assert begin(queue, (100, 512, 1000, 4)) == hip.OK
+    spans = sorted(zip(list(memory), (100, 512, 1000, 4)))
+    assert all(p % 256 == 0 for p, _ in spans) and all(a + n <= b for (a, n), (b, _) in zip(spans, spans[1:]))
+    assert [L.zdraw_hip_buffer_length(h) for h in handles] == [100, 512, 1000, 4]
+    assert begin(queue, (4, 4, 4, 4)) == hip.UNAVAILABLE  # taken
+    L.zdraw_hip_host_operands_end(queue)
+    assert begin(queue, (4, 4, 4, 4)) == hip.OK
+    L.zdraw_hip_host_operands_end(queue)
+    L.zdraw_hip_release_queue(queue)
+    # a call that finds it taken makes buffers of its own
+    rng = np.random.default_rng(5)
+    q, k, v = (rng.standard_normal((200, 2, 128), dtype=np.float32) for _ in range(3))
+    cfg = host.Config(200, 2, 2, 128, False, 0)
+    want = ctx.run(q, k, v, cfg)
+    assert begin(ctx.queue, (4, 4, 4, 4)) == hip.OK
+    C.memset(memory[0], 0x7B, 4)
+    assert np.array_equal(ctx.run(q, k, v, cfg), want)
+    assert C.string_at(memory[0], 4) == b"\x7b" * 4
+    L.zdraw_hip_host_operands_end(ctx.queue)

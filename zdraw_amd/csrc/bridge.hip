@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -58,6 +59,14 @@ struct Buffer {
     // such buffers have anything read from them cached (the norm weights' maximum).
     bool stable;
 };
+// Operands in host memory on their way through a blocking call: pinned memory that the kernels read and write in
+// place, kept by the queue from one call to the next, for one call at a time.
+struct HostOperands {
+    std::atomic<bool> busy{false};
+    char* base = nullptr;
+    size_t len = 0;
+    Buffer buf[4] = {};
+};
 constexpr int kScratchSlots = 8; // per queue: slots 0-6 as below, 7 = staged norm weights
 constexpr int kCallerSlots = 7;  // zdraw_hip_attn_scratch hands these out (metal_api.m:6147-6191)
 struct Queue {
@@ -67,6 +76,7 @@ struct Queue {
     // grow-only slots owned by the queue whose work uses them, so that two queues never share a
     // byte of it; freed with the queue.
     Buffer* scratch[kScratchSlots] = {};
+    HostOperands host;
 };
 struct Pipeline {
     int kind; // 0 = attention_block_mfma, 1 = qk_norm_rope, 2 = gemm_half
@@ -222,6 +232,12 @@ Buffer* queue_scratch(Queue* q, int slot, size_t bytes) {
     if (!q || slot < 0 || slot >= kScratchSlots || bytes == 0) return nullptr;
     return grow_slot(&q->scratch[slot], slot, bytes, [q] { (void)hipStreamSynchronize(q->stream); });
 }
+
+// The most pinned memory a queue keeps for operands in host memory (HostOperands). attention_fast.run, us, with
+// device buffers made for the call and in this memory: 2 heads, 64 tokens 81 -> 45, 256 118 -> 79, 1024 266 -> 227; 8
+// heads, 512 tokens 600 -> 435, 1024 (16 MB in all) 973 -> 763. Beyond it what bounds the call is its bytes over PCIe
+// either way, and the runtime's own staged copies keep up (24 heads, 1024 tokens 3073, 3282 in place).
+constexpr size_t kHostOperandBytes = size_t{16} << 20;
 
 // Whether what is enqueued now becomes part of a graph.
 bool capturing(const Queue* q) {
@@ -1211,6 +1227,7 @@ void zdraw_hip_release_queue(void* queue) {
             b = nullptr;
         }
     }
+    if (q->host.base) (void)hipHostFree(q->host.base);
     (void)hipStreamDestroy(q->stream);
     delete q;
 }
@@ -1318,6 +1335,47 @@ void zdraw_hip_release_buffer(void* buffer) {
 }
 
 void zdraw_hip_release_weight_buffer(void* buffer) { zdraw_hip_release_buffer(buffer); }
+
+int zdraw_hip_host_operands_begin(void* queue, const size_t bytes[4], void* handles[4], uint8_t* memory[4]) {
+    Queue* q = static_cast<Queue*>(queue);
+    if (!q || !bytes || !handles || !memory) return ZDRAW_HIP_ERR_HANDLE;
+    size_t at[4], total = 0;
+    for (int i = 0; i < 4; i++) {
+        if (bytes[i] == 0 || bytes[i] > kHostOperandBytes) return ZDRAW_HIP_UNAVAILABLE;
+        at[i] = total;
+        total += (bytes[i] + 255) & ~size_t{255};
+    }
+    if (total > kHostOperandBytes || capturing(q)) return ZDRAW_HIP_UNAVAILABLE;
+    HostOperands& h = q->host;
+    if (h.busy.exchange(true, std::memory_order_acquire)) return ZDRAW_HIP_UNAVAILABLE;
+    if (h.len < total) {
+        // (in powers of two from 1 MB on: a range of sizes settles after few allocations)
+        size_t want = size_t{1} << 20;
+        while (want < total) want *= 2;
+        void* p = nullptr;
+        if (hipStreamSynchronize(q->stream) != hipSuccess || hipHostMalloc(&p, want, hipHostMallocCoherent) != hipSuccess) {
+            (void)hipGetLastError(); // or the next launch would report it
+            h.busy.store(false, std::memory_order_release);
+            return ZDRAW_HIP_UNAVAILABLE;
+        }
+        if (h.base) (void)hipHostFree(h.base);
+        h.base = static_cast<char*>(p);
+        h.len = want;
+    }
+    for (int i = 0; i < 4; i++) {
+        h.buf[i] = Buffer{h.base + at[i], bytes[i], false, false};
+        handles[i] = &h.buf[i];
+        memory[i] = reinterpret_cast<uint8_t*>(h.base + at[i]);
+    }
+    return ZDRAW_HIP_OK;
+}
+
+void zdraw_hip_host_operands_end(void* queue) {
+    Queue* q = static_cast<Queue*>(queue);
+    if (!q) return;
+    (void)hipStreamSynchronize(q->stream); // a call that failed half way may have left work behind (idle: 0.2 us)
+    q->host.busy.store(false, std::memory_order_release);
+}
 
 // ---------------------------------------------------------------- pipelines
 void* zdraw_hip_compile(void* device, const char* source, const char* entry, char* error_buf, size_t error_len) {

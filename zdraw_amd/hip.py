@@ -103,6 +103,8 @@ SYMBOLS = {
     "zdraw_hip_buffer_length": (_sz, [_vp]),
     "zdraw_hip_buffer_device_ptr": (_vp, [_vp]),
     "zdraw_hip_release_buffer": (None, [_vp]),
+    "zdraw_hip_host_operands_begin": (_int, [_vp, C.POINTER(_sz), C.POINTER(_vp), C.POINTER(_vp)]),
+    "zdraw_hip_host_operands_end": (None, [_vp]),
     "zdraw_hip_compile": (_vp, [_vp, C.c_char_p, C.c_char_p, C.c_char_p, _sz]),
     "zdraw_hip_release_pipeline": (None, [_vp]),
     "zdraw_hip_pipeline_threads": (_sz, [_vp]),

@@ -157,6 +157,23 @@ Error Context::run(float* out, size_t out_len, const float* q, size_t q_len, con
     if (cfg.causal || cfg.kv_heads != cfg.heads) return Error::UnsupportedShape;
     ZdrawAttnParams params;
     if (!paramsFor(cfg, &params)) return Error::InvalidShape;
+    if (q && k && v && out) {
+        // through the queue's pinned memory, which the kernels read and write in place: no device
+        // buffer, no blocking upload, one wait
+        const size_t bytes[4] = {q_len * sizeof(float), k_len * sizeof(float), v_len * sizeof(float), out_len * sizeof(float)};
+        void* handles[4];
+        uint8_t* memory[4];
+        if (zdraw_hip_host_operands_begin(queue, bytes, handles, memory) == ZDRAW_HIP_OK) {
+            std::memcpy(memory[0], q, bytes[0]);
+            std::memcpy(memory[1], k, bytes[1]);
+            std::memcpy(memory[2], v, bytes[2]);
+            const Error done = fromCode(zdraw_hip_run_attention(queue, picked.pipeline, handles[0], handles[1], handles[2],
+                                                                handles[3], &params, (uint32_t)picked.kernel, picked.threads));
+            if (done == Error::Ok) std::memcpy(out, memory[3], bytes[3]);
+            zdraw_hip_host_operands_end(queue);
+            return done;
+        }
+    }
     // mattn.zig:349-374 (runFresh): upload q/k/v, one dispatch, read back.
     Buffer qb = Buffer::fromBytes(device, q, q_len * sizeof(float));
     Buffer kb = Buffer::fromBytes(device, k, k_len * sizeof(float));
