@@ -33,6 +33,7 @@ constexpr int64_t kThinTokens = 8192;
 
 template <typename TIn, int MODE, int G>
 __global__ void __launch_bounds__(kPrepTokens * 64) qk_prepass_kernel(const PrepPair pair) {
+    touch_args<sizeof(PrepPair)>();
     // grid z = operand * batch + segment; the choice is uniform over the workgroup
     const int op = (int)blockIdx.z / pair.op[0].batch;
     const PrepArgs& p = pair.op[op];
