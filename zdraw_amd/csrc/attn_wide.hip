@@ -61,7 +61,7 @@ constexpr int V_RING = NSK * K_SLOT;
 constexpr int P_RING = V_RING + NSV * V_SLOT;  // two slots of the exponentiated blocks
 constexpr int P_SLOT = NW * 2 * 1024;          // 2 KB a wave
 constexpr size_t kLdsBytes = (size_t)P_RING + 2 * P_SLOT + 16384; // 160 KB: the last 16 KB hold query rows only
-constexpr float kTau = 8.0f;      // log2 headroom of the lazy softmax maximum (attn_wide_finish_kernel)
+constexpr float kTau = 8.0f;      // log2 headroom of the lazy softmax maximum (attn_wide_safe_kernel)
 constexpr float kRowSumLimit = 0x1p90f; // a row sum past this flags its tile: a P beyond 2^90 may be on its way to overflow
 constexpr int RA = 6;             // K fragments read ahead of their MFMA
 constexpr int VA = 3;             // V fragment pairs read ahead
@@ -291,10 +291,10 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
     // largest score of the range's first block. It never moves, so nothing is ever rescaled
     // (any branch that touches the 256 accumulation registers inside the loop costs hundreds of
     // spills). fp32 and bf16 share one exponent
-    // range, so a later score may lie far above the reference (P up to 2^kHeadroom and beyond)
-    // or far below it without any loss; only a row whose scores climb more than kHeadroom above
+    // range, so a later score may lie far above the reference (P up to 2^90)
+    // or far below it without any loss; only a row whose scores climb some 90 (log2) above
     // its first block's is out of reach. Such a row shows in its row sum: the wave then flags the
-    // query tile, and attn_wide_finish_kernel, which follows every launch, forms flagged tiles
+    // query tile, and attn_wide_safe_kernel, which follows every launch, forms flagged tiles
     // again with a running maximum.
     float mc[2];
 #pragma unroll
@@ -439,7 +439,7 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
         l_tot[r] = pair_sum(row_pair_sum(l_run[r]));
         out_of_reach |= !(l_tot[r] <= kRowSumLimit);
     }
-    // a row sum past 2^kHeadroom (or not a number): some score left the reach of the fixed reference
+    // a row sum past kRowSumLimit (or not a number): some score left the reach of the fixed reference
     if (__any(out_of_reach) && el == 0) a.redo[tile] = 1;
     // the partner's reference points and row sums, through P's first slot (every wave is done with it)
     __syncthreads();
@@ -470,7 +470,7 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// The tiles that attn_wide_kernel flagged (a score more than 2^kHeadroom above its row's first
+// The tiles that attn_wide_kernel flagged (a score some 90, log2, above its row's first
 // block), formed again with a lazy running maximum. A workgroup is four waves and owns 128 query
 // rows and HALF of the 512 output dims over all keys (both workgroups of a tile form the full
 // scores: 48 MFMAs per wave and block where 32 would do); with 128 accumulation registers per
@@ -770,7 +770,9 @@ size_t wide_part_bytes(int tokens, int splits) {
 // blocks): the number whose estimate is the smallest. A full round over the CUs takes kFullUs per
 // block of a range (the power limit), a thinly filled one kThinUs (a wave's own chain), in between
 // in proportion; every range's share of O goes to memory and back once. The constants are a fit to
-// 1 to 8 ranges of 256 to 18432 tokens; the rule's pick is the measured best or within 4 % of it, so
+// 1 to 8 ranges of 256 to 18432 tokens; the rule's pick is the measured best or within 4 % of it
+// (with the 32 x 32 x 16 form of the kernel; with this one within 3 %, but at 2560 tokens 58.7 us with five for 55.5 with eight
+// and at 8192 157.3 with three for 151.5 with four; constants that take those put 7104 tokens at three instead of four: at 7168 142 for 129), so
 // ranges that save less than 3 % are not worth their shares (1019904 tokens would take six ranges and 12 GB
 // for 1.5 %), and neither are shares of more than kMaxShareBytes, which the queue keeps (33024 tokens: six
 // ranges, 389 MB, a quarter of the time by the estimate; 18432: three, 108 MB, 11 %).
