@@ -1111,9 +1111,8 @@ def test_running_maximum_moves_its_reference_point_late(ctx, name, tokens, heads
     assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
 
 
-# A masked row's reference point stays at 0 while its first block's maximum lies within 16 (log2, 11.1 nats)
-# of it: first admitted blocks inside and outside that band on both sides of 0, close to its edges, and
-# later keys that leave the scores' start at 0, move it, or follow a move
+# A masked row's first admitted block sets its reference point wherever its maximum lies: on both sides of 0, near
+# it and far from it, with later keys that leave the reference where it is, or move it
 @pytest.mark.parametrize("knob", [2, 4, 0], ids=["whole", "parts", "default"])
 @pytest.mark.parametrize("first", [-30.0, -12.0, -10.0, 0.0, 10.0, 12.0, 30.0])
 @pytest.mark.parametrize("late", [0.0, 14.0, 45.0])
@@ -1132,6 +1131,28 @@ def test_masked_first_blocks_about_the_zero_reference(ctx, first, late, knob):
     got = _plain_fused(ctx, q, k, v, in_dtype=hip.BF16, key_pad=pad, knob=knob)
     want = zo.attention_token_list(q, k, v, zo.Config(tokens, heads, heads, 128), list(range(tokens)), key_pad=pad)
     refimpl.check_close(got, want, "first block about the zero reference")
+
+
+# The largest score of a row's first block is its reference point, so that key's probability is exactly 1 (any other
+# reference rounds it to bf16, up to 2^-9 off). A row that this key decides (the others 50 nats below: 2e-19 of the
+# row at 1490 tokens) returns the key's value but for the roundings of a few f32 operations on it.
+@pytest.mark.parametrize("knob", [2, 4, 0], ids=["whole", "parts", "default"])
+@pytest.mark.parametrize("first", [-10.0, -3.3, 3.3, 10.0, 30.0])
+@pytest.mark.parametrize("masked", [True, False])
+def test_row_that_one_key_of_its_first_block_decides_returns_its_value(ctx, masked, first, knob):
+    say(f"first block {first} nats, masked {masked}, knob {knob}")
+    tokens, heads, dead = 1490, 2, 64 if masked else 0
+    u = np.full(128, 1.0 / np.sqrt(128.0), np.float32)
+    v = np.random.default_rng(8).standard_normal((tokens, heads, 128), dtype=np.float32)
+    q, k = np.empty_like(v), np.empty_like(v)
+    q[:] = np.float32(4.0) * u
+    k[:] = np.float32((first - 50.0) * np.sqrt(128.0) / 4.0) * u
+    k[dead + 5] = np.float32(first * np.sqrt(128.0) / 4.0) * u
+    v = host.bf16_bits_to_f32(host.f32_to_bf16_bits(v))
+    pad = (np.arange(tokens) < dead).astype(np.uint8) if masked else None
+    got = _plain_fused(ctx, q, k, v, in_dtype=hip.BF16, key_pad=pad, knob=knob)
+    want = np.broadcast_to(v[dead + 5], got.shape)
+    assert np.abs(got - want).max() <= 2.0 ** -20 * np.abs(want).max()
 
 
 def test_running_maximum_with_a_key_padding_mask_and_planted_keys(ctx):

@@ -59,7 +59,6 @@ constexpr int MAX_BLOCKS = 1024;  // key-block list capacity (tokens <= 32768)
 // (scores to +-60) 24 heads of 4608 tokens 250 -> 242 us at 16 instead of 8. P stays at or below
 // 2^20, so that V may reach 2^107 before a product leaves f32.
 constexpr float kTau = 16.0f;
-constexpr float kZeroRef = 16.0f; // a first block whose row maximum lies within this of 0 leaves the reference point at 0
 
 // Ring depth: 8 stages when one workgroup owns the CU (blocks are stored four
 // steps ahead of their first use, so one barrier per two steps orders every
@@ -148,19 +147,16 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     // through the register file, and at the board's power limit that is worth clock: -2 % of the
     // kernel's time. It costs a few registers (the compiler writes these MFMAs' results to other
     // registers than their inputs) and four lane exchanges per block, so only the builds with
-    // room take it: prepared operands, and not the running maximum with a mask in two key groups
-    // (that build then spills inside the loop). (Giving the scores that form too would double the MFMA
-    // instructions on a vector issue port that the softmax already half fills.) Of the masked running-maximum
-    // builds that of one key group has the registers (36 bytes spilled outside the steps, 16 in them):
-    // with the scores' start below 24 heads of 4064 of 4608 tokens 214 -> 203.5 us, 10 000 tokens in two calls 3160 -> 3025.
-    constexpr bool PV16 = DMA && (!MASKED || KG == 1);
+    // room take it: prepared operands, and not the running maximum together with a mask (that
+    // build then spills inside the loop; with its reference points held at 0 it has the room, 24 heads of 4064 of 4608
+    // tokens 214 -> 203.5 us, but a row's largest P is then no longer exactly 1 and rounds like the rest). (Giving the scores that form too would double the MFMA
+    // instructions on a vector issue port that the softmax already half fills.)
+    constexpr bool PV16 = DMA && (!MASKED || (BOUNDED && KG == 1));
     constexpr int KSTAGE = DMA ? KB * D : KS_ELEMS; // elements per ring stage
     constexpr int VSTAGE = DMA ? KB * D : VS_ELEMS;
     // a block enters the ring AHEAD steps before S needs its K (direct loads: one more step, to land)
     constexpr int AHEAD = NST == 8 ? (DMA ? 5 : 4) : 2;
-    // slots between an LDS fragment read and its MFMA (the masked running-maximum build of one key group: the
-    // shorter distance, for its registers. 10 000 tokens: 1 % slower with the longer one)
-    constexpr int LA = DMA && !(MASKED && !BOUNDED && KG == 1) ? kLdsLookaheadDirect : kLdsLookahead;
+    constexpr int LA = DMA ? kLdsLookaheadDirect : kLdsLookahead; // slots between an LDS fragment read and its MFMA
     constexpr int RB = kReadBatch;      // slots whose reads are issued together (divides 16 and LA)
     // Wave priority while an MFMA is being issued. The register-staged builds gain from it (the
     // masked one loses 13 % without). The direct-to-LDS build runs 5 % fewer cycles per
@@ -556,13 +552,6 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     float negm[QB]; // (one value per lane: every element of the accumulator starts from it)
 #pragma unroll
     for (int qi = 0; qi < QB; qi++) negm[qi] = 0.f;
-    // The masked build of one key group starts the scores from an inline 0 as long as every reference
-    // point of the wave is 0 (wave-uniform): the sixteen moves that fill the accumulator from negm,
-    // and eight more that the compiler adds there, stand between two MFMAs. A first block whose row
-    // maximum lies within kZeroRef of 0 leaves the reference there: QK-normalised scores do. The other
-    // builds hide the moves: with the branch 4608 unmasked tokens 211 -> 214 us, 1536 37.1 -> 38.4.
-    constexpr bool REFZERO = REFACC && MASKED && KG == 1;
-    bool ref_zero = true;
 
     // LDS byte addresses of this lane's fragments in ring stage 0; a stage, a key half (kb)
     // and a row half add constants. K: key row l32, dims 16 s + 8 h .. +7 (8 addresses, the
@@ -736,26 +725,6 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                 }
             } else {
                 const int st = slot >> 1;
-                if constexpr (REFZERO) {
-                    if (slot == 0) {
-                        // (the empty statement keeps the two branches from being merged into one MFMA
-                        // whose C operand would have to be sixteen registers either way)
-                        if (ref_zero) {
-                            f32x16 z;
-#pragma unroll
-                            for (int j = 0; j < 16; j++) z[j] = 0.f;
-                            s_next[0] = score_mfma(kf[0], qf[0][0], z);
-                            asm volatile("" : "+v"(s_next[0]));
-                        } else {
-                            f32x16 z;
-#pragma unroll
-                            for (int j = 0; j < 16; j++) z[j] = negm[0];
-                            s_next[0] = score_mfma(kf[0], qf[0][0], z);
-                        }
-                        if (MFMA_PRIO) __builtin_amdgcn_s_setprio(0);
-                        return;
-                    }
-                }
 #pragma unroll
                 for (int qi = 0; qi < QB; qi++)
                     s_next[qi] = score_mfma(kf[st], qf[qi][st], s_next[qi]);
@@ -779,12 +748,10 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                         }
             }
         }
-        if constexpr (!REFZERO) {
 #pragma unroll
-            for (int qi = 0; qi < QB; qi++)
+        for (int qi = 0; qi < QB; qi++)
 #pragma unroll
-                for (int j = 0; j < 16; j++) s_next[qi][j] = REFACC ? negm[qi] : 0.f;
-        }
+            for (int j = 0; j < 16; j++) s_next[qi][j] = REFACC ? negm[qi] : 0.f;
 
         float mc[QB], alpha[QB], psum[QB];
         unsigned pc[QB][8] = {}; // P as packed bf16 pairs
@@ -922,8 +889,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                     const float ref = (REFACC && m_run[qi] != -INFINITY) ? m_run[qi] : 0.f;
                     const float mlc = pair_max(fmaxf(t0, t3)) + ref;
                     const bool up = mlc > m_run[qi] + kTau;
-                    const bool at_zero = REFZERO && m_run[qi] == -INFINITY && fabsf(mlc) <= kZeroRef;
-                    const float m_new = !up ? m_run[qi] : at_zero ? 0.f : mlc;
+                    const float m_new = up ? mlc : m_run[qi];
                     const float ref_new = (m_new == -INFINITY) ? 0.f : m_new;
                     mc[qi] = ref_new - ref;
                     alpha[qi] = __builtin_amdgcn_exp2f(m_run[qi] - ref_new);
@@ -938,7 +904,6 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                             s_next[qi][j] -= mc[qi];
                             negm[qi] = -ref_new;
                         }
-                        if constexpr (REFZERO) ref_zero = !__any(negm[qi] != 0.f);
                     }
                     l_run[qi] *= alpha[qi];
                     if constexpr (PV16) {
