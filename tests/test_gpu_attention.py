@@ -1155,6 +1155,28 @@ def test_row_that_one_key_of_its_first_block_decides_returns_its_value(ctx, mask
     assert np.abs(got - want).max() <= 2.0 ** -20 * np.abs(want).max()
 
 
+# Three blocks of keys 15.5 (log2) above the first one, with values up to 2^112: against a reference point that stays where it
+# is 32 probabilities of 2^15.5 add up to 2^132, past f32. 7.5 above, the reference does stay and the sum is at most
+# 3 * 32 * 2^7.5 * 2^112 < 2^127. In units of 2^112, the bf16 attention bar.
+@pytest.mark.parametrize("in_dtype,knob", [(hip.BF16, 2), (hip.BF16, 4), (hip.BF16, 0), (hip.F32, 2)], ids=["whole", "parts", "default", "f32"])
+@pytest.mark.parametrize("valid", [0, 1400])
+@pytest.mark.parametrize("log2_above", [7.5, 15.5])
+def test_running_maximum_with_values_near_the_end_of_the_range(ctx, valid, in_dtype, knob, log2_above):
+    say(f"valid {valid} knob {knob} {log2_above} above")
+    tokens, heads = 1504, 2
+    rng = np.random.default_rng(int(2 * log2_above) + valid)
+    u = np.full(128, 1.0 / np.sqrt(128.0), np.float32)
+    q, k, v = (np.zeros((tokens, heads, 128), np.float32) for _ in range(3))
+    q[:] = np.float32(4.0) * u
+    for b in (5, 20, 35):  # one block in each part and key group but the first
+        k[32 * b:32 * b + 32] = np.float32(log2_above * np.log(2.0) * np.sqrt(128.0) / 4.0) * u
+    rb = lambda a: host.bf16_bits_to_f32(host.f32_to_bf16_bits(a))
+    q, k, v = rb(q), rb(k), rb(rng.uniform(-1.0, 1.0, v.shape).astype(np.float32))
+    got = _plain_fused(ctx, q, k, v * np.float32(2.0 ** 112), valid=valid, in_dtype=in_dtype, knob=knob)
+    want = zo.attention_run(q, k, v, zo.Config(tokens, heads, heads, 128, False, valid))
+    refimpl.check_close(got * np.float32(2.0 ** -112), want, "values near the end of the range")
+
+
 def test_running_maximum_with_a_key_padding_mask_and_planted_keys(ctx):
     # the boolean key mask build (block list compacted, mask words in LDS): whole blocks are
     # dropped, planted keys sit right after a dropped stretch and inside a partly masked block

@@ -54,11 +54,10 @@ constexpr int VPITCH = D + 32;    // 320 B rows: a 32-lane transposing read cove
 constexpr int KS_ELEMS = KB * KPITCH;
 constexpr int VS_ELEMS = KB * VPITCH;
 constexpr int MAX_BLOCKS = 1024;  // key-block list capacity (tokens <= 32768)
-// log2 headroom of the lazy softmax maximum: a row's reference point moves when a score lies this far above it.
-// More headroom, fewer moves, each of which costs a block its exponentials twice: with norm weights near 3
-// (scores to +-60) 24 heads of 4608 tokens 250 -> 242 us at 16 instead of 8. P stays at or below
-// 2^20, so that V may reach 2^107 before a product leaves f32.
-constexpr float kTau = 16.0f;
+// log2 headroom of the lazy softmax maximum: a row's reference point moves when a score lies this far above it. Every
+// P is at most 2^(kTau + 4), so that V may reach 2^115 before a product leaves f32. (16 instead of 8 moves fewer
+// references, with norm weights near 3 24 heads of 4608 tokens 250 -> 242 us, but overflows from V = 2^107 on.)
+constexpr float kTau = 8.0f;
 
 // Ring depth: 8 stages when one workgroup owns the CU (blocks are stored four
 // steps ahead of their first use, so one barrier per two steps orders every
@@ -872,8 +871,8 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             // takes the exponentials again and rescales O and the denominator.
             bool redo = false;
 #pragma unroll
-            for (int qi = 0; qi < QB; qi++) redo |= !(psum[qi] <= 0x1p20f) || m_run[qi] == -INFINITY;
-            static_assert(kTau == 16.0f, "the watch threshold is 16 * 2^kTau");
+            for (int qi = 0; qi < QB; qi++) redo |= !(psum[qi] <= 16.0f * 256.0f) || m_run[qi] == -INFINITY;
+            static_assert(kTau == 8.0f, "the watch threshold is 16 * 2^kTau");
             if (__any(redo)) {
 #pragma unroll
                 for (int qi = 0; qi < QB; qi++) {
