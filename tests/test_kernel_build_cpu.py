@@ -45,3 +45,22 @@ def test_wide_head_kernel_leaves_m0_alone_and_no_load_reads_a_scalar_register_to
     src = os.path.join(build.CSRC, "attn_wide.hip")
     bad = build.m0_writes(src, "attn_wide_kernel") + build.vmem_sgpr_hazards(src) + build.vmem_sgpr_hazards(os.path.join(build.CSRC, "gemm_half.hip"))
     assert not bad, "\n".join(bad[:20])
+
+
+@pytest.mark.skipif(not (os.path.exists("/opt/rocm/bin/hipcc") or shutil.which("hipcc")), reason="needs hipcc")
+@pytest.mark.parametrize("name", ["attn_fwd.hip", "attn_wide.hip", "gemm_half.hip", "qk_prepass.hip"])
+def test_no_kernel_reads_past_its_arguments(name):
+    # the head of a kernel loads a word of each of its arguments' cache lines through the argument pointer
+    # (attn_device.hpp, touch_args): all of them have to lie within the segment that the kernel is launched with
+    bad = build.kernarg_overreads(os.path.join(build.CSRC, name))
+    assert not bad, "\n".join(bad[:20])
+
+
+@pytest.mark.parametrize("load,over", [("s_load_dword s6, s[0:1], 0x3c", False), ("s_load_dword s6, s[0:1], 0x40", True),
+                                       ("s_load_dwordx4 s[8:11], s[0:1], 0x30", False), ("s_load_dwordx4 s[8:11], s[0:1], 0x34", True),
+                                       ("s_mov_b64 s[4:5], s[0:1]\n\ts_cmp_lg_u32 s4, 0\n\ts_load_dword s6, s[4:5], 0x40", True),
+                                       ("s_load_dwordx2 s[0:1], s[0:1], 0x38\n\ts_load_dword s6, s[0:1], 0x40", False)])
+def test_the_check_of_reads_past_the_arguments_sees_them(monkeypatch, load, over):
+    asm = f"kern:\n; %bb.0:\n\t{load}\n\ts_endpgm\n\t.amdhsa_kernel kern\n\t\t.amdhsa_kernarg_size 64\n\t\t.amdhsa_user_sgpr_dispatch_ptr 0\n\t.end_amdhsa_kernel"
+    monkeypatch.setattr(build, "_device_asm", lambda *_: asm.split("\n"))
+    assert bool(build.kernarg_overreads("")) == over

@@ -161,6 +161,52 @@ def vmem_sgpr_hazards(src: str, extra_flags=()) -> list[str]:
     return bad
 
 
+def kernarg_overreads(src: str, extra_flags=()) -> list[str]:
+    """Compiles `src` to gfx950 assembly and lists every scalar load from a kernel's argument pointer that ends
+    past the kernel's argument segment. The compiler sizes the segment by what the kernel declares and uses (the
+    grid size and its like are there only in kernels that read them), not by loads that the source makes through the
+    pointer itself (attn_device.hpp, touch_args): nothing guarantees memory behind it."""
+    import re
+    lines = [l.split(";")[0].strip() for l in _device_asm(src, extra_flags)]
+    sizes, first = {}, {}  # per kernel: bytes of the segment, first register of the pointer
+    name = ""
+    for text in lines:
+        m = re.match(r"^\.amdhsa_(\w+)\s+(\S+)$", text)
+        if not m:
+            continue
+        key, value = m.groups()
+        if key == "kernel":
+            name = value
+            first[name] = 0
+        elif key == "kernarg_size":
+            sizes[name] = int(value)
+        elif key in ("user_sgpr_dispatch_ptr", "user_sgpr_queue_ptr") and int(value):
+            first[name] += 2  # these come ahead of it in the registers
+    bad, kernel, pointers = [], "", set()
+    for text in lines:
+        m = re.match(r"^([\w$.]+):$", text)
+        if m and not text.startswith("."):
+            kernel = m.group(1)
+            pointers = {first[kernel]} if kernel in first else set()
+            continue
+        if not pointers:
+            continue
+        m = re.match(r"^s_load_dword(?:x(\d+))?\s+[^,]+,\s*s\[(\d+):\d+\],\s*(0x[0-9a-f]+|\d+)$", text)
+        if m and int(m.group(2)) in pointers:
+            end = int(m.group(3), 0) + 4 * int(m.group(1) or 1)
+            if end > sizes[kernel]:
+                bad.append(f"{kernel}: {text} reads to {end} of {sizes[kernel]} bytes of arguments")
+        copy = re.match(r"^s_mov_b64\s+s\[(\d+):\d+\],\s*s\[(\d+):\d+\]$", text)
+        copied = bool(copy) and int(copy.group(2)) in pointers
+        m = re.match(r"^(?:s_(?!cmp|bitcmp|store|waitcnt|cbranch|branch)\w+|v_read\w+)\s+s(?:(\d+)|\[(\d+):(\d+)\])", text)
+        if m:  # what is written over is a pointer no longer
+            lo, hi = (int(m.group(1)),) * 2 if m.group(1) else (int(m.group(2)), int(m.group(3)))
+            pointers -= set(range(lo - 1, hi + 1))
+        if copied:
+            pointers.add(int(copy.group(1)))
+    return bad
+
+
 def wide_mfma_hazards(extra_flags=()) -> list[str]:
     """The same check for the wide-head kernel (attn_wide.hip, attn_wide_kernel): all of its MFMAs
     are assembly statements, its 256 accumulation registers hold O^T for the whole walk, and every
@@ -211,17 +257,17 @@ def build_host(verbose: bool = False) -> str:
 def check_hand_scheduled_kernels(verbose: bool = False):
     """The GEMM's hand-placed MFMAs and its M0 held across loads are safe only as long as the
     compiler puts nothing of its own in between: a toolchain that does fails the build here."""
-    files = [os.path.join(CSRC, f) for f in ("attn_fwd.hip", "attn_wide.hip", "gemm_half.hip")]
+    files = [os.path.join(CSRC, f) for f in ("attn_fwd.hip", "attn_wide.hip", "gemm_half.hip", "qk_prepass.hip")]
     from concurrent.futures import ThreadPoolExecutor
     with ThreadPoolExecutor(max_workers=len(files)) as pool:  # one compilation per file, kept for all checks
         list(pool.map(_device_asm, files))
     bad = m0_writes() + m0_writes(files[1], "attn_wide_kernel") + tied_mfma_hazards() + wide_mfma_hazards()
     for f in files:
-        bad += vmem_sgpr_hazards(f)
+        bad += vmem_sgpr_hazards(f) + kernarg_overreads(f)
     if bad:
         raise RuntimeError("a kernel compiled to code that breaks its hand-written schedule:\n  " + "\n  ".join(bad))
     if verbose:
-        print("hand-scheduled kernels: no foreign M0 write, no accumulator touched inside an MFMA run, no load on a scalar register just written")
+        print("hand-scheduled kernels: no foreign M0 write, no accumulator touched inside an MFMA run, no load on a scalar register just written, no read past a kernel's arguments")
 
 
 def build_all(verbose: bool = False):
