@@ -50,8 +50,8 @@ def test_wide_head_kernel_leaves_m0_alone_and_no_load_reads_a_scalar_register_to
 @pytest.mark.skipif(not (os.path.exists("/opt/rocm/bin/hipcc") or shutil.which("hipcc")), reason="needs hipcc")
 @pytest.mark.parametrize("name", ["attn_fwd.hip", "attn_wide.hip", "gemm_half.hip", "qk_prepass.hip"])
 def test_no_kernel_reads_past_its_arguments(name):
-    # the head of a kernel loads a word of each of its arguments' cache lines through the argument pointer
-    # (attn_device.hpp, touch_args): all of them have to lie within the segment that the kernel is launched with
+    # the head of the pre-pass loads a word of each of its arguments' cache lines through the argument pointer
+    # (qk_prepass.hip, touch_args): all of them have to lie within the segment that the kernel is launched with
     bad = build.kernarg_overreads(os.path.join(build.CSRC, name))
     assert not bad, "\n".join(bad[:20])
 

@@ -165,7 +165,7 @@ def kernarg_overreads(src: str, extra_flags=()) -> list[str]:
     """Compiles `src` to gfx950 assembly and lists every scalar load from a kernel's argument pointer that ends
     past the kernel's argument segment. The compiler sizes the segment by what the kernel declares and uses (the
     grid size and its like are there only in kernels that read them), not by loads that the source makes through the
-    pointer itself (attn_device.hpp, touch_args): nothing guarantees memory behind it."""
+    pointer itself (qk_prepass.hip, touch_args): nothing guarantees memory behind it."""
     import re
     lines = [l.split(";")[0].strip() for l in _device_asm(src, extra_flags)]
     sizes, first = {}, {}  # per kernel: bytes of the segment, first register of the pointer

@@ -22,24 +22,6 @@ typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int D = kHeadDim;
 
-// One word of every cache line of a kernel's BYTES of arguments, in one round trip. (Of the arguments themselves only: what
-// the runtime keeps behind them, the grid size among it, exists in the kernels that read it and in no others.)
-// The compiler loads arguments where they are first used: each line is a miss to memory (the host has just
-// written them) that the next waits for, at the head of every workgroup's chain. Calls, us: 24 heads bf16, 768 tokens, five
-// blocks 135.1 -> 131.8, 4 x 1536, two blocks 300.2 -> 297.5; 2 heads f32 256 tokens 29.8 -> 28.8, 8 heads 100 tokens 28.3 -> 27.0.
-template <size_t BYTES>
-__device__ __forceinline__ void touch_args() {
-    constexpr int N = (int)((BYTES + 63) / 64);
-    static_assert(N >= 1 && N <= 12, "one operand per line below");
-    static_assert(BYTES % 4 == 0 && 64 * (N - 1) + 4 <= BYTES, "the last word lies within the arguments");
-    typedef const __attribute__((address_space(4))) unsigned* args_t;
-    const args_t p = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
-    unsigned x[12];
-#pragma unroll
-    for (int i = 0; i < 12; i++) x[i] = p[16 * (i < N ? i : N - 1)];
-    asm volatile("" ::"s"(x[0]), "s"(x[1]), "s"(x[2]), "s"(x[3]), "s"(x[4]), "s"(x[5]), "s"(x[6]), "s"(x[7]), "s"(x[8]), "s"(x[9]), "s"(x[10]), "s"(x[11]));
-}
-
 // ---------------------------------------------------------------- raw loads
 // Eight consecutive head_dim elements as they come from memory.
 template <typename T> struct Raw8;

@@ -170,7 +170,6 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     unsigned* const bmask = reinterpret_cast<unsigned*>(blocks + MAX_BLOCKS); // bit j: key j of the block is excluded
     __shared__ int s_count[MASKED ? MAX_BLOCKS / 64 : 1]; // admitted blocks of every 64
 
-    touch_args<sizeof(AttnArgs)>();
     unsigned long long clk_c0 = 0, clk_r0 = 0;
     if (a.clock_probe) {
         clk_c0 = __builtin_readcyclecounter();
@@ -1328,7 +1327,6 @@ constexpr int kMaxSplits = 16; // parts per key-split tile
 // pays one memory round trip instead of one per part.
 template <int NZ>
 __global__ void __launch_bounds__(256) attn_merge_kernel(const AttnArgs a, int block_rows) {
-    touch_args<sizeof(AttnArgs)>();
     const int r = (int)blockIdx.x * 8 + (int)(threadIdx.x >> 5); // row among tail_tiles x block_rows
     const int t = r / block_rows;
     const int rr = r - t * block_rows;

@@ -74,7 +74,6 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 // f32 -> bf16 with a scale, 8 elements per thread; blockIdx.y selects the operand.
 __global__ void __launch_bounds__(256) wide_round_kernel(const WidePrepArgs p) {
-    touch_args<sizeof(WidePrepArgs)>();
     const int op = (int)blockIdx.y;
     // the launch that precedes every attention launch also clears its redo flags
     if (op == 0 && blockIdx.x == 0)
@@ -146,7 +145,6 @@ __device__ __forceinline__ void acc_drain() {
 }
 
 __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
-    touch_args<sizeof(WideArgs)>();
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -724,7 +722,6 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_safe_kernel(const WideArgs a)
 // before the first is used, with no branch between them.
 template <int NP>
 __global__ void __launch_bounds__(256) wide_merge_kernel(const WideArgs a) {
-    touch_args<sizeof(WideArgs)>();
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; // (row, dim / 4)
     const int64_t row = i / (WD / 4);
     if (row >= a.tokens) return;

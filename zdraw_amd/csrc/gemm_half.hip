@@ -421,7 +421,6 @@ constexpr int SLOT = BM * BK * 2; // one operand's half of a slab: 32 KB
 constexpr size_t kRingLdsBytes = 5 * (size_t)SLOT; // 160 KB
 template <bool F16, typename TC>
 __global__ void __launch_bounds__(256, 1) gemm_ring_kernel(const GemmArgs g) {
-    touch_args<sizeof(GemmArgs)>();
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -626,7 +625,6 @@ constexpr size_t pipe_lds_bytes(int ti, int tj, int st) { return (size_t)st * (s
 
 template <bool F16, typename TC, int TI, int TJ, int ST, bool RAG>
 __global__ void __launch_bounds__(256, 1) gemm_pipe_kernel(const GemmArgs g) {
-    touch_args<sizeof(GemmArgs)>();
     constexpr int TBM = 32 * TI, TBN = 32 * TJ;
     constexpr int STAGE = (TBM + TBN) * BK * 2; // bytes: A rows then W rows
     constexpr int NM = TI * TJ;                 // MFMAs of a step
@@ -798,7 +796,6 @@ __global__ void __launch_bounds__(256, 1) gemm_pipe_kernel(const GemmArgs g) {
 constexpr int kMaxKSplits = 8;
 template <bool F16, typename TC>
 __global__ void __launch_bounds__(256) gemm_merge_kernel(const GemmArgs g) {
-    touch_args<sizeof(GemmArgs)>();
     constexpr int ES = (int)sizeof(TC);
     constexpr int PITCH = 128 * ES + 16; // bytes per staged row
     __shared__ __attribute__((aligned(16))) unsigned char stage[32 * PITCH];
