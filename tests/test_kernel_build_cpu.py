@@ -64,3 +64,34 @@ def test_the_check_of_reads_past_the_arguments_sees_them(monkeypatch, load, over
     asm = f"kern:\n; %bb.0:\n\t{load}\n\ts_endpgm\n\t.amdhsa_kernel kern\n\t\t.amdhsa_kernarg_size 64\n\t\t.amdhsa_user_sgpr_dispatch_ptr 0\n\t.end_amdhsa_kernel"
     monkeypatch.setattr(build, "_device_asm", lambda *_: asm.split("\n"))
     assert bool(build.kernarg_overreads("")) == over
+
+
+@pytest.mark.skipif(not (os.path.exists("/opt/rocm/bin/hipcc") or shutil.which("hipcc")), reason="needs hipcc")
+@pytest.mark.parametrize("name", ["attn_fwd.hip", "attn_wide.hip", "gemm_half.hip"])
+def test_no_result_of_an_assembly_mfma_is_used_early(name):
+    # attn_wide.hip forms its scores in ordinary registers with assembly MFMAs: what reads them has to
+    # stand as far behind as the compiler would have put it
+    bad = build.early_mfma_result_uses(os.path.join(build.CSRC, name))
+    assert not bad, "\n".join(bad[:20])
+
+
+M = "v_mfma_f32_16x16x32_bf16 v[4:7], v[8:11], v[12:15], "
+
+
+@pytest.mark.parametrize("asm,early", [
+    (["!" + M + "v[4:7]", "s_nop 6", "v_max_f32_e32 v0, v5, v5"], True),
+    (["!" + M + "v[4:7]", "s_nop 7", "v_max_f32_e32 v0, v5, v5"], False),
+    (["!" + M + "v[4:7]", "s_nop 6", "v_mov_b32_e32 v7, 0"], True),  # written over
+    (["!" + M + "v[4:7]", "s_nop 6", "scratch_store_dwordx4 off, v[4:7], off"], True),  # spilled
+    (["!" + M + "0", "v_add_f32_e32 v0, v1, v2", "!" + M + "v[4:7]", "s_nop 6", "v_exp_f32_e32 v0, v4"], True),  # the chain's last counts
+    (["!" + M + "0", "!" + M + "v[4:7]", "s_nop 7", "v_exp_f32_e32 v0, v4"], False),
+    (["!" + M + "0", ".LBB0_1:", "s_nop 7", "v_exp_f32_e32 v0, v4"], True),  # others may come in here
+    ([M + "0", "v_exp_f32_e32 v0, v4"], False),  # the compiler's own
+    (["!" + M.replace("v[4:7]", "a[4:7]") + "a[4:7]", "v_exp_f32_e32 v0, v4"], False),
+])
+def test_the_check_of_early_uses_sees_them(monkeypatch, asm, early):
+    lines = ["kern:"]
+    for a in asm:
+        lines += [";;#ASMSTART", "\t" + a[1:], ";;#ASMEND"] if a.startswith("!") else ["\t" + a]
+    monkeypatch.setattr(build, "_device_asm", lambda *_: lines)
+    assert bool(build.early_mfma_result_uses("")) == early

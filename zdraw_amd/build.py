@@ -207,6 +207,49 @@ def kernarg_overreads(src: str, extra_flags=()) -> list[str]:
     return bad
 
 
+def early_mfma_result_uses(src: str, extra_flags=()) -> list[str]:
+    """Compiles `src` to gfx950 assembly and lists every instruction other than an MFMA that touches an ordinary
+    register which an assembly MFMA (v_mfma_f32_16x16x32) wrote fewer than eight wait states before. Eight is the distance that the
+    compiler keeps behind its own MFMAs of that form (v_mfma, s_nop 7, use); around assembly
+    statements it keeps none. Every instruction counts as one state, MFMAs too, which take longer. A branch or
+    a label within the distance is listed as well: what follows it is not known here."""
+    import re
+    states_needed = 8
+    vgpr = re.compile(r"\bv(?:(\d+)|\[(\d+):(\d+)\])")
+
+    def registers(text):
+        return {r for one, lo, hi in vgpr.findall(text) for r in (range(int(one), int(one) + 1) if one else range(int(lo), int(hi) + 1))}
+
+    bad, kernel, in_asm = [], "", False
+    flying = []  # [registers, wait states since, the MFMA]
+    for line in _device_asm(src, extra_flags):
+        if "#ASMSTART" in line or "#ASMEND" in line:
+            in_asm = "#ASMSTART" in line
+            continue
+        text = line.split(";")[0].strip()
+        if not text or (text.startswith(".") and not text.endswith(":")):
+            continue
+        if text.endswith(":") or re.match(r"^s_(c?branch|setpc|endpgm)", text):
+            if not text.startswith((".", "s_")):
+                kernel = text[:-1]
+            elif not text.startswith("s_endpgm"):
+                bad += [f"{kernel}: {mfma} | {states} wait states | {text}" for _, states, mfma in flying]
+            flying = []
+            continue
+        own = re.match(r"^v_mfma_f32_16x16x32\S*\s+(v\[\d+:\d+\])", text) if in_asm else None
+        if not text.startswith("v_mfma"):
+            bad += [f"{kernel}: {mfma} | {states} wait states | {text}" for regs, states, mfma in flying if regs & registers(text)]
+        if own:
+            flying = [f for f in flying if not f[0] & registers(own.group(1))]  # the chain's next: waits by itself
+        nop = re.match(r"^s_nop\s+(\d+)", text)
+        for f in flying:
+            f[1] += int(nop.group(1)) + 1 if nop else 1
+        flying = [f for f in flying if f[1] < states_needed]
+        if own:
+            flying.append([registers(own.group(1)), 0, text])
+    return bad
+
+
 def wide_mfma_hazards(extra_flags=()) -> list[str]:
     """The same check for the wide-head kernel (attn_wide.hip, attn_wide_kernel): all of its MFMAs
     are assembly statements, its 256 accumulation registers hold O^T for the whole walk, and every
@@ -263,11 +306,11 @@ def check_hand_scheduled_kernels(verbose: bool = False):
         list(pool.map(_device_asm, files))
     bad = m0_writes() + m0_writes(files[1], "attn_wide_kernel") + tied_mfma_hazards() + wide_mfma_hazards()
     for f in files:
-        bad += vmem_sgpr_hazards(f) + kernarg_overreads(f)
+        bad += vmem_sgpr_hazards(f) + kernarg_overreads(f) + early_mfma_result_uses(f)
     if bad:
         raise RuntimeError("a kernel compiled to code that breaks its hand-written schedule:\n  " + "\n  ".join(bad))
     if verbose:
-        print("hand-scheduled kernels: no foreign M0 write, no accumulator touched inside an MFMA run, no load on a scalar register just written, no read past a kernel's arguments")
+        print("hand-scheduled kernels: no foreign M0 write, no accumulator touched inside an MFMA run, no load on a scalar register just written, no read past a kernel's arguments, no MFMA result used early")
 
 
 def build_all(verbose: bool = False):

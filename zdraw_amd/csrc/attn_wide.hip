@@ -284,7 +284,9 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    acc_drain(); // the scores are read next
+    // The scores are read next: they go through the wait, or the compiler, for which they are ready, reads them ahead of it.
+    asm volatile("s_nop 15" : "+v"(sv[0][0]), "+v"(sv[0][1]), "+v"(sv[1][0]), "+v"(sv[1][1]));
+    __builtin_amdgcn_sched_barrier(0);
     // Softmax in the exp2 domain (the scale rides on Q) against ONE reference point per row: the
     // largest score of the range's first block. It never moves, so nothing is ever rescaled
     // (any branch that touches the 256 accumulation registers inside the loop costs hundreds of
