@@ -95,3 +95,31 @@ def test_the_check_of_early_uses_sees_them(monkeypatch, asm, early):
         lines += [";;#ASMSTART", "\t" + a[1:], ";;#ASMEND"] if a.startswith("!") else ["\t" + a]
     monkeypatch.setattr(build, "_device_asm", lambda *_: lines)
     assert bool(build.early_mfma_result_uses("")) == early
+
+
+@pytest.mark.skipif(not (os.path.exists("/opt/rocm/bin/hipcc") or shutil.which("hipcc")), reason="needs hipcc")
+def test_no_load_of_the_attention_kernel_reads_a_scalar_register_too_early():
+    bad = build.vmem_sgpr_hazards(os.path.join(build.CSRC, "attn_fwd.hip"))
+    assert not bad, "\n".join(bad[:20])
+
+
+LOAD = "buffer_load_dwordx4 v4, s[8:11], s5 offen lds"
+
+
+@pytest.mark.parametrize("asm,early", [
+    (["v_readfirstlane_b32 s5, v1", LOAD], True),
+    (["v_readfirstlane_b32 s5, v1", "s_cmp_lg_u32 s5, 0", LOAD], True),  # only reads it
+    (["v_readfirstlane_b32 s5, v1", "s_bitcmp1_b32 s5, 0", LOAD], True),
+    (["v_readfirstlane_b32 s5, v1", "s_nop 3", LOAD], True),
+    (["v_readfirstlane_b32 s5, v1", "s_nop 4", LOAD], False),
+    (["v_readfirstlane_b32 s5, v1", "s_cmp_lg_u32 s5, 0", "s_nop 3", LOAD], False),
+    (["v_readfirstlane_b32 s5, v1", "s_mov_b32 s5, s6", LOAD], False),  # written over
+    (["v_readfirstlane_b32 s5, v1", "s_mov_b64 s[4:5], s[6:7]", LOAD], False),
+    (["v_readfirstlane_b32 s5, v1", "s_add_u32 s6, s5, 4", LOAD], True),
+    (["v_readlane_b32 s10, v255, 3", LOAD], True),  # the descriptor
+    (["v_cmp_gt_i32_e64 s[4:5], s6, v0", LOAD], True),
+    (["v_readfirstlane_b32 s6, v1", LOAD], False),
+])
+def test_the_check_of_scalar_registers_sees_early_reads(monkeypatch, asm, early):
+    monkeypatch.setattr(build, "_device_asm", lambda *_: ["kern:"] + asm)
+    assert bool(build.vmem_sgpr_hazards("")) == early

@@ -130,32 +130,34 @@ def tied_mfma_hazards(src: str = os.path.join(CSRC, "gemm_half.hip"), extra_flag
 
 def vmem_sgpr_hazards(src: str, extra_flags=()) -> list[str]:
     """Compiles `src` to gfx950 assembly and lists every memory instruction that reads a scalar register
-    which a vector instruction (v_readlane, v_readfirstlane) wrote fewer than five wait states before. The
+    which a vector instruction (v_readlane, v_readfirstlane, a compare into a register) wrote fewer than five wait states before. The
     hardware does not wait for such a write; the compiler keeps the distance for its own loads, not for the
     direct-to-LDS loads, which are assembly statements: with a stale descriptor or offset they would reach
     anywhere. Scalar registers restored from a spill ahead of such a load are the usual way to get there."""
     import re
     lines = [l.split(";")[0].strip() for l in _device_asm(src, extra_flags)]
     lines = [l for l in lines if l and (not l.startswith(".") or l.endswith(":"))]
-    write = re.compile(r"^v_read(?:first)?lane_b32(?:_e32|_e64)?\s+s(\d+)\b")
+    scalars = re.compile(r"\bs(?:(\d+)|\[(\d+):(\d+)\])")
+
+    def registers(text):
+        return {r for one, lo, hi in scalars.findall(text) for r in (range(int(one), int(one) + 1) if one else range(int(lo), int(hi) + 1))}
+
     bad, kernel = [], ""
     for i, text in enumerate(lines):
         if text.endswith(":") and not text.startswith("."):
             kernel = text[:-1]
-        m = write.match(text)
-        if not m:
+        if not re.match(r"^v_\w+\s+s[\d\[]", text):
             continue
-        reg, states = int(m.group(1)), 0
+        written, states = registers(text.split(",")[0]), 0
         for later in lines[i + 1:i + 12]:
-            if states >= 5 or re.match(rf"^s_\S+\s+s{reg}\b", later):
-                break  # far enough, or written again by the scalar unit
-            if re.match(r"^(buffer|global|flat|scratch)_", later):
-                read = {int(x) for x in re.findall(r"\bs(\d+)\b", later)}
-                for lo, hi in re.findall(r"\bs\[(\d+):(\d+)\]", later):
-                    read |= set(range(int(lo), int(hi) + 1))
-                if reg in read:
-                    bad.append(f"{kernel}: {text} | {states} wait states | {later}")
-                    break
+            # far enough, or written again by the scalar unit (compares and bit tests only read their first operand)
+            if re.match(r"^s_(?!cmp|bitcmp)\w+\s+s[\d\[]", later):
+                written -= registers(later.split(",")[0])
+            if states >= 5 or not written:
+                break
+            if re.match(r"^(buffer|global|flat|scratch)_", later) and written & registers(later):
+                bad.append(f"{kernel}: {text} | {states} wait states | {later}")
+                break
             nop = re.match(r"^s_nop\s+(\d+)", later)
             states += int(nop.group(1)) + 1 if nop else 0 if later.endswith(":") else 1
     return bad
