@@ -187,8 +187,9 @@ void zdraw_hip_release_weight_buffer(void* buffer);
 /* No reference counterpart: unified memory needs no copy, and uploads into fresh device memory cost a small
  * blocking call more than its kernels. Room for four operands in host memory: handles[i] is a buffer of
  * bytes[i] over the pinned host memory at memory[i], which the caller fills and the kernels read and write where
- * it is. It belongs to the queue, for one caller at a time, until _end; the work on it must be over by
- * then. ZDRAW_HIP_UNAVAILABLE (use buffers of your own) when another caller has it, for more than 16 MB,
+ * it is. It belongs to the queue, for one caller at a time, until that caller's thread calls _end (which waits for the
+ * queue); _end follows a begin that returned ZDRAW_HIP_OK and no other, and on a thread that does not hold the memory
+ * it does nothing. ZDRAW_HIP_UNAVAILABLE (use buffers of your own) when another caller has it, for more than 16 MB,
  * under capture, or where no such memory is left. */
 int zdraw_hip_host_operands_begin(void* queue, const size_t bytes[4], void* handles[4], uint8_t* memory[4]);
 void zdraw_hip_host_operands_end(void* queue);

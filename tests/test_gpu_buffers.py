@@ -8,6 +8,7 @@ that is not device memory, and whose contents the library must never cache.
 """
 import ctypes as C
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -307,3 +308,39 @@ def test_host_operands_belong_to_one_call_at_a_time(ctx):
     assert np.array_equal(ctx.run(q, k, v, cfg), want)
     assert C.string_at(memory[0], 4) == b"\x7b" * 4
     L.zdraw_hip_host_operands_end(ctx.queue)
+
+
+# A caller whose begin was refused and that ends all the same must not free what another holds: the third begin would
+# hand the same memory out under the first caller's kernels. Nor does an end without any begin.
+def test_host_operands_are_ended_by_their_holder_alone(ctx):
+    L = hip.lib()
+    queue = L.zdraw_hip_create_queue(ctx.device)
+    handles, memory = (C.c_void_p * 4)(), (C.c_void_p * 4)()
+
+    def begin(n, h, m):
+        return L.zdraw_hip_host_operands_begin(queue, (C.c_size_t * 4)(n, n, n, n), h, m)
+
+    def elsewhere(f):
+        box = []
+        t = threading.Thread(target=lambda: box.append(f()))
+        t.start()
+        t.join()
+        return box[0]
+
+    def refused():
+        rc = begin(4096, (C.c_void_p * 4)(), (C.c_void_p * 4)())
+        L.zdraw_hip_host_operands_end(queue)
+        return rc
+
+    L.zdraw_hip_host_operands_end(queue)
+    assert begin(512, handles, memory) == hip.OK
+    C.memset(memory[0], 0x5A, 512)
+    for _ in range(2):
+        assert elsewhere(refused) == hip.UNAVAILABLE
+    assert [L.zdraw_hip_buffer_length(h) for h in handles] == [512] * 4
+    assert C.string_at(memory[0], 512) == b"\x5a" * 512
+    L.zdraw_hip_host_operands_end(queue)
+    assert elsewhere(refused) == hip.OK  # free again, and ended by the thread that took it
+    assert begin(512, handles, memory) == hip.OK
+    L.zdraw_hip_host_operands_end(queue)
+    L.zdraw_hip_release_queue(queue)

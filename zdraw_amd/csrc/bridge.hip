@@ -21,6 +21,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <thread>
 #include <vector>
 
 using namespace zdraw;
@@ -62,7 +63,7 @@ struct Buffer {
 // Operands in host memory on their way through a blocking call: pinned memory that the kernels read and write in
 // place, kept by the queue from one call to the next, for one call at a time.
 struct HostOperands {
-    std::atomic<bool> busy{false};
+    std::atomic<std::thread::id> owner{}; // whose begin was answered with it (no thread: free)
     char* base = nullptr;
     size_t len = 0;
     Buffer buf[4] = {};
@@ -1347,7 +1348,9 @@ int zdraw_hip_host_operands_begin(void* queue, const size_t bytes[4], void* hand
     }
     if (total > kHostOperandBytes || capturing(q)) return ZDRAW_HIP_UNAVAILABLE;
     HostOperands& h = q->host;
-    if (h.busy.exchange(true, std::memory_order_acquire)) return ZDRAW_HIP_UNAVAILABLE;
+    std::thread::id nobody;
+    if (!h.owner.compare_exchange_strong(nobody, std::this_thread::get_id(), std::memory_order_acquire, std::memory_order_relaxed))
+        return ZDRAW_HIP_UNAVAILABLE;
     if (h.len < total) {
         // (in powers of two from 1 MB on: a range of sizes settles after few allocations)
         size_t want = size_t{1} << 20;
@@ -1355,7 +1358,7 @@ int zdraw_hip_host_operands_begin(void* queue, const size_t bytes[4], void* hand
         void* p = nullptr;
         if (hipStreamSynchronize(q->stream) != hipSuccess || hipHostMalloc(&p, want, hipHostMallocCoherent) != hipSuccess) {
             (void)hipGetLastError(); // or the next launch would report it
-            h.busy.store(false, std::memory_order_release);
+            h.owner.store(std::thread::id(), std::memory_order_release);
             return ZDRAW_HIP_UNAVAILABLE;
         }
         if (h.base) (void)hipHostFree(h.base);
@@ -1372,9 +1375,10 @@ int zdraw_hip_host_operands_begin(void* queue, const size_t bytes[4], void* hand
 
 void zdraw_hip_host_operands_end(void* queue) {
     Queue* q = static_cast<Queue*>(queue);
-    if (!q) return;
+    // (a caller whose begin was refused has nothing to end: the memory is another's, whose kernels may be running on it)
+    if (!q || q->host.owner.load(std::memory_order_relaxed) != std::this_thread::get_id()) return;
     (void)hipStreamSynchronize(q->stream); // a call that failed half way may have left work behind (idle: 0.2 us)
-    q->host.busy.store(false, std::memory_order_release);
+    q->host.owner.store(std::thread::id(), std::memory_order_release);
 }
 
 // ---------------------------------------------------------------- pipelines
