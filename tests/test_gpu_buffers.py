@@ -344,3 +344,35 @@ def test_host_operands_are_ended_by_their_holder_alone(ctx):
     assert begin(512, handles, memory) == hip.OK
     L.zdraw_hip_host_operands_end(queue)
     L.zdraw_hip_release_queue(queue)
+
+
+# Two contexts, a thread each, at once: every call finds its own queue's memory, which grows under it.
+def test_host_operands_of_two_queues_on_two_threads(ctx):
+    shapes = [(100, 1), (159, 3), (300, 2), (700, 3), (1024, 8), (64, 2)]
+    rng = np.random.default_rng(9)
+    work = []
+    for tokens, heads in shapes:
+        q, k, v = (rng.standard_normal((tokens, heads, 128), dtype=np.float32) for _ in range(3))
+        cfg = host.Config(tokens, heads, heads, 128, False, 0)
+        work.append((q, k, v, cfg, ctx.run_pooled(q, k, v, cfg)))
+    failures = []
+
+    def program(order):
+        c = host.Context.init()
+        try:
+            for i in order:
+                q, k, v, cfg, want = work[i]
+                if not np.array_equal(c.run(q, k, v, cfg).view(np.uint32), want.view(np.uint32)):
+                    failures.append(i)
+        except Exception as e:  # noqa: BLE001 (reported below, on the test's thread)
+            failures.append(e)
+        finally:
+            c.deinit()
+
+    n = len(work)
+    threads = [threading.Thread(target=program, args=(order,)) for order in (list(range(n)) * 3, list(reversed(range(n))) * 3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures

@@ -56,6 +56,31 @@ def test_wide_head_odd_numbers_of_blocks_on_every_row(ctx, tokens):
     refimpl.check_close(got, want, f"wide head, {tokens} tokens")
 
 
+# Rows whose scores against the first block of a key range are infinite or no numbers: the reference point is
+# taken from that block and starts every score behind it, so nothing of such a row may be used as it stands (its tile is formed
+# again with a running maximum). -inf: those keys weigh nothing. +inf, NaN: the row is NaN, as in the
+# oracle. The rows between them, and the tiles beside theirs, are ordinary. One range; two of nine blocks.
+@pytest.mark.parametrize("tokens", [256, 576])
+@pytest.mark.parametrize("kind", ["-inf", "+inf", "nan"])
+def test_wide_head_first_block_without_a_finite_maximum(ctx, tokens, kind):
+    rng = np.random.default_rng(70 + tokens)
+    q, k, v = draw(rng, tokens)
+    odd = np.zeros(tokens, bool)
+    odd[1:128:2] = True  # rows of the first tile
+    q[~odd, :, 0] = 0.0
+    k[:, :, 0] = 0.0
+    q[odd, :, 0] = np.float32("nan") if kind == "nan" else np.float32(2.0 ** 100)
+    for first in {0, 32 * (tokens // 64)} if kind != "nan" else ():
+        k[first:first + 32, :, 0] = np.float32(2.0 ** 60) * (1 if kind == "+inf" else -1)  # products of 2^160
+    got = ctx.run(q, k, v, host.Config(tokens, 1, 1, 512)).reshape(tokens, 1, 512)
+    want = zo.attention_run(q, k, v, zo.Config(tokens, 1, 1, 512))
+    refimpl.check_close(got[~odd], want[~odd], f"wide head, rows beside those with {kind}")
+    if kind == "-inf":
+        refimpl.check_close(got[odd], want[odd], "wide head, first blocks at -inf")
+    else:
+        assert np.isnan(want[odd]).all() and np.isnan(got[odd]).all()
+
+
 # Numbers of key blocks that the number of ranges does not divide (the last range is shorter),
 # half a query tile left over, three to seven ranges, and both sides of the length
 # where two ranges a tile outgrow one round; rows of the first, a middle and the last tile.
