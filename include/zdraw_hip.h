@@ -116,7 +116,11 @@ typedef struct ZdrawHipAttnExt {
      * Accuracy: Q' and K' are rounded to 16 bits before the product, so a score of s
      * nats carries an absolute error of about s * 2^-8 (bf16 operands) or s * 2^-11
      * (ZDRAW_HIP_F16 staging, see `staging`); scores reach sqrt(head_dim) * max|w_q| *
-     * max|w_k| = 11.3 nats with unit weights and grow with the product of the weights. */
+     * max|w_k| = 11.3 nats with unit weights and grow with the product of the weights.
+     * Range of V: the sums are kept in f32 against a reference point that a score may exceed. The
+     * running-maximum form lets a probability grow to 2^12 (a score of 8, log2, above the reference always fits, one more
+     * than 12 above moves it), the form without one to e^bound (2^63.5 at 44), the one-head kernel of width 512
+     * to 2^90: values beyond f32's largest divided by that and by the number of keys may overflow. */
     float score_bound;
     /* Element type in which the prepared Q and K are staged for the score product: 0 (or
      * ZDRAW_HIP_BF16) = bf16, ZDRAW_HIP_F16 = IEEE half, the staging type of the reference's

@@ -115,8 +115,9 @@ __device__ __forceinline__ void mfma_acc(f32x4& c, const bf16x8& x, const bf16x8
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(x), "v"(y));
 }
 // The same for the scores, in ordinary registers (the accumulation file is full): `FIRST` starts
-// the chain from zero. A tile's MFMAs are four apart; the scores are first read
-// by other instructions eight product MFMAs after the chain's last.
+// the chain from zero. A tile's MFMAs are four apart; in the key loop the scores are first read by other
+// instructions behind the third product MFMA after the chains' last, ahead of it through a wait whose operands they are. The
+// hardware needs eight wait states there, and zdraw_amd.build.early_mfma_result_uses holds the compiled code to them.
 template <bool FIRST>
 __device__ __forceinline__ void mfma_score(f32x4& c, const bf16x8& x, const bf16x8& y) {
     if constexpr (FIRST) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(x), "v"(y));
@@ -345,8 +346,8 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
     // offsets formed per load and the reference point subtracted from every score). Timing builds without
     // the loads -280, without the exchange of P -200, without K's or V's fragment reads -120 each, all of
     // them 2254. Fragments read further ahead change nothing; slots of half a K block, which spread the
-    // loads over both phases, cost more in addresses than they gave (3130). At 16384 tokens the clock is at
-    // 1.95-2.0 GHz with all CUs busy (1.59 GHz for the 32 x 32 x 16 form).
+    // loads over both phases, cost more in addresses than they gave (3130). At 16384 tokens the clock is
+    // 1.86 GHz (1.59 GHz for the 32 x 32 x 16 form).
     auto step = [&](auto ks_c, int b, const u32x4 (&pc)[2], u32x4 (&pn)[2]) __attribute__((always_inline)) {
         constexpr int KS = decltype(ks_c)::value;       // slot of K(b+1); K(b+2) is in the other
         constexpr int VS = KS ^ 1;                      // slot of V(b); V(b+1) goes to the other
