@@ -1195,7 +1195,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                 const f32x4 v = *(lds_turn_t)(turn + (unsigned)(i * 1024 + lane * 16));
                 if (r < rows) {
                     const int d = (l32 ^ (r & 15)) * 4;
-                    *reinterpret_cast<f32x4*>(base + r * stride + d) = v;
+                    store_through(base + r * stride + d, v);
                     if (row16) *reinterpret_cast<u32x2*>(row16 + (int64_t)r * (a.heads * D) + d) = round4(v, a.o16_dtype);
                 }
             }
@@ -1231,7 +1231,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                 const u32x4 row16 = *(lds_u32x4_t)(o_lds + (unsigned)(r * (D * 2) + (lane & 15) * 16));
                 const int orow = q0 + r;
                 if (orow < a.tokens)
-                    *reinterpret_cast<u32x4*>(obase + (int64_t)orow * a.o_ts + (((lane & 15) ^ (r & 15)) * 8)) = row16;
+                    store_through(obase + (int64_t)orow * a.o_ts + (((lane & 15) ^ (r & 15)) * 8), row16);
             }
         }
     } else {
@@ -1303,7 +1303,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                     const u32x4 row16 = *(lds_u32x4_t)(o_lds + (unsigned)(r * (D * 2) + (lane & 15) * 16));
                     const int orow = q0 + 32 * qi + r;
                     if (orow < a.tokens)
-                        *reinterpret_cast<u32x4*>(obase + (int64_t)orow * a.o_ts + (((lane & 15) ^ (r & 15)) * 8)) = row16;
+                        store_through(obase + (int64_t)orow * a.o_ts + (((lane & 15) ^ (r & 15)) * 8), row16);
                 }
             }
         }
@@ -1367,14 +1367,14 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const AttnArgs a, int b
     acc *= inv;
     const int64_t off = (int64_t)seg * a.o_bs + (int64_t)qrow * a.o_ts + (int64_t)head * a.o_hs + d0;
     if (a.out_dtype == kF32) {
-        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.o) + off) = acc;
+        store_through(reinterpret_cast<float*>(a.o) + off, acc);
         if (a.o16)
             *reinterpret_cast<u32x2*>(static_cast<unsigned short*>(a.o16) + (((int64_t)seg * a.tokens + qrow) * a.heads + head) * D + d0) = round4(acc, a.o16_dtype);
     } else if (a.out_dtype == kF16) {
         typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-        *reinterpret_cast<f16x4*>(reinterpret_cast<_Float16*>(a.o) + off) = __builtin_convertvector(acc, f16x4);
+        store_through(reinterpret_cast<_Float16*>(a.o) + off, __builtin_convertvector(acc, f16x4));
     } else {
-        *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16_t*>(a.o) + off) = __builtin_convertvector(acc, bf16x4);
+        store_through(reinterpret_cast<bf16_t*>(a.o) + off, __builtin_convertvector(acc, bf16x4));
     }
 }
 

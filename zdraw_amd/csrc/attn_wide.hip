@@ -465,7 +465,7 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
         float* op = (nsp > 1 ? a.part_o + ((int64_t)part * a.tokens + row0) * WD : a.o + (int64_t)row0 * WD) + 256 * dh;
 #pragma unroll
         for (int r = 0; r < 16; r++)
-            *reinterpret_cast<f32x4*>(op + (int64_t)r * WD + ((el ^ r) * 4)) = *(lds_f32x4_t)(turn + r * 1024 + el * 16);
+            store_through(op + (int64_t)r * WD + ((el ^ r) * 4), (f32x4)*(lds_f32x4_t)(turn + r * 1024 + el * 16));
         if (nsp > 1 && o < 2 && eg == 0) *reinterpret_cast<f32x2*>(a.part_ml + ((int64_t)part * a.tokens + row0 + ec) * 2) = ml;
     }
 }
@@ -747,7 +747,7 @@ __global__ void __launch_bounds__(256) wide_merge_kernel(const WideArgs a) {
         lt += ml[p][1] * w;
     }
     const float inv = lt > 0.f ? 1.0f / lt : 0.f;
-    *reinterpret_cast<f32x4*>(a.o + row * WD + 4 * c4) = acc * inv;
+    store_through(a.o + row * WD + 4 * c4, acc * inv);
 }
 
 } // namespace wide

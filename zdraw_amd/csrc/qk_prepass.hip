@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(kPrepTokens * 64) qk_prepass_kernel(const Prep
                     *reinterpret_cast<f32x4*>(dst) = f32x4{x[0], x[1], x[2], x[3]};
                     *reinterpret_cast<f32x4*>(dst + 4) = f32x4{x[4], x[5], x[6], x[7]};
                 } else {
-                    *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(p.y) + off) = p.out_dtype == kF16 ? pack_f16x8(x) : pack_bf16x8(x);
+                    store_through(reinterpret_cast<bf16_t*>(p.y) + off, p.out_dtype == kF16 ? pack_f16x8(x) : pack_bf16x8(x));
                 }
             }
         }
@@ -164,7 +164,7 @@ __global__ void __launch_bounds__(kPrepTokens * 64) qk_prepass_kernel(const Prep
                 *reinterpret_cast<f32x4*>(dst) = f32x4{x[0], x[1], x[2], x[3]};
                 *reinterpret_cast<f32x4*>(dst + 4) = f32x4{x[4], x[5], x[6], x[7]};
             } else {
-                *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(p.y) + off) = p.out_dtype == kF16 ? pack_f16x8(x) : pack_bf16x8(x);
+                store_through(reinterpret_cast<bf16_t*>(p.y) + off, p.out_dtype == kF16 ? pack_f16x8(x) : pack_bf16x8(x));
             }
         }
     }
