@@ -624,8 +624,8 @@ __global__ void __launch_bounds__(256, 1) gemm_ring_kernel(const GemmArgs g) {
 //     after the last of those reads the slab's one barrier (this wave's part of slab s + 1 has
 //     landed, everybody has slab s in registers: its stage is free);
 //   second step: the MFMAs on f1, the k 0..31 fragments of slab s + 1 are read into f0;
-//   from the barrier on, one load of slab s + ST per four MFMAs (the pace of the CU's address
-//     unit); what is left of them goes out in the next slab's first step, ahead of its barrier.
+//   from the barrier on, one load of slab s + ST per five MFMAs (fewer where a slab has fewer to a load);
+//     what is left of them goes out in the next slab's first step, ahead of its barrier.
 constexpr int vm_lgkm0(int vm) { return (vm & 15) | 0x70 | ((vm >> 4) << 14); }           // vmcnt(vm) lgkmcnt(0)
 constexpr int vm_only(int vm) { return (vm & 15) | 0xF70 | ((vm >> 4) << 14); }           // vmcnt(vm)
 constexpr size_t pipe_lds_bytes(int ti, int tj, int st) { return (size_t)st * (size_t)(ti + tj) * 32 * BK * 2; }
@@ -639,7 +639,11 @@ __global__ void __launch_bounds__(256, 1) gemm_pipe_kernel(const GemmArgs g) {
     constexpr int NL = TI + TJ;                 // loads of a wave per slab
     constexpr int RS = NM >= 32 ? 2 : 1;        // MFMAs per fragment read
     constexpr int TB = (NR - 1) * RS + 5 < NM - 1 ? (NR - 1) * RS + 5 : NM - 1; // the barrier follows this MFMA of the first step
-    constexpr int LS = 2 * NM / NL < 4 ? 2 * NM / NL : 4; // MFMAs per load
+    // MFMAs per load: five where a slab has that many (the three largest tiles), so that the loads spread over all of it;
+    // closer, they hold the waves at the memory queue. Launches, us, at 2, 3, 4, 5 and 6: 1024 x 3072 x 9216 65.0, 61.3, 57.1,
+    // 54.1-55.5, 54.4; 1632 x 3840 x 11520 140, 133, 132, 130, 130; 1632 x 3840 x 3840 60.8, 58.2, 56.4, 55.9, 56.0. Four against
+    // five over twelve products of 900 to 3000 rows: 0 to 4 % (3000 x 10272 x 2568 164.4 -> 158.4), none slower.
+    constexpr int LS = 2 * NM / NL < 5 ? 2 * NM / NL : 5;
     // load i goes out ahead of MFMA TB + 1 + LS i, counted from the start of the slab that frees its stage
     constexpr int IW = (2 * NM - (TB + 1) + LS - 1) / LS < NL ? (2 * NM - (TB + 1) + LS - 1) / LS : NL; // loads that go out within that slab
     static_assert(LS >= 1 && TB + 1 + LS * (NL - 1) <= 2 * NM + TB, "all loads of a slab are out by the next barrier");
