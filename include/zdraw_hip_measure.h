@@ -63,7 +63,7 @@ void zdraw_hip_wide_ranges(uint32_t tokens, uint32_t cus, uint32_t* ranges, uint
 void zdraw_hip_set_scratch_limit(size_t bytes);
 
 /* How many query tiles (128 rows) of the last wide-head launch had a score outgrow its row's
- * fixed reference point and were formed again by the running-maximum kernel (waits for that
+ * fixed reference point and were formed again with a running maximum (waits for that
  * launch). 0 on ordinary data; -1 if no wide-head launch has been made or the read failed. */
 int zdraw_hip_wide_redo_tiles(void);
 

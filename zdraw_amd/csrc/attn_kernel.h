@@ -139,7 +139,7 @@ struct WideArgs {
     float* part_o;  // f32 [splits][tokens][512]: unnormalised O of each key range
     float* part_ml; // f32 [splits][tokens][2]: its reference point and row sum
     int* redo;      // [wide_tiles(tokens)]: set by the kernel for a query tile (128 rows) whose scores outgrew the
-                    // fixed reference point; such tiles are formed again by the running-maximum kernel that follows
+                    // fixed reference point; the workgroup then forms its rows again with a running maximum
 };
 // f32 -> bf16 rounding of the three operands (Q with its scale) in one launch.
 struct WidePrepArgs {

@@ -61,8 +61,8 @@ constexpr int V_RING = NSK * K_SLOT;
 constexpr int P_RING = V_RING + NSV * V_SLOT;  // two slots of the exponentiated blocks
 constexpr int P_SLOT = NW * 2 * 1024;          // 2 KB a wave
 constexpr size_t kLdsBytes = (size_t)P_RING + 2 * P_SLOT + 16384; // 160 KB: the last 16 KB hold query rows only
-constexpr float kTau = 8.0f;      // log2 headroom of the lazy softmax maximum (attn_wide_safe_kernel)
-constexpr float kRowSumLimit = 0x1p90f; // a row sum past this flags its tile: a P beyond 2^90 may be on its way to overflow
+constexpr float kTau = 8.0f;      // log2 headroom of the lazy softmax maximum (safe::form_again)
+constexpr float kRowSumLimit = 0x1p90f; // a row sum past this has its tile's range formed again: a P beyond 2^90 may be on its way to overflow
 constexpr int RA = 6;             // K fragments read ahead of their MFMA
 constexpr int VA = 3;             // V fragment pairs read ahead
 constexpr int kMaxSplits = 8;     // key ranges per query tile
@@ -144,6 +144,253 @@ __device__ __forceinline__ void mfma_zero(f32x4& c, const bf16x8& z) {
 __device__ __forceinline__ void acc_drain() {
     asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
 }
+
+// ---------------------------------------------------------------------------------------------
+// The rows of a workgroup of attn_wide_kernel one of whose scores lies some 90 (log2) above its row's first block,
+// over the same key range, formed again with a lazy running maximum: one half of the 512 output dims at a time (the scores
+// of the range are formed for each), so that O^T takes 128 accumulation registers per wave and the compiler has
+// room to rescale it in place when a reference point moves. K blocks (32 KB) and V half-blocks (16 KB) cycle through three
+// LDS slots each. It runs behind the kernel's own epilogue, by the workgroup that found the row sum, where nothing of the
+// fast path is live any more: a kernel of its own behind every call, which this was, costs ordinary data its launch.
+// Calls, us, as a launch of its own -> here: 256 tokens 38.5 -> 37.2, 1024 43.7 -> 42.4, 2560 59.0 -> 57.7, 6208 111.3 -> 109.9,
+// 16384 438.1 -> 435.6. With every row formed again: 256 60 -> 77 (one workgroup takes both halves), 1024 88 -> 83, 6208
+// 330 -> 252, 16384 1224 -> 1134 (a launch of its own went over all keys, this over the range that needs it).
+namespace safe {
+constexpr int HALF = WD / 2;      // output dims per workgroup
+constexpr int V_SLOT = (NSL / 2) * TILE_BYTES; // half the dims of a V block: 16 KB
+constexpr int NS = 3;                          // slots per ring
+constexpr int V_RING = NS * K_SLOT;
+static_assert((size_t)NS * (K_SLOT + V_SLOT) <= wide::kLdsBytes, "144 of the kernel's 160 KB");
+
+// Output dims HALF dh .. of query tile `tile` over key blocks blk0 .. blk0 + nblk - 1, written as key range `part` of nsp
+// (nsp 1: the result). Every wave of the workgroup calls it, behind a barrier that ends all use of the LDS.
+__device__ __forceinline__ void form_again(const WideArgs& a, unsigned char* smem, int wave, int tile, int part, int nsp, int blk0, int nblk, int dh) {
+    int lane; // (formed here: kept from the kernel's start it would cost the key loop a register)
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+    const int l32 = lane & 31;
+    const int h = lane >> 5;
+    blk0 = __builtin_amdgcn_readfirstlane(blk0); // (uniform, and formed on the scalar unit from here on)
+    nblk = __builtin_amdgcn_readfirstlane(nblk);
+    const int q0 = tile * BQ + 32 * wave; // this wave's query rows
+
+    const unsigned lds0 = lds_address(smem);
+
+    // ---- Q fragments (B operand of S^T = K Q^T): query q0 + l32, dims 16 kk + 8 h .. +7
+    bf16x8 qf[32];
+    {
+        // rows past the end read the last row and are never stored
+        const bf16_t* qp = reinterpret_cast<const bf16_t*>(a.q) + (int64_t)min(q0 + l32, a.tokens - 1) * WD + 8 * h;
+#pragma unroll
+        for (int kk = 0; kk < 32; kk++) qf[kk] = *reinterpret_cast<const bf16x8*>(qp + 16 * kk);
+    }
+
+    // ---- block fetch. K: wave w fills tile w (dims 128 w .. +127) of the block, four rows per
+    // instruction. V: wave w fills rows 16 (w >> 1) .. +15 of tile (w & 1) of this workgroup's
+    // half. The lane that fills chunk position p of row r fetches the chunk the swizzle places
+    // there: K chunk c of row r sits at c ^ (r & 15), V chunk c at c ^ ((r & 3) << 2).
+    const unsigned span = (unsigned)a.tokens * (unsigned)(WD * 2);
+    const u32x4 k_rsrc = make_rsrc_words(a.k, span);
+    const u32x4 v_rsrc = make_rsrc_words(a.v, span);
+    unsigned fk_off[4], fv_off[4]; // K rows 4 j + 16 take the same chunks 16 rows further on
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int row = 4 * j + (lane >> 4);
+        const unsigned kc = (unsigned)((lane & 15) ^ (row & 15));
+        fk_off[j] = (unsigned)row * (WD * 2) + (unsigned)wave * (SL * 2) + kc * 16u;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int row = 16 * (wave >> 1) + 4 * j + (lane >> 4);
+        const unsigned vc = (unsigned)((lane & 15) ^ ((row & 3) << 2));
+        fv_off[j] = (unsigned)row * (WD * 2) + (unsigned)(2 * dh + (wave & 1)) * (SL * 2) + vc * 16u;
+    }
+    const unsigned fetch_k_lds = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)wave * TILE_BYTES);
+    const unsigned fetch_v_lds = __builtin_amdgcn_readfirstlane(lds0 + V_RING + (unsigned)(wave & 1) * TILE_BYTES + (unsigned)(16 * (wave >> 1)) * (SL * 2));
+    // the i-th (i < 12) load of the group that brings K block kb into K slot ks and V block vb into V slot vs
+    auto fetch_one = [&](int kb, int ks, int vb, int vs, int i) __attribute__((always_inline)) {
+        if (i < 8) {
+            const unsigned uo = (unsigned)(blk0 + (kb < nblk ? kb : nblk - 1)) * (unsigned)(KB * WD * 2) + (unsigned)(i >> 2) * (16 * WD * 2);
+            load_to_lds_16(k_rsrc, fetch_k_lds + (unsigned)ks * K_SLOT + (unsigned)(4 * i) * (SL * 2), fk_off[i & 3], uo);
+        } else {
+            const unsigned uo = (unsigned)(blk0 + (vb < nblk ? vb : nblk - 1)) * (unsigned)(KB * WD * 2);
+            load_to_lds_16(v_rsrc, fetch_v_lds + (unsigned)vs * V_SLOT + (unsigned)(4 * (i - 8)) * (SL * 2), fv_off[i - 8], uo);
+        }
+    };
+
+    // ---- fragment addresses in slot 0 (a tile and a slot add constants)
+    const int tr_row = (lane & 15) >> 2;
+    const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    // (pointers, so that the constant parts of an address go into the instruction's offset field)
+    typedef __attribute__((address_space(3))) unsigned char* lds_byte_t;
+    typedef const __attribute__((address_space(3))) bf16x8* lds_bf16x8_t;
+    typedef __attribute__((address_space(3))) s16x4* lds_s16x4_t;
+    const lds_byte_t lds_base = (lds_byte_t)smem;
+    lds_byte_t kfo[8], vfo[4];
+#pragma unroll
+    for (int kk = 0; kk < 8; kk++) kfo[kk] = lds_base + ((l32 * SL + (((2 * kk + h) ^ (l32 & 15)) * 8)) * 2);
+#pragma unroll
+    for (int blk = 0; blk < 4; blk++)
+        vfo[blk] = lds_base + V_RING + (((4 * h + tr_row) * SL + ((blk ^ tr_row) * 32) + tr_col) * 2);
+    auto k_read = [&](int slot, int kk) __attribute__((always_inline)) {
+        return *(lds_bf16x8_t)(kfo[kk & 7] + (slot * K_SLOT + (kk >> 3) * TILE_BYTES));
+    };
+
+    f32x16 oacc[8]; // O^T: lane = query l32, dims 256 dh + 32 blk + 8 i + 4 h + j
+#pragma unroll
+    for (int blk = 0; blk < 8; blk++)
+#pragma unroll
+        for (int j = 0; j < 16; j++) oacc[blk][j] = 0.f;
+    float m_run = -INFINITY, l_run = 0.f;
+
+    // ---- prologue: K(0..2), V(0..1) in; S(0); then K(3) requested
+#pragma unroll
+    for (int i = 0; i < 12; i++) fetch_one(0, 0, 0, 0, i);
+#pragma unroll
+    for (int i = 0; i < 12; i++) fetch_one(1, 1, 1, 1, i);
+#pragma unroll
+    for (int i = 0; i < 8; i++) fetch_one(2, 2, 0, 0, i);
+    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
+    __syncthreads();
+    f32x16 sv; // scores of the block the next step exponentiates: lane = query l32, element 4 i + j = key 8 i + 4 h + j
+    {
+        f32x16 s = zero16();
+#pragma unroll
+        for (int kk = 0; kk < 32; kk++) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k_read(0, kk), qf[kk], s, 0, 0, 0);
+        sv = s;
+    }
+    __syncthreads(); // K(0) has no reader left
+#pragma unroll
+    for (int i = 0; i < 4; i++) fetch_one(3, 0, 0, 0, i); // the first step sends the other eight of this group
+    bf16x8 kf[RA + 1]; // ring of fragments in flight
+#pragma unroll
+    for (int kk = 0; kk < RA; kk++) kf[kk] = k_read(1, kk);
+
+    // The running maximum moved (rare after the first blocks): O^T *= alpha, in place in the
+    // accumulation file. Written out by hand: left to the compiler, the two versions of O that
+    // meet after the branch cost more registers than there are.
+    auto rescale = [&](float alpha) __attribute__((always_inline)) {
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); // MFMA results are read next
+#pragma unroll
+        for (int blk = 0; blk < 8; blk++)
+#pragma unroll
+            for (int j = 0; j < 16; j++) {
+                float x = oacc[blk][j], t;
+                asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\ts_nop 0\n\tv_accvgpr_write_b32 %0, %1" : "+a"(x), "=&v"(t) : "v"(alpha));
+                oacc[blk][j] = x;
+            }
+        asm volatile("s_nop 7" ::: "memory"); // and feed the next MFMAs
+    };
+
+    // One step b with K(b+1) in K slot KS = (b + 1) % 3 and V(b) in V slot VS = b % 3:
+    //   S phase: the 32 MFMAs of S(b+1) = K(b+1) Q^T with the softmax of block b in their shadow;
+    //   barrier: K(b+2) and V(b) have landed (requested two steps ago), K(b+1) and V(b-1) have no
+    //            reader left;
+    //   PV phase: O += V(b)^T P(b)^T (16 MFMAs), the first fragments of K(b+2) read under them.
+    // The 12 loads that bring K(b+4) and V(b+2) into the two freed slots follow the barrier, 4
+    // under the PV phase and 8 under the next S phase.
+    auto step = [&](auto ks_c, auto vs_c, int b) __attribute__((always_inline)) {
+        constexpr int KS = decltype(ks_c)::value;       // slot of K(b+1); K(b+2) is in (KS + 1) % 3
+        constexpr int VS = decltype(vs_c)::value;       // slot of V(b); V(b-1) was in (VS + 2) % 3
+        constexpr int KN = (KS + 1) % 3;
+        f32x16 s;
+        float mloc = 0.f, mc = 0.f, alpha = 1.f, psum = 0.f, e_even = 0.f;
+        bool up = false;
+        unsigned pc[8];
+        s16x4 vlo[VA + 1], vhi[VA + 1];
+        // idx < 16: tile idx >> 3 of the half, key half (idx >> 2) & 1, 32-dim block idx & 3
+        auto v_read = [&](int idx) __attribute__((always_inline)) {
+            const lds_byte_t va = vfo[idx & 3] + (VS * V_SLOT + (idx >> 3) * TILE_BYTES + (16 * ((idx >> 2) & 1)) * (SL * 2));
+            vlo[idx % (VA + 1)] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)va);
+            vhi[idx % (VA + 1)] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(va + 8 * (SL * 2)));
+        };
+        __builtin_amdgcn_sched_barrier(0);
+        unrolled<32>([&](auto t_c) __attribute__((always_inline)) {
+            constexpr int t = decltype(t_c)::value;
+            // the previous barrier's group: K(b+3) into the slot K(b) left, V(b+1) into V(b-2)'s
+            if constexpr ((t & 3) == 0) fetch_one(b + 3, (KS + 2) % 3, b + 1, (VS + 1) % 3, 4 + (t >> 2));
+            if constexpr (t + RA < 32) kf[(t + RA) % (RA + 1)] = k_read(KS, t + RA);
+            if constexpr (t >= 28 && t - 28 < VA) v_read(t - 28);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[t % (RA + 1)], qf[t], t == 0 ? zero16() : s, 0, 0, 0);
+            // softmax of block b in the exp2 domain (the scale rides on Q) with a lazy maximum: the
+            // reference point moves only when this block's maximum exceeds it by more than kTau
+            if constexpr (t == 0) {
+                mloc = fmaxf(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])), fmaxf(fmaxf(sv[4], sv[5]), fmaxf(sv[6], sv[7])));
+            } else if constexpr (t == 1) {
+                mloc = fmaxf(mloc, fmaxf(fmaxf(fmaxf(sv[8], sv[9]), fmaxf(sv[10], sv[11])), fmaxf(fmaxf(sv[12], sv[13]), fmaxf(sv[14], sv[15]))));
+                const float mlc = pair_max(mloc);
+                up = mlc > m_run + kTau;
+                const float m_new = up ? mlc : m_run;
+                mc = (m_new == -INFINITY) ? 0.f : m_new;
+                alpha = __builtin_amdgcn_exp2f(m_run - mc);
+                m_run = m_new;
+            } else if constexpr (t >= 3 && t < 19) {
+                constexpr int e = t - 3; // one exponential per MFMA
+                const float x = __builtin_amdgcn_exp2f(sv[e] - mc);
+                psum += x;
+                if constexpr (e & 1) {
+                    f32x2 pp = {e_even, x};
+                    pc[e >> 1] = __builtin_bit_cast(unsigned, __builtin_convertvector(pp, bf16x2));
+                } else {
+                    e_even = x;
+                }
+            } else if constexpr (t == 19) {
+                l_run = l_run * alpha + psum;
+                if (__any(up)) rescale(alpha);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (t == 27) {
+                // every fragment of K(b+1) is in registers; K(b+2), V(b) have landed: everything but
+                // the 12 loads sent since the last barrier
+                __builtin_amdgcn_s_waitcnt(0x007C); // vmcnt(12) lgkmcnt(0)
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        });
+        const bf16x8 p0 = __builtin_bit_cast(bf16x8, u32x4{pc[0], pc[1], pc[2], pc[3]});
+        const bf16x8 p1 = __builtin_bit_cast(bf16x8, u32x4{pc[4], pc[5], pc[6], pc[7]});
+        unrolled<16>([&](auto i_c) __attribute__((always_inline)) {
+            constexpr int idx = decltype(i_c)::value;
+            if constexpr ((idx & 3) == 1) fetch_one(b + 4, KS, b + 2, (VS + 2) % 3, idx >> 2);
+            if constexpr (idx + VA < 16) v_read(idx + VA);
+            if constexpr (idx >= 16 - RA) kf[(idx - (16 - RA)) % (RA + 1)] = k_read(KN, idx - (16 - RA));
+            const bf16x8 vf = __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(vlo[idx % (VA + 1)], vhi[idx % (VA + 1)], 0, 1, 2, 3, 4, 5, 6, 7));
+            constexpr int ob = (idx >> 3) * 4 + (idx & 3);
+            oacc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, ((idx >> 2) & 1) ? p1 : p0, oacc[ob], 0, 0, 0);
+            if constexpr (idx == 4) sv = s; // the S MFMAs have drained by now
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+
+    int b = 0;
+    for (; b + 2 < nblk; b += 3) {
+        step(IC<1>{}, IC<0>{}, b);
+        step(IC<2>{}, IC<1>{}, b + 1);
+        step(IC<0>{}, IC<2>{}, b + 2);
+    }
+    if (b < nblk) step(IC<1>{}, IC<0>{}, b);
+    if (b + 1 < nblk) step(IC<2>{}, IC<1>{}, b + 1);
+    __builtin_amdgcn_s_waitcnt(0x0F70); // no direct load may outlive the workgroup's LDS
+
+    // ---- epilogue: O = O^T / l, or the range's share as it stands
+    const float l_tot = pair_sum(l_run);
+    if (q0 + l32 >= a.tokens) return; // (the lane joins the next half's barrier all the same: this is inlined)
+    const float scale = nsp > 1 ? 1.0f : l_tot > 0.f ? 1.0f / l_tot : 0.f;
+    float* op = (nsp > 1 ? a.part_o + ((int64_t)part * a.tokens + q0 + l32) * WD : a.o + (int64_t)(q0 + l32) * WD) + HALF * dh;
+    if (nsp > 1 && dh == 0 && h == 0) *reinterpret_cast<f32x2*>(a.part_ml + ((int64_t)part * a.tokens + q0 + l32) * 2) = f32x2{m_run, l_tot};
+#pragma unroll
+    for (int blk = 0; blk < 8; blk++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            f32x4 v;
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = oacc[blk][4 * i + j] * scale;
+            *reinterpret_cast<f32x4*>(op + 32 * blk + 8 * i + 4 * h) = v;
+        }
+}
+
+} // namespace safe
 
 __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -294,9 +541,8 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
     // spills). fp32 and bf16 share one exponent
     // range, so a later score may lie far above the reference (P up to 2^90)
     // or far below it without any loss; only a row whose scores climb some 90 (log2) above
-    // its first block's is out of reach. Such a row shows in its row sum: the wave then flags the
-    // query tile, and attn_wide_safe_kernel, which follows every launch, forms flagged tiles
-    // again with a running maximum.
+    // its first block's is out of reach. Such a row shows in its row sum, and the workgroup then
+    // forms its rows again with a running maximum (safe::form_again).
     float mc[2];
 #pragma unroll
     for (int r = 0; r < 2; r++) {
@@ -441,9 +687,12 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
         out_of_reach |= !(l_tot[r] <= kRowSumLimit);
     }
     // a row sum past kRowSumLimit (or not a number): some score left the reach of the fixed reference
-    if (__any(out_of_reach) && el == 0) a.redo[tile] = 1;
+    const bool mine_out = __any(out_of_reach);
+    if (mine_out && el == 0) a.redo[tile] = 1;
     // the partner's reference points and row sums, through P's first slot (every wave is done with it)
+    typedef __attribute__((address_space(3))) int* lds_int_t;
     __syncthreads();
+    if (el == 0) *(lds_int_t)(lds_base + (P_RING + BQ * 8 + wave * 4)) = mine_out ? 1 : 0;
     if (eg == 0) {
 #pragma unroll
         for (int r = 0; r < 2; r++) *(lds_f32x2_t)(lds_base + (P_RING + (wave * 32 + 16 * r + ec) * 8)) = f32x2{-neg[r][0], l_tot[r]};
@@ -468,256 +717,19 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
             store_through(op + (int64_t)r * WD + ((el ^ r) * 4), (f32x4)*(lds_f32x4_t)(turn + r * 1024 + el * 16));
         if (nsp > 1 && o < 2 && eg == 0) *reinterpret_cast<f32x2*>(a.part_ml + ((int64_t)part * a.tokens + row0 + ec) * 2) = ml;
     }
+    // what any wave of the workgroup found, read by all of them (nothing has been written there since the barrier)
+    int again = 0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) again |= *(lds_int_t)(lds_base + (P_RING + BQ * 8 + w * 4));
+    if (__builtin_amdgcn_readfirstlane(again) == 0) return;
+    __builtin_amdgcn_s_waitcnt(0x0F70); // the rows above are in memory before they are written again
+    for (int half = 0; half < 2; half++) {
+        __syncthreads(); // and nobody reads what is in the LDS
+        int dh2 = half;
+        asm volatile("" : "+s"(dh2)); // (nothing of a half is to be kept for the other)
+        safe::form_again(a, smem, wave, tile, part, nsp, blk0, nblk, dh2);
+    }
 }
-
-// ---------------------------------------------------------------------------------------------
-// The tiles that attn_wide_kernel flagged (a score some 90, log2, above its row's first
-// block), formed again with a lazy running maximum. A workgroup is four waves and owns 128 query
-// rows and HALF of the 512 output dims over all keys (both workgroups of a tile form the full
-// scores: 48 MFMAs per wave and block where 32 would do); with 128 accumulation registers per
-// wave the compiler has room to rescale O^T in place when a reference point moves. K blocks
-// (32 KB) and V half-blocks (16 KB) cycle through three LDS slots each. Launched after every
-// attn_wide_kernel launch; a workgroup whose tile is not flagged returns at once.
-namespace safe {
-constexpr int HALF = WD / 2;      // output dims per workgroup
-constexpr int V_SLOT = (NSL / 2) * TILE_BYTES; // half the dims of a V block: 16 KB
-constexpr int NS = 3;                          // slots per ring
-constexpr int V_RING = NS * K_SLOT;
-constexpr size_t kLdsBytes = (size_t)NS * (K_SLOT + V_SLOT); // 144 KB
-
-__global__ void __launch_bounds__(NT, 1) attn_wide_safe_kernel(const WideArgs a) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int l32 = lane & 31;
-    const int h = lane >> 5;
-    // workgroup = (query tile, half of the output dims), over all keys; only flagged tiles run
-    if (a.redo[(int)blockIdx.x >> 1] == 0) return; // uniform over the workgroup
-    const int dh = (int)blockIdx.x & 1;
-    constexpr int nsp = 1;
-    const int q0 = ((int)blockIdx.x >> 1) * BQ + 32 * wave; // this wave's query rows
-    const int blk0 = 0;
-    const int nblk = a.tokens / KB;
-
-    const unsigned lds0 = lds_address(smem);
-
-    // ---- Q fragments (B operand of S^T = K Q^T): query q0 + l32, dims 16 kk + 8 h .. +7
-    bf16x8 qf[32];
-    {
-        // rows past the end read the last row and are never stored
-        const bf16_t* qp = reinterpret_cast<const bf16_t*>(a.q) + (int64_t)min(q0 + l32, a.tokens - 1) * WD + 8 * h;
-#pragma unroll
-        for (int kk = 0; kk < 32; kk++) qf[kk] = *reinterpret_cast<const bf16x8*>(qp + 16 * kk);
-    }
-
-    // ---- block fetch. K: wave w fills tile w (dims 128 w .. +127) of the block, four rows per
-    // instruction. V: wave w fills rows 16 (w >> 1) .. +15 of tile (w & 1) of this workgroup's
-    // half. The lane that fills chunk position p of row r fetches the chunk the swizzle places
-    // there: K chunk c of row r sits at c ^ (r & 15), V chunk c at c ^ ((r & 3) << 2).
-    const unsigned span = (unsigned)a.tokens * (unsigned)(WD * 2);
-    const u32x4 k_rsrc = make_rsrc_words(a.k, span);
-    const u32x4 v_rsrc = make_rsrc_words(a.v, span);
-    unsigned fk_off[4], fv_off[4]; // K rows 4 j + 16 take the same chunks 16 rows further on
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int row = 4 * j + (lane >> 4);
-        const unsigned kc = (unsigned)((lane & 15) ^ (row & 15));
-        fk_off[j] = (unsigned)row * (WD * 2) + (unsigned)wave * (SL * 2) + kc * 16u;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int row = 16 * (wave >> 1) + 4 * j + (lane >> 4);
-        const unsigned vc = (unsigned)((lane & 15) ^ ((row & 3) << 2));
-        fv_off[j] = (unsigned)row * (WD * 2) + (unsigned)(2 * dh + (wave & 1)) * (SL * 2) + vc * 16u;
-    }
-    const unsigned fetch_k_lds = __builtin_amdgcn_readfirstlane(lds0 + (unsigned)wave * TILE_BYTES);
-    const unsigned fetch_v_lds = __builtin_amdgcn_readfirstlane(lds0 + V_RING + (unsigned)(wave & 1) * TILE_BYTES + (unsigned)(16 * (wave >> 1)) * (SL * 2));
-    // the i-th (i < 12) load of the group that brings K block kb into K slot ks and V block vb into V slot vs
-    auto fetch_one = [&](int kb, int ks, int vb, int vs, int i) __attribute__((always_inline)) {
-        if (i < 8) {
-            // (uniform, but the compiler may have formed it in a vector register)
-            const unsigned uo = __builtin_amdgcn_readfirstlane((unsigned)(blk0 + (kb < nblk ? kb : nblk - 1)) * (unsigned)(KB * WD * 2) + (unsigned)(i >> 2) * (16 * WD * 2));
-            load_to_lds_16(k_rsrc, fetch_k_lds + (unsigned)ks * K_SLOT + (unsigned)(4 * i) * (SL * 2), fk_off[i & 3], uo);
-        } else {
-            const unsigned uo = __builtin_amdgcn_readfirstlane((unsigned)(blk0 + (vb < nblk ? vb : nblk - 1)) * (unsigned)(KB * WD * 2));
-            load_to_lds_16(v_rsrc, fetch_v_lds + (unsigned)vs * V_SLOT + (unsigned)(4 * (i - 8)) * (SL * 2), fv_off[i - 8], uo);
-        }
-    };
-
-    // ---- fragment addresses in slot 0 (a tile and a slot add constants)
-    const int tr_row = (lane & 15) >> 2;
-    const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-    // (pointers, so that the constant parts of an address go into the instruction's offset field)
-    typedef __attribute__((address_space(3))) unsigned char* lds_byte_t;
-    typedef const __attribute__((address_space(3))) bf16x8* lds_bf16x8_t;
-    typedef __attribute__((address_space(3))) s16x4* lds_s16x4_t;
-    const lds_byte_t lds_base = (lds_byte_t)smem;
-    lds_byte_t kfo[8], vfo[4];
-#pragma unroll
-    for (int kk = 0; kk < 8; kk++) kfo[kk] = lds_base + ((l32 * SL + (((2 * kk + h) ^ (l32 & 15)) * 8)) * 2);
-#pragma unroll
-    for (int blk = 0; blk < 4; blk++)
-        vfo[blk] = lds_base + V_RING + (((4 * h + tr_row) * SL + ((blk ^ tr_row) * 32) + tr_col) * 2);
-    auto k_read = [&](int slot, int kk) __attribute__((always_inline)) {
-        return *(lds_bf16x8_t)(kfo[kk & 7] + (slot * K_SLOT + (kk >> 3) * TILE_BYTES));
-    };
-
-    f32x16 oacc[8]; // O^T: lane = query l32, dims 256 dh + 32 blk + 8 i + 4 h + j
-#pragma unroll
-    for (int blk = 0; blk < 8; blk++)
-#pragma unroll
-        for (int j = 0; j < 16; j++) oacc[blk][j] = 0.f;
-    float m_run = -INFINITY, l_run = 0.f;
-
-    // ---- prologue: K(0..2), V(0..1) in; S(0); then K(3) requested
-#pragma unroll
-    for (int i = 0; i < 12; i++) fetch_one(0, 0, 0, 0, i);
-#pragma unroll
-    for (int i = 0; i < 12; i++) fetch_one(1, 1, 1, 1, i);
-#pragma unroll
-    for (int i = 0; i < 8; i++) fetch_one(2, 2, 0, 0, i);
-    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
-    __syncthreads();
-    f32x16 sv; // scores of the block the next step exponentiates: lane = query l32, element 4 i + j = key 8 i + 4 h + j
-    {
-        f32x16 s = zero16();
-#pragma unroll
-        for (int kk = 0; kk < 32; kk++) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k_read(0, kk), qf[kk], s, 0, 0, 0);
-        sv = s;
-    }
-    __syncthreads(); // K(0) has no reader left
-#pragma unroll
-    for (int i = 0; i < 4; i++) fetch_one(3, 0, 0, 0, i); // the first step sends the other eight of this group
-    bf16x8 kf[RA + 1]; // ring of fragments in flight
-#pragma unroll
-    for (int kk = 0; kk < RA; kk++) kf[kk] = k_read(1, kk);
-
-    // The running maximum moved (rare after the first blocks): O^T *= alpha, in place in the
-    // accumulation file. Written out by hand: left to the compiler, the two versions of O that
-    // meet after the branch cost more registers than there are.
-    auto rescale = [&](float alpha) __attribute__((always_inline)) {
-        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); // MFMA results are read next
-#pragma unroll
-        for (int blk = 0; blk < 8; blk++)
-#pragma unroll
-            for (int j = 0; j < 16; j++) {
-                float x = oacc[blk][j], t;
-                asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\ts_nop 0\n\tv_accvgpr_write_b32 %0, %1" : "+a"(x), "=&v"(t) : "v"(alpha));
-                oacc[blk][j] = x;
-            }
-        asm volatile("s_nop 7" ::: "memory"); // and feed the next MFMAs
-    };
-
-    // One step b with K(b+1) in K slot KS = (b + 1) % 3 and V(b) in V slot VS = b % 3:
-    //   S phase: the 32 MFMAs of S(b+1) = K(b+1) Q^T with the softmax of block b in their shadow;
-    //   barrier: K(b+2) and V(b) have landed (requested two steps ago), K(b+1) and V(b-1) have no
-    //            reader left;
-    //   PV phase: O += V(b)^T P(b)^T (16 MFMAs), the first fragments of K(b+2) read under them.
-    // The 12 loads that bring K(b+4) and V(b+2) into the two freed slots follow the barrier, 4
-    // under the PV phase and 8 under the next S phase.
-    auto step = [&](auto ks_c, auto vs_c, int b) __attribute__((always_inline)) {
-        constexpr int KS = decltype(ks_c)::value;       // slot of K(b+1); K(b+2) is in (KS + 1) % 3
-        constexpr int VS = decltype(vs_c)::value;       // slot of V(b); V(b-1) was in (VS + 2) % 3
-        constexpr int KN = (KS + 1) % 3;
-        f32x16 s;
-        float mloc = 0.f, mc = 0.f, alpha = 1.f, psum = 0.f, e_even = 0.f;
-        bool up = false;
-        unsigned pc[8];
-        s16x4 vlo[VA + 1], vhi[VA + 1];
-        // idx < 16: tile idx >> 3 of the half, key half (idx >> 2) & 1, 32-dim block idx & 3
-        auto v_read = [&](int idx) __attribute__((always_inline)) {
-            const lds_byte_t va = vfo[idx & 3] + (VS * V_SLOT + (idx >> 3) * TILE_BYTES + (16 * ((idx >> 2) & 1)) * (SL * 2));
-            vlo[idx % (VA + 1)] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)va);
-            vhi[idx % (VA + 1)] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(va + 8 * (SL * 2)));
-        };
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int t = 0; t < 32; t++) {
-            // the previous barrier's group: K(b+3) into the slot K(b) left, V(b+1) into V(b-2)'s
-            if ((t & 3) == 0) fetch_one(b + 3, (KS + 2) % 3, b + 1, (VS + 1) % 3, 4 + (t >> 2));
-            if (t + RA < 32) kf[(t + RA) % (RA + 1)] = k_read(KS, t + RA);
-            if (t >= 28 && t - 28 < VA) v_read(t - 28);
-            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[t % (RA + 1)], qf[t], t == 0 ? zero16() : s, 0, 0, 0);
-            // softmax of block b in the exp2 domain (the scale rides on Q) with a lazy maximum: the
-            // reference point moves only when this block's maximum exceeds it by more than kTau
-            if (t == 0) {
-                mloc = fmaxf(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])), fmaxf(fmaxf(sv[4], sv[5]), fmaxf(sv[6], sv[7])));
-            } else if (t == 1) {
-                mloc = fmaxf(mloc, fmaxf(fmaxf(fmaxf(sv[8], sv[9]), fmaxf(sv[10], sv[11])), fmaxf(fmaxf(sv[12], sv[13]), fmaxf(sv[14], sv[15]))));
-                const float mlc = pair_max(mloc);
-                up = mlc > m_run + kTau;
-                const float m_new = up ? mlc : m_run;
-                mc = (m_new == -INFINITY) ? 0.f : m_new;
-                alpha = __builtin_amdgcn_exp2f(m_run - mc);
-                m_run = m_new;
-            } else if (t >= 3 && t < 19) {
-                const int e = t - 3; // one exponential per MFMA
-                const float x = __builtin_amdgcn_exp2f(sv[e] - mc);
-                psum += x;
-                if (e & 1) {
-                    f32x2 pp = {e_even, x};
-                    pc[e >> 1] = __builtin_bit_cast(unsigned, __builtin_convertvector(pp, bf16x2));
-                } else {
-                    e_even = x;
-                }
-            } else if (t == 19) {
-                l_run = l_run * alpha + psum;
-                if (__any(up)) rescale(alpha);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            if (t == 27) {
-                // every fragment of K(b+1) is in registers; K(b+2), V(b) have landed: everything but
-                // the 12 loads sent since the last barrier
-                __builtin_amdgcn_s_waitcnt(0x007C); // vmcnt(12) lgkmcnt(0)
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_s_barrier();
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        const bf16x8 p0 = __builtin_bit_cast(bf16x8, u32x4{pc[0], pc[1], pc[2], pc[3]});
-        const bf16x8 p1 = __builtin_bit_cast(bf16x8, u32x4{pc[4], pc[5], pc[6], pc[7]});
-#pragma unroll
-        for (int idx = 0; idx < 16; idx++) {
-            if ((idx & 3) == 1) fetch_one(b + 4, KS, b + 2, (VS + 2) % 3, idx >> 2);
-            if (idx + VA < 16) v_read(idx + VA);
-            if (idx >= 16 - RA) kf[(idx - (16 - RA)) % (RA + 1)] = k_read(KN, idx - (16 - RA));
-            const bf16x8 vf = __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(vlo[idx % (VA + 1)], vhi[idx % (VA + 1)], 0, 1, 2, 3, 4, 5, 6, 7));
-            const int ob = (idx >> 3) * 4 + (idx & 3);
-            oacc[ob] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, ((idx >> 2) & 1) ? p1 : p0, oacc[ob], 0, 0, 0);
-            if (idx == 4) sv = s; // the S MFMAs have drained by now
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-
-    int b = 0;
-    for (; b + 2 < nblk; b += 3) {
-        step(IC<1>{}, IC<0>{}, b);
-        step(IC<2>{}, IC<1>{}, b + 1);
-        step(IC<0>{}, IC<2>{}, b + 2);
-    }
-    if (b < nblk) step(IC<1>{}, IC<0>{}, b);
-    if (b + 1 < nblk) step(IC<2>{}, IC<1>{}, b + 1);
-    __builtin_amdgcn_s_waitcnt(0x0F70); // no direct load may outlive the workgroup's LDS
-
-    // ---- epilogue: O = O^T / l, or the range's share as it stands
-    const float l_tot = pair_sum(l_run);
-    if (q0 + l32 >= a.tokens) return;
-    const float inv_l = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-    float* op = a.o + (int64_t)(q0 + l32) * WD + HALF * dh;
-#pragma unroll
-    for (int blk = 0; blk < 8; blk++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            f32x4 v;
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = oacc[blk][4 * i + j] * inv_l;
-            *reinterpret_cast<f32x4*>(op + 32 * blk + 8 * i + 4 * h) = v;
-        }
-}
-
-} // namespace safe
 
 // Combines the key ranges of a split launch, in range order: with reference points m_p and row
 // sums l_p, O = sum_p 2^(m_p - m) O_p / sum_p 2^(m_p - m) l_p, m = max_p m_p. A thread owns four
@@ -824,17 +836,12 @@ hipError_t launch_wide_attention(const WideArgs& a, hipStream_t stream) {
         static_assert(wide::kMaxSplits == 8, "one case per number of ranges");
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
-    // flagged tiles (none on ordinary data) are formed again, over whatever the launches above left there
-    wide::safe::attn_wide_safe_kernel<<<dim3(tiles * 2u), dim3(wide::NT), wide::safe::kLdsBytes, stream>>>(a);
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 hipError_t wide_setup() {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&wide::attn_wide_kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)wide::kLdsBytes);
-    if (e != hipSuccess) return e;
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(&wide::safe::attn_wide_safe_kernel),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)wide::safe::kLdsBytes);
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(&wide::attn_wide_kernel),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)wide::kLdsBytes);
 }
 int wide_tiles(int tokens) { return (tokens + wide::BQ - 1) / wide::BQ; }
 

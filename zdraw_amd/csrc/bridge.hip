@@ -837,7 +837,7 @@ int check_pipeline(void* pipeline, uint32_t kernel, int want_kind) {
 }
 
 bool g_wide_setup_done = false;
-// the redo flags of the last wide-head launch (measurement aid: how many tiles took the safe kernel)
+// the redo flags of the last wide-head launch (measurement aid: how many tiles were formed twice)
 int* g_last_wide_redo = nullptr;
 int g_last_wide_tiles = 0;
 hipStream_t g_last_wide_stream = nullptr;
@@ -881,8 +881,8 @@ int enqueue_wide(Queue* queue, void* q, void* k, void* v, void* out, const Zdraw
         g_wide_setup_done = true;
     }
     // one flag per query tile (scratch slot 4): set by the kernel where a row's scores outgrow its
-    // fixed reference point, cleared by the rounding launch, read by the kernel that forms such
-    // tiles again
+    // fixed reference point and are formed again, cleared by the rounding launch (read by
+    // zdraw_hip_wide_redo_tiles only)
     Buffer* redo = queue_scratch(queue, 4, (size_t)wide_tiles((int)p->tokens) * sizeof(int));
     if (!redo) {
         set_err("scratch allocation failed");
