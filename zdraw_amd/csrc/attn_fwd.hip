@@ -124,6 +124,18 @@ __device__ __forceinline__ u32x2 round4(const f32x4& v, int dtype) {
 // waves, each over half of the keys, merged in LDS at the end: half the steps per workgroup and
 // twice the workgroups, for launches that leave CUs idle (launch_attention, shape 2). Every group
 // has a four-stage ring of its own and all of the schedule below; a step ends in a barrier.
+// The lane's number formed anew where it is needed once in a while. What is formed from it stays in registers across
+// the key loop otherwise: 228 to 256 of them and spills in the builds of prepared operands, 211 to 238 without, with the
+// wave's number in a scalar register. The masked running-maximum build so has room for the 16 x 16 product, and shorter
+// prologues pay where a launch is a few key blocks per wave: 24 heads, five blocks of 768 tokens 134.6 -> 130.5 us, of 1088
+// 181.1 -> 175.7; f32 rows of 24 heads, 4001 tokens 239.9 -> 235.5, 3000 tokens of which 2500 are keys 151.1 -> 147.7.
+// (The tail block's row offsets stay: formed again in a branch they cost 2 x 8704 tokens 0.5 %.)
+__device__ __forceinline__ int lane_again() {
+    int x;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
+    return x;
+}
+
 template <typename TIn, int KMODE, bool MASKED, bool BOUNDED, int QB, int NW, bool SF16 = false, int KG = 1>
 __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(const AttnArgs a) {
     constexpr int NT = NW * 64;
@@ -145,12 +157,13 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     // which a lane owns one query). The 16 x 16 form moves half the accumulator bytes per FLOP
     // through the register file, and at the board's power limit that is worth clock: -2 % of the
     // kernel's time. It costs a few registers (the compiler writes these MFMAs' results to other
-    // registers than their inputs) and four lane exchanges per block, so only the builds with
-    // room take it: prepared operands, and not the running maximum together with a mask (that
-    // build then spills inside the loop; with its reference points held at 0 it has the room, 24 heads of 4064 of 4608
-    // tokens 214 -> 203.5 us, but a row's largest P is then no longer exactly 1 and rounds like the rest). (Giving the scores that form too would double the MFMA
+    // registers than their inputs) and four lane exchanges per block. The one build of prepared operands without it, masked
+    // with two key groups, is a wave's chain and not the power limit, and the exchanges lengthen it: 24 heads, five
+    // blocks of 768 tokens with masked text 116.1 us without, 118.2 with it. Masked running maximum, one group, without -> with:
+    // 2 x 8704 tokens 3153 -> 3140, 4 x 1536 305.3 -> 303.1, 4464 tokens 520.1 -> 518.1 (two blocks each; error against float64
+    // the same). (Giving the scores that form too would double the MFMA
     // instructions on a vector issue port that the softmax already half fills.)
-    constexpr bool PV16 = DMA && (!MASKED || (BOUNDED && KG == 1));
+    constexpr bool PV16 = DMA && (!MASKED || KG == 1);
     constexpr int KSTAGE = DMA ? KB * D : KS_ELEMS; // elements per ring stage
     constexpr int VSTAGE = DMA ? KB * D : VS_ELEMS;
     // a block enters the ring AHEAD steps before S needs its K (direct loads: one more step, to land)
@@ -177,7 +190,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     }
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = DMA ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
     const int l32 = lane & 31;
     const int h = lane >> 5;
     const int grp = KG == 2 ? __builtin_amdgcn_readfirstlane(wave >> 2) : 0; // key group
@@ -300,7 +313,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     unsigned list_blk = 0, list_mask = 0;
     auto list_load = [&](int base) __attribute__((always_inline)) {
         list_base = base;
-        const int i = min(base + lane, last_own);
+        const int i = min(base + lane_again(), last_own);
         list_blk = kp ? (unsigned)blocks[i + i0] : (unsigned)(i + i0);
         list_mask = bmask[list_blk];
     };
@@ -735,14 +748,15 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             unsigned badm = MASKED ? (unsigned)__builtin_amdgcn_readlane((int)list_mask, b - list_base) : 0u;
             if (KG == 2 && b >= nown) badm = 0xffffffffu; // the idle step of the shorter half
             if (badm != 0u) { // wave-uniform: most blocks exclude nothing
+                const unsigned bad_h = badm >> (4 * (lane_again() >> 5)); // this lane's keys 4 h ..
 #pragma unroll
                 for (int qi = 0; qi < QB; qi++)
 #pragma unroll
                     for (int i = 0; i < 4; i++)
 #pragma unroll
                         for (int j = 0; j < 4; j++) {
-                            const int kk = 8 * i + 4 * h + j;
-                            s_cur[qi][4 * i + j] = ((badm >> kk) & 1u) ? -INFINITY : s_cur[qi][4 * i + j];
+                            const int kk = 8 * i + j;
+                            s_cur[qi][4 * i + j] = ((bad_h >> kk) & 1u) ? -INFINITY : s_cur[qi][4 * i + j];
                         }
             }
         }
@@ -909,7 +923,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                         // query 16 r + c16 comes from the lane that owns that query's scores
 #pragma unroll
                         for (int r = 0; r < 2; r++) {
-                            const float ar = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + c16), (int)__float_as_uint(alpha[qi])));
+                            const float ar = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + (lane_again() & 15)), (int)__float_as_uint(alpha[qi])));
 #pragma unroll
                             for (int dt = 0; dt < 8; dt++) oacc16[dt][r] *= ar;
                         }
@@ -1103,14 +1117,17 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
         if constexpr (DMA) __builtin_amdgcn_s_waitcnt(0x0F70); // no direct load may outlive the workgroup's LDS
     }
 
+    // (the lane's coordinates are formed again: kept across the key loop they would cost it registers)
+    [[maybe_unused]] const int elane = DMA ? lane_again() : lane;
+    [[maybe_unused]] const int el32 = elane & 31, eh = elane >> 5, ec16 = elane & 15, eg4 = elane >> 4;
     if constexpr (KG == 2) {
         // The second group's rows, reference points and denominators go through the idle ring to the
         // first, which adds them to its own (weighted by the distance of the reference points) and
         // stores: 64 KB in and out of LDS.
         typedef __attribute__((address_space(3))) f32x4* lds_f32x4_t;
         typedef __attribute__((address_space(3))) f32x2* lds_f32x2_t;
-        const unsigned xo = lds_address(Vs) + (unsigned)(gw * (64 * 64 * 4) + lane * 16); // 64 values a lane, 16 bytes at a time
-        const unsigned xm = lds_address(Ks) + (unsigned)(4 * (KSTAGE * 2) + gw * (64 * 8) + lane * 8);
+        const unsigned xo = lds_address(Vs) + (unsigned)(gw * (64 * 64 * 4) + elane * 16); // 64 values a lane, 16 bytes at a time
+        const unsigned xm = lds_address(Ks) + (unsigned)(4 * (KSTAGE * 2) + gw * (64 * 8) + elane * 8);
         __syncthreads(); // every wave is done with the ring
         if (grp != 0) {
             if constexpr (PV16) {
@@ -1139,8 +1156,8 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
         if constexpr (PV16 && !BOUNDED) { // the weights of query 16 r + c16 live with its scores
 #pragma unroll
             for (int r = 0; r < 2; r++) {
-                w0r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + c16), (int)__float_as_uint(w0)));
-                w1r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + c16), (int)__float_as_uint(w1)));
+                w0r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + ec16), (int)__float_as_uint(w0)));
+                w1r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + ec16), (int)__float_as_uint(w1)));
             }
         }
 #pragma unroll
@@ -1167,7 +1184,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
         float inv_r[2];
 #pragma unroll
         for (int r = 0; r < 2; r++)
-            inv_r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + c16), (int)__float_as_uint(inv_l)));
+            inv_r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + ec16), (int)__float_as_uint(inv_l)));
         const bool part = splits > 1; // unnormalised rows, reference point and denominator of a part of the keys
         if (part || a.out_dtype == kF32) {
             // f32 rows leave as the 16-bit ones below do, through 16 KB of LDS of the wave's own (16-byte
@@ -1181,7 +1198,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             for (int r = 0; r < 2; r++)
 #pragma unroll
                 for (int dt = 0; dt < 8; dt++)
-                    *(lds_turn_t)(turn + (unsigned)((16 * r + c16) * (D * 4) + (((4 * dt + g4) ^ c16) * 16))) = part ? oacc16[dt][r] : oacc16[dt][r] * inv_r[r];
+                    *(lds_turn_t)(turn + (unsigned)((16 * r + ec16) * (D * 4) + (((4 * dt + eg4) ^ ec16) * 16))) = part ? oacc16[dt][r] : oacc16[dt][r] * inv_r[r];
             const int64_t prow0 = (int64_t)blockIdx.x * BQ + gw * QR;
             float* const base = part ? a.part_o + prow0 * D
                                      : reinterpret_cast<float*>(a.o) + (int64_t)seg * a.o_bs + (int64_t)q0 * a.o_ts + (int64_t)head * a.o_hs;
@@ -1191,17 +1208,17 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
             unsigned short* const row16 = part || !a.o16 ? nullptr : static_cast<unsigned short*>(a.o16) + (((int64_t)seg * a.tokens + q0) * a.heads + head) * D;
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                const int r = 2 * i + h;
-                const f32x4 v = *(lds_turn_t)(turn + (unsigned)(i * 1024 + lane * 16));
+                const int r = 2 * i + eh;
+                const f32x4 v = *(lds_turn_t)(turn + (unsigned)(i * 1024 + elane * 16));
                 if (r < rows) {
-                    const int d = (l32 ^ (r & 15)) * 4;
+                    const int d = (el32 ^ (r & 15)) * 4;
                     store_through(base + r * stride + d, v);
                     if (row16) *reinterpret_cast<u32x2*>(row16 + (int64_t)r * (a.heads * D) + d) = round4(v, a.o16_dtype);
                 }
             }
-            if (part && h == 0) {
-                a.part_ml[(prow0 + l32) * 2] = BOUNDED ? 0.f : m_run[0];
-                a.part_ml[(prow0 + l32) * 2 + 1] = l_tot;
+            if (part && eh == 0) {
+                a.part_ml[(prow0 + el32) * 2] = BOUNDED ? 0.f : m_run[0];
+                a.part_ml[(prow0 + el32) * 2 + 1] = l_tot;
             }
         } else {
             // 16-bit output: a lane holds 8-byte pieces of two rows, which would leave the chip as
@@ -1222,16 +1239,16 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                     const f32x4 v = oacc16[dt][r] * inv_r[r];
                     const u32x2 bits = half ? __builtin_bit_cast(u32x2, __builtin_convertvector(v, f16x4))
                                             : __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
-                    *(lds_u32x2_t)(o_lds + (unsigned)((16 * r + c16) * (D * 2) + (((2 * dt + (g4 >> 1)) ^ c16) * 16) + 8 * (g4 & 1))) = bits;
+                    *(lds_u32x2_t)(o_lds + (unsigned)((16 * r + ec16) * (D * 2) + (((2 * dt + (eg4 >> 1)) ^ ec16) * 16) + 8 * (eg4 & 1))) = bits;
                 }
             unsigned short* const obase = reinterpret_cast<unsigned short*>(a.o) + (int64_t)seg * a.o_bs + (int64_t)head * a.o_hs;
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                const int r = 4 * j + (lane >> 4);
-                const u32x4 row16 = *(lds_u32x4_t)(o_lds + (unsigned)(r * (D * 2) + (lane & 15) * 16));
+                const int r = 4 * j + (elane >> 4);
+                const u32x4 row16 = *(lds_u32x4_t)(o_lds + (unsigned)(r * (D * 2) + (elane & 15) * 16));
                 const int orow = q0 + r;
                 if (orow < a.tokens)
-                    store_through(obase + (int64_t)orow * a.o_ts + (((lane & 15) ^ (r & 15)) * 8), row16);
+                    store_through(obase + (int64_t)orow * a.o_ts + (((elane & 15) ^ (r & 15)) * 8), row16);
             }
         }
     } else {
@@ -1239,10 +1256,10 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
         for (int qi = 0; qi < QB; qi++) {
             const float l_tot = pair_sum(l_run[qi]);
             const float inv_l = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-            const int qrow = q0 + 32 * qi + l32;
+            const int qrow = q0 + 32 * qi + el32;
             if (splits > 1) {
                 // unnormalised rows, reference point and denominator of this part
-                const int64_t prow = ((int64_t)blockIdx.x * BQ + gw * QR + 32 * qi + l32);
+                const int64_t prow = ((int64_t)blockIdx.x * BQ + gw * QR + 32 * qi + el32);
                 float* op = a.part_o + prow * D;
 #pragma unroll
                 for (int blk = 0; blk < 4; blk++)
@@ -1251,9 +1268,9 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                         f32x4 v;
 #pragma unroll
                         for (int j = 0; j < 4; j++) v[j] = oacc[qi][blk][4 * i + j];
-                        *reinterpret_cast<f32x4*>(op + 32 * blk + 8 * i + 4 * h) = v;
+                        *reinterpret_cast<f32x4*>(op + 32 * blk + 8 * i + 4 * eh) = v;
                     }
-                if (h == 0) {
+                if (eh == 0) {
                     a.part_ml[prow * 2] = BOUNDED ? 0.f : m_run[qi];
                     a.part_ml[prow * 2 + 1] = l_tot;
                 }
@@ -1267,11 +1284,11 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                             f32x4 v;
 #pragma unroll
                             for (int j = 0; j < 4; j++) v[j] = oacc[qi][blk][4 * i + j] * inv_l;
-                            *reinterpret_cast<f32x4*>(op + 32 * blk + 8 * i + 4 * h) = v;
+                            *reinterpret_cast<f32x4*>(op + 32 * blk + 8 * i + 4 * eh) = v;
                             if constexpr (DMA)
                                 if (a.o16)
                                     *reinterpret_cast<u32x2*>(static_cast<unsigned short*>(a.o16) + (((int64_t)seg * a.tokens + qrow) * a.heads + head) * D +
-                                                              32 * blk + 8 * i + 4 * h) = round4(v, a.o16_dtype);
+                                                              32 * blk + 8 * i + 4 * eh) = round4(v, a.o16_dtype);
                         }
                 }
             } else {
@@ -1294,16 +1311,16 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
                         for (int j = 0; j < 4; j++) v[j] = oacc[qi][blk][4 * i + j] * inv_l;
                         const u32x2 bits = half ? __builtin_bit_cast(u32x2, __builtin_convertvector(v, f16x4))
                                                 : __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
-                        *(lds_u32x2_t)(o_lds + (unsigned)(l32 * (D * 2) + (((4 * blk + i) ^ (l32 & 15)) * 16) + 8 * h)) = bits;
+                        *(lds_u32x2_t)(o_lds + (unsigned)(el32 * (D * 2) + (((4 * blk + i) ^ (el32 & 15)) * 16) + 8 * eh)) = bits;
                     }
                 unsigned short* const obase = reinterpret_cast<unsigned short*>(a.o) + (int64_t)seg * a.o_bs + (int64_t)head * a.o_hs;
 #pragma unroll
                 for (int j = 0; j < 8; j++) {
-                    const int r = 4 * j + (lane >> 4);
-                    const u32x4 row16 = *(lds_u32x4_t)(o_lds + (unsigned)(r * (D * 2) + (lane & 15) * 16));
+                    const int r = 4 * j + (elane >> 4);
+                    const u32x4 row16 = *(lds_u32x4_t)(o_lds + (unsigned)(r * (D * 2) + (elane & 15) * 16));
                     const int orow = q0 + 32 * qi + r;
                     if (orow < a.tokens)
-                        store_through(obase + (int64_t)orow * a.o_ts + (((lane & 15) ^ (r & 15)) * 8), row16);
+                        store_through(obase + (int64_t)orow * a.o_ts + (((elane & 15) ^ (r & 15)) * 8), row16);
                 }
             }
         }
@@ -1312,7 +1329,7 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     int64_t probe_slot = (int64_t)blockIdx.x - a.part_wgs;
     // (a slot per 256 query rows in either shape: of two workgroups that share them, the first's)
     if constexpr (KG == 2) probe_slot = (splits > 1 || (qb & 1)) ? -1 : (int64_t)bh * ((a.nqb + 1) >> 1) + (qb >> 1);
-    if (a.clock_probe && tid == 0 && probe_slot >= 0 && probe_slot < a.clock_cap) {
+    if (a.clock_probe && wave == 0 && elane == 0 && probe_slot >= 0 && probe_slot < a.clock_cap) {
         a.clock_probe[2 * probe_slot] = __builtin_readcyclecounter() - clk_c0;
         a.clock_probe[2 * probe_slot + 1] = __builtin_amdgcn_s_memrealtime() - clk_r0;
     }
