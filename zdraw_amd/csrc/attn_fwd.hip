@@ -1120,135 +1120,152 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
     // (the lane's coordinates are formed again: kept across the key loop they would cost it registers)
     [[maybe_unused]] const int elane = DMA ? lane_again() : lane;
     [[maybe_unused]] const int el32 = elane & 31, eh = elane >> 5, ec16 = elane & 15, eg4 = elane >> 4;
+    // O^T as the epilogue takes it: 16 / KG four-element pieces of the wave's 32 rows. PV16: piece 2 dt + r is tile
+    // dt of 16 dims, queries 16 r + c16, dims 4 g4 .. + 3 of it; otherwise piece 4 blk + i holds query l32, dims 8 i + 4 h
+    // .. + 3 of block blk of 32.
+    constexpr int NP = 16 / KG;
+    auto piece = [&](int n) __attribute__((always_inline)) -> f32x4 {
+        if constexpr (PV16) return oacc16[n >> 1][n & 1];
+        else return f32x4{oacc[0][n >> 2][4 * (n & 3)], oacc[0][n >> 2][4 * (n & 3) + 1], oacc[0][n >> 2][4 * (n & 3) + 2], oacc[0][n >> 2][4 * (n & 3) + 3]};
+    };
+    [[maybe_unused]] f32x4 own[NP];
+    [[maybe_unused]] unsigned turn_lds = 0; // KG = 2: 8 KB of LDS that only this wave uses from here on
     if constexpr (KG == 2) {
-        // The second group's rows, reference points and denominators go through the idle ring to the
-        // first, which adds them to its own (weighted by the distance of the reference points) and
-        // stores: 64 KB in and out of LDS.
+        // The two groups meet in the idle ring: of the rows that both have walked half of the keys for, each takes one
+        // half of the dims, with the other's share (weighted by the distance of the reference points), and finishes and stores
+        // that: 32 KB in and out of LDS each. (The first group alone, which this was, had four waves, one a SIMD, do 5 k of
+        // a launch's 30 k cycles: 24 heads, five blocks of 768 tokens 132.6 -> 129.2 us, one call of 700 f32 rows 40.9 -> 39.4.)
         typedef __attribute__((address_space(3))) f32x4* lds_f32x4_t;
         typedef __attribute__((address_space(3))) f32x2* lds_f32x2_t;
-        const unsigned xo = lds_address(Vs) + (unsigned)(gw * (64 * 64 * 4) + elane * 16); // 64 values a lane, 16 bytes at a time
-        const unsigned xm = lds_address(Ks) + (unsigned)(4 * (KSTAGE * 2) + gw * (64 * 8) + elane * 8);
+        const unsigned xo = lds_address(Vs) + (unsigned)(elane * 16); // 8 KB per wave, 16 bytes a lane at a time
+        const unsigned xm = lds_address(Ks) + (unsigned)(elane * 8);  // 512 bytes per wave
+        const unsigned mine = (unsigned)wave, other = (unsigned)(wave ^ 4);
         __syncthreads(); // every wave is done with the ring
-        if (grp != 0) {
-            if constexpr (PV16) {
+        if (grp == 0) {
 #pragma unroll
-                for (int i = 0; i < 16; i++) *(lds_f32x4_t)(xo + (unsigned)(i * 1024)) = oacc16[i >> 1][i & 1];
-            } else {
-#pragma unroll
-                for (int i = 0; i < 16; i++)
-                    *(lds_f32x4_t)(xo + (unsigned)(i * 1024)) =
-                        f32x4{oacc[0][i >> 2][4 * (i & 3)], oacc[0][i >> 2][4 * (i & 3) + 1], oacc[0][i >> 2][4 * (i & 3) + 2], oacc[0][i >> 2][4 * (i & 3) + 3]};
+            for (int i = 0; i < NP; i++) {
+                *(lds_f32x4_t)(xo + mine * (NP * 1024u) + (unsigned)(i * 1024)) = piece(NP + i);
+                own[i] = piece(i);
             }
-            *(lds_f32x2_t)xm = f32x2{m_run[0], l_run[0]};
+        } else {
+#pragma unroll
+            for (int i = 0; i < NP; i++) {
+                *(lds_f32x4_t)(xo + mine * (NP * 1024u) + (unsigned)(i * 1024)) = piece(i);
+                own[i] = piece(NP + i);
+            }
         }
+        *(lds_f32x2_t)(xm + mine * 512u) = f32x2{m_run[0], l_run[0]};
         __syncthreads();
-        if (grp != 0) return;
-        const f32x2 ml = *(lds_f32x2_t)xm;
-        float w0 = 1.f, w1 = 1.f;
+        const f32x2 ml = *(lds_f32x2_t)(xm + other * 512u);
+        float w_own = 1.f, w_other = 1.f;
         if constexpr (!BOUNDED) {
             const float m = fmaxf(m_run[0], ml[0]); // (a group without an admitted key has no reference: weight 0)
-            w0 = m_run[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[0] - m);
-            w1 = ml[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[0] - m);
+            w_own = m_run[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[0] - m);
+            w_other = ml[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[0] - m);
             m_run[0] = m;
         }
-        l_run[0] = l_run[0] * w0 + ml[1] * w1;
-        float w0r[2] = {w0, w0}, w1r[2] = {w1, w1};
+        // (both groups add the first group's share to the second's: one denominator for both halves of a row)
+        l_run[0] = grp == 0 ? l_run[0] * w_own + ml[1] * w_other : ml[1] * w_other + l_run[0] * w_own;
+        float wo[2] = {w_own, w_own}, wx[2] = {w_other, w_other};
         if constexpr (PV16 && !BOUNDED) { // the weights of query 16 r + c16 live with its scores
 #pragma unroll
             for (int r = 0; r < 2; r++) {
-                w0r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + ec16), (int)__float_as_uint(w0)));
-                w1r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + ec16), (int)__float_as_uint(w1)));
+                wo[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + ec16), (int)__float_as_uint(w_own)));
+                wx[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + ec16), (int)__float_as_uint(w_other)));
             }
         }
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const f32x4 x = *(lds_f32x4_t)(xo + (unsigned)(i * 1024));
-            if constexpr (PV16) {
-                oacc16[i >> 1][i & 1] = BOUNDED ? oacc16[i >> 1][i & 1] + x : oacc16[i >> 1][i & 1] * w0r[i & 1] + x * w1r[i & 1];
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int e = 4 * (i & 3) + j;
-                    oacc[0][i >> 2][e] = BOUNDED ? oacc[0][i >> 2][e] + x[j] : oacc[0][i >> 2][e] * w0 + x[j] * w1;
-                }
-            }
+        for (int i = 0; i < NP; i++) {
+            const f32x4 x = *(lds_f32x4_t)(xo + other * (NP * 1024u) + (unsigned)(i * 1024));
+            const int r = PV16 ? i & 1 : 0;
+            own[i] = BOUNDED ? own[i] + x : own[i] * wo[r] + x * wx[r];
         }
+        asm volatile("" ::: "memory");
+        turn_lds = lds_address(Vs) + other * (NP * 1024u); // what it held has been read, by this wave alone
+    } else if constexpr (DMA) {
+#pragma unroll
+        for (int i = 0; i < NP; i++) own[i] = piece(i);
     }
 
     // ---- epilogue: O = O^T / l
-    if constexpr (PV16) {
-        // The denominator lives with the scores (lane = query l32); the lane that holds query
-        // 16 r + c16 of O^T fetches it from there.
+    if constexpr (DMA) {
+        // Prepared 16-bit operands: the wave turns its 32 rows (KG = 2: the half of their dims that is its own) through LDS and
+        // stores them as whole rows (halves): straight from the lanes they are pieces of 8 to 64 bytes, which the CU's address
+        // unit takes one by one. (f32: 24 heads, 1024 tokens in two parts 24.7 -> 24.2 us; 30 heads, 4224 tokens, f32 rows
+        // 267.5 -> 266.) The 16-byte chunk c of row r sits at c ^ (r & SWZ).
         const float l_tot = pair_sum(l_run[0]);
         const float inv_l = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-        float inv_r[2];
-#pragma unroll
-        for (int r = 0; r < 2; r++)
-            inv_r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + ec16), (int)__float_as_uint(inv_l)));
-        const bool part = splits > 1; // unnormalised rows, reference point and denominator of a part of the keys
-        if (part || a.out_dtype == kF32) {
-            // f32 rows leave as the 16-bit ones below do, through 16 KB of LDS of the wave's own (16-byte
-            // chunk c of row r at c ^ (r & 15)) as whole 512-byte rows, two per instruction: straight from
-            // the lanes they are 64-byte pieces, which the CU's address unit takes one by one. (24 heads, 1024
-            // tokens in two parts 24.7 -> 24.2 us; 30 heads, 4224 tokens, f32 rows 267.5 -> 266.)
-            if constexpr (KG == 1) __syncthreads(); // every wave is done with the ring
-            typedef __attribute__((address_space(3))) f32x4* lds_turn_t;
-            const unsigned turn = KG == 2 ? lds_address(Vs) + (unsigned)(gw * (64 * 64 * 4)) : lds_address(smem) + (unsigned)(wave * (QR * D * 4));
+        float inv_r[2] = {inv_l, inv_l};
+        if constexpr (PV16) {
+            // The denominator lives with the scores (lane = query l32); the lane that holds query
+            // 16 r + c16 of O^T fetches it from there.
 #pragma unroll
             for (int r = 0; r < 2; r++)
+                inv_r[r] = __uint_as_float((unsigned)__builtin_amdgcn_ds_bpermute(4 * (16 * r + ec16), (int)__float_as_uint(inv_l)));
+        }
+        const bool part = splits > 1; // unnormalised rows, reference point and denominator of a part of the keys
+        const int dim0 = KG == 2 ? (D / 2) * grp : 0;
+        // piece n: its row and its first dim, of this wave's
+        auto row_of = [&](int n) __attribute__((always_inline)) { return PV16 ? 16 * (n & 1) + ec16 : el32; };
+        if constexpr (KG == 1) __syncthreads(); // every wave is done with the ring
+        if (part || a.out_dtype == kF32) {
+            typedef __attribute__((address_space(3))) f32x4* lds_turn_t;
+            constexpr int CPR = D / KG / 4, RPI = 64 / CPR, SWZ = 15; // chunks of a row, rows an instruction
+            const unsigned turn = KG == 2 ? turn_lds : lds_address(smem) + (unsigned)(wave * (QR * D * 4));
 #pragma unroll
-                for (int dt = 0; dt < 8; dt++)
-                    *(lds_turn_t)(turn + (unsigned)((16 * r + ec16) * (D * 4) + (((4 * dt + eg4) ^ ec16) * 16))) = part ? oacc16[dt][r] : oacc16[dt][r] * inv_r[r];
+            for (int n = 0; n < NP; n++) {
+                const int row = row_of(n), c = PV16 ? 4 * (n >> 1) + eg4 : 8 * (n >> 2) + 2 * (n & 3) + eh;
+                *(lds_turn_t)(turn + (unsigned)(row * (CPR * 16) + ((c ^ (row & SWZ)) * 16))) = part ? own[n] : own[n] * inv_r[PV16 ? n & 1 : 0];
+            }
             const int64_t prow0 = (int64_t)blockIdx.x * BQ + gw * QR;
-            float* const base = part ? a.part_o + prow0 * D
-                                     : reinterpret_cast<float*>(a.o) + (int64_t)seg * a.o_bs + (int64_t)q0 * a.o_ts + (int64_t)head * a.o_hs;
+            float* const base = (part ? a.part_o + prow0 * D
+                                      : reinterpret_cast<float*>(a.o) + (int64_t)seg * a.o_bs + (int64_t)q0 * a.o_ts + (int64_t)head * a.o_hs) + dim0;
             const int64_t stride = part ? (int64_t)D : a.o_ts;
             const int rows = part ? QR : a.tokens - q0;
             // (uniform) the rounded rows that the product behind this launch reads
-            unsigned short* const row16 = part || !a.o16 ? nullptr : static_cast<unsigned short*>(a.o16) + (((int64_t)seg * a.tokens + q0) * a.heads + head) * D;
+            unsigned short* const row16 = part || !a.o16 ? nullptr : static_cast<unsigned short*>(a.o16) + (((int64_t)seg * a.tokens + q0) * a.heads + head) * D + dim0;
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int r = 2 * i + eh;
+            for (int i = 0; i < QR / RPI; i++) {
+                const int r = RPI * i + elane / CPR;
                 const f32x4 v = *(lds_turn_t)(turn + (unsigned)(i * 1024 + elane * 16));
                 if (r < rows) {
-                    const int d = (el32 ^ (r & 15)) * 4;
+                    const int d = ((elane % CPR) ^ (r & SWZ)) * 4;
                     store_through(base + r * stride + d, v);
                     if (row16) *reinterpret_cast<u32x2*>(row16 + (int64_t)r * (a.heads * D) + d) = round4(v, a.o16_dtype);
                 }
             }
-            if (part && eh == 0) {
+            if (part && eh == 0 && grp == 0) {
                 a.part_ml[(prow0 + el32) * 2] = BOUNDED ? 0.f : m_run[0];
                 a.part_ml[(prow0 + el32) * 2 + 1] = l_tot;
             }
         } else {
-            // 16-bit output: a lane holds 8-byte pieces of two rows, which would leave the chip as
-            // 16 thirty-two-byte segments per store instruction. The wave turns its 32 x 128 tile
-            // through 8 KB of LDS (its own stage of the idle K ring, K layout: chunk c of row r
-            // at c ^ (r & 15)) and stores whole 256-byte rows, four per instruction.
-            if constexpr (KG == 1) __syncthreads(); // every wave is done with the ring
             typedef __attribute__((address_space(3))) u32x2* lds_u32x2_t;
             typedef const __attribute__((address_space(3))) u32x4* lds_u32x4_t;
             typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-            const unsigned o_lds = lds_address(Ks) + (unsigned)(wave * (KSTAGE * 2));
-            const bool half = a.out_dtype == kF16;
+            constexpr int CPR = D / KG / 8, RPI = 64 / CPR, SWZ = CPR - 1;
+            const unsigned turn = KG == 2 ? turn_lds : lds_address(Ks) + (unsigned)(wave * (KSTAGE * 2));
+            u32x2 bits[NP];
+            // (one branch for all of them: left inside the loop it is two a piece)
+            if (a.out_dtype == kF16) {
 #pragma unroll
-            for (int r = 0; r < 2; r++)
+                for (int n = 0; n < NP; n++) bits[n] = __builtin_bit_cast(u32x2, __builtin_convertvector(own[n] * inv_r[PV16 ? n & 1 : 0], f16x4));
+            } else {
 #pragma unroll
-                for (int dt = 0; dt < 8; dt++) {
-                    // row 16 r + c16, dims 16 dt + 4 g4 .. + 3: chunk 2 dt + g4 / 2, half g4 % 2
-                    const f32x4 v = oacc16[dt][r] * inv_r[r];
-                    const u32x2 bits = half ? __builtin_bit_cast(u32x2, __builtin_convertvector(v, f16x4))
-                                            : __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
-                    *(lds_u32x2_t)(o_lds + (unsigned)((16 * r + ec16) * (D * 2) + (((2 * dt + (eg4 >> 1)) ^ ec16) * 16) + 8 * (eg4 & 1))) = bits;
-                }
-            unsigned short* const obase = reinterpret_cast<unsigned short*>(a.o) + (int64_t)seg * a.o_bs + (int64_t)head * a.o_hs;
+                for (int n = 0; n < NP; n++) bits[n] = __builtin_bit_cast(u32x2, __builtin_convertvector(own[n] * inv_r[PV16 ? n & 1 : 0], bf16x4));
+            }
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int r = 4 * j + (elane >> 4);
-                const u32x4 row16 = *(lds_u32x4_t)(o_lds + (unsigned)(r * (D * 2) + (elane & 15) * 16));
+            for (int n = 0; n < NP; n++) {
+                const int row = row_of(n), c = PV16 ? 2 * (n >> 1) + (eg4 >> 1) : n, half = PV16 ? eg4 & 1 : eh;
+                *(lds_u32x2_t)(turn + (unsigned)(row * (CPR * 16) + ((c ^ (row & SWZ)) * 16) + 8 * half)) = bits[n];
+            }
+            unsigned short* const obase = reinterpret_cast<unsigned short*>(a.o) + (int64_t)seg * a.o_bs + (int64_t)head * a.o_hs + dim0;
+#pragma unroll
+            for (int j = 0; j < QR / RPI; j++) {
+                const int r = RPI * j + elane / CPR;
+                const u32x4 row16 = *(lds_u32x4_t)(turn + (unsigned)(j * 1024 + elane * 16));
                 const int orow = q0 + r;
                 if (orow < a.tokens)
-                    store_through(obase + (int64_t)orow * a.o_ts + (((elane & 15) ^ (r & 15)) * 8), row16);
+                    store_through(obase + (int64_t)orow * a.o_ts + (((elane % CPR) ^ (r & SWZ)) * 8), row16);
             }
         }
     } else {
@@ -1285,10 +1302,6 @@ __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(co
 #pragma unroll
                             for (int j = 0; j < 4; j++) v[j] = oacc[qi][blk][4 * i + j] * inv_l;
                             *reinterpret_cast<f32x4*>(op + 32 * blk + 8 * i + 4 * eh) = v;
-                            if constexpr (DMA)
-                                if (a.o16)
-                                    *reinterpret_cast<u32x2*>(static_cast<unsigned short*>(a.o16) + (((int64_t)seg * a.tokens + qrow) * a.heads + head) * D +
-                                                              32 * blk + 8 * i + 4 * eh) = round4(v, a.o16_dtype);
                         }
                 }
             } else {
