@@ -123,3 +123,30 @@ LOAD = "buffer_load_dwordx4 v4, s[8:11], s5 offen lds"
 def test_the_check_of_scalar_registers_sees_early_reads(monkeypatch, asm, early):
     monkeypatch.setattr(build, "_device_asm", lambda *_: ["kern:"] + asm)
     assert bool(build.vmem_sgpr_hazards("")) == early
+
+
+@pytest.mark.skipif(not (os.path.exists("/opt/rocm/bin/hipcc") or shutil.which("hipcc")), reason="needs hipcc")
+@pytest.mark.parametrize("name", ["attn_fwd.hip", "attn_wide.hip", "gemm_half.hip", "qk_prepass.hip"])
+def test_nothing_writes_the_data_of_a_store_right_behind_it(name):
+    # attn_device.hpp, store_through: the compiler knows of no store in an assembly statement
+    bad = build.early_store_data_writes(os.path.join(build.CSRC, name))
+    assert not bad, "\n".join(bad[:20])
+
+
+STORE = "global_store_dwordx4 v[2:3], v[4:7], off sc1"
+
+
+@pytest.mark.parametrize("asm,early", [
+    ([STORE, "v_add_u32_e32 v4, 1, v0"], True),
+    ([STORE, "s_nop 0", "v_add_u32_e32 v7, 1, v0"], True),
+    ([STORE, "s_nop 1", "v_add_u32_e32 v7, 1, v0"], False),
+    ([STORE, "s_add_u32 s0, s0, 1", "v_pk_mul_f16 v5, v0, v1"], True),
+    ([STORE, "s_nop 0", "v_add_u32_e32 v2, 1, v4"], False),  # the address, and reads
+    ([STORE, "s_nop 0", ".LBB0_1:", "v_mov_b64_e32 v[6:7], v[0:1]"], True),
+    ([STORE, "v_permlane32_swap_b32_e32 v0, v6"], True),
+    (["buffer_store_dwordx4 v[4:7], v2, s[0:3], 0 offen", "v_mov_b32_e32 v4, 0"], True),
+    (["global_store_dwordx2 v[2:3], v[4:5], off sc1", "v_mov_b32_e32 v4, 0"], False),
+])
+def test_the_check_of_store_data_sees_early_writes(monkeypatch, asm, early):
+    monkeypatch.setattr(build, "_device_asm", lambda *_: ["kern:"] + asm)
+    assert bool(build.early_store_data_writes("")) == early

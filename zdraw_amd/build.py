@@ -288,6 +288,39 @@ def wide_mfma_hazards(extra_flags=()) -> list[str]:
     return bad
 
 
+def early_store_data_writes(src: str, extra_flags=()) -> list[str]:
+    """Compiles `src` to gfx950 assembly and lists every vector instruction that writes a data register of a store of
+    more than 8 bytes per lane fewer than two wait states behind it. The store may still be reading that register; the
+    compiler keeps the distance behind its own stores, not behind those that are assembly statements."""
+    import re
+    lines = [l.split(";")[0].strip() for l in _device_asm(src, extra_flags)]
+    lines = [l for l in lines if l and (not l.startswith(".") or l.endswith(":"))]
+    vectors = re.compile(r"\bv(?:(\d+)|\[(\d+):(\d+)\])")
+
+    def registers(text):
+        return {r for one, lo, hi in vectors.findall(text) for r in (range(int(one), int(one) + 1) if one else range(int(lo), int(hi) + 1))}
+
+    bad, kernel = [], ""
+    for i, text in enumerate(lines):
+        if text.endswith(":") and not text.startswith("."):
+            kernel = text[:-1]
+        store = re.match(r"^(global|flat|scratch|buffer)_store_dwordx[34]\s+(.*)", text)
+        if not store:
+            continue
+        data, states = registers(store.group(2).split(",")[0 if store.group(1) == "buffer" else 1]), 0
+        for later in lines[i + 1:i + 4]:
+            if states >= 2:
+                break
+            # (an exchange of registers writes both of its operands)
+            ops = later.split(",")
+            if later.startswith("v_") and data & registers(",".join(ops[:2]) if "swap" in ops[0] else ops[0]):
+                bad.append(f"{kernel}: {text} | {states} wait states | {later}")
+                break
+            nop = re.match(r"^s_nop\s+(\d+)", later)
+            states += int(nop.group(1)) + 1 if nop else 0 if later.endswith(":") else 1
+    return bad
+
+
 def build_host(verbose: bool = False) -> str:
     os.makedirs(LIBDIR, exist_ok=True)
     srcs = [os.path.join(HOST, f) for f in sorted(os.listdir(HOST)) if f.endswith(".cc")]
@@ -308,11 +341,11 @@ def check_hand_scheduled_kernels(verbose: bool = False):
         list(pool.map(_device_asm, files))
     bad = m0_writes() + m0_writes(files[1], "attn_wide_kernel") + tied_mfma_hazards() + wide_mfma_hazards()
     for f in files:
-        bad += vmem_sgpr_hazards(f) + kernarg_overreads(f) + early_mfma_result_uses(f)
+        bad += vmem_sgpr_hazards(f) + early_store_data_writes(f) + kernarg_overreads(f) + early_mfma_result_uses(f)
     if bad:
         raise RuntimeError("a kernel compiled to code that breaks its hand-written schedule:\n  " + "\n  ".join(bad))
     if verbose:
-        print("hand-scheduled kernels: no foreign M0 write, no accumulator touched inside an MFMA run, no load on a scalar register just written, no read past a kernel's arguments, no MFMA result used early")
+        print("hand-scheduled kernels: no foreign M0 write, no accumulator touched inside an MFMA run, no load on a scalar register just written, no write of a store's data right behind it, no read past a kernel's arguments, no MFMA result used early")
 
 
 def build_all(verbose: bool = False):

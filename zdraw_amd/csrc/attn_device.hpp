@@ -106,13 +106,14 @@ __device__ __forceinline__ void load_to_lds_16_at(u32x4 rsrc, unsigned thread_of
 // in the eight L2s is written back when its last wave has ended, and the next launch waits for that: a pre-pass of 24
 // heads, 768 tokens ended 4.6 us before the attention kernel's first wave, now 3.2. For rows that leave as whole cache
 // lines from a launch another one follows; partial lines, and what a kernel itself reads again, stay with ordinary stores.
-// (The wait state keeps a vector instruction from writing the data registers right behind the store; the compiler
-// does not know that there is one.)
+// (The two wait states keep a vector instruction from writing the data registers while the store of 16 bytes still
+// reads them: the compiler, which keeps them behind a store of its own, does not know that there is one.
+// zdraw_amd.build.early_store_data_writes holds the compiled code to it. 8 bytes are read at once.)
 template <typename V>
 __device__ __forceinline__ void store_through(void* p, const V& v) {
     static_assert(sizeof(V) == 16 || sizeof(V) == 8, "two or four registers");
-    if constexpr (sizeof(V) == 16) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" : : "v"(p), "v"(v) : "memory");
-    else asm volatile("global_store_dwordx2 %0, %1, off sc1\n\ts_nop 0" : : "v"(p), "v"(v) : "memory");
+    if constexpr (sizeof(V) == 16) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
+    else asm volatile("global_store_dwordx2 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
 }
 
 __device__ __forceinline__ void unpack8(const Raw8<float>& r, float (&x)[8]) {

@@ -100,6 +100,18 @@ __device__ __forceinline__ u32x2 round4(const f32x4& v, int dtype) {
                          : __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
 }
 
+// The lane's number formed anew where it is needed once in a while. What is formed from it stays in registers across
+// the key loop otherwise: 228 to 256 of them and spills in the builds of prepared operands, 211 to 238 without, with the
+// wave's number in a scalar register. The masked running-maximum build so has room for the 16 x 16 product, and shorter
+// prologues pay where a launch is a few key blocks per wave: 24 heads, five blocks of 768 tokens 134.6 -> 130.5 us, of 1088
+// 181.1 -> 175.7; f32 rows of 24 heads, 4001 tokens 239.9 -> 235.5, 3000 tokens of which 2500 are keys 151.1 -> 147.7.
+// (The tail block's row offsets stay: formed again in a branch they cost 2 x 8704 tokens 0.5 %.)
+__device__ __forceinline__ int lane_again() {
+    int x;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
+    return x;
+}
+
 // QB = 32-query blocks per wave, NW = waves per workgroup. Built shapes:
 //   QB=1, NW=8: two waves per SIMD, 256 registers each (default);
 //   QB=1, NW=4: two workgroups per CU, each with its own LDS ring.
@@ -124,18 +136,6 @@ __device__ __forceinline__ u32x2 round4(const f32x4& v, int dtype) {
 // waves, each over half of the keys, merged in LDS at the end: half the steps per workgroup and
 // twice the workgroups, for launches that leave CUs idle (launch_attention, shape 2). Every group
 // has a four-stage ring of its own and all of the schedule below; a step ends in a barrier.
-// The lane's number formed anew where it is needed once in a while. What is formed from it stays in registers across
-// the key loop otherwise: 228 to 256 of them and spills in the builds of prepared operands, 211 to 238 without, with the
-// wave's number in a scalar register. The masked running-maximum build so has room for the 16 x 16 product, and shorter
-// prologues pay where a launch is a few key blocks per wave: 24 heads, five blocks of 768 tokens 134.6 -> 130.5 us, of 1088
-// 181.1 -> 175.7; f32 rows of 24 heads, 4001 tokens 239.9 -> 235.5, 3000 tokens of which 2500 are keys 151.1 -> 147.7.
-// (The tail block's row offsets stay: formed again in a branch they cost 2 x 8704 tokens 0.5 %.)
-__device__ __forceinline__ int lane_again() {
-    int x;
-    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
-    return x;
-}
-
 template <typename TIn, int KMODE, bool MASKED, bool BOUNDED, int QB, int NW, bool SF16 = false, int KG = 1>
 __global__ void __launch_bounds__(NW * 64, (QB == 2 ? 1 : 2)) attn_fwd_kernel(const AttnArgs a) {
     constexpr int NT = NW * 64;
