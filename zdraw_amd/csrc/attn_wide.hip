@@ -87,7 +87,9 @@ __global__ void __launch_bounds__(256) wide_round_kernel(const WidePrepArgs p) {
         const f32x4 b = *reinterpret_cast<const f32x4*>(src + 8 * i + 4);
         const float x[8] = {a[0] * scale, a[1] * scale, a[2] * scale, a[3] * scale,
                             b[0] * scale, b[1] * scale, b[2] * scale, b[3] * scale};
-        *reinterpret_cast<u32x4*>(dst + 8 * i) = pack_bf16x8(x);
+        // (through the L2: the attention launch starts 0.8 us sooner behind this one, calls of 6208 tokens 111.8 -> 110.9 us,
+        // of 16384 430.4 -> 429.6)
+        store_through(dst + 8 * i, pack_bf16x8(x));
     }
 }
 
