@@ -98,6 +98,16 @@ def test_wide_head_uneven_key_ranges_sampled_rows_and_rerun(ctx, tokens):
     assert (np.abs(got).max(axis=(1, 2)) > 0).all()
 
 
+# Lengths whose number of ranges rests on how the estimate rises with the fill of a round: six ranges with a last one of
+# four blocks, seven with one of four, eight of ten each, four that nearly fill a round, five over two rounds and a half.
+@pytest.mark.parametrize("tokens,want", [(1408, 6), (1600, 7), (2560, 8), (7424, 4), (16640, 5)])
+def test_wide_head_ranges_by_the_fill_of_a_round(ctx, tokens, want):
+    n, share = C.c_uint32(0), C.c_uint64(0)
+    hip.lib().zdraw_hip_wide_ranges(tokens, 256, C.byref(n), C.byref(share))
+    assert n.value == want
+    test_wide_head_uneven_key_ranges_sampled_rows_and_rerun(ctx, tokens)
+
+
 def test_wide_head_reference_case_sampled_rows_and_rerun(ctx):
     # metal/mattn_test.zig:138-230
     tokens = 6208

@@ -782,21 +782,24 @@ size_t wide_part_bytes(int tokens, int splits) {
 }
 // Key ranges per query tile (one workgroup each, of equal length but for the last, at least eight
 // blocks): the number whose estimate is the smallest. A full round over the CUs takes kFullUs per
-// block of a range (the power limit), a thinly filled one kThinUs (a wave's own chain), in between
+// block of a range (the power limit), one that fills up to kThinFill of them kThinUs (a wave's own chain), in between
 // in proportion; every range's share of O goes to memory and back once. The constants are a fit to
-// 1 to 8 ranges of 256 to 18432 tokens; the rule's pick is the measured best or within 4 % of it
-// (with the 32 x 32 x 16 form of the kernel; with this one within 3 %, but at 2560 tokens 58.7 us with five for 55.5 with eight
-// and at 8192 157.3 with three for 151.5 with four; constants that take those put 7104 tokens at three instead of four: at 7168 142 for 129), so
+// 1 to 8 ranges of 37 lengths from 256 to 18432 tokens, every number of ranges timed: the pick is the best or within 4 % of it, 0.6 %
+// in the mean (but at 1280 tokens: 48.9 us with five for 45.8 with four; a rule that rose in proportion to the fill from the
+// start took the widest split too late: us per call 1408 tokens 53.2 -> 47.5, 2560 57.0 -> 54.6,
+// 5248 93.9 -> 90.5, 7424 141.7 -> 131.6, 8192 157.2 -> 150.4, 21248 850.3 -> 730.1; of 49 lengths up to 35072 that the new
+// constants moved, none slower). 6208 tokens stay at four, 110.9 for 107.6 with five, whose shares take a quarter more. Estimates
+// leave out a call's other 25 us, so
 // ranges that save less than 3 % are not worth their shares (1019904 tokens would take six ranges and 12 GB
 // for 1.5 %), and neither are shares of more than kMaxShareBytes, which the queue keeps (33024 tokens: six
 // ranges, 389 MB, a quarter of the time by the estimate; 18432: three, 108 MB, 11 %).
-// (A power of two that divides the blocks, which this was before, left 6208 tokens, 194 blocks, at
+// (A power of two that divides the blocks, which this was at first, left 6208 tokens, 194 blocks, at
 // two ranges and 98 workgroups: call 152 us against 119 with four; 18432 tokens at one range:
 // 678 against 610 with three.)
 int wide_splits(int tokens, int cus) {
     constexpr size_t kMaxShareBytes = (size_t)512 << 20;
     constexpr float kMinGain = 0.03f;
-    constexpr float kFullUs = 1.6f, kThinUs = 1.16f, kRoundUs = 4.0f, kMergeUs = 3.0f, kShareBytesPerUs = 2.0e6f;
+    constexpr float kFullUs = 1.55f, kThinUs = 1.13f, kThinFill = 0.66f, kRoundUs = 5.5f, kMergeUs = 4.0f, kShareBytesPerUs = 3.3e6f;
     if (cus <= 0) return 1;
     const int tiles = (tokens + wide::BQ - 1) / wide::BQ;
     const int nblk = tokens / wide::KB;
@@ -808,7 +811,8 @@ int wide_splits(int tokens, int cus) {
         if (s > 1 && (per < 8 || (s - 1) * per >= nblk)) continue; // (no empty range)
         const int rounds = tiles * s / cus, last = tiles * s % cus;
         float us = (float)rounds * ((float)per * kFullUs + kRoundUs);
-        if (last) us += (float)per * fmaxf(kThinUs, kFullUs * (float)last / (float)cus) + kRoundUs;
+        const float past = fmaxf((float)last / (float)cus - kThinFill, 0.f) / (1.f - kThinFill);
+        if (last) us += (float)per * (kThinUs + (kFullUs - kThinUs) * past) + kRoundUs;
         if (s > 1) us += kMergeUs + (float)s * (float)tokens * (float)(wide::WD * sizeof(float)) / kShareBytesPerUs;
         if (s == 1) whole_us = us;
         if (us < best_us) { best_us = us; best = s; }
