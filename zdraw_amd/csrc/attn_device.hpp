@@ -104,8 +104,9 @@ __device__ __forceinline__ void load_to_lds_16_at(u32x4 rsrc, unsigned thread_of
 
 // A store of 8 or 16 bytes per lane that goes through the L2 to memory at once (device scope). What a kernel leaves dirty
 // in the eight L2s is written back when its last wave has ended, and the next launch waits for that: a pre-pass of 24
-// heads, 768 tokens ended 4.6 us before the attention kernel's first wave, now 3.2. For rows that leave as whole cache
-// lines from a launch another one follows; partial lines, and what a kernel itself reads again, stay with ordinary stores.
+// heads, 768 tokens ended 4.6 us before the attention kernel's first wave, now 3.2. For rows of whole cache lines, and f32
+// rows of any length, from a launch another one follows; 16-bit rows that lines do not divide (store_rows_lds, gemm_half.hip,
+// has both measured), the single elements at a row's end, and what a kernel itself reads again stay with ordinary stores.
 // (The two wait states keep a vector instruction from writing the data registers while the store of 16 bytes still
 // reads them: the compiler, which keeps them behind a store of its own, does not know that there is one.
 // zdraw_amd.build.early_store_data_writes holds the compiled code to it. 8 bytes are read at once.)

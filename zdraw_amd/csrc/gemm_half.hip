@@ -196,7 +196,7 @@ __device__ __forceinline__ void store_tile_lds32(const GemmArgs& g, void* c, con
 // CU's address unit takes one by one: a 256 x 160 tile of bf16 took 6 us that way.)
 template <typename TC, int TJ>
 constexpr int rows_wave_bytes() { return 32 * (16 * TJ * (int)sizeof(TC) + 16); }
-template <bool F16, typename TC, int TI, int TJ>
+template <bool F16, typename TC, int TI, int TJ, bool RAG>
 __device__ __forceinline__ void store_rows_lds(const GemmArgs& g, void* c, const f32x4 (&acc)[TI][TJ], unsigned lds_wave, int row0, int col0, int lane) {
     constexpr int ES = (int)sizeof(TC);
     constexpr int PITCH = 16 * TJ * ES + 16; // bytes per staged row
@@ -207,8 +207,13 @@ __device__ __forceinline__ void store_rows_lds(const GemmArgs& g, void* c, const
     // round end together, and their rows are then in memory when the last wave ends. Calls, us: q/k/v and output
     // products of 1024 and 512 f32 rows, hidden 3072, 180.6 -> 175.9; a segment of 1632 tokens, 30 heads, f32, two layers
     // 524.6 -> 517.1; 643 tokens 255.4 -> 249.9. Smaller tiles carry so little that the stores' own way shows: 139 and 108
-    // rows of bf16 96.0 -> 96.5.
-    constexpr bool THROUGH = TI * TJ >= 12;
+    // rows of bf16 96.0 -> 96.5. (A wave's part of a row need not be whole cache lines for that, it is 160 or 320 bytes in
+    // the 160-column tiles: segments of bf16 C, 30 heads, two layers, 1536 tokens 450.7 -> 444.8, 672 tokens 232.7 -> 229.0.)
+    // 16-bit rows of a length that lines do not divide lose: hidden 2568, through -> ordinary, 1675 and 512 rows 223.9 -> 220.8,
+    // 315 and 512 140.8 -> 139.4; f32 rows of that width gain, 2023 and 512 rows 283.2 -> 281.5. Such a C belongs to a
+    // product of as ragged a k, and that is what tells: a test of the address, with both stores behind it, costs the others
+    // up to 0.9 %.
+    constexpr bool THROUGH = TI * TJ >= 12 && (ES == 4 || !RAG);
     typedef __attribute__((address_space(3))) u32x2* lds_u32x2_t;
     typedef __attribute__((address_space(3))) f32x4* lds_f32x4_t;
     typedef const __attribute__((address_space(3))) u32x4* lds_u32x4_t;
@@ -795,7 +800,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pipe_kernel(const GemmArgs g) {
     __builtin_amdgcn_s_waitcnt(0x0F70); // this wave's direct loads (re-fetches past the end) have landed
     __syncthreads();                    // and everybody's: the stages are idle
     static_assert(4 * rows_wave_bytes<TC, TJ>() <= ST * STAGE, "the epilogue's rows fit the stages");
-    store_rows_lds<F16, TC, TI, TJ>(g, cp, acc, lds0 + (unsigned)(wave * rows_wave_bytes<TC, TJ>()), m0 + wm * (16 * TI), n0 + wn * (16 * TJ), lane);
+    store_rows_lds<F16, TC, TI, TJ, RAG>(g, cp, acc, lds0 + (unsigned)(wave * rows_wave_bytes<TC, TJ>()), m0 + wm * (16 * TI), n0 + wn * (16 * TJ), lane);
 }
 
 // Adds the parts of the k-split tiles in part order and writes C. A workgroup takes the 32 x
