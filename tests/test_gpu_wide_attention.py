@@ -99,7 +99,7 @@ def test_wide_head_uneven_key_ranges_sampled_rows_and_rerun(ctx, tokens):
 
 
 # Lengths whose number of ranges rests on how the estimate rises with the fill of a round: six ranges with a last one of
-# four blocks, seven with one of four, eight of ten each, four that nearly fill a round, five over two rounds and a half.
+# four blocks, seven with one of two, eight of ten each, four that nearly fill a round, five over two rounds and a half.
 @pytest.mark.parametrize("tokens,want", [(1408, 6), (1600, 7), (2560, 8), (7424, 4), (16640, 5)])
 def test_wide_head_ranges_by_the_fill_of_a_round(ctx, tokens, want):
     n, share = C.c_uint32(0), C.c_uint64(0)
@@ -165,12 +165,12 @@ def test_wide_head_sharp_softmax_and_large_scores(ctx):
         assert np.abs(want[i, 0] - v[j, 0]).max() < 1e-3  # the planted key really takes the whole row
 
 
-def test_wide_head_reference_point_moves_several_times(ctx):
+def test_wide_head_rows_overtaken_several_times_within_reach(ctx):
     # 1152 tokens (nine query tiles, 36 key blocks): rows whose best key so far is overtaken
-    # three times, 8 to 11 in the score each time, so the accumulated O is rescaled in place
-    # with earlier contributions still in it (each planted key keeps e^-8 .. e^-11 of the
-    # weight of the next); rows in every wave of a tile and in both halves of the output dims
-    # are checked against the oracle like all others.
+    # three times, 8 to 11 in the score each time (each planted key keeps e^-8 .. e^-11 of the
+    # weight of the next): within reach of the reference point, the first block's maximum, which
+    # stays where it is while the P of these keys grow to 2^40; rows in every wave of a tile and
+    # in both halves of the output dims are checked against the oracle like all others.
     tokens = 1152
     rng = np.random.default_rng(78)
     q, k, v = draw(rng, tokens)
@@ -181,16 +181,16 @@ def test_wide_head_reference_point_moves_several_times(ctx):
             k[j, 0] = level * unit
     got = ctx.run(q, k, v, host.Config(tokens, 1, 1, 512)).reshape(tokens, 1, 512)
     want = zo.attention_run(q, k, v, zo.Config(tokens, 1, 1, 512))
-    refimpl.check_close(got, want, "several moves of the reference point")
+    refimpl.check_close(got, want, "rows overtaken several times")
     for n, i in enumerate(rows):
         assert np.abs(want[i, 0] - v[1100 + n, 0]).max() < 1e-2  # the last planted key takes the row
 
 
-def test_wide_head_scores_that_outgrow_the_fixed_reference_take_the_safe_kernel(ctx):
-    # The fast kernel exponentiates every score of a row against the largest score of the first
-    # block of its key range and flags a query tile whose row sums show a score more than 2^90
-    # above that; flagged tiles are formed again by the running-maximum kernel that follows every
-    # launch. Ordinary data flags nothing; a key 75 nats (108 in log2) above a field of N(0, 1)
+def test_wide_head_scores_that_outgrow_the_fixed_reference_are_formed_again(ctx):
+    # The kernel exponentiates every score of a row against the largest score of the first
+    # block of its key range; a workgroup whose row sums show a score more than 2^90 above that
+    # flags its query tile and forms its rows of that range again with a running maximum.
+    # Ordinary data flags nothing; a key 75 nats (108 in log2) above a field of N(0, 1)
     # scores, late in a range, flags its tile and only that one, and the rows still match.
     L = hip.lib()
     tokens = 1024
@@ -216,6 +216,53 @@ def test_wide_head_scores_that_outgrow_the_fixed_reference_take_the_safe_kernel(
     refimpl.check_close(got[others], want[others], "rows beside the planted ones")
     for i, j in ((300, 900), (301, 901), (900, 1000)):
         assert np.abs(got[i, 0] - v[j, 0]).max() < 2e-2
+    again = ctx.run(q, k, v, cfg).reshape(tokens, 1, 512)
+    assert got.tobytes() == again.tobytes()
+
+
+def rounded_reference(q, k, v):
+    """Attention of one wide head in float64 on the operands the kernel multiplies: bf16, Q with its scale (exp2 domain)."""
+    def bf16(x):
+        return host.bf16_bits_to_f32(host.f32_to_bf16_bits(x)).reshape(x.shape)[:, 0].astype(np.float64)
+    s = bf16(q * np.float32(np.log2(np.e) / np.sqrt(512.0))) @ bf16(k).T
+    p = np.exp2(s - s.max(axis=1, keepdims=True))
+    p /= p.sum(axis=1, keepdims=True)
+    return p, (p @ bf16(v))[:, None]
+
+
+# Rows formed again with a running maximum, over key ranges of any number of blocks: the loop there takes three
+# blocks a trip, so 10, 7 and 4 blocks leave one over, 2 and 8 two, 9 none; ranges that end short (7, 4, 2); a row of a half-full last
+# tile (its other waves have no row). Each row climbs twice: its first block is ordinary, a run of keys lies 108 (log2) above, which the
+# fixed reference point cannot reach, and the last key another 9.5 above those, so that what has been summed is scaled by 2^-9.5
+# once it counts: the run keeps a share of the row that shows, in the sum and in O. Operands rounded as the kernel rounds them:
+# what is left is P and V in bf16, 2^-8 of the largest |V| (4.2) in all.
+@pytest.mark.parametrize("tokens,part,blocks", [(64, 0, 2), (128, 0, 4), (256, 0, 8), (576, 1, 9), (640, 0, 10), (640, 1, 10), (1088, 3, 7), (1408, 5, 4), (1600, 6, 2)])
+def test_wide_head_rows_formed_again_climb_twice(ctx, tokens, part, blocks):
+    L = hip.lib()
+    n, share = C.c_uint32(0), C.c_uint64(0)
+    L.zdraw_hip_wide_ranges(tokens, 256, C.byref(n), C.byref(share))
+    per = -(-(tokens // 32) // n.value)
+    first = part * per
+    assert part < n.value and min(per, tokens // 32 - first) == blocks, (n.value, per)
+    rng = np.random.default_rng(80 + tokens + part)
+    q, k, v = draw(rng, tokens)
+    rows = (5, tokens - 1)
+    last = 32 * (first + blocks) - 1
+    run = {}
+    for r, i in enumerate(rows):
+        unit = q[i, 0] / np.linalg.norm(q[i, 0])
+        per_bit = np.sqrt(512.0) / np.linalg.norm(q[i, 0]) / np.log2(np.e)  # |k| per unit of score (log2)
+        run[i] = np.arange(32 * (first + 1) + r, last - 1, 2)  # every other key between the first block and the last two keys
+        k[run[i], 0] = (108.0 * per_bit) * unit
+        v[run[i], 0] = rng.standard_normal(512, dtype=np.float32)  # (one vector: their share is not averaged away)
+        k[last - r, 0] = (117.5 * per_bit) * unit
+    weight, want = rounded_reference(q, k, v)
+    cfg = host.Config(tokens, 1, 1, 512)
+    got = ctx.run(q, k, v, cfg).reshape(tokens, 1, 512)
+    assert L.zdraw_hip_wide_redo_tiles() == len({i // 128 for i in rows})
+    refimpl.check_close(got, want, f"{tokens} tokens, a range of {blocks} blocks formed again")
+    for r, i in enumerate(rows):
+        assert 0.015 < weight[i, run[i]].sum() < 0.5 and weight[i, last - r] > 0.5
     again = ctx.run(q, k, v, cfg).reshape(tokens, 1, 512)
     assert got.tobytes() == again.tobytes()
 
