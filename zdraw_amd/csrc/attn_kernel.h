@@ -140,6 +140,7 @@ struct WideArgs {
     float* part_ml; // f32 [splits][tokens][2]: its reference point and row sum
     int* redo;      // [wide_tiles(tokens)]: set by the kernel for a query tile (128 rows) whose scores outgrew the
                     // fixed reference point; the workgroup then forms its rows again with a running maximum
+    int32_t halves; // 1: two workgroups per tile and range, each for one half of the output dims (wide_halves); 0: one
 };
 // f32 -> bf16 rounding of the three operands (Q with its scale) in one launch.
 struct WidePrepArgs {
@@ -155,6 +156,7 @@ int wide_block_rows();
 // Key ranges per query tile that fill a device of `cus` compute units (1: no split), and the
 // bytes of part_o followed by part_ml they need.
 int wide_splits(int tokens, int cus);
+int wide_halves(int tokens, int splits, int cus);
 int wide_tiles(int tokens); // query tiles (128 rows) = entries of WideArgs::redo
 size_t wide_part_bytes(int tokens, int splits);
 hipError_t launch_wide_round(const WidePrepArgs& args, hipStream_t stream);

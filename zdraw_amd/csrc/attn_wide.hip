@@ -155,8 +155,9 @@ __device__ __forceinline__ void acc_drain() {
 // LDS slots each. It runs behind the kernel's own epilogue, by the workgroup that found the row sum, where nothing of the
 // fast path is live any more: a kernel of its own behind every call, which this was, costs ordinary data its launch.
 // Calls, us, as a launch of its own -> here: 256 tokens 38.5 -> 37.2, 1024 43.7 -> 42.4, 2560 59.0 -> 57.7, 6208 111.3 -> 109.9,
-// 16384 438.1 -> 435.6. With every row formed again: 256 60 -> 77 (one workgroup takes both halves), 1024 88 -> 83, 6208
-// 330 -> 252, 16384 1224 -> 1134 (a launch of its own went over all keys, this over the range that needs it).
+// 16384 438.1 -> 435.6. With every row formed again: 256 59.6 -> 57.9, 512 68.9 -> 60.0, 1024 89 -> 65 (two workgroups take
+// a half each, wide_halves), 6208 330 -> 252, 16384 1224 -> 1134 (a launch of its own went over all keys, this over the range that
+// needs it; where the keys are one range of a full chip, 32768 tokens, a lone such tile takes twice as long).
 namespace safe {
 constexpr int HALF = WD / 2;      // output dims per workgroup
 constexpr int V_SLOT = (NSL / 2) * TILE_BYTES; // half the dims of a V block: 16 KB
@@ -403,11 +404,13 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
     const int g4 = lane >> 4;
     // workgroup = (key range, query tile), range-major, and each XCD takes one contiguous run of
     // that order (workgroups go to the XCDs in turn): the workgroups behind one L2 walk the same
-    // range, so a K/V block comes in once per XCD, not once per range as well.
+    // range, so a K/V block comes in once per XCD, not once per range as well. With a.halves, two workgroups in a row form
+    // the same and each stores, and where need be forms again, one half of the output dims (wide_halves).
     const int nsp = a.splits > 1 ? a.splits : 1;
-    const int tiles = (int)gridDim.x / nsp;
+    const int tiles = ((int)gridDim.x >> a.halves) / nsp;
     const int xcd = (int)blockIdx.x & 7, xrem = (int)gridDim.x & 7;
-    const int logical = ((int)blockIdx.x >> 3) + xcd * ((int)gridDim.x >> 3) + min(xcd, xrem);
+    const int wg = ((int)blockIdx.x >> 3) + xcd * ((int)gridDim.x >> 3) + min(xcd, xrem);
+    const int logical = wg >> a.halves;
     // (uniform, but the divisions run on the vector unit)
     const int part = __builtin_amdgcn_readfirstlane(logical / tiles);
     const int tile = logical - part * tiles;
@@ -710,6 +713,9 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
         const int row0 = tile * BQ + 32 * w + 16 * (o & 1);
         if (row0 >= a.tokens) continue; // (whole groups of 16 rows: tokens % 64 == 0)
         const f32x2 ml = *(lds_f32x2_t)(lds_base + (P_RING + (w * 32 + 16 * (o & 1) + ec) * 8));
+        // (one workgroup of two writes them, the one that would write them again)
+        if (nsp > 1 && o < 2 && eg == 0 && (wg & a.halves) == 0) *reinterpret_cast<f32x2*>(a.part_ml + ((int64_t)part * a.tokens + row0 + ec) * 2) = ml;
+        if (a.halves && dh != (wg & 1)) continue;
         const float scale = nsp > 1 ? 1.0f : ml[1] > 0.f ? 1.0f / ml[1] : 0.f;
 #pragma unroll
         for (int dt = 0; dt < 16; dt++) *(lds_f32x4_t)(turn + ec * 1024 + (((4 * dt + eg) ^ ec) * 16)) = oacc[dt][o] * scale;
@@ -717,7 +723,6 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
 #pragma unroll
         for (int r = 0; r < 16; r++)
             store_through(op + (int64_t)r * WD + ((el ^ r) * 4), (f32x4)*(lds_f32x4_t)(turn + r * 1024 + el * 16));
-        if (nsp > 1 && o < 2 && eg == 0) *reinterpret_cast<f32x2*>(a.part_ml + ((int64_t)part * a.tokens + row0 + ec) * 2) = ml;
     }
     // what any wave of the workgroup found, read by all of them (nothing has been written there since the barrier)
     int again = 0;
@@ -725,7 +730,7 @@ __global__ void __launch_bounds__(NT, 1) attn_wide_kernel(const WideArgs a) {
     for (int w = 0; w < NW; w++) again |= *(lds_int_t)(lds_base + (P_RING + BQ * 8 + w * 4));
     if (__builtin_amdgcn_readfirstlane(again) == 0) return;
     __builtin_amdgcn_s_waitcnt(0x0F70); // the rows above are in memory before they are written again
-    for (int half = 0; half < 2; half++) {
+    for (int half = wg & a.halves; half < 2; half += 1 + a.halves) {
         __syncthreads(); // and nobody reads what is in the LDS
         int dh2 = half;
         asm volatile("" : "+s"(dh2)); // (nothing of a half is to be kept for the other)
@@ -819,6 +824,16 @@ int wide_splits(int tokens, int cus) {
     }
     return best_us < whole_us * (1.f - kMinGain) ? best : 1;
 }
+// Whether two workgroups take each tile and range, each for one half of the output dims: where both together fill
+// no more than half of the CUs. Rows that are formed again are formed once per half, which one workgroup does in turn; two at
+// once lose nothing meanwhile, and each has half of the rows to store. us per call, one -> two, every row formed again: 64
+// tokens 53.4 -> 42.0, 256 77.1 -> 57.9, 512 79.5 -> 60.0, 1152 (45 workgroups) 86.4 -> 67.4; ordinary data 256 38.2 -> 38.2, 512
+// 40.8 -> 40.3, 960 43.0 -> 42.1, 1152 47.3 -> 46.8. Past the line both read K and V too often: ordinary 1664 tokens (91) 46.1 -> 46.4,
+// 2048 (128) 48.3 -> 49.3, 2560 (160) 53 -> 73.
+int wide_halves(int tokens, int splits, int cus) {
+    const int64_t wgs = (int64_t)wide_tiles(tokens) * (splits > 1 ? splits : 1);
+    return 4 * wgs <= cus ? 1 : 0;
+}
 
 hipError_t launch_wide_attention(const WideArgs& a, hipStream_t stream) {
     if (a.tokens <= 0 || a.tokens % wide_block_rows() != 0) return hipErrorInvalidValue;
@@ -827,8 +842,8 @@ hipError_t launch_wide_attention(const WideArgs& a, hipStream_t stream) {
     if (nsp > wide::kMaxSplits || (nsp - 1) * ((nblk + nsp - 1) / nsp) >= nblk) return hipErrorInvalidValue; // every range has a block
     if (nsp > 1 && (a.part_o == nullptr || a.part_ml == nullptr)) return hipErrorInvalidValue;
     const unsigned tiles = (unsigned)((a.tokens + wide::BQ - 1) / wide::BQ);
-    if (a.redo == nullptr) return hipErrorInvalidValue;
-    wide::attn_wide_kernel<<<dim3(tiles * (unsigned)nsp), dim3(wide::NT), wide::kLdsBytes, stream>>>(a);
+    if (a.redo == nullptr || (a.halves != 0 && a.halves != 1)) return hipErrorInvalidValue;
+    wide::attn_wide_kernel<<<dim3((tiles * (unsigned)nsp) << a.halves), dim3(wide::NT), wide::kLdsBytes, stream>>>(a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (nsp > 1) {

@@ -924,6 +924,7 @@ int enqueue_wide(Queue* queue, void* q, void* k, void* v, void* out, const Zdraw
             a.part_ml = a.part_o + (size_t)a.splits * (size_t)a.tokens * (size_t)wide_head_dim();
         }
     }
+    a.halves = wide_halves(a.tokens, a.splits, queue->dev->cus);
     TracePair tp{nullptr, nullptr};
     if (g_trace && hipEventCreate(&tp.a) == hipSuccess && hipEventCreate(&tp.b) == hipSuccess)
         (void)hipEventRecord(tp.a, stream);
