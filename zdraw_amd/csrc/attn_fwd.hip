@@ -101,7 +101,7 @@ __device__ __forceinline__ u32x2 round4(const f32x4& v, int dtype) {
 }
 
 // The lane's number formed anew where it is needed once in a while. What is formed from it stays in registers across
-// the key loop otherwise: 228 to 256 of them and spills in the builds of prepared operands, 211 to 238 without, with the
+// the key loop otherwise: 228 to 256 of them in the eight-wave builds of prepared operands, 208 to 234 without, with the
 // wave's number in a scalar register. The masked running-maximum build so has room for the 16 x 16 product, and shorter
 // prologues pay where a launch is a few key blocks per wave: 24 heads, five blocks of 768 tokens 134.6 -> 130.5 us, of 1088
 // 181.1 -> 175.7; f32 rows of 24 heads, 4001 tokens 239.9 -> 235.5, 3000 tokens of which 2500 are keys 151.1 -> 147.7.

@@ -157,7 +157,7 @@ __device__ __forceinline__ void acc_drain() {
 // Calls, us, as a launch of its own -> here: 256 tokens 38.5 -> 37.2, 1024 43.7 -> 42.4, 2560 59.0 -> 57.7, 6208 111.3 -> 109.9,
 // 16384 438.1 -> 435.6. With every row formed again: 256 59.6 -> 57.9, 512 68.9 -> 60.0, 1024 89 -> 65 (two workgroups take
 // a half each, wide_halves), 6208 330 -> 252, 16384 1224 -> 1134 (a launch of its own went over all keys, this over the range that
-// needs it; where the keys are one range of a full chip, 32768 tokens, a lone such tile takes twice as long).
+// needs it; where the keys are one range and the tiles more than 64, as with 32768 tokens, a lone such tile takes twice as long).
 namespace safe {
 constexpr int HALF = WD / 2;      // output dims per workgroup
 constexpr int V_SLOT = (NSL / 2) * TILE_BYTES; // half the dims of a V block: 16 KB
@@ -795,9 +795,9 @@ size_t wide_part_bytes(int tokens, int splits) {
 // 5248 93.9 -> 90.5, 7424 141.7 -> 131.6, 8192 157.2 -> 150.4, 21248 850.3 -> 730.1; of 49 lengths up to 35072 that the new
 // constants moved, none slower). 6208 tokens stay at four, 110.9 for 107.6 with five, whose shares take a quarter more. Estimates
 // leave out a call's other 25 us, so
-// ranges that save less than 3 % are not worth their shares (1019904 tokens would take six ranges and 12 GB
-// for 1.5 %), and neither are shares of more than kMaxShareBytes, which the queue keeps (33024 tokens: six
-// ranges, 389 MB, a quarter of the time by the estimate; 18432: three, 108 MB, 11 %).
+// ranges that save less than 3 % are not worth their shares (1019904 tokens would take five ranges and 10 GB
+// for 1.6 %), and neither are shares of more than kMaxShareBytes, which the queue keeps (33024 tokens: six
+// ranges, 389 MiB, 29 % of the time by the estimate; 18432: three, 108 MiB, 13 %).
 // (A power of two that divides the blocks, which this was at first, left 6208 tokens, 194 blocks, at
 // two ranges and 98 workgroups: call 152 us against 119 with four; 18432 tokens at one range:
 // 678 against 610 with three.)

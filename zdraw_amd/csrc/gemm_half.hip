@@ -644,7 +644,7 @@ __global__ void __launch_bounds__(256, 1) gemm_pipe_kernel(const GemmArgs g) {
     constexpr int NL = TI + TJ;                 // loads of a wave per slab
     constexpr int RS = NM >= 32 ? 2 : 1;        // MFMAs per fragment read
     constexpr int TB = (NR - 1) * RS + 5 < NM - 1 ? (NR - 1) * RS + 5 : NM - 1; // the barrier follows this MFMA of the first step
-    // MFMAs per load: five where a slab has that many (the three largest tiles), so that the loads spread over all of it;
+    // MFMAs per load: five where a slab has that many (192 x 192 and 256 x 160 tiles), so that the loads spread over all of it;
     // closer, they hold the waves at the memory queue. Launches, us, at 2, 3, 4, 5 and 6: 1024 x 3072 x 9216 65.0, 61.3, 57.1,
     // 54.1-55.5, 54.4; 1632 x 3840 x 11520 140, 133, 132, 130, 130; 1632 x 3840 x 3840 60.8, 58.2, 56.4, 55.9, 56.0. Four against
     // five over twelve products of 900 to 3000 rows: 0 to 4 % (3000 x 10272 x 2568 164.4 -> 158.4), none slower.
@@ -1026,7 +1026,8 @@ static int g_gemm_build = 1; // measurement knob (gemm_set_build)
 // A slab's time is its bytes (A and W rows of 128 bytes) at 55 to 66 GB/s: a CU has at most 32 KB of
 // loads in flight, in order, and memory answers after 600 ns, 55 GB/s (350 ns from the last-level
 // cache, 190 ns from L2: 93 and 173 GB/s; part of A comes from there). So a tile's bytes per FLOP decide, and they fall with its
-// size, until there are fewer tiles than CUs.
+// size, until there are fewer tiles than CUs. (The last two were timed with a load every four MFMAs; every five
+// takes 0 to 4 % off a launch of theirs.)
 struct PipeShape { int ti, tj, st; float slab_us, fix_us; };
 constexpr PipeShape kPipe[] = {
     {2, 2, 4, 0.30f, 4.0f}, {2, 3, 4, 0.31f, 4.0f}, {4, 2, 4, 0.385f, 4.5f}, {4, 3, 4, 0.446f, 4.5f}, {4, 4, 4, 0.54f, 5.0f},
