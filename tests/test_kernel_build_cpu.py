@@ -8,6 +8,7 @@ spill of an accumulator) would read the register before the MFMA has written it.
 The check compiles the file to gfx950 assembly and fails on any such instruction.
 """
 import os
+import re
 import shutil
 
 import pytest
@@ -150,3 +151,22 @@ STORE = "global_store_dwordx4 v[2:3], v[4:7], off sc1"
 def test_the_check_of_store_data_sees_early_writes(monkeypatch, asm, early):
     monkeypatch.setattr(build, "_device_asm", lambda *_: ["kern:"] + asm)
     assert bool(build.early_store_data_writes("")) == early
+
+
+@pytest.mark.skipif(not (os.path.exists("/opt/rocm/bin/hipcc") or shutil.which("hipcc")), reason="needs hipcc")
+def test_which_products_store_their_rows_through_the_l2():
+    # gemm_half.hip, store_rows_lds: tiles of 128 x 96 on, but not 16-bit C of a ragged k, whose rows begin
+    # anywhere in a cache line
+    kernel, seen = None, {}
+    for line in build._device_asm(os.path.join(build.CSRC, "gemm_half.hip")):
+        text = line.split(";")[0].strip()
+        name = re.match(r"^_ZN\w*gemm_pipe_kernelILb[01]E([ft])Li(\d)ELi(\d)ELi\d+ELb([01])E\w*:$", text)
+        if name or (text.endswith(":") and not text.startswith(".")):
+            kernel = text if name else None
+            if name:
+                seen[kernel] = (name.groups(), set())
+        elif kernel and text.startswith("global_store_dwordx4"):
+            seen[kernel][1].add("sc1" in text.split())
+    assert len(seen) == 72
+    for (c, ti, tj, ragged), through in seen.values():
+        assert through == {int(ti) * int(tj) >= 12 and (c == "f" or ragged == "0")}, (c, ti, tj, ragged)
