@@ -170,3 +170,23 @@ def test_which_products_store_their_rows_through_the_l2():
     assert len(seen) == 72
     for (c, ti, tj, ragged), through in seen.values():
         assert through == {int(ti) * int(tj) >= 12 and (c == "f" or ragged == "0")}, (c, ti, tj, ragged)
+
+
+@pytest.mark.skipif(not (os.path.exists("/opt/rocm/bin/hipcc") or shutil.which("hipcc")), reason="needs hipcc")
+def test_which_builds_form_the_lanes_number_again_for_the_key_block_list():
+    # attn_fwd.hip, list_load: of the masked builds that norm K in the tile load (eight waves) only those of bf16 rows
+    # with a bound; the others lose 1 to 14 % by it. (All form it in their steps' mask branches.)
+    kernel, seen = None, {}
+    for line in build._device_asm(os.path.join(build.CSRC, "attn_fwd.hip")):
+        text = line.split(";")[0].strip()
+        name = re.match(r"^_ZN\w*attn_fwd_kernelI(f|DF16b)Li([12])ELb1ELb([01])ELi1ELi8ELb0ELi1E\w*:$", text)
+        if name or (text.endswith(":") and not text.startswith(".")):
+            kernel = name.groups() if name else None
+            if name:
+                seen[kernel] = 0
+        elif kernel and text.startswith("v_mbcnt_lo"):
+            seen[kernel] += 1
+    assert len(seen) == 8
+    fewest = min(seen.values())
+    for (rows, _, bounded), n in seen.items():
+        assert (n > fewest) == (rows == "DF16b" and bounded == "1"), seen
