@@ -827,8 +827,8 @@ int wide_splits(int tokens, int cus) {
 // Whether two workgroups take each tile and range, each for one half of the output dims: where both together fill
 // no more than half of the CUs. Rows that are formed again are formed once per half, which one workgroup does in turn; two at
 // once lose nothing meanwhile, and each has half of the rows to store. us per call, one -> two, every row formed again: 64
-// tokens 53.4 -> 42.0, 256 77.1 -> 57.9, 512 79.5 -> 60.0, 1152 (45 workgroups) 86.4 -> 67.4; ordinary data 256 38.2 -> 38.2, 512
-// 40.8 -> 40.3, 960 43.0 -> 42.1, 1152 47.3 -> 46.8. Past the line both read K and V too often: ordinary 1664 tokens (91) 46.1 -> 46.4,
+// tokens 53.4 -> 42.0, 256 77.1 -> 57.9, 512 79.5 -> 60.0, 1152 (45 workgroups) 86.4 -> 67.4, 8192 in one range (64) 851 -> 604;
+// ordinary data 256 38.2 -> 38.2, 512 40.8 -> 40.3, 960 43.0 -> 42.1, 1152 47.3 -> 46.8, 8192 in one range 353.6 -> 353.1. Past the line both read K and V too often: ordinary 1664 tokens (91) 46.1 -> 46.4,
 // 2048 (128) 48.3 -> 49.3, 2560 (160) 53 -> 73.
 int wide_halves(int tokens, int splits, int cus) {
     const int64_t wgs = (int64_t)wide_tiles(tokens) * (splits > 1 ? splits : 1);
